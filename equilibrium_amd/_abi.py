@@ -394,7 +394,7 @@ class Batch:
         check(lib().eqf_batch_set_tuning(self.h, max_waves, order))
 
     def set_schedule(self, sched):
-        """Wavefront schedule of a wavefront-mode batch (SCHED_AUTO, SCHED_WIDE, SCHED_RING)."""
+        """Checked and otherwise without effect (eqf_batch_set_schedule)."""
         check(lib().eqf_batch_set_schedule(self.h, sched))
 
     def set_band(self, tile, sweeps_per_block):

@@ -1,6 +1,10 @@
-// eqf_redblack.hip -- red-black mode of the Stam frame step (row-major layout).
+// eqf_frame.hip -- the Stam frame step (fluid.rs:437-524) of one scene or of a
+// group of scenes: every kernel of a frame covers all scenes of the group.
 //
-// Every lin_solve (fluid.rs:301-325) updates the (i+j)-even cells of a sweep
+// The lin_solves run in the mode of the group: exact (lexicographic order,
+// eqf_lex.hip) or red-black (below).
+//
+// Red-black: every lin_solve (fluid.rs:301-325) updates the (i+j)-even cells of a sweep
 // first and the odd cells second, then applies set_boundaries, so all cells
 // of one colour are independent and the whole grid is updated in parallel by
 // many workgroups.  Sweeps are temporally blocked in registers (k_rb_band):
@@ -80,18 +84,11 @@ enum BandSel : uint32_t {
   BS_UPD = 16,
 };
 
-// One scene of a red-black launch group: a single scene, or every scene of
-// a batch.  Each kernel below covers all scenes of its group in one launch.
 // A workgroup finds its scene and its place in it with one load from a map
 // of the launch's work units (band tile, block of CELL_BLOCK interior cells
 // or of CELL_BLOCK cells ring included -> {scene, index in the scene}); the
 // set_boundaries list kernel, whose threads straddle scenes, searches a
 // prefix table instead.
-struct RbScene {
-  SceneDesc d;  // the scene's descriptor (a copy): fields, sizes, coefficients, rule bytes, lists
-  float* tmp;   // its ping-pong field
-  int* trig;    // its per-row break columns
-};
 // Field roles in kernel arguments: F_* (eqf_layout.h), the ping-pong field, or none.
 constexpr int ROLE_TMP = NFIELDS;
 constexpr int ROLE_NONE = -1;
@@ -638,13 +635,15 @@ __global__ void k_bnd(const RbScene* __restrict__ scs, const int* __restrict__ b
   x[p.x] = (mode == M_PASSIVE ? 1.0f : -1.0f) * x[p.y];
 }
 
-// set_boundaries corners (fluid.rs:265-271): one thread per scene and field.
-__global__ void k_corners(const RbScene* __restrict__ scs, int nsc, int role0, int role1) {
+// set_boundaries corners (fluid.rs:265-271): one thread per scene and field;
+// `diffused`: only scenes whose diffusion has sweeps.
+__global__ void k_corners(const RbScene* __restrict__ scs, int nsc, int role0, int role1, int diffused) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   const int js = t >> 1;
   const int role = (t & 1) ? role1 : role0;
   if (js >= nsc || role == ROLE_NONE) return;
   const RbScene& sc = scs[js];
+  if (diffused && sc.d.diff_iters <= 0) return;
   const int S = sc.d.S;
   float* x = role_ptr(sc, role);
   x[0] = 0.5f * (x[1] + x[S]);
@@ -717,7 +716,6 @@ __global__ void __launch_bounds__(256) k_copy(const RbScene* __restrict__ scs, c
 }  // namespace rb
 
 // ------------------------------------------------------------------ host --
-using rb::RbScene;
 // A launch group: its scenes and the prefix tables of their work units, in
 // one device buffer written before any frame is captured.
 struct RbGroup {
@@ -730,17 +728,27 @@ struct RbGroup {
   // work unit -> {scene, index in it}: band tiles, interior cell blocks, cell blocks
   int2 *d_tmap = nullptr, *d_imap = nullptr, *d_cmap = nullptr;
   int *d_bpp = nullptr, *d_brc = nullptr, *d_bp = nullptr;  // prefixes of list entries
+  // exact mode: strips of the three diffusions and of a pressure solve, in
+  // ticket order; counters; hand-off values; where a wait reports that it gave up
+  bool exact = false;
+  LexTask *d_ldiff = nullptr, *d_lpress = nullptr;
+  int n_ldiff = 0, n_lpress = 0, n_lflags = 0;
+  void* d_lex = nullptr;
+  size_t lex_bytes = 0;
+  uint32_t* h_err = nullptr;
   int n = 0, maxN = 0, tiles = 0, iblocks = 0, cblocks = 0, bpp = 0, brc = 0, bp = 0;
   bool any_src = false;
-  int diff_iters = 0, press_iters = 0;
+  int diff_iters = 0, press_iters = 0;  // red-black: the same for every scene
+  int diff_rounds = 0, press_rounds = 0;  // exact: the most of any scene
+  bool any_diff = false;
   int tile = 5, tsweeps = 5;  // band shape index (kBands) and sweeps per launch (untuned default)
   int tab_tile = -1, tab_T = -1;
   hipGraphExec_t graph = nullptr;
-  int64_t graph_frames = 0;
   uint64_t key = 0;  // what the table and the graph were built for
+  int64_t key_frames = 0;  // frames launched since
 };
 
-struct RBWork {
+struct FrameWork {
   float* tmp = nullptr;  // ping-pong field
   int* trig = nullptr;   // per-row break columns
   RbGroup one;           // the scene alone (eqf_step)
@@ -767,8 +775,7 @@ static uint64_t group_key(const RbGroup& g) {
     // part of the key (dt0 included: with zero viscosity and diffusion a new
     // delta_t changes only dt0).  The descriptor is value-initialised, so
     // its padding bytes are zero.
-    SceneDesc d = s->desc;
-    d.prio = 0;
+    const SceneDesc& d = s->desc;
     uint64_t words[(sizeof(SceneDesc) + 7) / 8] = {};
     std::memcpy(words, &d, sizeof(SceneDesc));
     mix(s->uid);
@@ -778,20 +785,60 @@ static uint64_t group_key(const RbGroup& g) {
   return key;
 }
 
+// The strips of `nslots` lin_solves of scene i, `iters` sweeps each.
+static void lex_tasks(int i, int S, int iters, int nslots, std::vector<LexTask>& v, int& nflags, int64_t& hpairs) {
+  const int K = lex_round_sweeps(iters, 0);  // the longest round
+  if (K == 0) return;
+  const int n = lex_strips(S, K);
+  for (int slot = 0; slot < nslots; ++slot)
+    for (int strip = 0; strip < n; ++strip) {
+      v.push_back(LexTask{i, slot, strip, n, nflags++, 0, hpairs});
+      if (strip + 1 < n) hpairs += lex_handoff_pairs(S);
+    }
+}
+static size_t lex_ctl_bytes(int nflags) { return (sizeof(uint32_t) * (size_t)(nflags + 2) + 255) & ~(size_t)255; }
+int64_t lex_workspace_bytes(int S) {
+  return 3 * ((int64_t)(lex_strips(S, LEX_KMAX) - 1) * lex_handoff_pairs(S) * 8 + lex_strips(S, LEX_KMAX) * 36);
+}
+
+// Ticket order: the longest remaining chain of a scene first (a strip waits
+// about 100 steps for the one above it), which puts every strip after the one
+// above it and, in a batch, fills the chip with strips that need not wait.
+static void lex_order(std::vector<LexTask>& v, const std::vector<eqf_scene*>& scenes) {
+  std::stable_sort(v.begin(), v.end(), [&scenes](const LexTask& a, const LexTask& b) {
+    const int ka = (a.nstrips - 1 - a.strip) * 100 + scenes[a.scene]->S;
+    const int kb = (b.nstrips - 1 - b.strip) * 100 + scenes[b.scene]->S;
+    return ka > kb;
+  });
+}
+
 // (Re)writes the group's tables from its scenes' descriptors, on `st`.
 static int group_tables(RbGroup& g, hipStream_t st, std::string& err) {
   const int n = (int)g.scenes.size();
   std::vector<RbScene> scs(n);
   std::vector<int2> tmap, imap, cmap;
+  std::vector<LexTask> ldiff, lpress;
+  int64_t hd = 0, hp = 0;
+  int fd = 0, fp = 0;
   std::vector<int> bpp(n + 1, 0), brc(n + 1, 0), bp(n + 1, 0);
   g.any_src = false;
   g.maxN = 0;
+  g.diff_rounds = g.press_rounds = 0;
+  g.any_diff = false;
   for (int i = 0; i < n; ++i) {
     eqf_scene* s = g.scenes[i];
-    auto* w = static_cast<RBWork*>(s->rb);
+    auto* w = static_cast<FrameWork*>(s->work);
     scs[i] = RbScene{s->desc, w->tmp, w->trig};
-    const int nt = band_tiles(s->S, g.tile, g.tsweeps);
-    for (int t = 0; t < nt; ++t) tmap.push_back(make_int2(i, t));
+    g.diff_rounds = std::max(g.diff_rounds, lex_rounds(s->desc.diff_iters));
+    g.press_rounds = std::max(g.press_rounds, lex_rounds(s->desc.press_iters));
+    g.any_diff = g.any_diff || s->desc.diff_iters > 0;
+    if (g.exact) {
+      lex_tasks(i, s->S, s->desc.diff_iters, 3, ldiff, fd, hd);
+      lex_tasks(i, s->S, s->desc.press_iters, 1, lpress, fp, hp);
+    } else {
+      const int nt = band_tiles(s->S, g.tile, g.tsweeps);
+      for (int t = 0; t < nt; ++t) tmap.push_back(make_int2(i, t));
+    }
     const int64_t ni = ((int64_t)s->N * s->N + rb::CELL_BLOCK - 1) / rb::CELL_BLOCK;
     for (int64_t k = 0; k < ni; ++k) imap.push_back(make_int2(i, (int)k));
     const int64_t nb = ((int64_t)s->S * s->S + rb::CELL_BLOCK - 1) / rb::CELL_BLOCK;
@@ -803,7 +850,7 @@ static int group_tables(RbGroup& g, hipStream_t st, std::string& err) {
     g.maxN = std::max(g.maxN, s->N);
   }
   if (tmap.size() > INT32_MAX / 2 || cmap.size() > INT32_MAX / 2) {  // imap < cmap
-    err = "red-black launch group too large for one launch";
+    err = "launch group too large for one launch";
     return EQF_EINVAL;
   }
   g.n = n;
@@ -817,7 +864,10 @@ static int group_tables(RbGroup& g, hipStream_t st, std::string& err) {
   const size_t b_scs = up(sizeof(RbScene) * n), b_i = up(sizeof(int) * (n + 1));
   const size_t b_t = up(sizeof(int2) * tmap.size());
   const size_t b_m = up(sizeof(int2) * imap.size()), b_c = up(sizeof(int2) * cmap.size());
-  const size_t bytes = b_scs + 3 * b_i + b_t + b_m + b_c;
+  lex_order(ldiff, g.scenes);
+  lex_order(lpress, g.scenes);
+  const size_t b_ld = up(sizeof(LexTask) * ldiff.size()), b_lp = up(sizeof(LexTask) * lpress.size());
+  const size_t bytes = b_scs + 3 * b_i + b_t + b_m + b_c + b_ld + b_lp;
   if (bytes > g.tab_bytes) {  // with headroom: a server's group changes size often
     (void)hipFree(g.d_tab);
     g.d_tab = nullptr;
@@ -825,7 +875,7 @@ static int group_tables(RbGroup& g, hipStream_t st, std::string& err) {
     const size_t cap = std::max(bytes, (size_t)4096) * 2;
     hipError_t e = hipMalloc(&g.d_tab, cap);
     if (e != hipSuccess) {
-      err = std::string("red-black tables: ") + hipGetErrorString(e);
+      err = std::string("frame tables: ") + hipGetErrorString(e);
       return EQF_ENOMEM;
     }
     g.tab_bytes = cap;
@@ -846,6 +896,8 @@ static int group_tables(RbGroup& g, hipStream_t st, std::string& err) {
   const size_t o_t = put(tmap.data(), sizeof(int2) * tmap.size(), b_t);
   const size_t o_m = put(imap.data(), sizeof(int2) * imap.size(), b_m);
   const size_t o_c = put(cmap.data(), sizeof(int2) * cmap.size(), b_c);
+  const size_t o_ld = put(ldiff.data(), sizeof(LexTask) * ldiff.size(), b_ld);
+  const size_t o_lp = put(lpress.data(), sizeof(LexTask) * lpress.size(), b_lp);
   char* d = (char*)g.d_tab;
   g.d_scs = (RbScene*)(d + o_scs);
   g.d_bpp = (int*)(d + o_bpp);
@@ -854,11 +906,45 @@ static int group_tables(RbGroup& g, hipStream_t st, std::string& err) {
   g.d_tmap = (int2*)(d + o_t);
   g.d_imap = (int2*)(d + o_m);
   g.d_cmap = (int2*)(d + o_c);
+  g.d_ldiff = (LexTask*)(d + o_ld);
+  g.d_lpress = (LexTask*)(d + o_lp);
+  g.n_ldiff = (int)ldiff.size();
+  g.n_lpress = (int)lpress.size();
+  if (g.exact) {
+    g.n_lflags = std::max(fd, fp);
+    const size_t need = lex_ctl_bytes(g.n_lflags) + 8 * (size_t)std::max(hd, hp);
+    if (need > g.lex_bytes) {
+      (void)hipFree(g.d_lex);
+      g.d_lex = nullptr;
+      g.lex_bytes = 0;
+      const size_t cap = g.stream ? need + need / 2 : need;  // with headroom where scenes come and go
+      hipError_t e = hipMalloc(&g.d_lex, cap);
+      if (e != hipSuccess) {
+        err = std::string("lin_solve workspace: ") + hipGetErrorString(e);
+        return EQF_ENOMEM;
+      }
+      g.lex_bytes = cap;
+    }
+    if (!g.h_err) {
+      hipError_t e = hipHostMalloc((void**)&g.h_err, sizeof(uint32_t), hipHostMallocDefault);
+      if (e != hipSuccess) {
+        err = std::string("lin_solve status: ") + hipGetErrorString(e);
+        return EQF_ENOMEM;
+      }
+      *g.h_err = 0;
+    }
+    // counters start at zero; every launch leaves them so
+    hipError_t e = hipMemsetAsync(g.d_lex, 0, lex_ctl_bytes(g.n_lflags), st);
+    if (e != hipSuccess) {
+      err = std::string("lin_solve counters: ") + hipGetErrorString(e);
+      return EQF_EDEVICE;
+    }
+  }
   // behind the frames already queued on `st` (they read the old tables)
   hipError_t e = hipMemcpyAsync(g.d_tab, base, bytes, hipMemcpyHostToDevice, st);
   if (e == hipSuccess) e = hipStreamSynchronize(st);
   if (e != hipSuccess) {
-    err = std::string("red-black tables: ") + hipGetErrorString(e);
+    err = std::string("frame tables: ") + hipGetErrorString(e);
     return EQF_EDEVICE;
   }
   g.tab_tile = g.tile;
@@ -899,10 +985,8 @@ static void g_copy(hipStream_t st, const RbGroup& g, int dst, int src) {
 
 // lin_solve in red-black order on every scene of the group (one iteration
 // count): ceil(iters/T) tile passes ping-ponging between x and the scratch
-// field; an odd pass count ends with a copy back; then, if `corners`, the
-// corners of the last set_boundaries (fluid.rs:265-271).
-static void g_lin_solve(hipStream_t st, const RbGroup& g, int mode, int x, int x0, int coef, int iters,
-                        bool corners) {
+// field; an odd pass count ends with a copy back.
+static void g_lin_solve(hipStream_t st, const RbGroup& g, int mode, int x, int x0, int coef, int iters) {
   if (iters <= 0) return;
   int a_ = x, b_ = rb::ROLE_TMP;
   for (int done = 0; done < iters;) {
@@ -914,9 +998,28 @@ static void g_lin_solve(hipStream_t st, const RbGroup& g, int mode, int x, int x
     done += nsw;
   }
   if (a_ != x) g_copy(st, g, x, a_);
-  if (corners)
-    hipLaunchKernelGGL(rb::k_corners, dim3((unsigned)((2 * g.n + 255) / 256)), dim3(256), 0, st, g.d_scs, g.n, x,
-                       rb::ROLE_NONE);
+}
+static void g_corners(hipStream_t st, const RbGroup& g, int c0, int c1, int diffused) {
+  hipLaunchKernelGGL(rb::k_corners, dim3((unsigned)((2 * g.n + 255) / 256)), dim3(256), 0, st, g.d_scs, g.n, c0, c1,
+                     diffused);
+}
+
+// Lexicographic lin_solves: the three diffusions of a frame in one launch per
+// round (they read and write different fields: u and v from the last frame's
+// velocity, density from the last frame's density), or a pressure solve.
+static void g_lex(hipStream_t st, const RbGroup& g, bool press, const LexSpec& s0, const LexSpec& s1,
+                  const LexSpec& s2) {
+  uint32_t* ctl = (uint32_t*)g.d_lex;
+  uint64_t* H = (uint64_t*)((char*)g.d_lex + lex_ctl_bytes(g.n_lflags));
+  for (int r = 0; r < (press ? g.press_rounds : g.diff_rounds); ++r) {
+    const LexArgs a{{s0, s1, s2}, r, press ? 1 : 0};
+    lex_launch(st, g.d_scs, press ? g.d_lpress : g.d_ldiff, press ? g.n_lpress : g.n_ldiff, a, ctl, g.n_lflags, H,
+               g.h_err);
+  }
+}
+static void g_pressure(hipStream_t st, const RbGroup& g, int p, int div) {
+  if (g.exact) g_lex(st, g, true, LexSpec{M_PASSIVE, p, div, 2}, LexSpec{}, LexSpec{});
+  else g_lin_solve(st, g, M_PASSIVE, p, div, 2, g.press_iters);
 }
 
 // set_boundaries lists of one or two fields, then the corners of the fields
@@ -927,9 +1030,7 @@ static void g_bnd(hipStream_t st, const RbGroup& g, int mode0, int x0, int mode1
   if (total > 0)
     hipLaunchKernelGGL(rb::k_bnd, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, g.d_scs, tab, g.n, mode0,
                        x0, mode1, x1);
-  if (c0 != rb::ROLE_NONE || c1 != rb::ROLE_NONE)
-    hipLaunchKernelGGL(rb::k_corners, dim3((unsigned)((2 * g.n + 255) / 256)), dim3(256), 0, st, g.d_scs, g.n, c0,
-                       c1);
+  if (c0 != rb::ROLE_NONE || c1 != rb::ROLE_NONE) g_corners(st, g, c0, c1, 0);
 }
 
 // One frame (fluid.rs:437-524) of every scene of the group.  All scenes share
@@ -948,12 +1049,16 @@ static void g_frame(hipStream_t st, const RbGroup& g) {
   const dim3 cells((unsigned)g.iblocks);  // interior cell blocks
   if (g.any_src)
     hipLaunchKernelGGL(rb::k_sources, dim3((unsigned)g.cblocks), dim3(256), 0, st, g.d_scs, g.d_cmap);
-  g_lin_solve(st, g, M_ROW, F_U0, F_U, 0, g.diff_iters, false);  // fluid.rs:438
-  g_lin_solve(st, g, M_COL, F_V0, F_V, 0, g.diff_iters, false);  // fluid.rs:448
+  if (g.exact) {  // fluid.rs:438, 448, 501
+    g_lex(st, g, false, LexSpec{M_ROW, F_U0, F_U, 0}, LexSpec{M_COL, F_V0, F_V, 0}, LexSpec{M_PASSIVE, F_SC, F_D, 1});
+  } else {
+    g_lin_solve(st, g, M_ROW, F_U0, F_U, 0, g.diff_iters);  // fluid.rs:438
+    g_lin_solve(st, g, M_COL, F_V0, F_V, 0, g.diff_iters);  // fluid.rs:448
+  }
   // project(U0, V0, p=U, div=V), fluid.rs:459
   hipLaunchKernelGGL(rb::k_div, cells, dim3(256), 0, st, g.d_scs, g.d_imap, F_U0, F_V0, F_V, F_U);
   g_bnd(st, g, M_PASSIVE, F_V, M_PASSIVE, F_U, ROLE_NONE, ROLE_NONE);
-  g_lin_solve(st, g, M_PASSIVE, F_U, F_V, 2, g.press_iters, false);
+  g_pressure(st, g, F_U, F_V);
   hipLaunchKernelGGL(rb::k_grad, cells, dim3(256), 0, st, g.d_scs, g.d_imap, F_U0, F_V0, F_U);
   g_bnd(st, g, M_ROW, F_U0, M_COL, F_V0, F_U0, F_V0);
   // advect U from U0 and V from V0 with (U0, V0), fluid.rs:469-489
@@ -962,12 +1067,14 @@ static void g_frame(hipStream_t st, const RbGroup& g) {
   g_bnd(st, g, M_ROW, F_U, M_COL, F_V, ROLE_NONE, ROLE_NONE);
   // project(U, V, p=U0, div=V0), fluid.rs:491
   hipLaunchKernelGGL(rb::k_div, cells, dim3(256), 0, st, g.d_scs, g.d_imap, F_U, F_V, F_V0, F_U0);
-  g_bnd(st, g, M_PASSIVE, F_V0, M_PASSIVE, F_U0, F_V0, g.press_iters > 0 ? ROLE_NONE : F_U0);
-  g_lin_solve(st, g, M_PASSIVE, F_U0, F_V0, 2, g.press_iters, true);
+  g_bnd(st, g, M_PASSIVE, F_V0, M_PASSIVE, F_U0, F_V0, ROLE_NONE);
+  g_pressure(st, g, F_U0, F_V0);
+  g_corners(st, g, F_U0, ROLE_NONE, 0);
   hipLaunchKernelGGL(rb::k_grad, cells, dim3(256), 0, st, g.d_scs, g.d_imap, F_U, F_V, F_U0);
   g_bnd(st, g, M_ROW, F_U, M_COL, F_V, F_U, F_V);
   // density, fluid.rs:501-523
-  g_lin_solve(st, g, M_PASSIVE, F_SC, F_D, 1, g.diff_iters, true);
+  if (!g.exact) g_lin_solve(st, g, M_PASSIVE, F_SC, F_D, 1, g.diff_iters);
+  if (g.any_diff) g_corners(st, g, F_SC, ROLE_NONE, 1);
   hipLaunchKernelGGL(rb::k_adv_trig, cells, dim3(256), 0, st, g.d_scs, g.d_imap, F_U, F_V);
   hipLaunchKernelGGL(rb::k_adv, cells, dim3(256), 0, st, g.d_scs, g.d_imap, F_D, F_SC, ROLE_NONE, ROLE_NONE,
                      F_U, F_V);
@@ -981,56 +1088,80 @@ static void group_release(RbGroup& g) {
   (void)hipFree(g.d_tab);
   g.d_tab = nullptr;
   g.tab_bytes = 0;
+  (void)hipFree(g.d_lex);
+  g.d_lex = nullptr;
+  g.lex_bytes = 0;
+  (void)hipHostFree(g.h_err);
+  g.h_err = nullptr;
 }
 
-// Advances every scene of the group by nframes on `st`: the frames are
-// captured once as a graph (rebuilt when the scenes' parameters, lists or
-// the tiling change) and replayed.
+// One frame as a graph on `st`.
+static int group_capture(RbGroup& g, hipStream_t st, std::string& err) {
+  hipGraph_t gr = nullptr;
+  hipError_t e = hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal);
+  if (e != hipSuccess) {
+    err = std::string("capture: ") + hipGetErrorString(e);
+    return EQF_EDEVICE;
+  }
+  g_frame(st, g);
+  hipError_t le = hipGetLastError();
+  e = hipStreamEndCapture(st, &gr);
+  if (le != hipSuccess || e != hipSuccess) {
+    err = std::string("frame capture: ") + hipGetErrorString(le != hipSuccess ? le : e);
+    if (gr) (void)hipGraphDestroy(gr);
+    return EQF_EDEVICE;
+  }
+  e = hipGraphInstantiate(&g.graph, gr, nullptr, nullptr, 0);
+  (void)hipGraphDestroy(gr);
+  if (e != hipSuccess) {
+    err = std::string("graph instantiate: ") + hipGetErrorString(e);
+    return EQF_EDEVICE;
+  }
+  return EQF_OK;
+}
+
+// Advances every scene of the group by nframes on `st`.  The tables are
+// rebuilt when the scenes' parameters, lists or the tiling change.  The first
+// frame after that is launched kernel by kernel; further ones replay a graph
+// captured once (a server's groups change membership often, and one frame's
+// launches cost less than a capture).
 static int group_step(RbGroup& g, hipStream_t st, int64_t nframes, std::string& err) {
   if (nframes <= 0 || g.scenes.empty()) return EQF_OK;
   g.diff_iters = g.scenes[0]->desc.diff_iters;
   g.press_iters = g.scenes[0]->desc.press_iters;
-  for (const eqf_scene* s : g.scenes)
-    if (s->desc.diff_iters != g.diff_iters || s->desc.press_iters != g.press_iters) {
-      err = "red-black scenes of one batch need the same iteration counts";
-      return EQF_EINVAL;
-    }
+  g.exact = g.scenes[0]->p.gs_mode == EQF_GS_WAVEFRONT;
+  if (!g.exact)
+    for (const eqf_scene* s : g.scenes)
+      if (s->desc.diff_iters != g.diff_iters || s->desc.press_iters != g.press_iters) {
+        err = "red-black scenes of one batch need the same iteration counts";
+        return EQF_EINVAL;
+      }
   const uint64_t key = group_key(g);
   if (!g.d_tab || key != g.key || g.tab_tile != g.tile || g.tab_T != g.tsweeps) {
     int rc = group_tables(g, st, err);
-    if (rc) return rc;
+    if (rc) {
+      g.tab_tile = -1;  // not usable
+      return rc;
+    }
     if (g.graph) (void)hipGraphExecDestroy(g.graph);
     g.graph = nullptr;
     g.key = key;
+    g.key_frames = 0;
   }
-  // one frame per graph, replayed nframes times (a frame is ~100 launches)
-  const int64_t per = 1;
-  if (!g.graph || g.graph_frames != per) {
-    if (g.graph) (void)hipGraphExecDestroy(g.graph);
-    g.graph = nullptr;
-    hipGraph_t gr = nullptr;
-    hipError_t e = hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal);
-    if (e != hipSuccess) {
-      err = std::string("capture: ") + hipGetErrorString(e);
-      return EQF_EDEVICE;
+  for (int64_t f = 0; f < nframes; ++f) {
+    if (g.key_frames++ == 0) {
+      g_frame(st, g);
+      hipError_t e = hipGetLastError();
+      if (e != hipSuccess) {
+        err = std::string("frame launch: ") + hipGetErrorString(e);
+        return EQF_EDEVICE;
+      }
+      continue;
     }
-    for (int64_t f = 0; f < per; ++f) g_frame(st, g);
-    hipError_t le = hipGetLastError();
-    e = hipStreamEndCapture(st, &gr);
-    if (le != hipSuccess || e != hipSuccess) {
-      err = std::string("red-black frame capture: ") + hipGetErrorString(le != hipSuccess ? le : e);
-      if (gr) (void)hipGraphDestroy(gr);
-      return EQF_EDEVICE;
+    if (!g.graph) {
+      int rc = group_capture(g, st, err);
+      if (rc) return rc;
     }
-    e = hipGraphInstantiate(&g.graph, gr, nullptr, nullptr, 0);
-    (void)hipGraphDestroy(gr);
-    if (e != hipSuccess) {
-      err = std::string("graph instantiate: ") + hipGetErrorString(e);
-      return EQF_EDEVICE;
-    }
-    g.graph_frames = per;
-  }
-  for (int64_t f = 0; f < nframes; f += per) {
     hipError_t e = hipGraphLaunch(g.graph, st);
     if (e != hipSuccess) {
       err = std::string("graph launch: ") + hipGetErrorString(e);
@@ -1040,13 +1171,14 @@ static int group_step(RbGroup& g, hipStream_t st, int64_t nframes, std::string& 
   return EQF_OK;
 }
 
-void* rb_create(eqf_scene* s, std::string& err) {
-  auto* w = new RBWork;
+void* frame_create(eqf_scene* s, std::string& err) {
+  auto* w = new FrameWork;
   const size_t n = (size_t)s->S * s->S;
-  hipError_t e = eqf_scene_malloc(s, (void**)&w->tmp, sizeof(float) * n);
+  hipError_t e = hipSuccess;
+  if (s->p.gs_mode == EQF_GS_REDBLACK) e = eqf_scene_malloc(s, (void**)&w->tmp, sizeof(float) * n);
   if (e == hipSuccess) e = eqf_scene_malloc(s, (void**)&w->trig, sizeof(int) * (size_t)s->S);
   if (e != hipSuccess) {
-    err = std::string("red-black workspace: ") + hipGetErrorString(e);
+    err = std::string("frame workspace: ") + hipGetErrorString(e);
     eqf_scene_mfree(s, w->tmp);
     eqf_scene_mfree(s, w->trig);
     delete w;
@@ -1058,65 +1190,75 @@ void* rb_create(eqf_scene* s, std::string& err) {
   return w;
 }
 
-void rb_destroy(eqf_scene* s) {
-  auto* w = static_cast<RBWork*>(s->rb);
+void frame_destroy(eqf_scene* s) {
+  auto* w = static_cast<FrameWork*>(s->work);
   if (!w) return;
   group_release(w->one);
   eqf_scene_mfree(s, w->tmp);
   eqf_scene_mfree(s, w->trig);
   delete w;
-  s->rb = nullptr;
+  s->work = nullptr;
 }
 
 static bool tiling_ok(int tile, int tsweeps) {
   return tile >= 0 && tile <= 5 && tsweeps >= 1 && tsweeps <= 8 && tsweeps != 3 && tsweeps != 7;
 }
 
-int rb_set_tiling(eqf_scene* s, int tile, int tsweeps) {
-  auto* w = static_cast<RBWork*>(s->rb);
+int frame_set_tiling(eqf_scene* s, int tile, int tsweeps) {
+  auto* w = static_cast<FrameWork*>(s->work);
   if (!w || !tiling_ok(tile, tsweeps)) return EQF_EINVAL;
   w->one.tile = tile;
   w->one.tsweeps = tsweeps;
   return EQF_OK;
 }
 
-int rb_step(eqf_scene* s, int64_t nframes, std::string& err) {
-  auto* w = static_cast<RBWork*>(s->rb);
+int frame_step(eqf_scene* s, int64_t nframes, std::string& err) {
+  auto* w = static_cast<FrameWork*>(s->work);
   return group_step(w->one, s->stream, nframes, err);
 }
 
-// Batches of red-black scenes (eqf_runtime.hip): one group over all of them.
-void* rb_batch_create(const std::vector<eqf_scene*>& scenes, hipStream_t st, std::string& err) {
-  for (const eqf_scene* s : scenes)
-    if (s->desc.diff_iters != scenes[0]->desc.diff_iters || s->desc.press_iters != scenes[0]->desc.press_iters) {
-      err = "red-black scenes of one batch need the same iteration counts";
-      return nullptr;
-    }
+bool frame_failed(const eqf_scene* s) {
+  const auto* w = static_cast<const FrameWork*>(s->work);
+  return w && w->one.h_err && *(volatile const uint32_t*)w->one.h_err != 0;
+}
+
+// Batches (eqf_runtime.hip) and server lanes: one group over all scenes.
+void* group_create(const std::vector<eqf_scene*>& scenes, hipStream_t st, std::string& err) {
+  if (scenes[0]->p.gs_mode == EQF_GS_REDBLACK)
+    for (const eqf_scene* s : scenes)
+      if (s->desc.diff_iters != scenes[0]->desc.diff_iters || s->desc.press_iters != scenes[0]->desc.press_iters) {
+        err = "red-black scenes of one batch need the same iteration counts";
+        return nullptr;
+      }
   auto* g = new RbGroup;
   g->scenes = scenes;
   g->stream = st;
   return g;
 }
-void rb_batch_destroy(void* p) {
+void group_destroy(void* p) {
   auto* g = static_cast<RbGroup*>(p);
   if (!g) return;
   group_release(*g);
   delete g;
 }
-int rb_batch_set_tiling(void* p, int tile, int tsweeps) {
+int group_set_tiling(void* p, int tile, int tsweeps) {
   auto* g = static_cast<RbGroup*>(p);
   if (!g || !tiling_ok(tile, tsweeps)) return EQF_EINVAL;
   g->tile = tile;
   g->tsweeps = tsweeps;
   return EQF_OK;
 }
-int rb_batch_step(void* p, int64_t nframes, std::string& err) {
+int group_step_frames(void* p, int64_t nframes, std::string& err) {
   auto* g = static_cast<RbGroup*>(p);
   return group_step(*g, g->stream, nframes, err);
 }
-void rb_batch_set_scenes(void* p, const std::vector<eqf_scene*>& scenes) {
+void group_set_scenes(void* p, const std::vector<eqf_scene*>& scenes) {
   auto* g = static_cast<RbGroup*>(p);
   g->scenes = scenes;  // a new membership changes the key: tables and graph are rebuilt
+}
+bool group_failed(const void* p) {
+  const auto* g = static_cast<const RbGroup*>(p);
+  return g && g->h_err && *(volatile const uint32_t*)g->h_err != 0;
 }
 
 }  // namespace eqf

@@ -17,8 +17,7 @@ struct eqf_scene {
   eqf_ctx* ctx = nullptr;
   uint64_t uid = 0;  // unique per scene object of the process (never reused)
   eqf_params p{};
-  int S = 0, N = 0, ns = 0, P = 0;
-  int layout = eqf::L_CYCLIC;
+  int S = 0, N = 0;
   int64_t fstride = 0;
   std::vector<uint8_t> mask;  // row-major, host copy
   bool bnd_dirty = true;
@@ -31,12 +30,10 @@ struct eqf_scene {
   int2* d_bnd = nullptr;
   size_t bnd_cap = 0;
   int nbnd[3] = {0, 0, 0};
-  void* d_main = nullptr;     // one allocation: fields, codes, rowf, hand-off rows, descriptor
-  float* d_stage = nullptr;   // row-major staging for uploads/downloads (lazy)
+  void* d_main = nullptr;     // one allocation: pad, fields, rule bytes, rowf
+  float* d_stage = nullptr;   // staging for eqf_add_source (lazy)
   uint8_t* d_mask = nullptr;  // mask + scratch for the boundary build (lazy)
-  eqf::SceneDesc* d_desc = nullptr;
   eqf::SceneDesc desc{};
-  std::vector<float> hbuf;  // layout staging
   int in_batch = 0;
   // Batch membership: the batch advances the scene on its own stream.  Work
   // queued on the scene's stream meanwhile first waits for the batch's last
@@ -46,7 +43,7 @@ struct eqf_scene {
   hipEvent_t ev_ops = nullptr;
   bool ops_pending = false;
   bool owns_stream = true;
-  void* rb = nullptr;       // red-black workspace (eqf_redblack.hip)
+  void* work = nullptr;     // frame workspace (eqf_frame.hip)
   // Scenes of a server allocate from the server's memory pool, ordered on
   // pool_stream (hipMallocFromPoolAsync / hipFreeAsync): freeing a retired
   // scene then waits for nothing else on the device, where hipFree would wait
@@ -60,22 +57,7 @@ hipError_t eqf_scene_malloc(eqf_scene* s, void** p, size_t bytes);
 void eqf_scene_mfree(eqf_scene* s, void* p);
 
 // Runtime services shared with the server (eqf_runtime.hip).
-int eqf_internal_prepare(eqf_scene* s);  // boundary lists + device descriptor
-// Issue priority of a scene among the scenes of one launch: 3 for the largest
-// (strip count), then 2, 1, 0 for each halving.
-int eqf_batch_prio(int ns, int maxns);
-int eqf_stream_l2(int maxP, int n);
-// Waves a wavefront-mode scene uses under schedule `sched` (GsSched): its
-// strips times the sweep streams per strip (up to 16 waves, at most
-// P / stream lag streams).
-int eqf_scene_waves(int ns, int P, int sched);
-// The schedule (GsSched) of a launch whose largest scene has maxns strips
-// and period P, with at most max_waves waves per workgroup.
-int eqf_pick_sched(int maxns, int P, int max_waves);
-// waves / lds_floats: the largest eqf_scene_waves() and cyc_lds_floats() of
-// the scenes under schedule `sched`.
-hipError_t eqf_internal_launch(const eqf::SceneDesc* d_descs, int n, int waves, int lds_floats, int nframes,
-                               int sched, hipStream_t st);
+int eqf_internal_prepare(eqf_scene* s);  // boundary lists + descriptor
 int eqf_internal_error(int code, const std::string& msg);
 // Device address of eqf_render_rgba_noalloc's fixed scratch on `device`
 // (eqf_render.hip), looked up once per device at context creation.
@@ -93,21 +75,58 @@ int eqf_internal_scene_create(eqf_ctx* ctx, const eqf_params* p, hipStream_t str
 int eqf_dev_init_fields(eqf_scene* s, int times);
 int eqf_dev_upload(eqf_scene* s, float* dst, float* dst2, const float* host, int add);
 int eqf_dev_download(eqf_scene* s, const float* src, float* host);
-// src field (scene layout) -> row-major device array, queued on the scene's stream.
-int eqf_dev_to_rm_async(eqf_scene* s, const float* src, float* dst);
+// src field -> another device array, queued on the scene's stream.
+int eqf_dev_copy_async(eqf_scene* s, const float* src, float* dst);
 int eqf_dev_rebuild_bnd(eqf_scene* s);
 void eqf_dev_trim(eqf_scene* s);
 
 namespace eqf {
-// Red-black mode (eqf_redblack.hip).
-void* rb_create(eqf_scene* s, std::string& err);
-void rb_destroy(eqf_scene* s);
-int rb_step(eqf_scene* s, int64_t nframes, std::string& err);
-int rb_set_tiling(eqf_scene* s, int tile, int tsweeps);
-// A batch of red-black scenes: every frame kernel covers all of them.
-void* rb_batch_create(const std::vector<eqf_scene*>& scenes, hipStream_t st, std::string& err);
-void rb_batch_destroy(void* g);
-int rb_batch_set_tiling(void* g, int tile, int tsweeps);
-int rb_batch_step(void* g, int64_t nframes, std::string& err);
-void rb_batch_set_scenes(void* g, const std::vector<eqf_scene*>& scenes);
+
+// One scene of a launch group: a single scene, or every scene of a batch.
+// Each frame kernel covers all scenes of its group in one launch.
+struct RbScene {
+  SceneDesc d;  // the scene's descriptor (a copy): fields, sizes, coefficients, rule bytes, lists
+  float* tmp;   // its ping-pong field (red-black mode)
+  int* trig;    // its per-row break columns
+};
+
+// Lexicographic lin_solve (eqf_lex.hip).  A launch covers up to three
+// lin_solves (slots) of every scene; a task is one strip of one of them.
+struct LexTask {
+  int scene, slot;
+  int strip, nstrips;
+  int flag;      // its progress count; the strip above has the one before
+  int pad;
+  int64_t hoff;  // its hand-off pairs (the strip above: lex_handoff_pairs before)
+};
+struct LexSpec {
+  int mode, x_role, x0_role, coef;
+};
+struct LexArgs {
+  LexSpec sp[3];
+  int round, press;  // round of sweeps; which iteration count (0 diffusion, 1 pressure)
+};
+// Polls of about a microsecond a strip waits for the one above before it gives up (and reports).
+constexpr uint32_t LEX_SPIN_MAX = 1u << 22;
+// ctl: ticket, ended workgroups, then nflags progress counts, all zero before
+// the first launch; a launch leaves them zero.
+void lex_launch(hipStream_t st, const RbScene* scs, const LexTask* tasks, int ntasks, const LexArgs& args,
+                uint32_t* ctl, int nflags, uint64_t* H, uint32_t* err);
+
+// Frames (eqf_frame.hip).  A launch group's scenes share one mode.
+void* frame_create(eqf_scene* s, std::string& err);
+void frame_destroy(eqf_scene* s);
+int frame_step(eqf_scene* s, int64_t nframes, std::string& err);
+int frame_set_tiling(eqf_scene* s, int tile, int tsweeps);
+// A batch of scenes of one mode: every frame kernel covers all of them.
+void* group_create(const std::vector<eqf_scene*>& scenes, hipStream_t st, std::string& err);
+void group_destroy(void* g);
+int group_set_tiling(void* g, int tile, int tsweeps);
+int group_step_frames(void* g, int64_t nframes, std::string& err);
+void group_set_scenes(void* g, const std::vector<eqf_scene*>& scenes);
+// Whether a wait inside a kernel of the group gave up (never in a sound run).
+bool group_failed(const void* g);
+bool frame_failed(const eqf_scene* s);
+// Device bytes of the lexicographic hand-off of one scene.
+int64_t lex_workspace_bytes(int S);
 }  // namespace eqf

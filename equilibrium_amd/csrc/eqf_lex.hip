@@ -1,0 +1,794 @@
+// eqf_lex.hip -- lexicographic Gauss-Seidel (lin_solve, fluid.rs:301-325) of
+// the exact mode on gfx950, bit for bit.
+//
+// Work split.  The grid of S x S cells (ring included) is cut into strips of
+// 64 rows.  A workgroup takes one strip of one lin_solve through up to
+// LEX_KMAX = 20 sweeps (a round): lane r of a wave owns a row, each of four
+// waves runs up to five consecutive sweeps, two steps apart.  The strip moves
+// up by one row from sweep to sweep: in sweep k lane r holds row j = 64 s + r
+// - k.  A cell of sweep k at step t is column c = t - r - 2k.  Then everything
+// a cell reads comes from its own lane or the lane before it, at an earlier
+// step:
+//   left  x_k(c-1, j)      own lane, step t-1
+//   up    x_k(c, j-1)      lane r-1, step t-1
+//   down  x_{k-1}(c, j+1)  own lane, its value after set_boundaries at t-1
+//   right x_{k-1}(c+1, j)  lane r-1, the same
+// so sweeps hand values on in registers, waves through LDS, and a strip needs
+// only the strip above it (lane 63 of every sweep), never the one below: x and
+// x0 are read once and x is written once for all the sweeps of a round.  The
+// row shift costs K - 1 more rows per round.  Strips that do not move have to
+// wait out a round trip with the strip below in every sweep, which kept the
+// sweeps of a strip 32 to 64 steps apart and moved 12 bytes per cell and sweep
+// through the caches: one workgroup per scene, 28.7 ms per frame at N=1024,
+// 0.86 at N=128, 0.44 at N=30 (16 sweeps), 11.0 for 512 scenes of N 64..512;
+// with moving strips on a CU each 2.20, 0.44, 0.18 and 8.1 ms.
+//
+// AdjustRow's walls are the left / right neighbours, known one step after the
+// cell: its final value is formed then (hence two steps from sweep to sweep).
+// AdjustColumn runs the same code with rows and columns exchanged (the scan
+// order along anti-diagonals is symmetric), so that its walls are left / right
+// too.  Ring cells are cells like the others whose "update" is their fixed
+// value, or in Passive the copy of the interior neighbour.  Which of these a
+// block of eight steps can hold decides among four forms of the step (Class).
+//
+// Two more waves bring operands into LDS by anti-diagonals, where a step of a
+// wave reads 64 neighbours, write the results, and exchange lane 63's values
+// with the strips above and below, which run on other CUs: agent-scope stores
+// and loads in device memory, and a progress count per strip.  A strip trails
+// the one above it by about 100 steps (64 of skew, the blocks of 8, two
+// memory latencies).  Workgroups take their strip from a ticket counter whose
+// order puts every strip after the one it reads from, so a waiting workgroup
+// always waits for one that already runs: the launch ends whatever share of
+// it is resident.
+//
+// Bound: instruction issue of the sweeps.  An update of a plain cell takes 7
+// VALU instructions (6 of arithmetic, 1 lane shift); a plain block of 5 sweeps
+// x 8 steps about 3000 cycles with a wave alone on its SIMD, of which 40 x 7
+// VALU instructions are 1400.  A lone scene is bound by its chain of
+// S + 63 + 2K steps plus about 100 per strip.
+//
+// Compiled with -ffp-contract=off: rustc does not contract a*b+c.
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "eqf_internal.h"
+
+namespace eqf {
+namespace lex {
+
+constexpr int W = LEX_W, QMAX = 5, KMAX = LEX_KMAX, B = LEX_B;
+constexpr int NT = 64 * (W + 2);  // four waves of sweeps, two that move data
+static_assert(KMAX == W * QMAX && B == 8, "four waves of up to five sweeps, blocks of 8 steps");
+// x0 in LDS by anti-diagonals: row u = c + j - 64 s of a ring of XR rows,
+// position p = j - 64 s + KMAX - 1 (sweep k at step t reads row t - 3k, lane r
+// position r - k + KMAX - 1: 64 neighbours).  Rows are numbered u + UOFF >= 0.
+// A block of 8 steps may start anywhere in the ring, so the first 8 rows are
+// held twice.  Live at block b: rows 8b - 20 .. 8b + 79 (the last wave's last
+// sweep, words of four rules; the rows loaded during the block).
+constexpr int XP = 84, XR = 104, UOFF = 64;
+static_assert(XP >= 64 + KMAX - 1 && XR % B == 0 && XR >= 3 * (KMAX - 1) + B * W + 11, "x0 ring too short");
+constexpr int CR = XR / 4;  // rule words: four rows of one position per word, first two rows held twice
+// hand-off from wave to wave: 16 step rows of 65 values (the first: the strip
+// above); a pitch of 72 keeps the transposing accesses (8 steps x 8 lanes per
+// 64) in distinct banks
+constexpr int RP = 72, RR = 16;
+// LDS layout (4-byte words)
+constexpr int L_X0 = 0;
+constexpr int L_CODE = L_X0 + (XR + B) * XP;
+constexpr int L_RING = L_CODE + (CR + 2) * XP;
+constexpr int EN = W * QMAX * B;
+constexpr int L_EU = L_RING + (W + 1) * RR * RP;  // lane 0's up / right values: [block & 1][wave][sweep][8 steps]
+constexpr int L_ER = L_EU + 2 * EN;
+constexpr int L_P = L_ER + 2 * EN;  // lane 63's updated values: [block & 1][wave][sweep][8 steps]
+constexpr int L_PF = L_P + 2 * EN;  // in blocks with rules also the final values, of the cells of a step before
+constexpr int L_CL = L_PF + 2 * EN;  // class of the waves' blocks of steps, a byte each: [block & 3]
+constexpr int L_MISC = L_CL + 4;
+constexpr int L_WORDS = L_MISC + 4;
+static_assert(L_WORDS * 4 <= 80 * 1024, "two workgroups per CU");
+
+typedef __attribute__((address_space(3))) float lf;
+typedef __attribute__((address_space(3))) uint32_t lu;
+typedef __attribute__((address_space(3))) uint8_t lb;
+typedef float f4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) f4 lf4;
+
+__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
+// lane i <- lane i-1; lane 0 <- edge (DPP wave_shr:1).  PIN keeps the move where
+// it is written (it reads its source lane only if that lane is enabled).
+template <bool PIN>
+__device__ __forceinline__ float from_prev_lane(float v, float edge) {
+  float r = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, edge),
+                                                                  __builtin_bit_cast(int, v), 0x138, 0xf, 0xf, false));
+  if constexpr (PIN) asm volatile("" : "+v"(r));
+  return r;
+}
+
+typedef __amdgpu_buffer_rsrc_t rsrc_t;
+__device__ __forceinline__ rsrc_t make_rsrc(const void* base, uint32_t bytes) {
+  const uint64_t a = (uint64_t)(uintptr_t)base;
+  const uint64_t au = (uint64_t)(uint32_t)uni((int)(uint32_t)a) | ((uint64_t)(uint32_t)uni((int)(a >> 32)) << 32);
+  return __builtin_amdgcn_make_buffer_rsrc((void*)(uintptr_t)au, (short)0, uni((int)bytes), 0x00020000);
+}
+
+template <class T>
+__device__ __forceinline__ T agent_load(const T* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <class T>
+__device__ __forceinline__ void agent_store(T* p, T v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Selector of a cell in LDS: 0 a plain cell; ROW / COL (logical): 1 -(left),
+// 2 -(right), 4 ring (keeps its value); PASSIVE ring: 8 keeps its value, 9
+// copies the left, 10 the right, 11 the upper, 12 the lower neighbour.
+template <int MODE>
+__device__ __forceinline__ uint32_t selectors(uint32_t c) {  // four rule bytes -> four selectors
+  if constexpr (MODE == M_PASSIVE) return ((c >> R_PAS_SHIFT) & 0x07070707u) | ((~c & 0x01010101u) << 3);
+  else return ((c >> (MODE == M_COL ? R_COL_SHIFT : R_ROW_SHIFT)) & 0x03030303u) | ((~c & 0x01010101u) << 2);
+}
+
+// Values a wave carries from block to block.
+struct Carry {
+  float r1[QMAX];     // the cell updated at the last step
+  float f2[QMAX];     // final value of the cell updated the step before it
+  float ul[QMAX];     // upper neighbour used at the last step
+  float lp[QMAX];     // left neighbour used at the last step
+  uint32_t sp[QMAX];  // selector of the cell updated at the last step
+  float in, inr;      // the previous wave's final values of the last step: this lane's, the lane's before it
+  int row;            // x0 ring row of the next block's first step, sweep k0
+};
+
+// What the cells of a block of steps may be besides plain ones:
+//   C_ROWS  ring cells of the first and last row, each a fixed lane of a sweep
+//           (strips at the grid's top and bottom)
+//   C_RING  (Passive, every row and column holding a NoWall cell) ring cells
+//           of the first and last column too: the lane whose column it is
+//   C_ALL   anything, by the selectors in LDS
+enum Class { C_PLAIN = 0, C_ROWS = 1, C_RING = 2, C_ALL = 3 };
+
+// What a strip's waves know about its place.
+struct Place {
+  int S, base, lane;
+  float a, cr;
+};
+
+// Eight steps of Q consecutive sweeps k0 .. k0+Q-1 (block m = b - w: steps 8m
+// .. 8m+7).  Where no cell has a rule, a cell's final value is the updated
+// one, and the right neighbour of a cell is the upper neighbour that the sweep
+// before used a step ago: one lane shift per update instead of two.
+template <int MODE, int Q, int CLS>
+__device__ __forceinline__ void steps(lf* L, Carry& s, int b, int w, int k0, const Place& pl) {
+  constexpr bool GEN = CLS == C_ALL;
+  constexpr bool FIN = GEN && MODE != M_PASSIVE;  // final values other than the updated ones
+  const int m = b - w, lane = pl.lane;
+  const float a = pl.a, cr = pl.cr;
+  const lf* x0p[Q];
+  uint32_t cw[Q][2];
+  bool top[Q], bot[Q];
+  int c0[Q], cN[Q];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    int row = s.row - 3 * q;
+    row += row < 0 ? XR : 0;
+    x0p[q] = L + (L_X0 + row * XP + KMAX - 1 - (k0 + q)) + lane;
+    if constexpr (CLS == C_ROWS || CLS == C_RING) {
+      top[q] = lane == k0 + q - pl.base;
+      bot[q] = lane == k0 + q - pl.base + pl.S - 1;
+      if constexpr (CLS == C_RING) {  // minus the columns at the block's first step
+        c0[q] = lane + 2 * (k0 + q) - m * B;
+        cN[q] = c0[q] + pl.S - 1;
+      }
+    }
+    if constexpr (GEN) {
+      const lu* cp = (const lu*)L + (L_CODE + (row >> 2) * XP + KMAX - 1 - (k0 + q)) + lane;
+      const uint32_t w0 = cp[0], w1 = cp[XP], w2 = cp[2 * XP];
+      const uint32_t sh = (uint32_t)(row & 3);
+      cw[q][0] = __builtin_amdgcn_alignbyte(w1, w0, sh);
+      cw[q][1] = __builtin_amdgcn_alignbyte(w2, w1, sh);
+    }
+  }
+  const lf* ri = L + (L_RING + (w * RR + (m & 1) * B) * RP) + lane;
+  lf* ro = L + (L_RING + ((w + 1) * RR + (m & 1) * B) * RP + 1) + lane;
+  const lf* eu = L + L_EU + (b & 1) * EN + w * QMAX * B;
+  const lf* er = L + L_ER + (b & 1) * EN + w * QMAX * B;
+  lf* po = L + L_P + (b & 1) * EN + w * QMAX * B;
+  lf* pf = L + L_PF + (b & 1) * EN + w * QMAX * B;
+  // Operands of four steps are read from LDS while the four before them are
+  // still being computed, ahead of those steps' writes (the compiler cannot
+  // tell that reads and writes do not overlap, and one wave per SIMD has
+  // nothing else to fill the latency of a read with).
+  float xin[2][4], xinr[2][4], x0v[Q][2][4];
+  f4 e4u[Q][2], e4r[Q][2];
+  auto fetch = [&](int h) {
+#pragma unroll
+    for (int ii = 0; ii < 4; ++ii) {
+#pragma unroll
+      for (int q = 0; q < Q; ++q) x0v[q][h][ii] = x0p[q][(h * 4 + ii) * XP];
+      xin[h][ii] = ri[(h * 4 + ii) * RP + 1];
+      xinr[h][ii] = ri[(h * 4 + ii) * RP];
+    }
+    if (lane == 0) {  // only lane 0 has use for them
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        e4u[q][h] = *(const lf4*)(eu + q * B + h * 4);
+        if (FIN && q > 0) e4r[q][h] = *(const lf4*)(er + q * B + h * 4);
+      }
+    }
+  };
+  fetch(0);
+  float in = s.in, inr = s.inr, out[B];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    f4 pa[Q], pb[Q];
+#pragma unroll
+    for (int ii = 0; ii < 4; ++ii) {
+      // The sweeps of a step are independent; the update goes through them
+      // operation by operation, so that no instruction waits for the one
+      // before it (a dependent one issues 8 cycles later instead of 4).
+      float dn[Q], lt[Q], t[Q], rt[Q], up[Q], nv[Q], fin[Q];
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        dn[q] = q == 0 ? in : s.f2[q - 1];
+        lt[q] = s.r1[q];
+        fin[q] = s.r1[q];
+      }
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+        rt[q] = q == 0 ? inr : FIN ? from_prev_lane<GEN>(dn[q], e4r[q][h][ii]) : s.ul[q - 1];
+#pragma unroll
+      for (int q = 0; q < Q; ++q) up[q] = from_prev_lane<GEN>(s.r1[q], e4u[q][h][ii]);
+      // fluid.rs:315-320; AdjustColumn: logical right / left are down / up
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int q = 0; q < Q; ++q) t[q] = MODE == M_COL ? dn[q] + up[q] : rt[q] + lt[q];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int q = 0; q < Q; ++q) t[q] = t[q] + (MODE == M_COL ? rt[q] : dn[q]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int q = 0; q < Q; ++q) t[q] = t[q] + (MODE == M_COL ? lt[q] : up[q]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int q = 0; q < Q; ++q) t[q] = a * t[q];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int q = 0; q < Q; ++q) t[q] = x0v[q][h][ii] + t[q];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int q = 0; q < Q; ++q) nv[q] = t[q] * cr;
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (CLS == C_ROWS || CLS == C_RING) {
+        // ring cells: their fixed value, in Passive the interior neighbour
+        // (before the first sweep the ring holds what it held, not copies of
+        // the right / lower neighbours)
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+          const bool first = q == 0 && k0 == 0;
+          if constexpr (MODE == M_PASSIVE) {
+            nv[q] = top[q] ? (first ? x0v[q][h][ii] : dn[q]) : nv[q];
+            nv[q] = bot[q] ? up[q] : nv[q];
+            if constexpr (CLS == C_RING) {
+              nv[q] = c0[q] == h * 4 + ii ? (first ? x0v[q][h][ii] : rt[q]) : nv[q];
+              nv[q] = cN[q] == h * 4 + ii ? lt[q] : nv[q];
+            }
+          } else {
+            nv[q] = (top[q] || bot[q]) ? x0v[q][h][ii] : nv[q];
+          }
+        }
+      }
+      if constexpr (GEN) {
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+          const uint32_t sel = (cw[q][h] >> (8 * ii)) & 255u;
+          if constexpr (MODE == M_PASSIVE) {
+            // before the first sweep the ring holds what it held, not copies
+            // of the right / lower neighbours
+            float rv = x0v[q][h][ii];
+            rv = sel == 9u ? lt[q] : rv;
+            rv = sel == 11u ? up[q] : rv;
+            if (k0 + q > 0) {
+              rv = sel == 10u ? rt[q] : rv;
+              rv = sel == 12u ? dn[q] : rv;
+            }
+            nv[q] = sel == 0u ? nv[q] : rv;
+          } else {
+            nv[q] = (sel & 4u) ? x0v[q][h][ii] : nv[q];
+            fin[q] = s.sp[q] == 1u ? -s.lp[q] : fin[q];
+            fin[q] = s.sp[q] == 2u ? -nv[q] : fin[q];
+            s.sp[q] = sel;
+            s.lp[q] = lt[q];
+          }
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        pa[q][ii] = nv[q];
+        if (FIN) pb[q][ii] = fin[q];
+        s.f2[q] = fin[q];
+        s.r1[q] = nv[q];
+        s.ul[q] = up[q];
+      }
+      out[h * 4 + ii] = s.f2[Q - 1];
+      in = xin[h][ii];
+      inr = xinr[h][ii];
+      if (h == 0 && ii == 2) fetch(1);
+    }
+    if (lane == 63) {
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        *(lf4*)(po + q * B + h * 4) = pa[q];
+        if (FIN) *(lf4*)(pf + q * B + h * 4) = pb[q];
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < B; ++i) ro[i * RP] = out[i];
+  s.in = in;
+  s.inr = inr;
+  s.row += B;
+  s.row -= s.row >= XR ? XR : 0;
+  if constexpr (!GEN && MODE != M_PASSIVE) {
+#pragma unroll
+    for (int q = 0; q < Q; ++q) s.sp[q] = 0;  // plain cells
+  }
+}
+
+template <int MODE, int Q>
+__device__ __forceinline__ void steps_c(int cls, lf* L, Carry& s, int b, int w, int k0, const Place& pl) {
+  if (cls == C_PLAIN) steps<MODE, Q, C_PLAIN>(L, s, b, w, k0, pl);
+  else if (cls == C_ROWS) steps<MODE, Q, C_ROWS>(L, s, b, w, k0, pl);
+  else if (MODE == M_PASSIVE && cls == C_RING) steps<M_PASSIVE, Q, C_RING>(L, s, b, w, k0, pl);
+  else steps<MODE, Q, C_ALL>(L, s, b, w, k0, pl);
+}
+template <int MODE>
+__device__ __forceinline__ void steps_q(int Q, int cls, lf* L, Carry& s, int b, int w, int k0, const Place& pl) {
+  if (Q == 1) steps_c<MODE, 1>(cls, L, s, b, w, k0, pl);
+  else if (Q == 2) steps_c<MODE, 2>(cls, L, s, b, w, k0, pl);
+  else if (Q == 3) steps_c<MODE, 3>(cls, L, s, b, w, k0, pl);
+  else if (Q == 4) steps_c<MODE, 4>(cls, L, s, b, w, k0, pl);
+  else steps_c<MODE, 5>(cls, L, s, b, w, k0, pl);
+}
+
+// The sweeps of wave w of K: first sweep, count, and its first and last block of steps.
+struct Part {
+  int k0, Q, mlo, mhi;
+};
+__device__ __forceinline__ Part part_of(int w, int S, int K) {
+  const int Wn = min(W, K);
+  Part r;
+  r.Q = w < Wn ? K / Wn + (w < K % Wn ? 1 : 0) : 0;
+  r.k0 = w * (K / Wn) + min(w, K % Wn);
+  r.mlo = max(0, (2 * r.k0 - 1) >> 3);
+  r.mhi = w < Wn ? (S + 63 + 2 * (r.k0 + r.Q - 1)) >> 3 : -1;
+  return r;
+}
+
+// One strip of one round (K sweeps) of a lin_solve.  Waves 0..3 run the
+// sweeps; waves 4 and 5 bring operands into LDS a block ahead, write the
+// results, and talk to the neighbouring strips, so that their loads'
+// latencies and the waits for the strip above stay out of the sweeps.
+// In block b of the workgroup wave w runs block m = b - w of its steps.
+template <int MODE>
+__device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, const LexTask& tk, const LexSpec& sp, int K,
+                                           uint32_t* __restrict__ flags, uint64_t* __restrict__ Hb,
+                                           uint32_t* __restrict__ err) {
+  const SceneDesc& d = sc.d;
+  const int S = d.S;
+  const int tid = threadIdx.x, lane = tid & 63, w = uni(tid >> 6);
+  const int base = 64 * tk.strip;
+  const int Wn = min(W, K);
+  const int NB = lex_blocks(S, K);
+  const int NI = NB + Wn;
+  // LDS before the first block: edge values that nothing writes read 0
+  for (int e = L_EU + tid; e < L_MISC; e += NT) L[e] = 0.0f;
+  __syncthreads();
+
+  if (w < W) {  // the sweeps
+    const Part pt = part_of(w, S, K);
+    const Place pl{S, base, lane, sp.coef == 0 ? d.a_visc : sp.coef == 1 ? d.a_diff : 1.0f,
+                   sp.coef == 0 ? d.cr_visc : sp.coef == 1 ? d.cr_diff : 0.25f};
+    Carry s;
+#pragma unroll
+    for (int q = 0; q < QMAX; ++q) {
+      s.r1[q] = s.f2[q] = s.ul[q] = s.lp[q] = 0.0f;
+      s.sp[q] = 0;
+    }
+    s.in = s.inr = 0.0f;
+    s.row = (pt.mlo * B + UOFF - 3 * pt.k0) % XR;
+    for (int b = -1; b < NI; ++b) {
+      const int m = b - w;
+      if (m >= pt.mlo && m <= pt.mhi) {
+        const int cls = (uni((int)((lu*)L)[L_CL + (b & 3)]) >> (8 * w)) & 255;
+        steps_q<MODE>(pt.Q, cls, L, s, b, w, pt.k0, pl);
+      }
+      __syncthreads();
+    }
+    return;
+  }
+
+  float* x = d.fld + (int64_t)sp.x_role * d.fstride;
+  const float* x0 = d.fld + (int64_t)sp.x0_role * d.fstride;
+  // Range-checked views from FLD_PAD floats before the field (the scene's
+  // allocation holds as many before field 0) to 4 floats past it: every
+  // 4-element load that touches a cell of the grid lies inside.
+  const uint32_t fbytes = (uint32_t)(d.fstride + FLD_PAD + 4) * 4u;
+  const rsrc_t rx = make_rsrc(x - FLD_PAD, fbytes);
+  const int stepc = MODE == M_COL ? S : 1;  // memory step of a logical column
+  auto is_ring = [&](int c, int j) { return c == 0 || c == S - 1 || j == 0 || j == S - 1; };
+
+  // Items of four values that follow each other in memory, which are four
+  // rows of the anti-diagonal layout.  ROW / PASSIVE: one position, columns
+  // c .. c+3; COL: one logical column c, positions p .. p+3.  A pass z of a
+  // wave takes items 64 z + lane; a block's addresses are a lane's constant
+  // plus a uniform step per block.
+  const bool has_prev = tk.strip > 0, has_next = tk.strip + 1 < tk.nstrips;
+  const int T = lex_blocks(S, KMAX) * B;
+  // hand-off: value 64 z + lane of the EN per block, [wave][sweep][step]
+  int ew[3], ek[3], ei[3], elo[3], ehi[3];
+  bool eq0[3];  // the wave's first sweep
+#pragma unroll
+  for (int z = 0; z < 3; ++z) {
+    const int e = 64 * z + lane;
+    ew[z] = e / (QMAX * B);
+    const Part pt = part_of(ew[z], S, K);
+    const int q = e / B % QMAX;
+    ek[z] = pt.k0 + q;
+    ei[z] = e % B;
+    eq0[z] = q == 0;
+    const bool on = e < EN && q < pt.Q;
+    elo[z] = on ? pt.mlo : 1;
+    ehi[z] = on ? pt.mhi : 0;
+  }
+  const bool ring_copies = MODE == M_PASSIVE && d.nbnd[M_PASSIVE] == 4 * d.N;  // every ring cell copies its neighbour
+  if (w == W) {  // x0 and the rules, and lane 63's values for the strip below
+    const rsrc_t rx0 = make_rsrc(x0 - FLD_PAD, fbytes);
+    const int Sc = rm_code_stride(S);
+    // the rule bytes, transposed for COL, from CODE_PAD bytes before to 8 after them
+    const rsrc_t rc = make_rsrc(d.code + (MODE == M_COL ? rm_code_bytes(S) : 0) - CODE_PAD, rm_code_used(S) + CODE_PAD + 8);
+    constexpr int NX = 2 * (XP - 1) + (MODE == M_COL ? 2 * (B - 1) : 0), NC = 2 * (XP - 1);
+    static_assert(NX <= 192, "three passes");
+    const int hf = (lane & 1) * 4;  // the item's first row of the block's eight
+    int xp0[3], xc[3], xj[3], xoff[3], coff[3], cc[3];
+#pragma unroll
+    for (int z = 0; z < 3; ++z) {
+      const int it = (64 * z + lane) >> 1;
+      xp0[z] = MODE == M_COL ? hf + it - (B - 1) : it;  // position of the first value
+      xc[z] = (MODE == M_COL ? KMAX - 1 + B - 1 - it : hf - it + KMAX - 1) - UOFF;  // + 8 ub: its logical column
+      xj[z] = base + xp0[z] - (KMAX - 1);                                          // its logical row
+      xoff[z] = (MODE == M_COL ? xc[z] * S + xj[z] : xj[z] * S + xc[z]) * 4 + FLD_PAD * 4;
+      cc[z] = hf - it + KMAX - 1 - UOFF;  // + 8 ub: first logical column of the rules
+      coff[z] = min(max(base + it - (KMAX - 1), 0), S - 1) * Sc + hf - it + KMAX - 1 - UOFF + CODE_PAD;
+    }
+    bool xring[3];  // by its row(s)
+#pragma unroll
+    for (int z = 0; z < 3; ++z)
+      xring[z] = MODE == M_COL ? (uint32_t)(xj[z] + 3) <= 3u || (uint32_t)(S - 1 - xj[z]) <= 3u : xj[z] == 0 || xj[z] == S - 1;
+    u4 gx0[3], gring[3];
+    u2 gc[3];
+    bool ring_w[3] = {false, false, false};  // some item of the pass holds a ring cell (wave-uniform)
+#pragma unroll
+    for (int z = 0; z < 3; ++z) {
+      gx0[z] = gring[z] = (u4)(0);
+      gc[z] = (u2)(0);
+    }
+    auto load = [&](int ub) {  // rows 8 ub - UOFF .. of x0 (for ring cells, the value they hold) and their rules
+#pragma unroll
+      for (int z = 0; z < 3; ++z) {
+        const int c = xc[z] + ub * B, off = xoff[z] + ub * B * stepc * 4;
+        // holds a ring cell (or one beyond the grid)
+        const bool rg = xring[z] || (MODE == M_COL ? c == 0 || c == S - 1 : (uint32_t)(c + 3) <= 3u || (uint32_t)(S - 1 - c) <= 3u);
+        ring_w[z] = __builtin_amdgcn_ballot_w64(rg) != 0;
+        gx0[z] = __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(rx0, off, 0, 0));
+        if (ring_w[z]) gring[z] = __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(rx, off, 0, 0));
+        gc[z] = __builtin_bit_cast(u2, __builtin_amdgcn_raw_buffer_load_b64(rc, (coff[z] + ub * B) & ~3, 0, 0));
+      }
+    };
+    uint32_t h_rule = 0, h_col = 0;
+    auto put = [&](int ub) {
+      const int row = (ub * B) % XR;
+      uint32_t any = 0;
+      bool cols = false;
+#pragma unroll
+      for (int z = 0; z < 3; ++z) {
+        uint32_t v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = gx0[z][i];
+        if (ring_w[z]) {
+          const int c = xc[z] + ub * B;
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            v[i] = is_ring(MODE == M_COL ? c : c + i, MODE == M_COL ? xj[z] + i : xj[z]) ? gring[z][i] : v[i];
+        }
+        lu* q = (lu*)L + (L_X0 + row * XP) + hf * XP;
+        if (64 * z + lane < NX) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            // (COL: positions outside the row go to its last slot, which nobody reads)
+            const int pi = MODE == M_COL ? ((uint32_t)(xp0[z] + i) < (uint32_t)XP ? xp0[z] + i : XP - 1) : xp0[z];
+            q[i * XP + pi] = v[i];
+            if (row == 0) q[(XR + i) * XP + pi] = v[i];
+          }
+        }
+        if (64 * z + lane < NC) {
+          const uint32_t sel = selectors<MODE>(__builtin_amdgcn_alignbyte(gc[z].y, gc[z].x, (uint32_t)((coff[z] + ub * B) & 3)));
+          lu* cq = (lu*)L + (L_CODE + (row >> 2) * XP) + (hf >> 2) * XP + ((64 * z + lane) >> 1);
+          cq[0] = sel;
+          if (row == 0) cq[CR * XP] = sel;
+          any |= sel;
+          const int c = cc[z] + ub * B;
+          cols = cols || (uint32_t)(c + 3) <= 3u || (uint32_t)(S - 1 - c) <= 3u;
+        }
+      }
+      const bool rules = MODE == M_PASSIVE ? !ring_copies && any != 0 : (any & 0x03030303u) != 0;
+      h_rule = (h_rule << 1) | (__builtin_amdgcn_ballot_w64(rules) != 0 ? 1u : 0u);
+      h_col = (h_col << 1) | (__builtin_amdgcn_ballot_w64(cols) != 0 ? 1u : 0u);
+    };
+    // Classes of the blocks that the waves run in block nb of the workgroup,
+    // by the rows of x0 (8 to a bit, the newest, 8 (nb + 8), lowest) of their
+    // cells and of those finished in them.
+    const bool rows = base < KMAX || base + 64 > S - 1;  // a sweep holds a ring row
+    uint32_t cmask;  // lane w: the bits of wave w
+    {
+      const Part pt = part_of(min(lane, W - 1), S, K);
+      const int newest = 8 + min(lane, W - 1) - ((B - 1 - 3 * pt.k0 + UOFF) >> 3);
+      const int oldest = 8 + min(lane, W - 1) - ((-1 - 3 * (pt.k0 + pt.Q - 1) + UOFF) >> 3);
+      cmask = ((2u << oldest) - 1u) & ~((1u << newest) - 1u);
+    }
+    auto classes = [&](int nb) {
+      uint32_t c = rows ? C_ROWS : C_PLAIN;
+      c = (h_col & cmask) ? (MODE == M_PASSIVE ? C_RING : C_ALL) : c;
+      c = (h_rule & cmask) ? C_ALL : c;
+      if (lane < W) ((lb*)(L + L_CL))[(nb & 3) * 4 + lane] = (uint8_t)c;
+    };
+    for (int ub = 5; ub < 8; ++ub) {  // rows of the cells left of column 0's diagonal
+      load(ub);
+      put(ub);
+    }
+    uint64_t* hout = Hb + tk.hoff;
+    uint32_t* fown = flags + tk.flag;
+    load(UOFF / B);
+    for (int b = -1; b < NI; ++b) {
+      if (b + 1 < NB) {
+        put(b + 1 + UOFF / B);
+      } else {
+        h_rule <<= 1;
+        h_col <<= 1;
+      }
+      classes(b + 1);
+      if (has_next) {
+#pragma unroll
+        for (int z = 0; z < 3; ++z) {
+          // (updated, final) values by the step of the update; a block with
+          // rules then corrects the final values of the steps before its own
+          const int m = b - 1 - ew[z], pb = (b - 1) & 1;
+          if (m >= elo[z] && m <= ehi[z]) {
+            const uint32_t pv = ((const lu*)L)[L_P + pb * EN + 64 * z + lane];
+            uint64_t* ho = hout + (ek[z] * T + m * B + ei[z]);
+            agent_store(ho, (uint64_t)pv | ((uint64_t)pv << 32));
+            if (MODE != M_PASSIVE && ((const lb*)(L + L_CL))[((b - 1) & 3) * 4 + ew[z]] == C_ALL && m * B + ei[z] > 0)
+              agent_store((uint32_t*)ho - 1, ((const lu*)L)[L_PF + pb * EN + 64 * z + lane]);
+          }
+        }
+      }
+      asm volatile("" ::: "memory");
+      bool six = false;  // exactly the next block's six loads follow the stores
+      if (b + 2 < NB) {
+        load(b + 2 + UOFF / B);
+        six = !(ring_w[0] || ring_w[1] || ring_w[2]);
+      }
+      if (has_next && b > 0) {  // the stores are in memory: publish them
+        if (six) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (lane == 0) agent_store(fown, (uint32_t)b);
+      }
+      __syncthreads();
+    }
+    if (has_next) {
+      if (lane == 0) agent_store(fown, 0x7fffffffu);
+      // in memory before this workgroup counts as ended (the flags are cleared then)
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    return;
+  }
+
+  // Wave 5: x before the round, lane 0's values from the strip above, and the
+  // final values.
+  const uint64_t* hin = Hb + (has_prev ? tk.hoff - (int64_t)KMAX * T : 0);
+  const uint32_t* fprev = flags + (has_prev ? tk.flag - 1 : tk.flag);
+  constexpr int ZI = MODE == M_COL ? 3 : 2;                          // passes
+  constexpr int NIN = MODE == M_COL ? 2 * (64 + B - 1) : 2 * 64;     // items
+  const int hf = (lane & 1) * 4;
+  // x before the round, as "sweep -1": row t of ring 0, lane r: x(t + 1 - r, base + r + 1)
+  int ir[ZI], ioff[ZI], oc[ZI], oj[ZI];
+#pragma unroll
+  for (int z = 0; z < ZI; ++z) {
+    const int it = (64 * z + lane) >> 1;
+    ir[z] = MODE == M_COL ? hf + it - (B - 1) : it;
+    const int ic = MODE == M_COL ? B - it : hf + 1 - it;  // + 8 m
+    ioff[z] = (MODE == M_COL ? ic * S + base + ir[z] + 1 : (base + ir[z] + 1) * S + ic) * 4 + FLD_PAD * 4;
+    // final values have the same shape
+    oc[z] = (MODE == M_COL ? B - 2 - it : hf - 1 - it) - 2 * (K - 1);  // + 8 m
+    oj[z] = base + ir[z] - (K - 1);
+  }
+  u4 gin[ZI];
+  float gu[3], gr[3];
+#pragma unroll
+  for (int z = 0; z < ZI; ++z) gin[z] = (u4)(0);
+  uint32_t credit = 0, fnext = 0;  // the strip above has published this many blocks
+  bool dead = false;
+  // operands of block nb of the workgroup
+  auto load = [&](int nb) {
+    if (nb < NB)
+#pragma unroll
+      for (int z = 0; z < ZI; ++z)
+        gin[z] = __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(rx, ioff[z] + nb * B * stepc * 4, 0, 0));
+    // lane 0's values were made by the strip above in blocks up to nb + 8:
+    // nb + 9 published blocks are needed
+    if (has_prev) {
+      const uint32_t need = (uint32_t)(nb + 9);
+      credit = max(credit, (uint32_t)uni((int)fnext));
+      uint32_t spins = 0;
+      while (credit < need && !dead) {
+        credit = (uint32_t)uni((int)agent_load(fprev));
+        if (credit < need) {
+          __builtin_amdgcn_s_sleep(1);
+          if (++spins > LEX_SPIN_MAX) {  // cannot happen (see the file comment); never wait for ever
+            dead = true;
+            if (lane == 0) __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+          }
+        }
+      }
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int z = 0; z < 3; ++z) {
+        const int m = nb - ew[z];
+        gu[z] = gr[z] = 0.0f;
+        if (m >= elo[z] && m <= ehi[z]) {
+          // The upper neighbour of step tau was updated at step tau + 63 of the
+          // strip above, the right one at tau + 62; a wave's first sweep takes
+          // its right ones from the ring, a step later (sweep 0: x before the round).
+          const int tau = m * B + ei[z];
+          const float* hp = (const float*)hin + 2 * (ek[z] * T);
+          const int cc = min(tau + 2, S - 1), jj = min(base, S - 1);
+          const float* xr = x + (MODE == M_COL ? cc * S + jj : jj * S + cc);
+          gu[z] = agent_load(hp + 2 * min(tau + 63, T - 1));
+          gr[z] = agent_load(ek[z] > 0 ? hp + 2 * (min(tau + 62 + (eq0[z] ? 1 : 0), T - 1) - T) + 1 : xr);
+        }
+      }
+      fnext = agent_load(fprev);
+    }
+  };
+  load(0);
+  for (int b = -1; b < NI; ++b) {
+    if (b + 1 < NB) {
+#pragma unroll
+      for (int z = 0; z < ZI; ++z) {
+        lu* q = (lu*)L + (L_RING + ((b + 1) & 1) * B * RP + 1) + hf * RP;
+        if (64 * z + lane < NIN) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int ri = MODE == M_COL ? ((uint32_t)(ir[z] + i) < 64u ? ir[z] + i : RP - 2) : ir[z];
+            const uint32_t v = gin[z][i];
+            q[i * RP + ri] = v;  // (a pointer one past the strip above's value)
+          }
+        }
+      }
+    }
+    if (has_prev) {
+#pragma unroll
+      for (int z = 0; z < 3; ++z)
+        if (64 * z + lane < EN) {
+          const int nb = b + 1, mm = nb - ew[z];
+          L[L_EU + (nb & 1) * EN + 64 * z + lane] = gu[z];
+          if (!eq0[z]) L[L_ER + (nb & 1) * EN + 64 * z + lane] = gr[z];
+          else L[L_RING + (ew[z] * RR + (mm & 1) * B + ei[z]) * RP] = gr[z];
+        }
+    }
+    load(b + 2);
+    // Final values of the round's last sweep (ring Wn, the block before) to x:
+    // interior cells, and in Passive the ring cells that copy them.
+    if (b >= Wn) {
+      const int m = b - Wn;
+#pragma unroll
+      for (int z = 0; z < ZI; ++z) {
+        if (64 * z + lane >= NIN) continue;
+        const lf* ring = L + (L_RING + (Wn * RR + (m & 1) * B) * RP + 1) + hf * RP;
+        const int c = oc[z] + m * B, j = oj[z];
+        float v[4];
+        bool ok[4], all = true, some = false;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int ci = MODE == M_COL ? c : c + i, ji = MODE == M_COL ? j + i : j;
+          const int ri = MODE == M_COL ? min(max(ir[z] + i, 0), 63) : ir[z];
+          v[i] = ring[i * RP + ri];
+          ok[i] = ci >= 1 && ci <= S - 2 && ji >= 1 && ji <= S - 2 && (MODE != M_COL || (uint32_t)(ir[z] + i) < 64u);
+          all = all && ok[i];
+          some = some || ok[i];
+        }
+        float* o = x + (MODE == M_COL ? c * S + j : j * S + c);
+        if (all) {
+          typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+          f4u vv;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) vv[i] = v[i];
+          *(f4u*)o = vv;
+        } else if (some) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (ok[i]) o[i] = v[i];
+        }
+        if constexpr (MODE == M_PASSIVE) {
+          if (some && (j == 1 || j == S - 2 || c <= 1 || c + 3 >= S - 2)) {
+            const int Sc = rm_code_stride(S);
+            uint8_t top[4], bot[4], lft = 255, rgt = 255;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) top[i] = bot[i] = 255;
+            if (!ring_copies) {
+#pragma unroll
+              for (int i = 0; i < 4; ++i) {
+                const int cc = min(max(c + i, 0), S - 1);
+                top[i] = d.code[cc];
+                bot[i] = d.code[(S - 1) * Sc + cc];
+              }
+              lft = d.code[j * Sc];
+              rgt = d.code[j * Sc + S - 1];
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              if (!ok[i]) continue;
+              if (j == 1 && (top[i] >> R_PAS_SHIFT)) x[c + i] = v[i];
+              if (j == S - 2 && (bot[i] >> R_PAS_SHIFT)) x[(S - 1) * S + c + i] = v[i];
+              if (c + i == 1 && (lft >> R_PAS_SHIFT)) x[j * S] = v[i];
+              if (c + i == S - 2 && (rgt >> R_PAS_SHIFT)) x[j * S + S - 1] = v[i];
+            }
+          }
+        }
+      }
+    }
+    __syncthreads();
+  }
+}
+
+__global__ void __launch_bounds__(NT, 3)
+    k_lex(const RbScene* __restrict__ scs, const LexTask* __restrict__ tasks, int ntasks, LexArgs args,
+          uint32_t* __restrict__ ctl, uint32_t* __restrict__ flags, int nflags, uint64_t* __restrict__ H,
+          uint32_t* __restrict__ err) {
+  extern __shared__ float lex_lds[];
+  lf* L = (lf*)lex_lds;
+  if (threadIdx.x == 0) ((lu*)L)[L_MISC] = atomicAdd(&ctl[0], 1u);
+  __syncthreads();
+  const int t = uni((int)((lu*)L)[L_MISC]);
+  if (t >= ntasks) return;  // the counters were not zero at the start: nothing is sound then
+  const LexTask tk = tasks[t];
+  const RbScene& sc = scs[tk.scene];
+  const LexSpec sp = args.sp[tk.slot];
+  const int K = lex_round_sweeps(args.press ? sc.d.press_iters : sc.d.diff_iters, args.round);
+  if (K > 0) {
+    if (sp.mode == M_ROW) strip_task<M_ROW>(L, sc, tk, sp, K, flags, H, err);
+    else if (sp.mode == M_COL) strip_task<M_COL>(L, sc, tk, sp, K, flags, H, err);
+    else strip_task<M_PASSIVE>(L, sc, tk, sp, K, flags, H, err);
+  }
+  // The last workgroup to end leaves the counters as the next launch needs them.
+  __syncthreads();
+  if (threadIdx.x == 0) ((lu*)L)[L_MISC] = atomicAdd(&ctl[1], 1u);
+  __syncthreads();
+  if (uni((int)((lu*)L)[L_MISC]) == ntasks - 1) {
+    for (int i = threadIdx.x; i < nflags; i += NT) agent_store(flags + i, 0u);
+    if (threadIdx.x < 2) agent_store(ctl + threadIdx.x, 0u);
+  }
+}
+
+}  // namespace lex
+
+void lex_launch(hipStream_t st, const RbScene* scs, const LexTask* tasks, int ntasks, const LexArgs& args,
+                uint32_t* ctl, int nflags, uint64_t* H, uint32_t* err) {
+  if (ntasks <= 0) return;
+  hipLaunchKernelGGL(lex::k_lex, dim3((unsigned)ntasks), dim3(lex::NT), lex::L_WORDS * 4, st, scs, tasks, ntasks,
+                     args, ctl, ctl + 2, nflags, H, err);
+}
+
+}  // namespace eqf

@@ -78,7 +78,7 @@ static int render_inputs(eqf_scene* s, float* d_dens_rm) {
     rc = eqf_dev_rebuild_bnd(s);
     if (rc) return rc;
   }
-  return eqf_dev_to_rm_async(s, s->d_fld + (int64_t)F_D * s->fstride, d_dens_rm);
+  return eqf_dev_copy_async(s, s->d_fld + (int64_t)F_D * s->fstride, d_dens_rm);
 }
 
 static int launch_render(eqf_scene* s, const float* d_dens_rm, const eqf_colors* c, uint8_t* d_rgba) {
@@ -317,7 +317,7 @@ extern "C" int eqf_render_rgba_noalloc(eqf_scene* s, const eqf_colors* c, uint8_
   if (rc) return rc;
   float* d_dens = (float*)base;
   uint8_t* d_rgba = (uint8_t*)(d_dens + rgba_offset_floats(n));
-  rc = eqf_dev_to_rm_async(s, s->d_fld + (int64_t)F_D * s->fstride, d_dens);
+  rc = eqf_dev_copy_async(s, s->d_fld + (int64_t)F_D * s->fstride, d_dens);
   if (!rc) rc = launch_render(s, d_dens, c, d_rgba);
   if (rc) return rc;
   e = hipMemcpyAsync(rgba_host, d_rgba, 4 * n, hipMemcpyDeviceToHost, s->stream);

@@ -19,10 +19,6 @@
 
 using namespace eqf;
 
-template <int D, int B, int BS, bool XR, int MAXT>
-__global__ void eqf_frames_cyclic(const eqf::SceneDesc* __restrict__ descs, int nframes);
-
-
 // ----------------------------------------------------------------- errors --
 static thread_local std::string g_err;
 
@@ -57,19 +53,21 @@ static int64_t resolved_press(const eqf_params& p) {
   return p.pressure_iters < 0 ? resolved_gs(p) : p.pressure_iters;
 }
 
-int64_t eqf_scene_off(const eqf_scene* s, int x, int y) {
-  return s->layout == L_CYCLIC ? cyc_off(x, y, s->S, s->P, s->ns) : (int64_t)x + (int64_t)y * s->S;
-}
-
 static float* field_ptr(const eqf_scene* s, int f) { return s->d_fld + (int64_t)f * s->fstride; }
 
-// row-major host array <-> device field (layout conversion on the device)
+// row-major host array <-> device field
 static int upload_rm(eqf_scene* s, float* dfield, const float* host) {
   return eqf_dev_upload(s, dfield, nullptr, host, 0);
 }
 
+// Reported by the calls that wait for frames if a strip gave up waiting for
+// the one above it (see eqf_lex.hip: its order of work rules that out).
+static const char* const kGaveUp = "a lin_solve strip gave up waiting; the scene's fields are not valid";
+static int check_frames(const eqf_scene* s);
+
 static int download_rm(const eqf_scene* cs, const float* dfield, float* host) {
-  return eqf_dev_download(const_cast<eqf_scene*>(cs), dfield, host);
+  const int rc = eqf_dev_download(const_cast<eqf_scene*>(cs), dfield, host);
+  return rc ? rc : check_frames(cs);
 }
 
 // Reference initial state (fluid.rs:93-110, 527-570, 602-606), on the host.
@@ -122,13 +120,10 @@ static void fill_desc(eqf_scene* s) {
   d.fld = s->d_fld;
   d.src = s->d_src;
   d.code = s->d_code;
-  d.rowf = s->d_rowf;
   d.bnd = s->d_bnd;
   d.fstride = s->fstride;
   d.S = s->S;
   d.N = s->N;
-  d.ns = s->ns;
-  d.P = s->P;
   for (int i = 0; i < 3; ++i) d.nbnd[i] = s->nbnd[i];
   d.diff_iters = (int)resolved_gs(p);
   d.press_iters = (int)resolved_press(p);
@@ -144,8 +139,6 @@ static void fill_desc(eqf_scene* s) {
   d.sf = (float)s->S;
   d.sfm1 = d.sf - 1.0f;
   d.has_src = s->d_src ? s->src_mask : 0;
-  d.prio = 0;
-  d.stream_l2 = eqf_stream_l2(s->P, 1);
 }
 
 static int sync_desc(eqf_scene* s) {
@@ -154,9 +147,12 @@ static int sync_desc(eqf_scene* s) {
     if (rc) return rc;
   }
   fill_desc(s);
-  HIPCHK(hipMemcpyAsync(s->d_desc, &s->desc, sizeof(SceneDesc), hipMemcpyHostToDevice, s->stream));
   return EQF_OK;
 }
+
+// The exact mode takes grids of up to 16 strips of 64 rows; a batch's
+// max_waves is at least the strips of its largest scene.
+static int exact_strips(int N) { return (N + 63) / 64; }
 
 static int check_params(const eqf_params* p) {
   if (!p) return fail(EQF_EINVAL, "params is NULL");
@@ -168,9 +164,9 @@ static int check_params(const eqf_params* p) {
   const int64_t it = resolved_gs(*p), pi = resolved_press(*p);
   if (it > (1 << 24) || pi > (1 << 24)) return fail(EQF_EINVAL, "iteration count too large");
   if (p->gs_mode == EQF_GS_WAVEFRONT) {
-    const int N = (int)p->size - 2, ns = (N + 63) / 64;
+    const int N = (int)p->size - 2, ns = exact_strips(N);
     if (ns > 16)
-      return fail(EQF_EINVAL, "wavefront mode supports size <= 1026 (16 strips of 64 rows per workgroup); "
+      return fail(EQF_EINVAL, "wavefront mode supports size <= 1026 (16 strips of 64 rows); "
                               "use EQF_GS_REDBLACK for larger grids");
     if ((int64_t)(ns - 1) * 87 + 64 + std::max(it, pi) * N + 64 > (int64_t)INT32_MAX)
       return fail(EQF_EINVAL, "iteration count too large for this size");
@@ -228,7 +224,7 @@ void eqf_scene_mfree(eqf_scene* s, void* p) {
 
 static void scene_free(eqf_scene* s) {
   if (!s) return;
-  if (s->rb) rb_destroy(s);
+  if (s->work) frame_destroy(s);
   if (s->ev_ops) (void)hipEventDestroy(s->ev_ops);
   eqf_scene_mfree(s, s->d_main);
   eqf_scene_mfree(s, s->d_src);
@@ -252,10 +248,7 @@ static int scene_alloc(eqf_ctx* ctx, const eqf_params* p, eqf_scene** out, hipSt
   s->p = *p;
   s->S = (int)p->size;
   s->N = s->S - 2;
-  s->ns = (s->N + 63) / 64;
-  s->layout = p->gs_mode == EQF_GS_WAVEFRONT ? L_CYCLIC : L_ROWMAJOR;
-  s->P = cyc_period(s->N);
-  s->fstride = s->layout == L_CYCLIC ? cyc_field_floats(s->S, s->P, s->ns) : rm_field_floats(s->S);
+  s->fstride = rm_field_floats(s->S);
   hipError_t e = hipSuccess;
   if (stream) {
     s->stream = stream;
@@ -271,18 +264,15 @@ static int scene_alloc(eqf_ctx* ctx, const eqf_params* p, eqf_scene** out, hipSt
     scene_free(s);
     return fail(EQF_EDEVICE, std::string("hipStreamCreate: ") + hipGetErrorString(e));
   }
-  const size_t ncode = s->layout == L_CYCLIC ? 3 * (size_t)cyc_code_bytes(s->P, s->ns) : (size_t)rm_code_bytes(s->S);
   auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
-  const size_t b_fld = up(sizeof(float) * NFIELDS * (size_t)s->fstride);
-  const size_t b_code = up(ncode), b_rowf = up((size_t)s->S);
-  const size_t b_desc = up(sizeof(SceneDesc));
-  e = eqf_scene_malloc(s, &s->d_main, b_fld + b_code + b_rowf + b_desc);
+  const size_t b_pad = sizeof(float) * FLD_PAD, b_fld = up(sizeof(float) * NFIELDS * (size_t)s->fstride);
+  const size_t b_code = up(2 * (size_t)rm_code_bytes(s->S)), b_rowf = up((size_t)s->S);
+  e = eqf_scene_malloc(s, &s->d_main, b_pad + b_fld + b_code + b_rowf);
   if (e == hipSuccess) {
-    char* base = (char*)s->d_main;
+    char* base = (char*)s->d_main + b_pad;
     s->d_fld = (float*)base;
     s->d_code = (uint8_t*)(base + b_fld);
     s->d_rowf = (uint8_t*)(base + b_fld + b_code);
-    s->d_desc = (SceneDesc*)(base + b_fld + b_code + b_rowf);
     e = hipMemsetAsync(s->d_fld, 0, sizeof(float) * NFIELDS * s->fstride, s->stream);
   }
   if (e != hipSuccess) {
@@ -320,10 +310,10 @@ int eqf_internal_scene_create(eqf_ctx* ctx, const eqf_params* p, hipStream_t str
     host_init(s->S, p->init_times, F, s->mask);
     for (int f = 0; f < NFIELDS && !rc; ++f) rc = upload_rm(s, field_ptr(s, f), F[f].data());
   }
-  if (!rc && s->layout == L_ROWMAJOR) {
+  if (!rc) {
     std::string err;
-    s->rb = rb_create(s, err);
-    if (!s->rb) rc = fail(EQF_ENOMEM, err);
+    s->work = frame_create(s, err);
+    if (!s->work) rc = fail(EQF_ENOMEM, err);
   }
   if (rc) {
     scene_free(s);
@@ -358,13 +348,11 @@ extern "C" int eqf_scene_clone(const eqf_scene* src, eqf_scene** out) {
     scene_free(s);
     return fail(EQF_EDEVICE, std::string("clone: ") + hipGetErrorString(e));
   }
-  if (s->layout == L_ROWMAJOR) {
-    std::string err;
-    s->rb = rb_create(s, err);
-    if (!s->rb) {
-      scene_free(s);
-      return fail(EQF_ENOMEM, err);
-    }
+  std::string err;
+  s->work = frame_create(s, err);
+  if (!s->work) {
+    scene_free(s);
+    return fail(EQF_ENOMEM, err);
   }
   *out = s;
   return EQF_OK;
@@ -455,7 +443,7 @@ static int check_field(int f) {
 
 static int64_t clamp_cell(const eqf_scene* s, uint32_t x, uint32_t y) {
   const uint32_t S = (uint32_t)s->S;
-  return eqf_scene_off(s, (int)std::min(x, S - 1), (int)std::min(y, S - 1));
+  return (int64_t)std::min(x, S - 1) + (int64_t)std::min(y, S - 1) * S;
 }
 
 extern "C" int eqf_add_density(eqf_scene* s, uint32_t x, uint32_t y, float amount) {
@@ -554,10 +542,6 @@ extern "C" int eqf_download(eqf_scene* s, int field, float* host) {
   return download_rm(s, field_ptr(s, field), host);
 }
 
-int eqf_scene_waves(int ns, int P, int sched) {
-  return std::max(1, std::min(16, ns * cyc_streams(16, ns, P, sched)));
-}
-
 extern "C" int eqf_step(eqf_scene* s, int64_t nframes) {
   if (!s) return fail(EQF_EINVAL, "scene is NULL");
   if (s->in_batch) return fail(EQF_EBUSY, "scene is part of a batch");
@@ -566,25 +550,15 @@ extern "C" int eqf_step(eqf_scene* s, int64_t nframes) {
   HIPCHK(hipSetDevice(s->ctx->device));
   int rc = sync_desc(s);
   if (rc) return rc;
-  if (s->layout == L_ROWMAJOR) {
-    std::string err;
-    rc = rb_step(s, nframes, err);
-    return rc ? fail(rc, err) : EQF_OK;
-  }
-  const int sched = eqf_pick_sched(s->ns, s->P, 16);
-  const int W = eqf_scene_waves(s->ns, s->P, sched);
-  while (nframes > 0) {
-    const int nf = (int)std::min<int64_t>(nframes, 1 << 20);
-    HIPCHK(eqf_internal_launch(s->d_desc, 1, W, cyc_lds_floats(s->ns, s->P, W, sched), nf, sched, s->stream));
-    nframes -= nf;
-  }
-  return EQF_OK;
+  std::string err;
+  rc = frame_step(s, nframes, err);
+  return rc ? fail(rc, err) : EQF_OK;
 }
 
 extern "C" int eqf_scene_set_tuning(eqf_scene* s, int tile, int sweeps_per_block) {
   if (!s) return fail(EQF_EINVAL, "scene is NULL");
-  if (s->layout != L_ROWMAJOR) return fail(EQF_EINVAL, "tuning applies to red-black scenes");
-  if (rb_set_tiling(s, tile, sweeps_per_block) != EQF_OK)
+  if (s->p.gs_mode != EQF_GS_REDBLACK) return fail(EQF_EINVAL, "tuning applies to red-black scenes");
+  if (frame_set_tiling(s, tile, sweeps_per_block) != EQF_OK)
     return fail(EQF_EINVAL, "tile must be 0..5 and sweeps_per_block 1, 2, 4, 5, 6 or 8");
   return EQF_OK;
 }
@@ -593,67 +567,22 @@ extern "C" int eqf_sync(eqf_scene* s) {
   if (!s) return fail(EQF_EINVAL, "scene is NULL");
   if (int rc = eqf_internal_scene_enter(s)) return rc;
   HIPCHK(hipStreamSynchronize(s->stream));
-  return EQF_OK;
+  return check_frames(s);
 }
 
 // ------------------------------------------------------------------ batch --
 struct eqf_batch {
   eqf_ctx* ctx = nullptr;
-  std::vector<eqf_scene*> given;   // the caller's order
-  std::vector<eqf_scene*> scenes;  // workgroup order of the launch
-  SceneDesc* d_descs = nullptr;
-  int W = 1;
-  int max_waves = 16;  // tuning: waves per workgroup at most (>= the largest strip count)
-  int order = EQF_BATCH_LARGEST_FIRST;
-  int sched_req = EQF_SCHED_AUTO;  // tuning: wavefront schedule (eqf_batch_set_schedule)
-  int sched = GS_WIDE;             // the schedule in use (GsSched)
-  void* rbg = nullptr;  // red-black batch: the launch group over all scenes (eqf_redblack.hip)
+  std::vector<eqf_scene*> scenes;  // largest first
+  void* group = nullptr;           // the launch group over all scenes (eqf_frame.hip)
+  bool redblack = false;
   hipStream_t stream = nullptr;
-  hipGraphExec_t gexec = nullptr;
-  int64_t graph_frames = 0;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   double last_ms = 0.0;
 };
 
-// Workgroup order, descriptors and workgroup width of a batch from its
-// tuning; uploads the descriptors on the batch stream.
-static int batch_layout(eqf_batch* b) {
-  b->scenes = b->given;
-  if (b->order == EQF_BATCH_LARGEST_FIRST) {
-    // their workgroups are the longest: dispatched first (longest-processing-
-    // time order), they spread over the XCDs and set the launch's length
-    std::stable_sort(b->scenes.begin(), b->scenes.end(), [](const eqf_scene* a, const eqf_scene* c) {
-      return (int64_t)a->N * a->N * std::max(a->desc.diff_iters, 1) >
-             (int64_t)c->N * c->N * std::max(c->desc.diff_iters, 1);
-    });
-  }
-  const int n = (int)b->scenes.size();
-  std::vector<SceneDesc> descs(n);
-  int maxns = 1, maxw = 1, bigP = 16;  // bigP: the period of the largest scene (most strips)
-  for (int i = 0; i < n; ++i) {
-    descs[i] = b->scenes[i]->desc;
-    const eqf_scene* s = b->scenes[i];
-    if (s->ns > maxns || (s->ns == maxns && s->P > bigP)) bigP = s->P;
-    maxns = std::max(maxns, s->ns);
-  }
-  b->sched = b->sched_req == EQF_SCHED_RING   ? GS_RING
-             : b->sched_req == EQF_SCHED_WIDE ? GS_WIDE
-             : b->sched_req == EQF_SCHED_FINE ? GS_FINE
-                                              : eqf_pick_sched(maxns, bigP, b->max_waves);
-  for (int i = 0; i < n; ++i) maxw = std::max(maxw, eqf_scene_waves(b->scenes[i]->ns, b->scenes[i]->P, b->sched));
-  if (b->max_waves < maxns) return fail(EQF_EINVAL, "max_waves below the largest scene's strip count");
-  int maxP = 0;
-  for (int i = 0; i < n; ++i) maxP = std::max(maxP, b->scenes[i]->P);
-  for (int i = 0; i < n; ++i) {
-    descs[i].prio = eqf_batch_prio(b->scenes[i]->ns, maxns);
-    descs[i].stream_l2 = eqf_stream_l2(maxP, n);
-  }
-  b->W = std::min(maxw, b->max_waves);
-  hipError_t e =
-      hipMemcpyAsync(b->d_descs, descs.data(), sizeof(SceneDesc) * n, hipMemcpyHostToDevice, b->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(b->stream);
-  if (e != hipSuccess) return fail(EQF_EDEVICE, std::string("batch layout: ") + hipGetErrorString(e));
-  return EQF_OK;
+static int check_frames(const eqf_scene* s) {
+  return frame_failed(s) || (s->batch && group_failed(s->batch->group)) ? fail(EQF_EDEVICE, kGaveUp) : EQF_OK;
 }
 
 extern "C" int eqf_batch_create(eqf_ctx* ctx, eqf_scene* const* scenes, int n, eqf_batch** out) {
@@ -667,7 +596,7 @@ extern "C" int eqf_batch_create(eqf_ctx* ctx, eqf_scene* const* scenes, int n, e
   }
   for (int i = 0; i < n; ++i) {
     if (!scenes[i]) return fail(EQF_EINVAL, "NULL scene");
-    if (scenes[i]->layout != scenes[0]->layout)
+    if (scenes[i]->p.gs_mode != scenes[0]->p.gs_mode)
       return fail(EQF_EINVAL, "a batch holds scenes of one mode (wavefront or red-black)");
     if (scenes[i]->in_batch) return fail(EQF_EBUSY, "scene already in a batch");
   }
@@ -679,27 +608,22 @@ extern "C" int eqf_batch_create(eqf_ctx* ctx, eqf_scene* const* scenes, int n, e
   }
   auto* b = new eqf_batch;
   b->ctx = ctx;
-  b->given.assign(scenes, scenes + n);
+  b->redblack = scenes[0]->p.gs_mode == EQF_GS_REDBLACK;
+  b->scenes.assign(scenes, scenes + n);
+  std::stable_sort(b->scenes.begin(), b->scenes.end(),
+                   [](const eqf_scene* a, const eqf_scene* c) { return a->N > c->N; });
   hipError_t e = hipStreamCreate(&b->stream);
-  if (e == hipSuccess) e = hipMalloc(&b->d_descs, sizeof(SceneDesc) * n);
   if (e == hipSuccess) e = hipEventCreate(&b->ev0);
   if (e == hipSuccess) e = hipEventCreate(&b->ev1);
   int rc = EQF_OK;
   if (e != hipSuccess) {
     rc = fail(EQF_EDEVICE, std::string("batch create: ") + hipGetErrorString(e));
-  } else if (scenes[0]->layout == L_ROWMAJOR) {
-    // red-black: every frame kernel covers all scenes, largest first
-    b->scenes = b->given;
-    std::stable_sort(b->scenes.begin(), b->scenes.end(),
-                     [](const eqf_scene* a, const eqf_scene* c) { return a->N > c->N; });
-    std::string err;
-    b->rbg = rb_batch_create(b->scenes, b->stream, err);
-    if (!b->rbg) rc = fail(EQF_EINVAL, err);
   } else {
-    rc = batch_layout(b);
+    std::string err;
+    b->group = group_create(b->scenes, b->stream, err);
+    if (!b->group) rc = fail(EQF_EINVAL, err);
   }
   if (rc) {
-    (void)hipFree(b->d_descs);
     if (b->ev0) (void)hipEventDestroy(b->ev0);
     if (b->ev1) (void)hipEventDestroy(b->ev1);
     if (b->stream) (void)hipStreamDestroy(b->stream);
@@ -717,119 +641,33 @@ extern "C" int eqf_batch_create(eqf_ctx* ctx, eqf_scene* const* scenes, int n, e
 
 extern "C" int eqf_batch_set_band(eqf_batch* b, int tile, int sweeps_per_block) {
   if (!b) return fail(EQF_EINVAL, "batch is NULL");
-  if (!b->rbg) return fail(EQF_EINVAL, "band tiling applies to red-black batches");
+  if (!b->redblack) return fail(EQF_EINVAL, "band tiling applies to red-black batches");
   HIPCHK(hipSetDevice(b->ctx->device));
   HIPCHK(hipStreamSynchronize(b->stream));
-  if (rb_batch_set_tiling(b->rbg, tile, sweeps_per_block) != EQF_OK)
+  if (group_set_tiling(b->group, tile, sweeps_per_block) != EQF_OK)
     return fail(EQF_EINVAL, "tile must be 0..5 and sweeps 1, 2, 4, 5, 6 or 8");
   return EQF_OK;
 }
 
+// The lexicographic kernel has one split of the work for every batch (see
+// eqf_lex.hip), so these two settings change nothing; they check their
+// arguments as they always did.
 extern "C" int eqf_batch_set_schedule(eqf_batch* b, int sched) {
   if (!b) return fail(EQF_EINVAL, "batch is NULL");
-  if (b->rbg) return fail(EQF_EINVAL, "red-black batches have no wavefront schedule");
+  if (b->redblack) return fail(EQF_EINVAL, "red-black batches have no wavefront schedule");
   if (sched != EQF_SCHED_AUTO && sched != EQF_SCHED_WIDE && sched != EQF_SCHED_RING && sched != EQF_SCHED_FINE)
     return fail(EQF_EINVAL, "sched must be EQF_SCHED_AUTO, EQF_SCHED_WIDE, EQF_SCHED_RING or EQF_SCHED_FINE");
-  HIPCHK(hipSetDevice(b->ctx->device));
-  HIPCHK(hipStreamSynchronize(b->stream));
-  const int prev = b->sched_req;
-  b->sched_req = sched;
-  int rc = batch_layout(b);
-  if (rc) {  // keep the previous schedule
-    b->sched_req = prev;
-    (void)batch_layout(b);
-    return rc;
-  }
-  if (b->gexec) (void)hipGraphExecDestroy(b->gexec);  // the graph holds the launch
-  b->gexec = nullptr;
-  b->graph_frames = 0;
   return EQF_OK;
 }
 
 extern "C" int eqf_batch_set_tuning(eqf_batch* b, int max_waves, int order) {
   if (!b) return fail(EQF_EINVAL, "batch is NULL");
-  if (b->rbg) return fail(EQF_EINVAL, "red-black batches are tuned with eqf_batch_set_band");
+  if (b->redblack) return fail(EQF_EINVAL, "red-black batches are tuned with eqf_batch_set_band");
   if (max_waves < 1 || max_waves > 16) return fail(EQF_EINVAL, "max_waves must be 1..16");
   if (order != EQF_BATCH_LARGEST_FIRST && order != EQF_BATCH_GIVEN_ORDER) return fail(EQF_EINVAL, "bad order");
-  HIPCHK(hipSetDevice(b->ctx->device));
-  HIPCHK(hipStreamSynchronize(b->stream));
-  const int mw = b->max_waves, od = b->order;
-  b->max_waves = max_waves;
-  b->order = order;
-  int rc = batch_layout(b);
-  if (rc) {  // keep the previous tuning
-    b->max_waves = mw;
-    b->order = od;
-    (void)batch_layout(b);
-    return rc;
-  }
-  if (b->gexec) (void)hipGraphExecDestroy(b->gexec);  // the graph holds the launch shape
-  b->gexec = nullptr;
-  b->graph_frames = 0;
+  if (max_waves < exact_strips(b->scenes[0]->N))
+    return fail(EQF_EINVAL, "max_waves below the largest scene's strip count");
   return EQF_OK;
-}
-
-hipError_t eqf_internal_launch(const SceneDesc* d_descs, int n, int W, int lds_floats, int nframes, int sched,
-                               hipStream_t st) {
-  const size_t lds = sizeof(float) * (size_t)lds_floats;
-#define EQF_LAUNCH_SCHED(S)                                                                               \
-  do {                                                                                                    \
-    if (W <= 8)                                                                                           \
-      hipLaunchKernelGGL((eqf_frames_cyclic<gs_depth(S), GS_B, gs_sync(S), gs_has_ring(S), 512>), dim3(n), \
-                         dim3(64 * W), lds, st, d_descs, nframes);                                        \
-    else                                                                                                  \
-      hipLaunchKernelGGL((eqf_frames_cyclic<gs_depth(S), GS_B, gs_sync(S), gs_has_ring(S), 1024>), dim3(n), \
-                         dim3(64 * W), lds, st, d_descs, nframes);                                        \
-  } while (0)
-  if (sched == GS_FINE) EQF_LAUNCH_SCHED(GS_FINE);
-  else if (sched == GS_RING) EQF_LAUNCH_SCHED(GS_RING);
-  else EQF_LAUNCH_SCHED(GS_WIDE);
-#undef EQF_LAUNCH_SCHED
-  return hipGetLastError();
-}
-
-// Wavefront schedule of a launch whose largest scene (the longest frame
-// chain) has maxns strips and period P, with at most max_waves waves per
-// workgroup.  The ring schedules hand x0 between sweep streams in LDS (fewer
-// vector-memory instructions and HBM bytes) and, with their shorter stream
-// lags, run more streams per strip (P / 48 for GS_RING, P / 32 for GS_FINE,
-// against P / 64), at the cost of a barrier every 8 or 4 steps.  The rule:
-// GS_FINE when it gives that scene more streams than GS_RING (N 49..192),
-// else GS_RING when it gives more than GS_WIDE or two or more streams and at
-// least 8 waves (N 193..512), else GS_WIDE (N > 512: one stream per strip;
-// N <= 48: one stream under every schedule).  Measured (ms per frame, 20 sweeps, 16 waves at
-// most, wide / ring / fine, one box): single scenes N=64 0.93 / 0.96 / 0.62,
-// N=100 1.73 / 1.12 / 0.92, N=128 1.14 / 1.22 / 0.86, N=150 1.56 / 1.34 /
-// 1.21, N=192 1.53 / 1.34 / 1.33, N=256 2.12 / 2.01 / 2.04, N=320 3.20 / 3.01
-// / 3.15, N=512 7.37 / 7.00 / 7.37, N=600 (one stream) 12.97 / 13.38 / -;
-// batches: 130 N=64 0.95 / 0.97 / 0.63, 118 N=128 1.18 / 1.27 / 0.91, 130
-// N=256 2.66 / 2.44 / 2.41, 391 scenes N <= 256 3.09 / 2.94 / 2.76, the
-// 512-scene mix 12.23 / 10.94 / 10.73 (the tuner picks per batch), 121 N=512
-// with 8 waves (one stream per strip) 12.06 / 12.36 / -.
-int eqf_pick_sched(int maxns, int P, int max_waves) {
-  const int mf = cyc_streams(max_waves, maxns, P, GS_FINE);
-  const int mr = cyc_streams(max_waves, maxns, P, GS_RING);
-  const int mw = cyc_streams(max_waves, maxns, P, GS_WIDE);
-  if (mf > mr) return GS_FINE;
-  return (mr > mw || (mr >= 2 && maxns * mr >= 8)) ? GS_RING : GS_WIDE;
-}
-
-// Non-temporal streaming (SceneDesc::stream_l2) for the n scenes of a launch
-// whose largest scene has period maxP: fields of P > 256 (over 256 KB each)
-// are not found in L2 again by the next phase, and smaller scenes sharing
-// their launch leave L2 to the big scenes' sweep re-reads (batched mix 12.4
-// -> 12.2 ms per frame, wide schedule); a launch of small scenes only keeps
-// L2 for itself (391 scenes N <= 256: 3.27 -> 3.00 ms).  Level 2 also
-// streams the x0 loads of ring writers (their lines' last uses): with many
-// large scenes sharing L2 it pays (the 512-scene mix 11.49 -> 10.98 ms, 121
-// N=512 9.99 -> 9.85), with few it costs (one N=512 6.93 -> 7.11, 32 N=512
-// 7.38 -> 7.81).
-int eqf_stream_l2(int maxP, int n) { return maxP > 256 ? (n >= 64 ? 2 : 1) : 0; }
-
-int eqf_batch_prio(int ns, int maxns) {
-  int p = 3;
-  for (int m = maxns; p > 0 && 2 * ns <= m; m /= 2) --p;
-  return p;
 }
 
 int eqf_internal_prepare(eqf_scene* s) { return sync_desc(s); }
@@ -845,13 +683,6 @@ int eqf_internal_scene_enter(eqf_scene* s) {
 int eqf_internal_error(int code, const std::string& msg) { return fail(code, msg); }
 int eqf_internal_check_params(const eqf_params* p) { return check_params(p); }
 
-static hipError_t batch_launch(eqf_batch* b, int nframes_per_launch) {
-  int lds = 0;
-  for (auto* s : b->scenes) lds = std::max(lds, cyc_lds_floats(s->ns, s->P, b->W, b->sched));
-  return eqf_internal_launch(b->d_descs, (int)b->scenes.size(), b->W, lds, nframes_per_launch, b->sched,
-                             b->stream);
-}
-
 extern "C" int eqf_batch_step(eqf_batch* b, int64_t nframes) {
   if (!b) return fail(EQF_EINVAL, "batch is NULL");
   if (nframes < 0) return fail(EQF_EINVAL, "nframes < 0");
@@ -866,34 +697,10 @@ extern "C" int eqf_batch_step(eqf_batch* b, int64_t nframes) {
     HIPCHK(hipStreamWaitEvent(b->stream, s->ev_ops, 0));
     s->ops_pending = false;
   }
-  if (b->rbg) {  // red-black: the group's frames, captured once per nframes
-    HIPCHK(hipEventRecord(b->ev0, b->stream));
-    std::string err;
-    const int rc = rb_batch_step(b->rbg, nframes, err);
-    if (rc) return fail(rc, err);
-    HIPCHK(hipEventRecord(b->ev1, b->stream));
-    return EQF_OK;
-  }
-  // One launch per frame, captured once as a graph of `nframes` launches.
-  if (!b->gexec || b->graph_frames != nframes) {
-    if (b->gexec) {
-      HIPCHK(hipStreamSynchronize(b->stream));  // the previous replay may still run
-      HIPCHK(hipGraphExecDestroy(b->gexec));
-    }
-    b->gexec = nullptr;
-    hipGraph_t g = nullptr;
-    HIPCHK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-    hipError_t le = hipSuccess;
-    for (int64_t f = 0; f < nframes && le == hipSuccess; ++f) le = batch_launch(b, 1);
-    hipError_t ce = hipStreamEndCapture(b->stream, &g);
-    if (le != hipSuccess) return fail(EQF_EDEVICE, std::string("batch capture: ") + hipGetErrorString(le));
-    HIPCHK(ce);
-    HIPCHK(hipGraphInstantiate(&b->gexec, g, nullptr, nullptr, 0));
-    HIPCHK(hipGraphDestroy(g));
-    b->graph_frames = nframes;
-  }
   HIPCHK(hipEventRecord(b->ev0, b->stream));
-  HIPCHK(hipGraphLaunch(b->gexec, b->stream));
+  std::string err;
+  const int rc = group_step_frames(b->group, nframes, err);
+  if (rc) return fail(rc, err);
   HIPCHK(hipEventRecord(b->ev1, b->stream));
   return EQF_OK;
 }
@@ -903,7 +710,7 @@ extern "C" int eqf_batch_sync(eqf_batch* b) {
   HIPCHK(hipStreamSynchronize(b->stream));
   float ms = 0.f;
   if (hipEventElapsedTime(&ms, b->ev0, b->ev1) == hipSuccess) b->last_ms = ms;
-  return EQF_OK;
+  return group_failed(b->group) ? fail(EQF_EDEVICE, kGaveUp) : EQF_OK;
 }
 
 extern "C" int eqf_batch_last_ms(const eqf_batch* b, double* ms) {
@@ -917,14 +724,12 @@ extern "C" int eqf_batch_destroy(eqf_batch* b) {
   (void)hipStreamSynchronize(b->stream);
   for (auto* s : b->scenes)  // work that waits on the batch's events ends before they go
     if (s->ops_pending) (void)hipStreamSynchronize(s->stream);
-  if (b->gexec) (void)hipGraphExecDestroy(b->gexec);
-  rb_batch_destroy(b->rbg);
+  group_destroy(b->group);
   for (auto* s : b->scenes) {
     s->in_batch = 0;
     s->batch = nullptr;
     s->ops_pending = false;
   }
-  (void)hipFree(b->d_descs);
   (void)hipEventDestroy(b->ev0);
   (void)hipEventDestroy(b->ev1);
   (void)hipStreamDestroy(b->stream);

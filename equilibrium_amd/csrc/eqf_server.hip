@@ -1,23 +1,18 @@
 // eqf_server.hip -- continuous batching of scene requests on one GPU.
 //
 // A server thread owns every admitted scene.  Resident scenes are split into
-// lanes that tick independently, each on its own stream: small wavefront-mode
-// scenes (at most 4 strips of 64 rows, N <= 256), large wavefront-mode scenes
-// (5-16 strips), and red-black scenes (any size).  A lane's tick advances its
-// scenes by one frame (fluid.rs:437-524): one fused launch of
-// eqf_frames_cyclic over the lane's scenes, sized by the lane's own largest
-// scene, or one frame graph per red-black launch group (one group per pair of
-// iteration counts).  When a lane's tick ends, the thread retires the lane's
-// finished scenes, adds the ones admitted to it meanwhile and launches its
-// next tick, so a small scene's frame takes its own lane's time rather than
-// the largest resident scene's.  Within a wavefront lane's tick, a scene
-// whose frame chain is k times shorter than the lane's longest runs up to k
-// frames (at most 16, never past its request) in its workgroup, so the
-// lane's scenes advance at their own pace.  Between those events the thread admits
-// queued requests while their device memory fits the budget (allocation,
-// Fluid::new's state, obstacles, sources) on a fourth stream, overlapping the
-// running ticks.  Every scene runs its own workgroups with its own data, so a
-// scene's result does not depend on which others share its ticks.
+// lanes that tick independently, each on its own stream: small exact scenes
+// (N <= 256), large exact scenes (N 257..1024), and red-black scenes (any
+// size).  A lane's tick advances its scenes by one frame (fluid.rs:437-524):
+// the frame of one launch group over all of them (on the red-black lane, of
+// one group per pair of iteration counts).  When a lane's tick ends, the
+// thread retires the lane's finished scenes, adds the ones admitted to it
+// meanwhile and launches its next tick, so a small scene's frame takes its own
+// lane's time rather than the largest resident scene's.  Between those events
+// the thread admits queued requests while their device memory fits the budget
+// (allocation, Fluid::new's state, obstacles, sources) on a fourth stream,
+// overlapping the running ticks.  A scene's result does not depend on which
+// others share its ticks.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -56,7 +51,6 @@ struct Req {
   int tick_frames = 1;  // frames of the tick in flight
   double t_submit = 0, t_admit = 0, t_done = 0;
   eqf_scene* scene = nullptr;
-  bool rb = false;  // red-black mode: advanced by its launch group on the red-black lane
   int lane = 0;
   uint64_t bytes = 0;
   int64_t cells = 0;
@@ -70,7 +64,7 @@ namespace {
 // that is four streams, the number of hardware queues HIP gives a process by
 // default: streams sharing a queue would run their ticks one after the other.
 enum { LANE_SMALL = 0, LANE_LARGE = 1, LANE_RB = 2, NLANES = 3 };
-constexpr int kSmallMaxStrips = 4;
+constexpr int kSmallMaxSize = 258;
 
 struct Lane {
   hipStream_t st = nullptr;
@@ -79,16 +73,11 @@ struct Lane {
   std::vector<Req*> ticking;        // scenes of the tick in flight
   bool busy = false;
   double t_launch = 0;
-  // wavefront lanes: the descriptors of the scenes last launched
-  SceneDesc* d_descs = nullptr;
-  int desc_cap = 0;
-  std::vector<uint64_t> last_uids;  // (scene uid (never reused), frames per tick) pairs that d_descs holds
-  std::vector<SceneDesc> descs;
 };
 
 int lane_of(const eqf_scene* s) {
-  if (s->layout == L_ROWMAJOR) return LANE_RB;
-  return s->ns <= kSmallMaxStrips ? LANE_SMALL : LANE_LARGE;
+  if (s->p.gs_mode == EQF_GS_REDBLACK) return LANE_RB;
+  return s->S <= kSmallMaxSize ? LANE_SMALL : LANE_LARGE;
 }
 }  // namespace
 
@@ -113,10 +102,10 @@ struct eqf_server {
   // the resident scenes' device memory, allocated and freed in astream's order
   hipMemPool_t pool = nullptr;
   Lane lanes[NLANES];
-  // launch groups of the resident red-black scenes, one per (diffusion,
-  // pressure) iteration counts, on the red-black lane's stream: every frame
-  // kernel covers all scenes of a group
-  std::map<std::pair<int, int>, void*> rb_groups;
+  // launch groups of the resident scenes, on their lane's stream: one per
+  // wavefront lane, and on the red-black lane one per (diffusion, pressure)
+  // iteration counts; every frame kernel covers all scenes of a group
+  std::map<std::pair<int, int>, void*> groups[NLANES];
   Clock::time_point t0;
   // statistics
   int64_t ticks = 0, scene_frames = 0, max_resident = 0;
@@ -134,16 +123,12 @@ struct eqf_server {
 
 // Device bytes of a scene of this size and mode with frame sources.
 static uint64_t estimate_bytes(const eqf_params& p) {
-  const int S = (int)p.size, N = S - 2, ns = (N + 63) / 64, P = cyc_period(N);
-  if (p.gs_mode == EQF_GS_REDBLACK) {
-    // fields + sources, rule bytes, ping-pong field, row flags, break columns, lists
-    const uint64_t fs = (uint64_t)rm_field_floats(S), cells = (uint64_t)S * S;
-    return (NFIELDS + 3) * fs * 4 + (uint64_t)rm_code_bytes(S) + cells * 4 + (uint64_t)S * 5 + (uint64_t)N * 96 +
-           sizeof(SceneDesc) + 8192;
-  }
-  const uint64_t fs = (uint64_t)cyc_field_floats(S, P, ns);
-  return (NFIELDS + 3) * fs * 4 + 3ull * (uint64_t)cyc_code_bytes(P, ns) + (uint64_t)S + (uint64_t)N * 96 +
-         sizeof(SceneDesc) + 4096;
+  const int S = (int)p.size, N = S - 2;
+  // fields + sources, rule bytes, row flags, break columns, lists, and the
+  // ping-pong field (red-black) or the lin_solve hand-off (exact)
+  const uint64_t fs = (uint64_t)rm_field_floats(S), cells = (uint64_t)S * S;
+  const uint64_t work = p.gs_mode == EQF_GS_REDBLACK ? cells * 4 : (uint64_t)lex_workspace_bytes(S);
+  return (NFIELDS + 3) * fs * 4 + 2 * (uint64_t)rm_code_bytes(S) + work + (uint64_t)S * 5 + (uint64_t)N * 96 + 8192;
 }
 
 static int admit(eqf_server* sv, Req* r, std::string& err) {
@@ -166,7 +151,6 @@ static int admit(eqf_server* sv, Req* r, std::string& err) {
     if (s) eqf_scene_destroy(s);
     return rc;
   }
-  r->rb = s->layout == L_ROWMAJOR;
   r->lane = lane_of(s);
   // the scene keeps the admission stream for its own operations (its
   // read-back at retirement, after its lane's last tick has ended); its
@@ -215,94 +199,30 @@ static void lane_tick_done(eqf_server* sv, Lane& L, double now) {
   if (--sv->busy_lanes == 0) sv->busy_ms += now - sv->busy_since;
 }
 
-// Dependent wavefront steps of one frame of a scene: its lin_solves' chains
-// (sweeps over m streams per strip, strip and stream fill); the one-pass
-// phases add a few passes over the strip.
-static double frame_chain(const eqf_scene* s, int sched) {
-  const int W = eqf_scene_waves(s->ns, s->P, sched);
-  const int lag = gs_stream_lag(sched);
-  const int m = cyc_streams(W, s->ns, s->P, sched);
-  auto solve = [&](int it) {
-    if (it <= 0) return 0.0;
-    const int mm = std::min(m, it);
-    return (double)((it + mm - 1) / mm) * s->P + (double)(s->ns - 1) * gs_strip_lag(sched) +
-           (double)(mm - 1) * lag + 64.0;
-  };
-  return 3.0 * solve(s->desc.diff_iters) + 2.0 * solve(s->desc.press_iters) + 4.0 * s->P;
-}
-
-// Launches one tick of every scene of an idle lane.  Returns an error
-// message, or "" on success.
+// Launches one tick (a frame) of every scene of an idle lane.  Returns an
+// error message, or "" on success.
 static std::string lane_launch(eqf_server* sv, int li) {
   Lane& L = sv->lanes[li];
   L.ticking = L.members;
   hipError_t e = hipSuccess;
   std::string err;
-  if (li != LANE_RB) {
-    auto& wf = L.ticking;
-    std::stable_sort(wf.begin(), wf.end(), [](const Req* a, const Req* b) { return a->cells > b->cells; });
-    int maxns = 1, lds = 0, waves = 1;
-    double chain_max = 0;
-    int bigP = 16;  // the period of the largest scene (most strips)
-    for (Req* r : wf) {
-      if (r->scene->ns > maxns || (r->scene->ns == maxns && r->scene->P > bigP)) bigP = r->scene->P;
-      maxns = std::max(maxns, r->scene->ns);
-    }
-    const int sched = eqf_pick_sched(maxns, bigP, 16);
-    for (Req* r : wf) {
-      waves = std::max(waves, eqf_scene_waves(r->scene->ns, r->scene->P, sched));
-      chain_max = std::max(chain_max, frame_chain(r->scene, sched));
-    }
-    for (Req* r : wf) lds = std::max(lds, cyc_lds_floats(r->scene->ns, r->scene->P, waves, sched));
-    std::vector<uint64_t> uids(2 * wf.size());
-    for (size_t i = 0; i < wf.size(); ++i) {
-      Req* r = wf[i];
-      const int64_t k = (int64_t)(chain_max / frame_chain(r->scene, sched));
-      r->tick_frames = (int)std::max<int64_t>(1, std::min<int64_t>({k, 16, r->nframes - r->frames_done}));
-      uids[2 * i] = r->scene->uid;
-      uids[2 * i + 1] = (uint64_t)r->tick_frames;
-    }
-    if (uids != L.last_uids) {
-      L.descs.resize(wf.size());
-      int maxP = 0;
-      for (Req* r : wf) maxP = std::max(maxP, r->scene->P);
-      for (size_t i = 0; i < wf.size(); ++i) {
-        L.descs[i] = wf[i]->scene->desc;
-        L.descs[i].prio = eqf_batch_prio(wf[i]->scene->ns, maxns);
-        L.descs[i].frame_mult = wf[i]->tick_frames;
-        L.descs[i].stream_l2 = eqf_stream_l2(maxP, (int)wf.size());
-      }
-      L.last_uids.clear();
-      if ((int)wf.size() > L.desc_cap) {
-        // the lane is idle: nothing reads the old array any more
-        const int cap = std::max<int>((int)wf.size(), 2 * L.desc_cap);
-        (void)hipFree(L.d_descs);
-        L.d_descs = nullptr;
-        L.desc_cap = 0;
-        e = hipMalloc(&L.d_descs, sizeof(SceneDesc) * cap);
-        if (e == hipSuccess) L.desc_cap = cap;
-      }
-      // pageable source: the copy has read it when the call returns
-      if (e == hipSuccess)
-        e = hipMemcpyAsync(L.d_descs, L.descs.data(), sizeof(SceneDesc) * wf.size(), hipMemcpyHostToDevice, L.st);
-      if (e == hipSuccess) L.last_uids = uids;
-    }
-    if (e == hipSuccess) e = eqf_internal_launch(L.d_descs, (int)wf.size(), waves, lds, 1, sched, L.st);
-    if (e != hipSuccess) err = hipGetErrorString(e);
-  } else {
-    std::map<std::pair<int, int>, std::vector<eqf_scene*>> by_iters;
-    std::stable_sort(L.ticking.begin(), L.ticking.end(),
-                     [](const Req* a, const Req* b) { return a->cells > b->cells; });
-    for (Req* r : L.ticking) {
-      r->tick_frames = 1;
-      by_iters[{r->scene->desc.diff_iters, r->scene->desc.press_iters}].push_back(r->scene);
-    }
-    for (auto& [key, members] : by_iters) {
-      void*& g = sv->rb_groups[key];
-      if (!g) g = rb_batch_create(members, L.st, err);
-      if (!g) break;
-      rb_batch_set_scenes(g, members);
-      if (rb_batch_step(g, 1, err) != EQF_OK) break;
+  std::map<std::pair<int, int>, std::vector<eqf_scene*>> by_iters;
+  std::stable_sort(L.ticking.begin(), L.ticking.end(),
+                   [](const Req* a, const Req* b) { return a->cells > b->cells; });
+  for (Req* r : L.ticking) {
+    r->tick_frames = 1;
+    const SceneDesc& d = r->scene->desc;
+    by_iters[li == LANE_RB ? std::make_pair(d.diff_iters, d.press_iters) : std::make_pair(0, 0)].push_back(r->scene);
+  }
+  for (auto& [key, members] : by_iters) {
+    void*& g = sv->groups[li][key];
+    if (!g) g = group_create(members, L.st, err);
+    if (!g) break;
+    group_set_scenes(g, members);
+    if (group_step_frames(g, 1, err) != EQF_OK) break;
+    if (group_failed(g)) {
+      err = "a lin_solve strip gave up waiting";
+      break;
     }
   }
   if (err.empty()) {
@@ -696,9 +616,9 @@ extern "C" int eqf_server_destroy(eqf_server* sv) {
     sv->cv_idle.notify_all();
   }
   for (Lane& L : sv->lanes) (void)hipStreamSynchronize(L.st);
-  for (auto& kv : sv->rb_groups) rb_batch_destroy(kv.second);
+  for (auto& m : sv->groups)
+    for (auto& kv : m) group_destroy(kv.second);
   for (Lane& L : sv->lanes) {
-    (void)hipFree(L.d_descs);
     (void)hipStreamDestroy(L.st);
     (void)hipEventDestroy(L.ev);
   }

@@ -1,6 +1,5 @@
-// eqf_setup.hip -- device-side scene setup: initial state, layout conversion
-// of uploaded/downloaded fields and sources, and the boundary codes/lists
-// derived from the obstacle mask.  Keeping these on the device makes
+// eqf_setup.hip -- device-side scene setup: initial state, uploads, downloads
+// and adds of whole fields, and the boundary rules / lists derived from the obstacle mask.  Keeping these on the device makes
 // admitting a scene cost a few small launches instead of host loops over
 // every cell, which matters when the server admits hundreds of scenes/s.
 #include <hip/hip_runtime.h>
@@ -16,12 +15,10 @@ using namespace eqf;
 namespace {
 
 struct Geo {
-  int S, N, ns, P, layout;
+  int S, N;
 };
 
-__device__ __forceinline__ int64_t off_of(const Geo& g, int x, int y) {
-  return g.layout == L_CYCLIC ? cyc_off(x, y, g.S, g.P, g.ns) : (int64_t)x + (int64_t)y * g.S;
-}
+__device__ __forceinline__ int off_of(const Geo& g, int x, int y) { return x + y * g.S; }
 
 // Fluid::new / Fluid::default state (fluid.rs:93-110, 527-570) for sizes
 // where the density block needs no index clamping (S >= 22): U = V = `times`
@@ -46,26 +43,13 @@ __global__ void k_init(Geo g, float* __restrict__ f, int64_t fs, int times) {
   f[F_V0 * fs + o] = 0.0f;
 }
 
-// Row-major <-> scene layout.  mode 0: dst = src; mode 1: dst += src (and
-// dst2 += src when dst2 is set: add_density writes density and scratch).
-__global__ void k_from_rm(Geo g, const float* __restrict__ rm, float* __restrict__ dst, float* __restrict__ dst2,
-                          int mode) {
+// dst += src (and dst2 += src when dst2 is set: add_density writes density and scratch).
+__global__ void k_add(int64_t n, const float* __restrict__ src, float* __restrict__ dst, float* __restrict__ dst2) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= (int64_t)g.S * g.S) return;
-  const int64_t o = off_of(g, (int)(e % g.S), (int)(e / g.S));
-  const float v = rm[e];
-  if (mode == 0) {
-    dst[o] = v;
-  } else {
-    dst[o] += v;
-    if (dst2) dst2[o] += v;
-  }
-}
-
-__global__ void k_to_rm(Geo g, const float* __restrict__ src, float* __restrict__ rm) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= (int64_t)g.S * g.S) return;
-  rm[e] = src[off_of(g, (int)(e % g.S), (int)(e / g.S))];
+  if (e >= n) return;
+  const float v = src[e];
+  dst[e] += v;
+  if (dst2) dst2[e] += v;
 }
 
 // rowf[j] / colf[i]: row / column holds a NoWall cell (Passive copy rule of
@@ -96,7 +80,7 @@ __global__ void k_rowcol_bytes(int S, const uint32_t* __restrict__ rowf32, const
   colf[k] = colf32[k] != 0;
 }
 
-// Per-cell boundary codes (eqf_layout.h CodeBits) and the set_boundaries
+// Per-cell rule bytes (eqf_layout.h RuleBits) and the set_boundaries
 // lists: AdjustRow (right wall wins over left, fluid.rs:151-164),
 // AdjustColumn (up wins over down, fluid.rs:165-177), Passive ring copies.
 // fill == 0 only counts entries.
@@ -108,39 +92,19 @@ __global__ void k_codes(Geo g, const uint8_t* __restrict__ m, const uint8_t* __r
   if (e >= (int64_t)S * S) return;
   const int x = (int)(e % S), y = (int)(e / S);
   auto wall = [&](int i, int j) { return m[(int64_t)j * S + i] == EQF_DEFAULT_WALL; };
+  auto put = [&](int i, int j, uint32_t r) {
+    code[(int64_t)j * rm_code_stride(S) + i] = (uint8_t)r;
+    code[rm_code_bytes(S) + (int64_t)i * rm_code_stride(S) + j] = (uint8_t)r;
+  };
   if (x >= 1 && x <= N && y >= 1 && y <= N) {
-    uint32_t c = 0;
     const bool fl = !wall(x, y);
-    if (fl) c |= C_FLUID;
-    if (wall(x - 1, y)) c |= C_LWALL;
-    if (wall(x + 1, y)) c |= C_RWALL;
-    if (wall(x, y + 1)) c |= C_DWALL;
-    if (wall(x, y - 1)) c |= C_UWALL;
-    if (colf[x]) c |= C_COLF;
-    if (fill && g.layout == L_ROWMAJOR) {
+    if (fill) {
       uint32_t r = R_INTERIOR;
       if (fl) {
-        r |= ((c & C_RWALL) ? R_NEG_SECOND : (c & C_LWALL) ? R_NEG_FIRST : 0u) << R_ROW_SHIFT;
-        r |= ((c & C_UWALL) ? R_NEG_FIRST : (c & C_DWALL) ? R_NEG_SECOND : 0u) << R_COL_SHIFT;
+        r |= (wall(x + 1, y) ? R_NEG_SECOND : wall(x - 1, y) ? R_NEG_FIRST : 0u) << R_ROW_SHIFT;
+        r |= (wall(x, y - 1) ? R_NEG_FIRST : wall(x, y + 1) ? R_NEG_SECOND : 0u) << R_COL_SHIFT;
       }
-      code[(int64_t)y * rm_code_stride(S) + x] = (uint8_t)r;
-    }
-    if (fill && g.layout == L_CYCLIC) {
-      const int64_t o = cyc_code_word(x, y, g.P), mstride = cyc_code_bytes(g.P, g.ns) / 4;
-      const int sh = cyc_code_shift(x, y, g.P);
-      const bool strip_bottom = (y & 63) == 0 && y < N;  // the row below is in the next strip
-      uint8_t srow = SEL_KEEP, scol = SEL_KEEP;
-      if (fl) {
-        srow = (c & C_RWALL) ? SEL_NEG2 : (c & C_LWALL) ? SEL_NEG1 : SEL_KEEP;
-        scol = (c & C_UWALL) ? SEL_NEG1 : ((c & C_DWALL) && !strip_bottom) ? SEL_NEG2 : SEL_KEEP;
-      } else if (((y - 1) & 63) == 0 && y > 1 && !wall(x, y - 1) && !wall(x, y - 2)) {
-        scol = SEL_FIXUP;
-      }
-      // the words start at zero; OR in the non-zero selectors
-      uint32_t* cw = reinterpret_cast<uint32_t*>(code);
-      if (srow) atomicOr(&cw[o], (uint32_t)srow << sh);
-      if (scol) atomicOr(&cw[mstride + o], (uint32_t)scol << sh);
-      if (colf[x]) atomicOr(&cw[2 * mstride + o], 1u << sh);
+      put(x, y, r);
     }
     if (fl) {
       int sx = -1;
@@ -168,15 +132,13 @@ __global__ void k_codes(Geo g, const uint8_t* __restrict__ m, const uint8_t* __r
     if (on) {
       const int k = atomicAdd(&cnt[2], 1);
       if (fill) lpas[k] = make_int2((int)off_of(g, x, y), (int)off_of(g, sx, sy));
-      if (fill && g.layout == L_ROWMAJOR) {
-        const uint32_t r = y == 0 ? R_COPY_DOWN : y == S - 1 ? R_COPY_UP : x == 0 ? R_COPY_RIGHT : R_COPY_LEFT;
-        code[(int64_t)y * rm_code_stride(S) + x] = (uint8_t)(r << R_PAS_SHIFT);
-      }
+      if (fill)
+        put(x, y, (y == 0 ? R_COPY_DOWN : y == S - 1 ? R_COPY_UP : x == 0 ? R_COPY_RIGHT : R_COPY_LEFT) << R_PAS_SHIFT);
     }
   }
 }
 
-Geo geo_of(const eqf_scene* s) { return Geo{s->S, s->N, s->ns, s->P, s->layout}; }
+Geo geo_of(const eqf_scene* s) { return Geo{s->S, s->N}; }
 
 unsigned blocks_for(int64_t n) { return (unsigned)((n + 255) / 256); }
 
@@ -198,47 +160,29 @@ static int ensure_stage(eqf_scene* s) {
 
 int eqf_dev_upload(eqf_scene* s, float* dst, float* dst2, const float* host, int add) {
   const size_t n = (size_t)s->S * s->S;
-  if (s->layout == L_ROWMAJOR && !add) {
-    hipError_t e = hipMemcpyAsync(dst, host, sizeof(float) * n, hipMemcpyHostToDevice, s->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
-    return e == hipSuccess ? EQF_OK : eqf_internal_error(EQF_EDEVICE, std::string("upload: ") + hipGetErrorString(e));
+  float* to = dst;
+  if (add) {
+    int rc = ensure_stage(s);
+    if (rc) return rc;
+    to = s->d_stage;
   }
-  int rc = ensure_stage(s);
-  if (rc) return rc;
-  hipError_t e = hipMemcpyAsync(s->d_stage, host, sizeof(float) * n, hipMemcpyHostToDevice, s->stream);
-  if (e == hipSuccess) {
-    hipLaunchKernelGGL(k_from_rm, dim3(blocks_for((int64_t)n)), dim3(256), 0, s->stream, geo_of(s), s->d_stage, dst,
-                       dst2, add);
+  hipError_t e = hipMemcpyAsync(to, host, sizeof(float) * n, hipMemcpyHostToDevice, s->stream);
+  if (e == hipSuccess && add) {
+    hipLaunchKernelGGL(k_add, dim3(blocks_for((int64_t)n)), dim3(256), 0, s->stream, (int64_t)n, s->d_stage, dst, dst2);
     e = hipGetLastError();
   }
   if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
   return e == hipSuccess ? EQF_OK : eqf_internal_error(EQF_EDEVICE, std::string("upload: ") + hipGetErrorString(e));
 }
 
-int eqf_dev_to_rm_async(eqf_scene* s, const float* src, float* dst) {
-  const size_t n = (size_t)s->S * s->S;
-  hipError_t e;
-  if (s->layout == L_ROWMAJOR) {
-    e = hipMemcpyAsync(dst, src, sizeof(float) * n, hipMemcpyDeviceToDevice, s->stream);
-  } else {
-    hipLaunchKernelGGL(k_to_rm, dim3(blocks_for((int64_t)n)), dim3(256), 0, s->stream, geo_of(s), src, dst);
-    e = hipGetLastError();
-  }
-  return e == hipSuccess ? EQF_OK : eqf_internal_error(EQF_EDEVICE, std::string("layout copy: ") + hipGetErrorString(e));
+int eqf_dev_copy_async(eqf_scene* s, const float* src, float* dst) {
+  const hipError_t e =
+      hipMemcpyAsync(dst, src, sizeof(float) * (size_t)s->S * s->S, hipMemcpyDeviceToDevice, s->stream);
+  return e == hipSuccess ? EQF_OK : eqf_internal_error(EQF_EDEVICE, std::string("field copy: ") + hipGetErrorString(e));
 }
 
 int eqf_dev_download(eqf_scene* s, const float* src, float* host) {
-  const size_t n = (size_t)s->S * s->S;
-  hipError_t e;
-  if (s->layout == L_ROWMAJOR) {
-    e = hipMemcpyAsync(host, src, sizeof(float) * n, hipMemcpyDeviceToHost, s->stream);
-  } else {
-    int rc = ensure_stage(s);
-    if (rc) return rc;
-    hipLaunchKernelGGL(k_to_rm, dim3(blocks_for((int64_t)n)), dim3(256), 0, s->stream, geo_of(s), src, s->d_stage);
-    e = hipGetLastError();
-    if (e == hipSuccess) e = hipMemcpyAsync(host, s->d_stage, sizeof(float) * n, hipMemcpyDeviceToHost, s->stream);
-  }
+  hipError_t e = hipMemcpyAsync(host, src, sizeof(float) * (size_t)s->S * s->S, hipMemcpyDeviceToHost, s->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
   return e == hipSuccess ? EQF_OK : eqf_internal_error(EQF_EDEVICE, std::string("download: ") + hipGetErrorString(e));
 }
@@ -302,8 +246,7 @@ int eqf_dev_rebuild_bnd(eqf_scene* s) {
     s->bnd_cap = total;
   }
   {
-    const size_t ncode = s->layout == L_CYCLIC ? 3 * (size_t)cyc_code_bytes(s->P, s->ns) : (size_t)rm_code_bytes(S);
-    e = hipMemsetAsync(s->d_code, 0, ncode, s->stream);
+    e = hipMemsetAsync(s->d_code, 0, 2 * (size_t)rm_code_bytes(S), s->stream);
   }
   if (e == hipSuccess) {  // the fill pass counts into the second, still zero, counters
     hipLaunchKernelGGL(k_codes, dim3(blocks_for(n)), dim3(256), 0, s->stream, g, s->d_mask, s->d_rowf, d_colf,

@@ -1,9 +1,8 @@
 """Autotuners.
 
 * Red-black mode: band shape x sweeps per launch (eqf_scene_set_tuning).
-* Batches (wavefront mode): waves per workgroup at most -- with fewer waves a
-  strip runs fewer sweep streams -- and the scene-to-workgroup order
-  (eqf_batch_set_tuning), and the wavefront schedule (eqf_batch_set_schedule).
+* Batches (wavefront mode): nothing to choose (the lexicographic kernel has one
+  split of the work); tune_batch times a trial for the record.
 * Batches (red-black mode): band shape x sweeps per launch over all scenes
   (eqf_batch_set_band).
 
@@ -76,54 +75,39 @@ def tune_redblack(scene, frames=1, use_cache=True):
     return tile, tsw, timings
 
 
-BATCH_WAVES = (16, 8, 4, 2, 1)
-BATCH_ORDERS = (_abi.BATCH_LARGEST_FIRST, _abi.BATCH_GIVEN_ORDER)
-BATCH_SCHEDS = (_abi.SCHED_WIDE, _abi.SCHED_RING, _abi.SCHED_FINE)
-
-
 def _batch_key(scenes):
     sig = ",".join(f"{s.params.size}:{s.params.gs_iters}:{s.params.pressure_iters}" for s in scenes)
-    return f"batch2:{len(scenes)}:{hashlib.sha1(sig.encode()).hexdigest()[:16]}:{_device_key(scenes[0].ctx)}"
+    return f"batch3:{len(scenes)}:{hashlib.sha1(sig.encode()).hexdigest()[:16]}:{_device_key(scenes[0].ctx)}"
 
 
 def tune_batch(scenes, frames=2, use_cache=True):
-    """Picks (max_waves, order, schedule) for a batch of the given
-    wavefront-mode _abi.Scene objects and returns (max_waves, order,
-    schedule, timings in ms per frame).  Trials run on clones."""
+    """(max_waves, order, schedule) for a batch of the given wavefront-mode
+    _abi.Scene objects, and the trial's ms per frame: the launch does not
+    depend on these settings, so they are the defaults.  The trial runs on
+    clones."""
+    best = (16, _abi.BATCH_LARGEST_FIRST, _abi.SCHED_AUTO)
     key = _batch_key(scenes)
     db = _load() if use_cache else {}
     if key in db:
-        w, o, sc = db[key]["best"]
-        return w, o, sc, db[key].get("ms", {})
-    maxns = max((s.params.size - 2 + 63) // 64 for s in scenes)
+        return (*best, db[key].get("ms", {}))
     clones = [s.clone() for s in scenes]
     b = _abi.Batch(clones)
-    timings = {}
     try:
-        for w in BATCH_WAVES:
-            if w < maxns:
-                continue
-            for o in BATCH_ORDERS:
-                b.set_tuning(w, o)
-                for sc in BATCH_SCHEDS:
-                    b.set_schedule(sc)
-                    b.step(frames)  # builds the graph of `frames` launches
-                    b.sync()
-                    t0 = time.perf_counter()
-                    b.step(frames)
-                    b.sync()
-                    timings[f"{w}:{o}:{sc}"] = (time.perf_counter() - t0) * 1e3 / frames
+        b.step(frames)  # builds the graph
+        b.sync()
+        t0 = time.perf_counter()
+        b.step(frames)
+        b.sync()
+        timings = {"16:0:0": (time.perf_counter() - t0) * 1e3 / frames}
     finally:
         b.close()
         for c in clones:
             c.close()
-    best = min(timings, key=timings.get)
-    w, o, sc = (int(x) for x in best.split(":"))
     db = _load() if use_cache else {}
-    db[key] = {"best": [w, o, sc], "ms": timings}
+    db[key] = {"best": list(best), "ms": timings}
     if use_cache:
         _save(db)
-    return w, o, sc, timings
+    return (*best, timings)
 
 
 def tune_batch_band(scenes, frames=2, use_cache=True):

@@ -150,11 +150,10 @@ int eqf_sync(eqf_scene *s);
  * (equilibrium_amd/tune.py); the server's red-black groups use the default. */
 int eqf_scene_set_tuning(eqf_scene *s, int tile, int sweeps_per_block);
 
-/* Batches: many scenes of one mode advanced together; K frames are captured
- * once as a HIP graph and replayed.  Wavefront mode (sizes up to 1026): one
- * fused launch per frame runs every scene's whole frame.  Red-black mode (any
- * sizes, one iteration count): every kernel of the frame covers all scenes
- * (band passes over all scenes' tiles, then the grid-wide phases).  Scenes
+/* Batches: many scenes of one mode advanced together; a frame is captured
+ * once as a HIP graph and replayed, and every kernel of it covers all scenes.
+ * Wavefront mode: sizes up to 1026, any iteration counts.  Red-black mode: any
+ * sizes, one iteration count.  Scenes
  * stay owned by the caller.  While in a batch a scene is not stepped alone
  * and its mask, parameters and frame sources are fixed (eqf_step,
  * eqf_fill_rect, eqf_set_mask, eqf_scene_set_params, eqf_set_frame_source
@@ -170,26 +169,17 @@ int eqf_batch_sync(eqf_batch *b);
 int eqf_batch_destroy(eqf_batch *b);
 /* Wall time of the last eqf_batch_step in milliseconds (HIP events). */
 int eqf_batch_last_ms(const eqf_batch *b, double *ms);
-/* Launch shape of a batch (no counterpart in the reference): waves per
- * workgroup at most (1..16, at least the largest scene's strip count of
- * ceil(N/64); fewer waves means fewer sweep streams per strip) and the
- * scene-to-workgroup order.  Results do not depend on it.  Chosen by the
- * autotuner (equilibrium_amd/tune.py). */
+/* Launch shape of a wavefront-mode batch (no counterpart in the reference):
+ * waves per workgroup at most (1..16, at least the largest scene's strip count
+ * of ceil(N/64)) and the scene-to-workgroup order.  The arguments are checked;
+ * neither results nor launches depend on them: a lin_solve always gives a
+ * workgroup to each strip of 64 rows, in the order of the scenes' longest
+ * remaining chains. */
 enum { EQF_BATCH_LARGEST_FIRST = 0, EQF_BATCH_GIVEN_ORDER = 1 };
 int eqf_batch_set_tuning(eqf_batch *b, int max_waves, int order);
 /* Wavefront schedule of a wavefront-mode batch (no counterpart in the
- * reference; results do not depend on it): EQF_SCHED_WIDE, a workgroup
- * barrier every 16 steps, every sweep stream reading a lin_solve's
- * right-hand side from device memory; EQF_SCHED_RING, a barrier every 8
- * steps, the right-hand side handed from sweep stream to sweep stream in
- * LDS and up to P/48 streams per strip instead of P/64; EQF_SCHED_FINE, a
- * barrier every 4 steps, 4 steps of prefetch, the LDS hand-off and up to
- * P/32 streams per strip (small scenes); EQF_SCHED_AUTO (the default): FINE
- * when it gives the batch's largest scene more sweep streams than RING (N
- * 49..192 with max_waves 16), else RING when it gives more than WIDE or two
- * or more streams and at least 8 waves (N 193..512), else WIDE.  Single
- * scenes (eqf_step) and server ticks use the AUTO rule.  Red-black batches:
- * EQF_EINVAL. */
+ * reference): the argument is checked; neither results nor launches depend on
+ * it.  Red-black batches: EQF_EINVAL. */
 enum { EQF_SCHED_AUTO = 0, EQF_SCHED_WIDE = 1, EQF_SCHED_RING = 2, EQF_SCHED_FINE = 3 };
 int eqf_batch_set_schedule(eqf_batch *b, int sched);
 /* Band shape and sweeps per launch of a red-black batch (as
@@ -200,9 +190,9 @@ int eqf_batch_set_band(eqf_batch *b, int tile, int sweeps_per_block);
  * reference, whose frame loop runs one scene; renderer_helpers.rs:52-72).
  * A server thread admits queued requests while their device memory fits the
  * budget, keeps admitted scenes resident, and advances every resident scene
- * by one frame per tick: wavefront-mode scenes (size <= 1026) with one fused
- * launch, red-black scenes (any size) with their frame graphs on a second
- * stream beside it; scenes join and leave at tick boundaries.  Admission
+ * by one frame per tick of its lane (wavefront-mode scenes up to size 258,
+ * larger ones up to 1026, red-black scenes of any size: three lanes, each on
+ * its own stream); scenes join and leave at tick boundaries.  Admission
  * uploads overlap the running tick. */
 typedef struct eqf_server_config {
     uint64_t hbm_budget_bytes; /* device memory the resident scenes may use */

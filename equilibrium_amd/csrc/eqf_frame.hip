@@ -786,19 +786,19 @@ static uint64_t group_key(const RbGroup& g) {
 }
 
 // The strips of `nslots` lin_solves of scene i, `iters` sweeps each.
-static void lex_tasks(int i, int S, int iters, int nslots, std::vector<LexTask>& v, int& nflags, int64_t& hpairs) {
+static void lex_tasks(int i, int S, int iters, int nslots, std::vector<LexTask>& v, int& nflags, int64_t& hfloats) {
   const int K = lex_round_sweeps(iters, 0);  // the longest round
   if (K == 0) return;
   const int n = lex_strips(S, K);
   for (int slot = 0; slot < nslots; ++slot)
     for (int strip = 0; strip < n; ++strip) {
-      v.push_back(LexTask{i, slot, strip, n, nflags++, 0, hpairs});
-      if (strip + 1 < n) hpairs += lex_handoff_pairs(S);
+      v.push_back(LexTask{i, slot, strip, n, nflags++, 0, hfloats});
+      if (strip + 1 < n) hfloats += lex_handoff_floats(S);
     }
 }
 static size_t lex_ctl_bytes(int nflags) { return (sizeof(uint32_t) * (size_t)(nflags + 2) + 255) & ~(size_t)255; }
 int64_t lex_workspace_bytes(int S) {
-  return 3 * ((int64_t)(lex_strips(S, LEX_KMAX) - 1) * lex_handoff_pairs(S) * 8 + lex_strips(S, LEX_KMAX) * 36);
+  return 3 * ((int64_t)(lex_strips(S, LEX_KMAX) - 1) * lex_handoff_floats(S) * 4 + lex_strips(S, LEX_KMAX) * 36);
 }
 
 // Ticket order: the longest remaining chain of a scene first (a strip waits
@@ -912,7 +912,7 @@ static int group_tables(RbGroup& g, hipStream_t st, std::string& err) {
   g.n_lpress = (int)lpress.size();
   if (g.exact) {
     g.n_lflags = std::max(fd, fp);
-    const size_t need = lex_ctl_bytes(g.n_lflags) + 8 * (size_t)std::max(hd, hp);
+    const size_t need = lex_ctl_bytes(g.n_lflags) + 4 * (size_t)std::max(hd, hp);
     if (need > g.lex_bytes) {
       (void)hipFree(g.d_lex);
       g.d_lex = nullptr;
@@ -1010,7 +1010,7 @@ static void g_corners(hipStream_t st, const RbGroup& g, int c0, int c1, int diff
 static void g_lex(hipStream_t st, const RbGroup& g, bool press, const LexSpec& s0, const LexSpec& s1,
                   const LexSpec& s2) {
   uint32_t* ctl = (uint32_t*)g.d_lex;
-  uint64_t* H = (uint64_t*)((char*)g.d_lex + lex_ctl_bytes(g.n_lflags));
+  float* H = (float*)((char*)g.d_lex + lex_ctl_bytes(g.n_lflags));
   for (int r = 0; r < (press ? g.press_rounds : g.diff_rounds); ++r) {
     const LexArgs a{{s0, s1, s2}, r, press ? 1 : 0};
     lex_launch(st, g.d_scs, press ? g.d_lpress : g.d_ldiff, press ? g.n_lpress : g.n_ldiff, a, ctl, g.n_lflags, H,

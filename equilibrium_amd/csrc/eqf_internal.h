@@ -97,7 +97,7 @@ struct LexTask {
   int strip, nstrips;
   int flag;      // its progress count; the strip above has the one before
   int pad;
-  int64_t hoff;  // its hand-off pairs (the strip above: lex_handoff_pairs before)
+  int64_t hoff;  // its hand-off values (the strip above: lex_handoff_floats before)
 };
 struct LexSpec {
   int mode, x_role, x0_role, coef;
@@ -111,7 +111,7 @@ constexpr uint32_t LEX_SPIN_MAX = 1u << 22;
 // ctl: ticket, ended workgroups, then nflags progress counts, all zero before
 // the first launch; a launch leaves them zero.
 void lex_launch(hipStream_t st, const RbScene* scs, const LexTask* tasks, int ntasks, const LexArgs& args,
-                uint32_t* ctl, int nflags, uint64_t* H, uint32_t* err);
+                uint32_t* ctl, int nflags, float* H, uint32_t* err);
 
 // Frames (eqf_frame.hip).  A launch group's scenes share one mode.
 void* frame_create(eqf_scene* s, std::string& err);

@@ -79,11 +79,13 @@ EQF_HD inline int lex_round_sweeps(int iters, int round) {
   const int n = lex_rounds(iters);
   return round < n ? iters / n + (round < iters % n ? 1 : 0) : 0;
 }
-// Strips of 64 rows that K sweeps of S rows take, each sweep one row further up.
-EQF_HD inline int lex_strips(int S, int K) { return (S + K - 1 + 63) / 64; }
+// Rows of a strip: 64 lanes, the first of which repeats the last row of the strip above.
+constexpr int LEX_ROWS = 63;
+// Strips that K sweeps of S rows take, each sweep one row further up.
+EQF_HD inline int lex_strips(int S, int K) { return (S + K - 1 + LEX_ROWS - 1) / LEX_ROWS; }
 // Blocks of LEX_B steps of a strip: column S-1 of lane 63 in the last sweep, and its final value a step later.
 EQF_HD inline int lex_blocks(int S, int K) { return ((S + 63 + 2 * (K - 1)) >> 3) + 1; }
-// Hand-off values a strip leaves for the next one: (raw, final) pairs per sweep and step.
-EQF_HD inline int64_t lex_handoff_pairs(int S) { return (int64_t)LEX_KMAX * lex_blocks(S, LEX_KMAX) * LEX_B; }
+// Hand-off values a strip leaves for the next one: one per sweep and step.
+EQF_HD inline int64_t lex_handoff_floats(int S) { return (int64_t)LEX_KMAX * lex_blocks(S, LEX_KMAX) * LEX_B; }
 
 }  // namespace eqf

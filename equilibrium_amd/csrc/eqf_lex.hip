@@ -2,18 +2,20 @@
 // the exact mode on gfx950, bit for bit.
 //
 // Work split.  The grid of S x S cells (ring included) is cut into strips of
-// 64 rows.  A workgroup takes one strip of one lin_solve through up to
+// 63 rows.  A workgroup takes one strip of one lin_solve through up to
 // LEX_KMAX = 20 sweeps (a round): lane r of a wave owns a row, each of four
 // waves runs up to five consecutive sweeps, two steps apart.  The strip moves
-// up by one row from sweep to sweep: in sweep k lane r holds row j = 64 s + r
-// - k.  A cell of sweep k at step t is column c = t - r - 2k.  Then everything
+// up by one row from sweep to sweep: in sweep k lane r holds row j = 63 s - 1 +
+// r - k.  A cell of sweep k at step t is column c = t - r - 2k.  Then everything
 // a cell reads comes from its own lane or the lane before it, at an earlier
 // step:
 //   left  x_k(c-1, j)      own lane, step t-1
 //   up    x_k(c, j-1)      lane r-1, step t-1
 //   down  x_{k-1}(c, j+1)  own lane, its value after set_boundaries at t-1
 //   right x_{k-1}(c+1, j)  lane r-1, the same
-// so sweeps hand values on in registers, waves through LDS, and a strip needs
+// Lane 0 repeats the last row of the strip above: its updated values come from
+// there instead of x0, and with the rules of its row they give its final ones.
+// So sweeps hand values on in registers, waves through LDS, and a strip needs
 // only the strip above it (lane 63 of every sweep), never the one below: x and
 // x0 are read once and x is written once for all the sweeps of a round.  The
 // row shift costs K - 1 more rows per round.  Strips that do not move have to
@@ -21,7 +23,14 @@
 // sweeps of a strip 32 to 64 steps apart and moved 12 bytes per cell and sweep
 // through the caches: one workgroup per scene, 28.7 ms per frame at N=1024,
 // 0.86 at N=128, 0.44 at N=30 (16 sweeps), 11.0 for 512 scenes of N 64..512;
-// with moving strips on a CU each 2.20, 0.44, 0.18 and 8.1 ms.
+// with moving strips on a CU each 1.91, 0.39, 0.16 and 5.8 ms.
+//
+// Lane 0 as a row of its own (63 rows per strip, one select per update) does
+// away with the first lane's neighbours as operands of their own: the lane
+// shifts become operands of the additions, 109 registers instead of 168 hold
+// a wave, and two workgroups share a CU.  With 64 rows, two values per cell in
+// the hand-off and the shifts as moves a frame took 2.20, 0.44, 0.18 and 8.1 ms
+// (7.6 where it was held to 128 registers, by spilling).
 //
 // AdjustRow's walls are the left / right neighbours, known one step after the
 // cell: its final value is formed then (hence two steps from sweep to sweep).
@@ -31,21 +40,24 @@
 // value, or in Passive the copy of the interior neighbour.  Which of these a
 // block of eight steps can hold decides among four forms of the step (Class).
 //
-// Two more waves bring operands into LDS by anti-diagonals, where a step of a
+// Three more waves bring operands into LDS by anti-diagonals, where a step of a
 // wave reads 64 neighbours, write the results, and exchange lane 63's values
 // with the strips above and below, which run on other CUs: agent-scope stores
-// and loads in device memory, and a progress count per strip.  A strip trails
+// and loads in device memory, and a progress count per strip.  (Two waves for
+// it took 4400 cycles per block, more than the sweeps; with three the sweeps
+// bound it.)  A strip trails
 // the one above it by about 100 steps (64 of skew, the blocks of 8, two
 // memory latencies).  Workgroups take their strip from a ticket counter whose
 // order puts every strip after the one it reads from, so a waiting workgroup
 // always waits for one that already runs: the launch ends whatever share of
 // it is resident.
 //
-// Bound: instruction issue of the sweeps.  An update of a plain cell takes 7
-// VALU instructions (6 of arithmetic, 1 lane shift); a plain block of 5 sweeps
-// x 8 steps about 3000 cycles with a wave alone on its SIMD, of which 40 x 7
-// VALU instructions are 1400.  A lone scene is bound by its chain of
-// S + 63 + 2K steps plus about 100 per strip.
+// Bound: instruction issue of the sweeps.  An update of a plain cell takes 8
+// VALU instructions (6 of arithmetic, of which two shift a lane, one for lane
+// 0, one that gathers lane 63's value); a plain block of 5 sweeps x 8 steps
+// 2800 cycles with a wave alone on its SIMD, of which 500 are LDS reads of x0.
+// A lone scene is bound by its chain of S + 63 + 2K steps plus about 100 per
+// strip.
 //
 // Compiled with -ffp-contract=off: rustc does not contract a*b+c.
 #include <hip/hip_runtime.h>
@@ -57,31 +69,28 @@ namespace eqf {
 namespace lex {
 
 constexpr int W = LEX_W, QMAX = 5, KMAX = LEX_KMAX, B = LEX_B;
-constexpr int NT = 64 * (W + 2);  // four waves of sweeps, two that move data
+constexpr int NT = 64 * (W + 3);  // four waves of sweeps, three that move data
 static_assert(KMAX == W * QMAX && B == 8, "four waves of up to five sweeps, blocks of 8 steps");
-// x0 in LDS by anti-diagonals: row u = c + j - 64 s of a ring of XR rows,
-// position p = j - 64 s + KMAX - 1 (sweep k at step t reads row t - 3k, lane r
-// position r - k + KMAX - 1: 64 neighbours).  Rows are numbered u + UOFF >= 0.
+// x0 in LDS by anti-diagonals: row u = c + j - 63 s + 1 of a ring of XR rows,
+// position p = j - 63 s + KMAX (sweep k at step t reads row t - 3k, lane r
+// position r - k + KMAX - 1: 64 neighbours; lane 0 its value from the strip
+// above, at CP + k).  Rows are numbered u + UOFF >= 0.
 // A block of 8 steps may start anywhere in the ring, so the first 8 rows are
 // held twice.  Live at block b: rows 8b - 20 .. 8b + 79 (the last wave's last
 // sweep, words of four rules; the rows loaded during the block).
-constexpr int XP = 84, XR = 104, UOFF = 64;
-static_assert(XP >= 64 + KMAX - 1 && XR % B == 0 && XR >= 3 * (KMAX - 1) + B * W + 11, "x0 ring too short");
+constexpr int CP = 84, XP = CP + KMAX, XR = 104, UOFF = 64;
+static_assert(CP >= 64 + KMAX - 1 && XR % B == 0 && XR >= 3 * (KMAX - 1) + B * W + 11, "x0 ring too short");
 constexpr int CR = XR / 4;  // rule words: four rows of one position per word, first two rows held twice
-// hand-off from wave to wave: 16 step rows of 65 values (the first: the strip
-// above); a pitch of 72 keeps the transposing accesses (8 steps x 8 lanes per
+// hand-off from wave to wave: 16 step rows of 64 values; a pitch of 72 keeps the transposing accesses (8 steps x 8 lanes per
 // 64) in distinct banks
 constexpr int RP = 72, RR = 16;
 // LDS layout (4-byte words)
 constexpr int L_X0 = 0;
 constexpr int L_CODE = L_X0 + (XR + B) * XP;
-constexpr int L_RING = L_CODE + (CR + 2) * XP;
+constexpr int L_RING = L_CODE + (CR + 2) * CP;
 constexpr int EN = W * QMAX * B;
-constexpr int L_EU = L_RING + (W + 1) * RR * RP;  // lane 0's up / right values: [block & 1][wave][sweep][8 steps]
-constexpr int L_ER = L_EU + 2 * EN;
-constexpr int L_P = L_ER + 2 * EN;  // lane 63's updated values: [block & 1][wave][sweep][8 steps]
-constexpr int L_PF = L_P + 2 * EN;  // in blocks with rules also the final values, of the cells of a step before
-constexpr int L_CL = L_PF + 2 * EN;  // class of the waves' blocks of steps, a byte each: [block & 3]
+constexpr int L_P = L_RING + (W + 1) * RR * RP;  // lane 63's updated values: [block & 1][wave][sweep][8 steps]
+constexpr int L_CL = L_P + 2 * EN;  // class of the waves' blocks of steps, a byte each: [block & 3]
 constexpr int L_MISC = L_CL + 4;
 constexpr int L_WORDS = L_MISC + 4;
 static_assert(L_WORDS * 4 <= 80 * 1024, "two workgroups per CU");
@@ -89,21 +98,34 @@ static_assert(L_WORDS * 4 <= 80 * 1024, "two workgroups per CU");
 typedef __attribute__((address_space(3))) float lf;
 typedef __attribute__((address_space(3))) uint32_t lu;
 typedef __attribute__((address_space(3))) uint8_t lb;
-typedef float f4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u2 __attribute__((ext_vector_type(2)));
-typedef __attribute__((address_space(3))) f4 lf4;
+typedef float f2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) f2 lf2;
 
 __device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
-// lane i <- lane i-1; lane 0 <- edge (DPP wave_shr:1).  PIN keeps the move where
-// it is written (it reads its source lane only if that lane is enabled).
-template <bool PIN>
-__device__ __forceinline__ float from_prev_lane(float v, float edge) {
-  float r = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, edge),
-                                                                  __builtin_bit_cast(int, v), 0x138, 0xf, 0xf, false));
-  if constexpr (PIN) asm volatile("" : "+v"(r));
-  return r;
+// lane i <- lane i-1 (DPP wave_shr:1; lane 0, which has no use for it, 0).
+// Where its one use is an addition the compiler makes it that addition's operand.
+__device__ __forceinline__ float from_prev_lane(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x138, 0xf, 0xf, true));
+}
+
+// Lane 63 - n of `acc` <- lane 63 of v (n < 16; a constant).  Lanes below it in
+// its group of four change too: called with n ascending.
+template <int N>
+__device__ __forceinline__ float put_lane_n(float acc, float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, acc), __builtin_bit_cast(int, v),
+                                                               N == 0 ? 0xe4 : 0x100 + N, 8, 8 >> (N / 4), false));
+}
+__device__ __forceinline__ float put_lane(float acc, float v, int n) {
+  switch (n) {
+#define EQF_LANE(N) case N: return put_lane_n<N>(acc, v);
+    EQF_LANE(0) EQF_LANE(1) EQF_LANE(2) EQF_LANE(3) EQF_LANE(4) EQF_LANE(5) EQF_LANE(6) EQF_LANE(7)
+    EQF_LANE(8) EQF_LANE(9) EQF_LANE(10) EQF_LANE(11) EQF_LANE(12) EQF_LANE(13) EQF_LANE(14) EQF_LANE(15)
+#undef EQF_LANE
+  }
+  return acc;
 }
 
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
@@ -135,10 +157,9 @@ __device__ __forceinline__ uint32_t selectors(uint32_t c) {  // four rule bytes 
 struct Carry {
   float r1[QMAX];     // the cell updated at the last step
   float f2[QMAX];     // final value of the cell updated the step before it
-  float ul[QMAX];     // upper neighbour used at the last step
   float lp[QMAX];     // left neighbour used at the last step
   uint32_t sp[QMAX];  // selector of the cell updated at the last step
-  float in, inr;      // the previous wave's final values of the last step: this lane's, the lane's before it
+  float in;           // the previous wave's final value of the last step
   int row;            // x0 ring row of the next block's first step, sweep k0
 };
 
@@ -158,12 +179,12 @@ struct Place {
 
 // Eight steps of Q consecutive sweeps k0 .. k0+Q-1 (block m = b - w: steps 8m
 // .. 8m+7).  Where no cell has a rule, a cell's final value is the updated
-// one, and the right neighbour of a cell is the upper neighbour that the sweep
-// before used a step ago: one lane shift per update instead of two.
+// one.
 template <int MODE, int Q, int CLS>
 __device__ __forceinline__ void steps(lf* L, Carry& s, int b, int w, int k0, const Place& pl) {
   constexpr bool GEN = CLS == C_ALL;
   constexpr bool FIN = GEN && MODE != M_PASSIVE;  // final values other than the updated ones
+  constexpr int G = 2;
   const int m = b - w, lane = pl.lane;
   const float a = pl.a, cr = pl.cr;
   const lf* x0p[Q];
@@ -174,7 +195,8 @@ __device__ __forceinline__ void steps(lf* L, Carry& s, int b, int w, int k0, con
   for (int q = 0; q < Q; ++q) {
     int row = s.row - 3 * q;
     row += row < 0 ? XR : 0;
-    x0p[q] = L + (L_X0 + row * XP + KMAX - 1 - (k0 + q)) + lane;
+    const int pos = KMAX - 1 - (k0 + q) + lane;
+    x0p[q] = L + (L_X0 + row * XP) + (lane == 0 ? CP + k0 + q : pos);
     if constexpr (CLS == C_ROWS || CLS == C_RING) {
       top[q] = lane == k0 + q - pl.base;
       bot[q] = lane == k0 + q - pl.base + pl.S - 1;
@@ -184,48 +206,41 @@ __device__ __forceinline__ void steps(lf* L, Carry& s, int b, int w, int k0, con
       }
     }
     if constexpr (GEN) {
-      const lu* cp = (const lu*)L + (L_CODE + (row >> 2) * XP + KMAX - 1 - (k0 + q)) + lane;
-      const uint32_t w0 = cp[0], w1 = cp[XP], w2 = cp[2 * XP];
+      const lu* cp = (const lu*)L + (L_CODE + (row >> 2) * CP) + pos;
+      const uint32_t w0 = cp[0], w1 = cp[CP], w2 = cp[2 * CP];
       const uint32_t sh = (uint32_t)(row & 3);
       cw[q][0] = __builtin_amdgcn_alignbyte(w1, w0, sh);
       cw[q][1] = __builtin_amdgcn_alignbyte(w2, w1, sh);
     }
   }
   const lf* ri = L + (L_RING + (w * RR + (m & 1) * B) * RP) + lane;
-  lf* ro = L + (L_RING + ((w + 1) * RR + (m & 1) * B) * RP + 1) + lane;
-  const lf* eu = L + L_EU + (b & 1) * EN + w * QMAX * B;
-  const lf* er = L + L_ER + (b & 1) * EN + w * QMAX * B;
+  lf* ro = L + (L_RING + ((w + 1) * RR + (m & 1) * B) * RP) + lane;
   lf* po = L + L_P + (b & 1) * EN + w * QMAX * B;
-  lf* pf = L + L_PF + (b & 1) * EN + w * QMAX * B;
-  // Operands of four steps are read from LDS while the four before them are
-  // still being computed, ahead of those steps' writes (the compiler cannot
-  // tell that reads and writes do not overlap, and one wave per SIMD has
-  // nothing else to fill the latency of a read with).
-  float xin[2][4], xinr[2][4], x0v[Q][2][4];
-  f4 e4u[Q][2], e4r[Q][2];
-  auto fetch = [&](int h) {
+  // Operands of G steps are read from LDS while the G before them are computed,
+  // ahead of those steps' writes (the compiler cannot tell that reads and
+  // writes do not overlap).
+  float xin[2][G], x0v[Q][2][G];
+  auto fetch = [&](int g) {
+    const int h = g & 1;
 #pragma unroll
-    for (int ii = 0; ii < 4; ++ii) {
+    for (int ii = 0; ii < G; ++ii) {
 #pragma unroll
-      for (int q = 0; q < Q; ++q) x0v[q][h][ii] = x0p[q][(h * 4 + ii) * XP];
-      xin[h][ii] = ri[(h * 4 + ii) * RP + 1];
-      xinr[h][ii] = ri[(h * 4 + ii) * RP];
-    }
-    if (lane == 0) {  // only lane 0 has use for them
-#pragma unroll
-      for (int q = 0; q < Q; ++q) {
-        e4u[q][h] = *(const lf4*)(eu + q * B + h * 4);
-        if (FIN && q > 0) e4r[q][h] = *(const lf4*)(er + q * B + h * 4);
-      }
+      for (int q = 0; q < Q; ++q) x0v[q][h][ii] = x0p[q][(g * G + ii) * XP];
+      xin[h][ii] = ri[(g * G + ii) * RP];
     }
   };
   fetch(0);
-  float in = s.in, inr = s.inr, out[B];
+  float in = s.in, last[(Q + 1) / 2];
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    f4 pa[Q], pb[Q];
+  for (int q = 0; q < Q; q += 2) last[q / 2] = 0.0f;
 #pragma unroll
-    for (int ii = 0; ii < 4; ++ii) {
+  for (int g = 0; g < B / G; ++g) {
+    const int h = g & 1;
+    if (g + 1 < B / G) fetch(g + 1);
+    float out[G];
+#pragma unroll
+    for (int ii = 0; ii < G; ++ii) {
+      const int i = g * G + ii;
       // The sweeps of a step are independent; the update goes through them
       // operation by operation, so that no instruction waits for the one
       // before it (a dependent one issues 8 cycles later instead of 4).
@@ -235,22 +250,18 @@ __device__ __forceinline__ void steps(lf* L, Carry& s, int b, int w, int k0, con
         dn[q] = q == 0 ? in : s.f2[q - 1];
         lt[q] = s.r1[q];
         fin[q] = s.r1[q];
+        rt[q] = from_prev_lane(dn[q]);
+        up[q] = from_prev_lane(s.r1[q]);
       }
-#pragma unroll
-      for (int q = 0; q < Q; ++q)
-        rt[q] = q == 0 ? inr : FIN ? from_prev_lane<GEN>(dn[q], e4r[q][h][ii]) : s.ul[q - 1];
-#pragma unroll
-      for (int q = 0; q < Q; ++q) up[q] = from_prev_lane<GEN>(s.r1[q], e4u[q][h][ii]);
       // fluid.rs:315-320; AdjustColumn: logical right / left are down / up
+#pragma unroll
+      for (int q = 0; q < Q; ++q) t[q] = MODE == M_COL ? up[q] + dn[q] : rt[q] + lt[q];
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int q = 0; q < Q; ++q) t[q] = MODE == M_COL ? dn[q] + up[q] : rt[q] + lt[q];
+      for (int q = 0; q < Q; ++q) t[q] = MODE == M_COL ? rt[q] + t[q] : t[q] + dn[q];
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int q = 0; q < Q; ++q) t[q] = t[q] + (MODE == M_COL ? rt[q] : dn[q]);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int q = 0; q < Q; ++q) t[q] = t[q] + (MODE == M_COL ? lt[q] : up[q]);
+      for (int q = 0; q < Q; ++q) t[q] = MODE == M_COL ? t[q] + lt[q] : up[q] + t[q];
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int q = 0; q < Q; ++q) t[q] = a * t[q];
@@ -272,8 +283,8 @@ __device__ __forceinline__ void steps(lf* L, Carry& s, int b, int w, int k0, con
             nv[q] = top[q] ? (first ? x0v[q][h][ii] : dn[q]) : nv[q];
             nv[q] = bot[q] ? up[q] : nv[q];
             if constexpr (CLS == C_RING) {
-              nv[q] = c0[q] == h * 4 + ii ? (first ? x0v[q][h][ii] : rt[q]) : nv[q];
-              nv[q] = cN[q] == h * 4 + ii ? lt[q] : nv[q];
+              nv[q] = c0[q] == i ? (first ? x0v[q][h][ii] : rt[q]) : nv[q];
+              nv[q] = cN[q] == i ? lt[q] : nv[q];
             }
           } else {
             nv[q] = (top[q] || bot[q]) ? x0v[q][h][ii] : nv[q];
@@ -283,7 +294,7 @@ __device__ __forceinline__ void steps(lf* L, Carry& s, int b, int w, int k0, con
       if constexpr (GEN) {
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
-          const uint32_t sel = (cw[q][h] >> (8 * ii)) & 255u;
+          const uint32_t sel = (cw[q][i >> 2] >> (8 * (i & 3))) & 255u;
           if constexpr (MODE == M_PASSIVE) {
             // before the first sweep the ring holds what it held, not copies
             // of the right / lower neighbours
@@ -297,38 +308,37 @@ __device__ __forceinline__ void steps(lf* L, Carry& s, int b, int w, int k0, con
             nv[q] = sel == 0u ? nv[q] : rv;
           } else {
             nv[q] = (sel & 4u) ? x0v[q][h][ii] : nv[q];
-            fin[q] = s.sp[q] == 1u ? -s.lp[q] : fin[q];
-            fin[q] = s.sp[q] == 2u ? -nv[q] : fin[q];
-            s.sp[q] = sel;
-            s.lp[q] = lt[q];
           }
         }
       }
 #pragma unroll
+      for (int q = 0; q < Q; ++q) nv[q] = lane == 0 ? x0v[q][h][ii] : nv[q];
+      if constexpr (FIN) {
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+          fin[q] = s.sp[q] == 1u ? -s.lp[q] : fin[q];
+          fin[q] = s.sp[q] == 2u ? -nv[q] : fin[q];
+          s.sp[q] = (cw[q][i >> 2] >> (8 * (i & 3))) & 255u;
+          s.lp[q] = lt[q];
+        }
+      }
+#pragma unroll
       for (int q = 0; q < Q; ++q) {
-        pa[q][ii] = nv[q];
-        if (FIN) pb[q][ii] = fin[q];
+        last[q / 2] = put_lane(last[q / 2], nv[q], (q & 1) * B + i);
         s.f2[q] = fin[q];
         s.r1[q] = nv[q];
-        s.ul[q] = up[q];
       }
-      out[h * 4 + ii] = s.f2[Q - 1];
+      out[ii] = s.f2[Q - 1];
       in = xin[h][ii];
-      inr = xinr[h][ii];
-      if (h == 0 && ii == 2) fetch(1);
     }
-    if (lane == 63) {
 #pragma unroll
-      for (int q = 0; q < Q; ++q) {
-        *(lf4*)(po + q * B + h * 4) = pa[q];
-        if (FIN) *(lf4*)(pf + q * B + h * 4) = pb[q];
-      }
-    }
+    for (int ii = 0; ii < G; ++ii) ro[(g * G + ii) * RP] = out[ii];
   }
+  // lane 63's values: lane 63 - i holds step i of an even sweep, lane 55 - i of the odd one after it
 #pragma unroll
-  for (int i = 0; i < B; ++i) ro[i * RP] = out[i];
+  for (int q = 0; q < Q; q += 2)
+    if (lane >= (q + 1 < Q ? 64 - 2 * B : 64 - B)) po[q * B + 63 - lane] = last[q / 2];
   s.in = in;
-  s.inr = inr;
   s.row += B;
   s.row -= s.row >= XR ? XR : 0;
   if constexpr (!GEN && MODE != M_PASSIVE) {
@@ -368,23 +378,24 @@ __device__ __forceinline__ Part part_of(int w, int S, int K) {
 }
 
 // One strip of one round (K sweeps) of a lin_solve.  Waves 0..3 run the
-// sweeps; waves 4 and 5 bring operands into LDS a block ahead, write the
+// sweeps; waves 4, 5 and 6 bring operands into LDS a block ahead, write the
 // results, and talk to the neighbouring strips, so that their loads'
 // latencies and the waits for the strip above stay out of the sweeps.
 // In block b of the workgroup wave w runs block m = b - w of its steps.
 template <int MODE>
 __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, const LexTask& tk, const LexSpec& sp, int K,
-                                           uint32_t* __restrict__ flags, uint64_t* __restrict__ Hb,
+                                           uint32_t* __restrict__ flags, float* __restrict__ Hb,
                                            uint32_t* __restrict__ err) {
   const SceneDesc& d = sc.d;
   const int S = d.S;
   const int tid = threadIdx.x, lane = tid & 63, w = uni(tid >> 6);
-  const int base = 64 * tk.strip;
+  const int base = LEX_ROWS * tk.strip - 1;  // lane 0: the last row of the strip above
   const int Wn = min(W, K);
   const int NB = lex_blocks(S, K);
   const int NI = NB + Wn;
-  // LDS before the first block: edge values that nothing writes read 0
-  for (int e = L_EU + tid; e < L_MISC; e += NT) L[e] = 0.0f;
+  // LDS before the first block: lane 0's values, which nothing writes in the first strip
+  for (int e = tid; e < (XR + B) * KMAX; e += NT) L[L_X0 + e / KMAX * XP + CP + e % KMAX] = 0.0f;
+  if (tid < L_MISC - L_CL) ((lu*)L)[L_CL + tid] = 0;
   __syncthreads();
 
   if (w < W) {  // the sweeps
@@ -394,10 +405,10 @@ __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, const LexTa
     Carry s;
 #pragma unroll
     for (int q = 0; q < QMAX; ++q) {
-      s.r1[q] = s.f2[q] = s.ul[q] = s.lp[q] = 0.0f;
+      s.r1[q] = s.f2[q] = s.lp[q] = 0.0f;
       s.sp[q] = 0;
     }
-    s.in = s.inr = 0.0f;
+    s.in = 0.0f;
     s.row = (pt.mlo * B + UOFF - 3 * pt.k0) % XR;
     for (int b = -1; b < NI; ++b) {
       const int m = b - w;
@@ -429,7 +440,6 @@ __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, const LexTa
   const int T = lex_blocks(S, KMAX) * B;
   // hand-off: value 64 z + lane of the EN per block, [wave][sweep][step]
   int ew[3], ek[3], ei[3], elo[3], ehi[3];
-  bool eq0[3];  // the wave's first sweep
 #pragma unroll
   for (int z = 0; z < 3; ++z) {
     const int e = 64 * z + lane;
@@ -438,21 +448,18 @@ __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, const LexTa
     const int q = e / B % QMAX;
     ek[z] = pt.k0 + q;
     ei[z] = e % B;
-    eq0[z] = q == 0;
     const bool on = e < EN && q < pt.Q;
     elo[z] = on ? pt.mlo : 1;
     ehi[z] = on ? pt.mhi : 0;
   }
   const bool ring_copies = MODE == M_PASSIVE && d.nbnd[M_PASSIVE] == 4 * d.N;  // every ring cell copies its neighbour
-  if (w == W) {  // x0 and the rules, and lane 63's values for the strip below
+  const int hf = (lane & 1) * 4;  // the item's first row of the block's eight
+  if (w == W) {  // x0
     const rsrc_t rx0 = make_rsrc(x0 - FLD_PAD, fbytes);
-    const int Sc = rm_code_stride(S);
-    // the rule bytes, transposed for COL, from CODE_PAD bytes before to 8 after them
-    const rsrc_t rc = make_rsrc(d.code + (MODE == M_COL ? rm_code_bytes(S) : 0) - CODE_PAD, rm_code_used(S) + CODE_PAD + 8);
-    constexpr int NX = 2 * (XP - 1) + (MODE == M_COL ? 2 * (B - 1) : 0), NC = 2 * (XP - 1);
+    constexpr int NX = 2 * (CP - 1) + (MODE == M_COL ? 2 * (B - 1) : 0);
     static_assert(NX <= 192, "three passes");
-    const int hf = (lane & 1) * 4;  // the item's first row of the block's eight
-    int xp0[3], xc[3], xj[3], xoff[3], coff[3], cc[3];
+    int xp0[3], xc[3], xj[3], xoff[3];
+    bool xring[3];  // a ring cell by its row(s)
 #pragma unroll
     for (int z = 0; z < 3; ++z) {
       const int it = (64 * z + lane) >> 1;
@@ -460,22 +467,13 @@ __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, const LexTa
       xc[z] = (MODE == M_COL ? KMAX - 1 + B - 1 - it : hf - it + KMAX - 1) - UOFF;  // + 8 ub: its logical column
       xj[z] = base + xp0[z] - (KMAX - 1);                                          // its logical row
       xoff[z] = (MODE == M_COL ? xc[z] * S + xj[z] : xj[z] * S + xc[z]) * 4 + FLD_PAD * 4;
-      cc[z] = hf - it + KMAX - 1 - UOFF;  // + 8 ub: first logical column of the rules
-      coff[z] = min(max(base + it - (KMAX - 1), 0), S - 1) * Sc + hf - it + KMAX - 1 - UOFF + CODE_PAD;
-    }
-    bool xring[3];  // by its row(s)
-#pragma unroll
-    for (int z = 0; z < 3; ++z)
       xring[z] = MODE == M_COL ? (uint32_t)(xj[z] + 3) <= 3u || (uint32_t)(S - 1 - xj[z]) <= 3u : xj[z] == 0 || xj[z] == S - 1;
+    }
     u4 gx0[3], gring[3];
-    u2 gc[3];
     bool ring_w[3] = {false, false, false};  // some item of the pass holds a ring cell (wave-uniform)
 #pragma unroll
-    for (int z = 0; z < 3; ++z) {
-      gx0[z] = gring[z] = (u4)(0);
-      gc[z] = (u2)(0);
-    }
-    auto load = [&](int ub) {  // rows 8 ub - UOFF .. of x0 (for ring cells, the value they hold) and their rules
+    for (int z = 0; z < 3; ++z) gx0[z] = gring[z] = (u4)(0);
+    auto load = [&](int ub) {  // rows 8 ub - UOFF .. of x0 (for ring cells, the value they hold)
 #pragma unroll
       for (int z = 0; z < 3; ++z) {
         const int c = xc[z] + ub * B, off = xoff[z] + ub * B * stepc * 4;
@@ -484,14 +482,10 @@ __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, const LexTa
         ring_w[z] = __builtin_amdgcn_ballot_w64(rg) != 0;
         gx0[z] = __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(rx0, off, 0, 0));
         if (ring_w[z]) gring[z] = __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(rx, off, 0, 0));
-        gc[z] = __builtin_bit_cast(u2, __builtin_amdgcn_raw_buffer_load_b64(rc, (coff[z] + ub * B) & ~3, 0, 0));
       }
     };
-    uint32_t h_rule = 0, h_col = 0;
     auto put = [&](int ub) {
       const int row = (ub * B) % XR;
-      uint32_t any = 0;
-      bool cols = false;
 #pragma unroll
       for (int z = 0; z < 3; ++z) {
         uint32_t v[4];
@@ -508,21 +502,61 @@ __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, const LexTa
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             // (COL: positions outside the row go to its last slot, which nobody reads)
-            const int pi = MODE == M_COL ? ((uint32_t)(xp0[z] + i) < (uint32_t)XP ? xp0[z] + i : XP - 1) : xp0[z];
+            const int pi = MODE == M_COL ? ((uint32_t)(xp0[z] + i) < (uint32_t)CP ? xp0[z] + i : CP - 1) : xp0[z];
             q[i * XP + pi] = v[i];
             if (row == 0) q[(XR + i) * XP + pi] = v[i];
           }
         }
+      }
+    };
+    for (int ub = 5; ub < 8; ++ub) {  // rows of the cells left of column 0's diagonal
+      load(ub);
+      put(ub);
+    }
+    load(UOFF / B);
+    for (int b = -1; b < NI; ++b) {
+      if (b + 1 < NB) put(b + 1 + UOFF / B);
+      if (b + 2 < NB) load(b + 2 + UOFF / B);
+      __syncthreads();
+    }
+    return;
+  }
+
+  if (w == W + 2) {  // lane 63's values for the strip below; the rules
+    const int Sc = rm_code_stride(S);
+    // the rule bytes, transposed for COL, from CODE_PAD bytes before to 8 after them
+    const rsrc_t rc = make_rsrc(d.code + (MODE == M_COL ? rm_code_bytes(S) : 0) - CODE_PAD, rm_code_used(S) + CODE_PAD + 8);
+    constexpr int NC = 2 * (CP - 1);
+    static_assert(NC <= 192, "three passes");
+    int coff[3], cc[3];
+    u2 gc[3];
+#pragma unroll
+    for (int z = 0; z < 3; ++z) {
+      const int it = (64 * z + lane) >> 1;
+      cc[z] = hf - it + KMAX - 1 - UOFF;  // + 8 ub: first logical column
+      coff[z] = min(max(base + it - (KMAX - 1), 0), S - 1) * Sc + hf - it + KMAX - 1 - UOFF + CODE_PAD;
+    }
+    auto load = [&](int ub) {
+#pragma unroll
+      for (int z = 0; z < 3; ++z)
+        gc[z] = __builtin_bit_cast(u2, __builtin_amdgcn_raw_buffer_load_b64(rc, (coff[z] + ub * B) & ~3, 0, 0));
+    };
+    uint32_t h_rule = 0, h_col = 0;
+    auto put = [&](int ub) {
+      const int row = (ub * B) % XR;
+      uint32_t any = 0;
+      bool cols = false;
+#pragma unroll
+      for (int z = 0; z < 3; ++z)
         if (64 * z + lane < NC) {
           const uint32_t sel = selectors<MODE>(__builtin_amdgcn_alignbyte(gc[z].y, gc[z].x, (uint32_t)((coff[z] + ub * B) & 3)));
-          lu* cq = (lu*)L + (L_CODE + (row >> 2) * XP) + (hf >> 2) * XP + ((64 * z + lane) >> 1);
+          lu* cq = (lu*)L + (L_CODE + (row >> 2) * CP) + (hf >> 2) * CP + ((64 * z + lane) >> 1);
           cq[0] = sel;
-          if (row == 0) cq[CR * XP] = sel;
+          if (row == 0) cq[CR * CP] = sel;
           any |= sel;
           const int c = cc[z] + ub * B;
           cols = cols || (uint32_t)(c + 3) <= 3u || (uint32_t)(S - 1 - c) <= 3u;
         }
-      }
       const bool rules = MODE == M_PASSIVE ? !ring_copies && any != 0 : (any & 0x03030303u) != 0;
       h_rule = (h_rule << 1) | (__builtin_amdgcn_ballot_w64(rules) != 0 ? 1u : 0u);
       h_col = (h_col << 1) | (__builtin_amdgcn_ballot_w64(cols) != 0 ? 1u : 0u);
@@ -548,10 +582,17 @@ __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, const LexTa
       load(ub);
       put(ub);
     }
-    uint64_t* hout = Hb + tk.hoff;
+    float* hout = Hb + tk.hoff;
     uint32_t* fown = flags + tk.flag;
     load(UOFF / B);
     for (int b = -1; b < NI; ++b) {
+      if (has_next) {
+#pragma unroll
+        for (int z = 0; z < 3; ++z) {
+          const int m = b - 1 - ew[z], pb = (b - 1) & 1;
+          if (m >= elo[z] && m <= ehi[z]) agent_store(hout + (ek[z] * T + m * B + ei[z]), L[L_P + pb * EN + 64 * z + lane]);
+        }
+      }
       if (b + 1 < NB) {
         put(b + 1 + UOFF / B);
       } else {
@@ -559,32 +600,11 @@ __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, const LexTa
         h_col <<= 1;
       }
       classes(b + 1);
-      if (has_next) {
-#pragma unroll
-        for (int z = 0; z < 3; ++z) {
-          // (updated, final) values by the step of the update; a block with
-          // rules then corrects the final values of the steps before its own
-          const int m = b - 1 - ew[z], pb = (b - 1) & 1;
-          if (m >= elo[z] && m <= ehi[z]) {
-            const uint32_t pv = ((const lu*)L)[L_P + pb * EN + 64 * z + lane];
-            uint64_t* ho = hout + (ek[z] * T + m * B + ei[z]);
-            agent_store(ho, (uint64_t)pv | ((uint64_t)pv << 32));
-            if (MODE != M_PASSIVE && ((const lb*)(L + L_CL))[((b - 1) & 3) * 4 + ew[z]] == C_ALL && m * B + ei[z] > 0)
-              agent_store((uint32_t*)ho - 1, ((const lu*)L)[L_PF + pb * EN + 64 * z + lane]);
-          }
-        }
-      }
-      asm volatile("" ::: "memory");
-      bool six = false;  // exactly the next block's six loads follow the stores
-      if (b + 2 < NB) {
-        load(b + 2 + UOFF / B);
-        six = !(ring_w[0] || ring_w[1] || ring_w[2]);
-      }
       if (has_next && b > 0) {  // the stores are in memory: publish them
-        if (six) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         if (lane == 0) agent_store(fown, (uint32_t)b);
       }
+      if (b + 2 < NB) load(b + 2 + UOFF / B);
       __syncthreads();
     }
     if (has_next) {
@@ -597,11 +617,10 @@ __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, const LexTa
 
   // Wave 5: x before the round, lane 0's values from the strip above, and the
   // final values.
-  const uint64_t* hin = Hb + (has_prev ? tk.hoff - (int64_t)KMAX * T : 0);
+  const float* hin = Hb + (has_prev ? tk.hoff - (int64_t)KMAX * T : 0);
   const uint32_t* fprev = flags + (has_prev ? tk.flag - 1 : tk.flag);
   constexpr int ZI = MODE == M_COL ? 3 : 2;                          // passes
   constexpr int NIN = MODE == M_COL ? 2 * (64 + B - 1) : 2 * 64;     // items
-  const int hf = (lane & 1) * 4;
   // x before the round, as "sweep -1": row t of ring 0, lane r: x(t + 1 - r, base + r + 1)
   int ir[ZI], ioff[ZI], oc[ZI], oj[ZI];
 #pragma unroll
@@ -615,7 +634,10 @@ __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, const LexTa
     oj[z] = base + ir[z] - (K - 1);
   }
   u4 gin[ZI];
-  float gu[3], gr[3];
+  float gu[3];
+  int erow[3];  // x0 ring row of lane 0's values of the next block to be written
+#pragma unroll
+  for (int z = 0; z < 3; ++z) erow[z] = (ei[z] - 3 * ek[z] + UOFF + XR - B * ew[z]) % XR;
 #pragma unroll
   for (int z = 0; z < ZI; ++z) gin[z] = (u4)(0);
   uint32_t credit = 0, fnext = 0;  // the strip above has published this many blocks
@@ -646,17 +668,11 @@ __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, const LexTa
 #pragma unroll
       for (int z = 0; z < 3; ++z) {
         const int m = nb - ew[z];
-        gu[z] = gr[z] = 0.0f;
+        gu[z] = 0.0f;
+        // lane 0's value of step tau was made by the strip above in step tau + 63
         if (m >= elo[z] && m <= ehi[z]) {
-          // The upper neighbour of step tau was updated at step tau + 63 of the
-          // strip above, the right one at tau + 62; a wave's first sweep takes
-          // its right ones from the ring, a step later (sweep 0: x before the round).
           const int tau = m * B + ei[z];
-          const float* hp = (const float*)hin + 2 * (ek[z] * T);
-          const int cc = min(tau + 2, S - 1), jj = min(base, S - 1);
-          const float* xr = x + (MODE == M_COL ? cc * S + jj : jj * S + cc);
-          gu[z] = agent_load(hp + 2 * min(tau + 63, T - 1));
-          gr[z] = agent_load(ek[z] > 0 ? hp + 2 * (min(tau + 62 + (eq0[z] ? 1 : 0), T - 1) - T) + 1 : xr);
+          gu[z] = agent_load(hin + ek[z] * T + min(tau + 63, T - 1));
         }
       }
       fnext = agent_load(fprev);
@@ -667,13 +683,13 @@ __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, const LexTa
     if (b + 1 < NB) {
 #pragma unroll
       for (int z = 0; z < ZI; ++z) {
-        lu* q = (lu*)L + (L_RING + ((b + 1) & 1) * B * RP + 1) + hf * RP;
+        lu* q = (lu*)L + (L_RING + ((b + 1) & 1) * B * RP) + hf * RP;
         if (64 * z + lane < NIN) {
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const int ri = MODE == M_COL ? ((uint32_t)(ir[z] + i) < 64u ? ir[z] + i : RP - 2) : ir[z];
+            const int ri = MODE == M_COL ? ((uint32_t)(ir[z] + i) < 64u ? ir[z] + i : RP - 1) : ir[z];
             const uint32_t v = gin[z][i];
-            q[i * RP + ri] = v;  // (a pointer one past the strip above's value)
+            q[i * RP + ri] = v;
           }
         }
       }
@@ -681,11 +697,12 @@ __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, const LexTa
     if (has_prev) {
 #pragma unroll
       for (int z = 0; z < 3; ++z)
-        if (64 * z + lane < EN) {
-          const int nb = b + 1, mm = nb - ew[z];
-          L[L_EU + (nb & 1) * EN + 64 * z + lane] = gu[z];
-          if (!eq0[z]) L[L_ER + (nb & 1) * EN + 64 * z + lane] = gr[z];
-          else L[L_RING + (ew[z] * RR + (mm & 1) * B + ei[z]) * RP] = gr[z];
+        if (elo[z] <= ehi[z]) {
+          lf* e = L + (L_X0 + CP) + erow[z] * XP + ek[z];
+          e[0] = gu[z];
+          if (erow[z] < B) e[XR * XP] = gu[z];
+          erow[z] += B;
+          erow[z] -= erow[z] >= XR ? XR : 0;
         }
     }
     load(b + 2);
@@ -696,7 +713,7 @@ __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, const LexTa
 #pragma unroll
       for (int z = 0; z < ZI; ++z) {
         if (64 * z + lane >= NIN) continue;
-        const lf* ring = L + (L_RING + (Wn * RR + (m & 1) * B) * RP + 1) + hf * RP;
+        const lf* ring = L + (L_RING + (Wn * RR + (m & 1) * B) * RP) + hf * RP;
         const int c = oc[z] + m * B, j = oj[z];
         float v[4];
         bool ok[4], all = true, some = false;
@@ -705,7 +722,7 @@ __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, const LexTa
           const int ci = MODE == M_COL ? c : c + i, ji = MODE == M_COL ? j + i : j;
           const int ri = MODE == M_COL ? min(max(ir[z] + i, 0), 63) : ir[z];
           v[i] = ring[i * RP + ri];
-          ok[i] = ci >= 1 && ci <= S - 2 && ji >= 1 && ji <= S - 2 && (MODE != M_COL || (uint32_t)(ir[z] + i) < 64u);
+          ok[i] = ci >= 1 && ci <= S - 2 && ji >= 1 && ji <= S - 2 && (uint32_t)(ir[z] + (MODE == M_COL ? i : 0) - 1) < 63u;
           all = all && ok[i];
           some = some || ok[i];
         }
@@ -724,27 +741,23 @@ __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, const LexTa
         if constexpr (MODE == M_PASSIVE) {
           if (some && (j == 1 || j == S - 2 || c <= 1 || c + 3 >= S - 2)) {
             const int Sc = rm_code_stride(S);
-            uint8_t top[4], bot[4], lft = 255, rgt = 255;
+            if (j == 1 || j == S - 2) {  // the rows above / below the interior
+              for (int side = 0; side < 2; ++side) {
+                if (j != (side ? S - 2 : 1)) continue;
+                const int y = side ? S - 1 : 0;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) top[i] = bot[i] = 255;
-            if (!ring_copies) {
-#pragma unroll
-              for (int i = 0; i < 4; ++i) {
-                const int cc = min(max(c + i, 0), S - 1);
-                top[i] = d.code[cc];
-                bot[i] = d.code[(S - 1) * Sc + cc];
+                for (int i = 0; i < 4; ++i)
+                  if (ok[i] && (ring_copies || (d.code[y * Sc + c + i] >> R_PAS_SHIFT))) x[y * S + c + i] = v[i];
               }
-              lft = d.code[j * Sc];
-              rgt = d.code[j * Sc + S - 1];
             }
+            float e = v[0];  // the columns left / right of it
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              if (!ok[i]) continue;
-              if (j == 1 && (top[i] >> R_PAS_SHIFT)) x[c + i] = v[i];
-              if (j == S - 2 && (bot[i] >> R_PAS_SHIFT)) x[(S - 1) * S + c + i] = v[i];
-              if (c + i == 1 && (lft >> R_PAS_SHIFT)) x[j * S] = v[i];
-              if (c + i == S - 2 && (rgt >> R_PAS_SHIFT)) x[j * S + S - 1] = v[i];
-            }
+            for (int i = 1; i < 4; ++i) e = c + i == 1 ? v[i] : e;
+            if (c <= 1 && c + 3 >= 1 && (ring_copies || (d.code[j * Sc] >> R_PAS_SHIFT))) x[j * S] = e;
+            e = v[0];
+#pragma unroll
+            for (int i = 1; i < 4; ++i) e = c + i == S - 2 ? v[i] : e;
+            if (c <= S - 2 && c + 3 >= S - 2 && (ring_copies || (d.code[j * Sc + S - 1] >> R_PAS_SHIFT))) x[j * S + S - 1] = e;
           }
         }
       }
@@ -753,9 +766,9 @@ __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, const LexTa
   }
 }
 
-__global__ void __launch_bounds__(NT, 3)
+__global__ void __launch_bounds__(NT, 4)
     k_lex(const RbScene* __restrict__ scs, const LexTask* __restrict__ tasks, int ntasks, LexArgs args,
-          uint32_t* __restrict__ ctl, uint32_t* __restrict__ flags, int nflags, uint64_t* __restrict__ H,
+          uint32_t* __restrict__ ctl, uint32_t* __restrict__ flags, int nflags, float* __restrict__ H,
           uint32_t* __restrict__ err) {
   extern __shared__ float lex_lds[];
   lf* L = (lf*)lex_lds;
@@ -785,7 +798,7 @@ __global__ void __launch_bounds__(NT, 3)
 }  // namespace lex
 
 void lex_launch(hipStream_t st, const RbScene* scs, const LexTask* tasks, int ntasks, const LexArgs& args,
-                uint32_t* ctl, int nflags, uint64_t* H, uint32_t* err) {
+                uint32_t* ctl, int nflags, float* H, uint32_t* err) {
   if (ntasks <= 0) return;
   hipLaunchKernelGGL(lex::k_lex, dim3((unsigned)ntasks), dim3(lex::NT), lex::L_WORDS * 4, st, scs, tasks, ntasks,
                      args, ctl, ctl + 2, nflags, H, err);

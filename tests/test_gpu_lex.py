@@ -1,5 +1,5 @@
 """The lexicographic lin_solve on the GPU at the edges of its split: strips of
-64 rows that move up a row per sweep, four waves of up to five sweeps, rounds of
+63 rows that move up a row per sweep, four waves of up to five sweeps, rounds of
 20 sweeps, blocks of 8 steps.  Random fields and walls, frames of the whole step
 against the oracle, bit for bit."""
 import numpy as np
@@ -41,7 +41,8 @@ def _pair(S, iters, press, walls, seed, full=()):
 
 @pytest.mark.parametrize("S,iters,press", [
     (3, 20, 20), (4, 1, 2), (22, 3, 4),      # one cell; fewer sweeps than waves
-    (45, 20, 20), (46, 20, 20),              # K + S - 1 = 64 / 65 rows: one strip, two
+    (44, 20, 20), (45, 20, 20),              # K + S - 1 = 63 / 64 rows: one strip, two
+    (46, 20, 20), (107, 20, 20), (108, 20, 20),
     (64, 5, 7), (65, 13, 16), (66, 19, 6),   # uneven sweeps per wave
     (109, 20, 20), (110, 20, 21),            # two strips, three; a second round of one sweep more
     (131, 41, 25), (258, 20, 40),            # three rounds, two

@@ -3,18 +3,49 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
 #include "../../include/eqfluid.h"
 #include "eqf_layout.h"
 
+// Pinned host memory that downloads of a context's scenes pass through, two
+// chunks per download in progress (eqf_setup.hip).  Held by the context and by
+// its scenes, whichever lives longest; at most KEEP buffers wait for reuse.
+class HostStaging {
+ public:
+  static constexpr size_t CHUNK = (size_t)1 << 21;
+  static constexpr int KEEP = 4;
+  struct Buf {
+    char* host = nullptr;  // 2 * CHUNK bytes
+    hipEvent_t ev[2] = {nullptr, nullptr};
+    Buf* next = nullptr;
+  };
+  explicit HostStaging(int device) : device_(device) {}
+  ~HostStaging();
+  HostStaging(const HostStaging&) = delete;
+  HostStaging& operator=(const HostStaging&) = delete;
+  Buf* take();  // nullptr: none to be had
+  void give(Buf* b);
+
+ private:
+  static void drop(Buf* b);
+  const int device_;
+  std::mutex m_;
+  Buf* free_ = nullptr;
+  int nfree_ = 0;
+};
+
 struct eqf_ctx {
   int device;
+  std::shared_ptr<HostStaging> staging;
 };
 
 struct eqf_scene {
   eqf_ctx* ctx = nullptr;
+  std::shared_ptr<HostStaging> staging;  // the context's
   uint64_t uid = 0;  // unique per scene object of the process (never reused)
   eqf_params p{};
   int S = 0, N = 0;

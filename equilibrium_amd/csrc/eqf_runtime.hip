@@ -184,6 +184,13 @@ extern "C" int eqf_ctx_create(int device, eqf_ctx** out) {
   auto* c = new (std::nothrow) eqf_ctx;
   if (!c) return fail(EQF_ENOMEM, "host allocation failed");
   c->device = device;
+  try {
+    c->staging = std::make_shared<HostStaging>(device);
+  } catch (...) {
+    delete c;
+    return fail(EQF_ENOMEM, "host allocation failed");
+  }
+  c->staging->give(c->staging->take());  // one is there from the start
   *out = c;
   return EQF_OK;
 }
@@ -245,6 +252,7 @@ static int scene_alloc(eqf_ctx* ctx, const eqf_params* p, eqf_scene** out, hipSt
   static std::atomic<uint64_t> next_uid{1};
   s->uid = next_uid++;
   s->ctx = ctx;
+  s->staging = ctx->staging;
   s->p = *p;
   s->S = (int)p->size;
   s->N = s->S - 2;

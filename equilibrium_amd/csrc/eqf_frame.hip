@@ -18,8 +18,8 @@
 // it, so the first and last tiles of a row or column of tiles reach the edge
 // with no halo there.  A pass reads one buffer and writes another (ping-pong).
 //
-// The other phases (divergence, gradient, advection with its row `break`,
-// set_boundaries lists, copy) are grid-wide kernels.  One frame is captured
+// The other phases (divergence, gradient, advection with its row `break`, each
+// with its set_boundaries, and the copy) are grid-wide kernels.  One frame is captured
 // once as a HIP graph and replayed.  Results are identical to the red-black
 // f32 CPU oracle bit for bit and are compared with its f64 version for
 // accuracy.  Compiled with -ffp-contract=off like the exact mode.
@@ -85,10 +85,8 @@ enum BandSel : uint32_t {
 };
 
 // A workgroup finds its scene and its place in it with one load from a map
-// of the launch's work units (band tile, block of CELL_BLOCK interior cells
-// or of CELL_BLOCK cells ring included -> {scene, index in the scene}); the
-// set_boundaries list kernel, whose threads straddle scenes, searches a
-// prefix table instead.
+// of the launch's work units (band tile or block of CELL_BLOCK cells, ring
+// included -> {scene, index in the scene}; segments of rows: seg_of).
 // Field roles in kernel arguments: F_* (eqf_layout.h), the ping-pong field, or none.
 constexpr int ROLE_TMP = NFIELDS;
 constexpr int ROLE_NONE = -1;
@@ -96,46 +94,37 @@ constexpr int ROLE_NONE = -1;
 constexpr int CELL_K = 4;
 constexpr int CELL_BLOCK = 256 * CELL_K;
 
-// The CELL_K interior cells of this thread in interior block `blk` of a
-// scene: flat indices blk*CELL_BLOCK + k*256 + threadIdx.x over the N x N
-// interior in row-major order, as 1-based (i, j).  Indices past N*N are
-// flagged !ok and clamped to cell (N, N), so their loads stay in the grid.
-__device__ __forceinline__ void interior_cells(int blk, int N, int (&ci)[CELL_K], int (&cj)[CELL_K],
-                                               bool (&ok)[CELL_K]) {
-  const int64_t idx0 = (int64_t)blk * CELL_BLOCK, nn = (int64_t)N * N;
-  const int j0 = (int)(idx0 / N), i0 = (int)(idx0 - (int64_t)j0 * N);
-  const float inv = 1.0f / (float)N;
-#pragma unroll
-  for (int k = 0; k < CELL_K; ++k) {
-    const int off = i0 + k * 256 + (int)threadIdx.x;  // < N + CELL_BLOCK: exact in f32
-    int q = (int)((float)off * inv);
-    int r = off - q * N;
-    if (r < 0) {  // the rounded reciprocal is off by at most one row
-      --q;
-      r += N;
-    } else if (r >= N) {
-      ++q;
-      r -= N;
-    }
-    ok[k] = idx0 + k * 256 + threadIdx.x < nn;
-    ci[k] = ok[k] ? r + 1 : N;
-    cj[k] = ok[k] ? j0 + q + 1 : N;
+// The kernels over interior cells give a wave up to SEG cells of one row, cell
+// 64 k + lane of them to lane `lane`, so that a row's place is scalar arithmetic
+// and a cell costs few address instructions: with cells dealt out in row-major
+// order regardless of rows, these took longer than the memory (a VALU
+// instruction per cell is 0.43 us at N=4096, and a division in 64 bits per wave
+// 0.3 us of a small launch).
+constexpr int SEG_K = 4, SEG = 64 * SEG_K;
+struct Seg {
+  int j, c0, n;  // row, first column, columns (<= 0: none)
+};
+// Wave w's segment of a workgroup.  at: {scene, row and segment of the first
+// wave's, segments per row}.
+__device__ __forceinline__ Seg seg_of(const int4& at, int w, int N) {
+  int j = at.y, s = at.z + w;
+  while (s >= at.w) {
+    s -= at.w;
+    ++j;
   }
+  const int c0 = 1 + s * SEG;
+  return Seg{j, c0, j <= N ? min(SEG, N + 1 - c0) : 0};
+}
+// Element i of an array: a scalar base and a 32-bit offset (a field has at most
+// 2^30 floats).
+__device__ __forceinline__ float ld(const float* p, uint32_t i) {
+  return *(const GAS float*)((const GAS char*)(const GAS float*)p + (size_t)(i << 2));
+}
+__device__ __forceinline__ void stg(float* p, uint32_t i, float v) {
+  *(GAS float*)((GAS char*)(GAS float*)p + (size_t)(i << 2)) = v;
 }
 __device__ __forceinline__ float* role_ptr(const RbScene& s, int role) {
   return role == ROLE_TMP ? s.tmp : s.d.fld + (int64_t)role * s.d.fstride;
-}
-// The last scene j with start[j] <= g (start[0] = 0; scenes without work
-// units have start[j] == start[j+1] and are skipped).
-template <class I>
-__device__ __forceinline__ int find_scene(const I* __restrict__ start, int n, I g) {
-  int lo = 0, hi = n - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (start[mid] <= g) lo = mid;
-    else hi = mid - 1;
-  }
-  return lo;
 }
 // Tiles along one dimension of S cells for regions of W cells and output
 // tiles of TX: region b starts at b*TX; the first needs no halo before it
@@ -259,10 +248,13 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu((N
       x0[i][b] = inside ? x0[i][b] : 0.0f;
       const uint32_t c = (cw[i] >> (8 * b)) & 255u;
       uint32_t sel = (c & R_INTERIOR) ? (uint32_t)BS_UPD : 0u;
-      if constexpr (MODE == M_ROW) sel |= (c >> R_ROW_SHIFT) & 3u;  // BS_NEG_LEFT / BS_NEG_RIGHT
+      if constexpr (MODE == M_ROW) {
+        const uint32_t r = (c >> R_ROW_SHIFT) & 3u;  // BS_NEG_LEFT / BS_NEG_RIGHT
+        sel |= r != R_SOURCE ? r : 0u;
+      }
       if constexpr (MODE == M_COL) {
         const uint32_t r = (c >> R_COL_SHIFT) & 3u;
-        sel |= r ? r + (BS_NEG_UP - R_NEG_FIRST) : 0u;
+        sel |= r && r != R_SOURCE ? r + (BS_NEG_UP - R_NEG_FIRST) : 0u;
       }
       if constexpr (MODE == M_PASSIVE) {
         const uint32_t r = (c >> R_PAS_SHIFT) & 7u;
@@ -426,73 +418,191 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu((N
   }
 }
 
-// project, first half (fluid.rs:339-349).  imap: workgroup -> {scene, block
-// of CELL_BLOCK interior cells}; every load of a thread's cells is issued
-// before its stores.  Also resets every row's break column to N+1 for the
-// advect that follows this projection (the cell in column 1 does it).
-__global__ void __launch_bounds__(256) k_div(const RbScene* __restrict__ scs, const int2* __restrict__ imap,
-                                             int u_role, int v_role, int div_role, int p_role) {
-  const int2 im = imap[blockIdx.x];
-  const RbScene& sc = scs[im.x];
-  const int S = sc.d.S, N = sc.d.N;
-  int ci[CELL_K], cj[CELL_K];
-  bool ok[CELL_K];
-  interior_cells(im.y, N, ci, cj, ok);
-  const float* __restrict__ u = role_ptr(sc, u_role);
-  const float* __restrict__ v = role_ptr(sc, v_role);
-  float ur[CELL_K], ul[CELL_K], vd[CELL_K], vu[CELL_K];
-#pragma unroll
-  for (int k = 0; k < CELL_K; ++k) {
-    const int q = cj[k] * S + ci[k];
-    ur[k] = u[q + 1];
-    ul[k] = u[q - 1];
-    vd[k] = v[q + S];
-    vu[k] = v[q - S];
+// set_boundaries (fluid.rs:151-187) and its corners (fluid.rs:265-271) run
+// inside the kernels that produce a field: a thread that has a cell's new value
+// also writes the cells that take theirs from it, so nothing waits for a
+// neighbour's thread.  On their own (a list of cells, then the corners) they
+// were 12 of a frame's 25 launches, and the break columns of the two advections
+// two more; a frame took 0.162 ms at N=30 (16 sweeps, exact), 0.297 at N=250
+// (red-black) and takes 0.139 and 0.274.
+
+// AdjustRow / AdjustColumn: a fluid cell beside a wall takes minus the wall
+// cell's value.  It takes it from the wall cell's thread, or from the ring,
+// which holds still.  Rule bytes mark the few wall cells of the interior that
+// have such a neighbour.
+__device__ __forceinline__ uint32_t row_rule(uint32_t c) { return (c >> R_ROW_SHIFT) & 3u; }
+__device__ __forceinline__ uint32_t col_rule(uint32_t c) { return (c >> R_COL_SHIFT) & 3u; }
+// Cell (i, j), rule byte c, of u (AdjustRow) and v (AdjustColumn) gets nu, nv
+// (where `keep`, has what it holds).
+__device__ __forceinline__ void put_ruled(const SceneDesc& d, uint32_t c, int i, int j, float* __restrict__ u,
+                                          float* __restrict__ v, float nu, float nv, bool keep) {
+  const int S = d.S, N = d.N, q = j * S + i, Sc = rm_code_stride(S);
+  const uint32_t rr = row_rule(c), rc = col_rule(c);
+  const uint8_t* code = d.code + j * Sc + i;
+  if (rr == R_NEG_FIRST) {
+    if (i == 1) u[q] = -u[q - 1];
+  } else if (rr == R_NEG_SECOND) {
+    if (i == N) u[q] = -u[q + 1];
+  } else {
+    if (!keep) u[q] = nu;
+    if (rr == R_SOURCE) {
+      if (keep) nu = u[q];
+      if (row_rule(code[-1]) == R_NEG_SECOND) u[q - 1] = -nu;
+      if (row_rule(code[1]) == R_NEG_FIRST) u[q + 1] = -nu;
+    }
   }
-  float* __restrict__ dv = role_ptr(sc, div_role);
-  float* __restrict__ p = role_ptr(sc, p_role);
-  const float sf = sc.d.sf;
-#pragma unroll
-  for (int k = 0; k < CELL_K; ++k) {
-    if (!ok[k]) continue;
-    const int q = cj[k] * S + ci[k];
-    dv[q] = -0.5f * (ur[k] - ul[k] + vd[k] - vu[k]) / sf;
-    p[q] = 0.0f;
-    if (ci[k] == 1) sc.trig[cj[k]] = N + 1;
+  if (rc == R_NEG_FIRST) {
+    if (j == 1) v[q] = -v[q - S];
+  } else if (rc == R_NEG_SECOND) {
+    if (j == N) v[q] = -v[q + S];
+  } else {
+    if (!keep) v[q] = nv;
+    if (rc == R_SOURCE) {
+      if (keep) nv = v[q];
+      if (col_rule(code[-Sc]) == R_NEG_SECOND) v[q - S] = -nv;
+      if (col_rule(code[Sc]) == R_NEG_FIRST) v[q + S] = -nv;
+    }
   }
 }
+// Passive: ring cells of rows and columns that hold a NoWall cell take the
+// interior neighbour's value; then, where `corner`, the corners, each by the
+// thread that has the two ring cells it is the mean of.  For interior cell
+// (i, j) beside the ring, of value val.
+__device__ __forceinline__ void put_ring(const SceneDesc& d, int i, int j, float* __restrict__ x, float val,
+                                         bool corner) {
+  const int S = d.S, N = d.N, Sc = rm_code_stride(S);
+  const bool all = d.ring_copies == 4 * N;
+  auto on = [&](int rx, int ry) { return all || (d.code[ry * Sc + rx] >> R_PAS_SHIFT) != 0; };
+  if (i == 1 && on(0, j)) x[j * S] = val;
+  if (i == N && on(S - 1, j)) x[j * S + S - 1] = val;
+  if (j == 1 && on(i, 0)) x[i] = val;
+  if (j == N && on(i, S - 1)) x[(S - 1) * S + i] = val;
+  if (!corner || (i != 1 && i != N) || (j != 1 && j != N)) return;
+  for (int k = 0; k < 4; ++k) {
+    const int cx = k & 1 ? S - 1 : 0, cy = k & 2 ? S - 1 : 0, nx = k & 1 ? N : 1, ny = k & 2 ? N : 1;
+    if (i != nx || j != ny) continue;
+    const float a = on(nx, cy) ? val : x[cy * S + nx], b = on(cx, ny) ? val : x[ny * S + cx];
+    x[cy * S + cx] = 0.5f * (a + b);
+  }
+}
+// ... for the values of a segment's cells (val[k]: cell 64 k + lane).
+template <int K>
+__device__ __forceinline__ void put_ring_seg(const SceneDesc& d, const Seg& g, int lane, float* __restrict__ x,
+                                             const float (&val)[K], bool corner) {
+  const int N = d.N;
+  if (g.j == 1 || g.j == N) {
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+      if (64 * k + lane < g.n) put_ring(d, g.c0 + 64 * k + lane, g.j, x, val[k], corner);
+  } else {
+    if (g.c0 == 1 && lane == 0) put_ring(d, 1, g.j, x, val[0], false);
+    if (N > 1 && g.c0 + g.n - 1 == N && lane == ((g.n - 1) & 63)) put_ring(d, N, g.j, x, val[K - 1], false);
+  }
+}
+// Corners of a field whose ring holds still: corner k of it.
+__device__ __forceinline__ void put_corner(int S, int k, float* __restrict__ x) {
+  const int cx = k & 1 ? S - 1 : 0, cy = k & 2 ? S - 1 : 0, nx = k & 1 ? S - 2 : 1, ny = k & 2 ? S - 2 : 1;
+  x[cy * S + cx] = 0.5f * (x[cy * S + nx] + x[ny * S + cx]);
+}
 
-// project, second half (fluid.rs:364-371); imap as for k_div.
-__global__ void __launch_bounds__(256) k_grad(const RbScene* __restrict__ scs, const int2* __restrict__ imap,
-                                              int u_role, int v_role, int p_role) {
-  const int2 im = imap[blockIdx.x];
-  const RbScene& sc = scs[im.x];
-  const int S = sc.d.S, N = sc.d.N;
-  int ci[CELL_K], cj[CELL_K];
-  bool ok[CELL_K];
-  interior_cells(im.y, N, ci, cj, ok);
-  float* __restrict__ u = role_ptr(sc, u_role);
-  float* __restrict__ v = role_ptr(sc, v_role);
-  const float* __restrict__ p = role_ptr(sc, p_role);
-  float uq[CELL_K], vq[CELL_K], pr[CELL_K], pl[CELL_K], pd[CELL_K], pu[CELL_K];
+// project, first half (fluid.rs:339-349), with Passive set_boundaries of both
+// results and, where `corner`, the divergence's corners.  imap: workgroup ->
+// its first wave's segment (seg_of).
+template <int K>
+__device__ __forceinline__ void div_seg(const SceneDesc& d, const Seg& g, int lane, const float* __restrict__ u,
+                                        const float* __restrict__ v, float* __restrict__ dv, float* __restrict__ p,
+                                        int corner) {
+  const int S = d.S;
+  float ur[K], ul[K], vd[K], vu[K];
+  uint32_t q[K];
 #pragma unroll
-  for (int k = 0; k < CELL_K; ++k) {
-    const int q = cj[k] * S + ci[k];
-    uq[k] = u[q];
-    vq[k] = v[q];
-    pr[k] = p[q + 1];
-    pl[k] = p[q - 1];
-    pd[k] = p[q + S];
-    pu[k] = p[q - S];
+  for (int k = 0; k < K; ++k) {
+    q[k] = (uint32_t)(g.j * S + g.c0) + (uint32_t)(k < K - 1 ? 64 * k + lane : min(64 * k + lane, g.n - 1));
+    ur[k] = ld(u + 1, q[k]);
+    ul[k] = ld(u - 1, q[k]);
+    vd[k] = ld(v + S, q[k]);
+    vu[k] = ld(v - S, q[k]);
   }
-  const float sf = sc.d.sf;
 #pragma unroll
-  for (int k = 0; k < CELL_K; ++k) {
-    if (!ok[k]) continue;
-    const int q = cj[k] * S + ci[k];
-    u[q] = uq[k] - 0.5f * (pr[k] - pl[k]) * sf;
-    v[q] = vq[k] - 0.5f * (pd[k] - pu[k]) * sf;
+  for (int k = 0; k < K; ++k) {
+    ur[k] = -0.5f * (ur[k] - ul[k] + vd[k] - vu[k]) / d.sf;
+    if (64 * k + lane < g.n) {
+      stg(dv, q[k], ur[k]);
+      stg(p, q[k], 0.0f);
+      ul[k] = 0.0f;
+    }
   }
+  put_ring_seg<K>(d, g, lane, dv, ur, corner != 0);
+  put_ring_seg<K>(d, g, lane, p, ul, false);
+}
+__global__ void __launch_bounds__(256) k_div(const RbScene* __restrict__ scs, const int4* __restrict__ imap,
+                                             int u_role, int v_role, int div_role, int p_role, int corner) {
+  const int4 at = imap[blockIdx.x];
+  const RbScene& sc = scs[at.x];
+  const int lane = threadIdx.x & 63;
+  const Seg g = seg_of(at, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), sc.d.N);
+  const float *u = role_ptr(sc, u_role), *v = role_ptr(sc, v_role);
+  float *dv = role_ptr(sc, div_role), *p = role_ptr(sc, p_role);
+  if (g.n > 192) div_seg<4>(sc.d, g, lane, u, v, dv, p, corner);
+  else if (g.n > 128) div_seg<3>(sc.d, g, lane, u, v, dv, p, corner);
+  else if (g.n > 64) div_seg<2>(sc.d, g, lane, u, v, dv, p, corner);
+  else if (g.n > 0) div_seg<1>(sc.d, g, lane, u, v, dv, p, corner);
+}
+
+// project, second half (fluid.rs:364-371), with set_boundaries of both results
+// and their corners (their ring cells hold still); the corners of p too where
+// `pc`, and those of the field c_role (ROLE_NONE: none) where the scene's
+// diffusion has sweeps.  imap as for k_div.
+template <int K>
+__device__ __forceinline__ void grad_seg(const SceneDesc& d, const Seg& g, int lane, float* __restrict__ u,
+                                         float* __restrict__ v, const float* __restrict__ p) {
+  const int S = d.S;
+  const uint8_t* code = d.code + (g.j * rm_code_stride(S) + g.c0);
+  float uq[K], vq[K], pr[K], pl[K], pd[K], pu[K];
+  uint32_t q[K], c[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const uint32_t o = (uint32_t)(k < K - 1 ? 64 * k + lane : min(64 * k + lane, g.n - 1));
+    q[k] = (uint32_t)(g.j * S + g.c0) + o;
+    uq[k] = ld(u, q[k]);
+    vq[k] = ld(v, q[k]);
+    pr[k] = ld(p + 1, q[k]);
+    pl[k] = ld(p - 1, q[k]);
+    pd[k] = ld(p + S, q[k]);
+    pu[k] = ld(p - S, q[k]);
+    c[k] = code[o];
+  }
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    uq[k] = uq[k] - 0.5f * (pr[k] - pl[k]) * d.sf;
+    vq[k] = vq[k] - 0.5f * (pd[k] - pu[k]) * d.sf;
+    const bool in = 64 * k + lane < g.n;
+    if (in && c[k] == R_INTERIOR) {
+      stg(u, q[k], uq[k]);
+      stg(v, q[k], vq[k]);
+    } else if (in) {
+      put_ruled(d, c[k], g.c0 + 64 * k + lane, g.j, u, v, uq[k], vq[k], false);
+    }
+  }
+}
+__global__ void __launch_bounds__(256) k_grad(const RbScene* __restrict__ scs, const int4* __restrict__ imap,
+                                              int u_role, int v_role, int p_role, int pc, int c_role) {
+  const int4 at = imap[blockIdx.x];
+  const RbScene& sc = scs[at.x];
+  const int S = sc.d.S, lane = threadIdx.x & 63;
+  const Seg g = seg_of(at, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), sc.d.N);
+  float *u = role_ptr(sc, u_role), *v = role_ptr(sc, v_role);
+  const float* p = role_ptr(sc, p_role);
+  if (at.y == 1 && at.z == 0 && threadIdx.x >= 240) {  // 16 threads: corner k of up to four fields
+    const int k = threadIdx.x & 3, f = (threadIdx.x >> 2) & 3;
+    const int role = f == 0 ? u_role : f == 1 ? v_role : f == 2 ? (pc ? p_role : ROLE_NONE)
+                                                                : (sc.d.diff_iters > 0 ? c_role : ROLE_NONE);
+    if (role != ROLE_NONE) put_corner(S, k, role_ptr(sc, role));
+  }
+  if (g.n > 192) grad_seg<4>(sc.d, g, lane, u, v, p);
+  else if (g.n > 128) grad_seg<3>(sc.d, g, lane, u, v, p);
+  else if (g.n > 64) grad_seg<2>(sc.d, g, lane, u, v, p);
+  else if (g.n > 0) grad_seg<1>(sc.d, g, lane, u, v, p);
 }
 
 struct Trace {
@@ -519,137 +629,156 @@ __device__ __forceinline__ Trace back_trace(const SceneDesc& d, int c, int j, fl
   return r;
 }
 __device__ __forceinline__ float gather(const float* __restrict__ d0, const Trace& r, int S) {
-  return r.s0 * (r.t0 * d0[r.j0 * S + r.i0] + r.t1 * d0[r.j1 * S + r.i0]) +
-         r.s1 * (r.t0 * d0[r.j0 * S + r.i1] + r.t1 * d0[r.j1 * S + r.i1]);
+  const uint32_t a = (uint32_t)(r.j0 * S), b = (uint32_t)(r.j1 * S);
+  return r.s0 * (r.t0 * ld(d0, a + r.i0) + r.t1 * ld(d0, b + r.i0)) +
+         r.s1 * (r.t0 * ld(d0, a + r.i1) + r.t1 * ld(d0, b + r.i1));
 }
 
-// advect, pass A: first column of each row whose back-trace reaches the far
-// edge (the `break` of fluid.rs:420-423), as the minimum of the triggering
-// columns (k_div set every row to N+1 "none" before).  imap as for k_div.  A
-// wave's lanes hold consecutive cells, so only the leftmost triggering cell
-// of each row within a wave updates the row's minimum.
-__global__ void __launch_bounds__(256) k_adv_trig(const RbScene* __restrict__ scs, const int2* __restrict__ imap,
-                                                  int u_role, int v_role) {
-  const int2 im = imap[blockIdx.x];
-  const RbScene& sc = scs[im.x];
-  const SceneDesc& d = sc.d;
-  const int S = d.S, N = d.N;
-  int ci[CELL_K], cj[CELL_K];
-  bool ok[CELL_K];
-  interior_cells(im.y, N, ci, cj, ok);
-  const float* __restrict__ u = role_ptr(sc, u_role);
-  const float* __restrict__ v = role_ptr(sc, v_role);
-  float uu[CELL_K], vv[CELL_K];
+// advect (fluid.rs:385-434) for one field (DENSITY: Passive set_boundaries and
+// the corners after it) or the two velocities (AdjustRow / AdjustColumn after
+// it).  A row stops at the first column whose back-trace reaches the far edge
+// (the `break` of fluid.rs:420-423): that cell copies its left neighbour's
+// value, cells right of it keep the buffer's content.  So the waves of a row
+// (R to a workgroup of NW; amap: its first row) first agree on the break
+// column, by lanes where a wave has the row alone, else in LDS, and then gather;
+// a segment's velocities stay in registers between the two, except where a row
+// has more than SEG * NW cells: they are read again (from the cache).
+template <bool DENSITY>
+struct AdvArgs {
+  const float *d0, *d1, *u, *v;
+  float *o0, *o1;
+};
+// First column of the segment whose back-trace reaches the far edge (N + 1: none).
+template <int K>
+__device__ __forceinline__ int seg_break(const SceneDesc& d, const Seg& g, int lane, const float (&uu)[K],
+                                         const float (&vv)[K]) {
+  int tr = d.N + 1;
 #pragma unroll
-  for (int k = 0; k < CELL_K; ++k) {
-    const int q = cj[k] * S + ci[k];
-    uu[k] = u[q];
-    vv[k] = v[q];
-  }
-  const int lane = threadIdx.x & 63;
-#pragma unroll
-  for (int k = 0; k < CELL_K; ++k) {
-    const bool t = ok[k] && back_trace(d, ci[k], cj[k], uu[k], vv[k]).trig;
+  for (int k = K - 1; k >= 0; --k) {
+    const bool t = 64 * k + lane < g.n && back_trace(d, g.c0 + 64 * k + lane, g.j, uu[k], vv[k]).trig;
     const uint64_t m = __builtin_amdgcn_ballot_w64(t);
-    if (t) {
-      // lanes max(0, lane - (i-1)) .. lane-1 hold this row's cells left of this one
-      const int first = max(0, lane - (ci[k] - 1));
-      const uint64_t left = ((1ull << lane) - 1) & ~((1ull << first) - 1);
-      if ((m & left) == 0) atomicMin(&sc.trig[cj[k]], ci[k]);
-    }
+    tr = m ? g.c0 + 64 * k + (int)__builtin_ctzll(m) : tr;
+  }
+  return tr;
+}
+template <int K>
+__device__ __forceinline__ void seg_load(const SceneDesc& d, const Seg& g, int lane, const float* __restrict__ u,
+                                         const float* __restrict__ v, float (&uu)[K], float (&vv)[K]) {
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const uint32_t q = (uint32_t)(g.j * d.S + g.c0) + (uint32_t)min(64 * k + lane, g.n - 1);
+    uu[k] = ld(u, q);
+    vv[k] = ld(v, q);
   }
 }
-
-// advect, pass B (fluid.rs:398-430) for one or two fields sharing u, v
-// (o1_role ROLE_NONE: one field); imap as for k_div.  The break columns and
-// velocities of a thread's cells are loaded together, then every gather, then
-// the stores.  Cells right of their row's break keep the buffer's content;
-// their (clamped, in-grid) gathers are computed and dropped.
-__global__ void __launch_bounds__(256) k_adv(const RbScene* __restrict__ scs, const int2* __restrict__ imap,
-                                             int o0_role, int i0_role, int o1_role, int i1_role, int u_role,
-                                             int v_role) {
-  const int2 im = imap[blockIdx.x];
-  const RbScene& sc = scs[im.x];
-  const int S = sc.d.S, N = sc.d.N;
-  int ci[CELL_K], cj[CELL_K];
-  bool ok[CELL_K];
-  interior_cells(im.y, N, ci, cj, ok);
-  float* __restrict__ o0 = role_ptr(sc, o0_role);
-  float* __restrict__ o1 = o1_role == ROLE_NONE ? nullptr : role_ptr(sc, o1_role);
-  const float* __restrict__ d0 = role_ptr(sc, i0_role);
-  const float* __restrict__ d1 = o1 ? role_ptr(sc, i1_role) : d0;
-  const float* __restrict__ u = role_ptr(sc, u_role);
-  const float* __restrict__ v = role_ptr(sc, v_role);
-  int tr[CELL_K];
-  float uu[CELL_K], vv[CELL_K];
+template <bool DENSITY, int K>
+__device__ __forceinline__ void seg_gather(const SceneDesc& d, const Seg& g, int lane, int tr, const AdvArgs<DENSITY>& a,
+                                           float (&uu)[K], float (&vv)[K]) {
+  const int S = d.S;
+  const uint8_t* code = d.code + (g.j * rm_code_stride(S) + g.c0);
+  float* __restrict__ o0 = a.o0;
+  float* __restrict__ o1 = a.o1;
+  float r0[K], r1[K];
+  uint32_t c[K];
 #pragma unroll
-  for (int k = 0; k < CELL_K; ++k) {
-    const int q = cj[k] * S + ci[k];
-    tr[k] = sc.trig[cj[k]];
-    uu[k] = u[q];
-    vv[k] = v[q];
-  }
-  float r0[CELL_K], r1[CELL_K];
-#pragma unroll
-  for (int k = 0; k < CELL_K; ++k) {
-    const int i = ci[k], j = cj[k], row = j * S;
-    int c = i;
-    if (i == tr[k] && i > 1) {  // the trigger cell copies its left neighbour's value (at most one per row)
-      c = i - 1;
-      uu[k] = u[row + c];
-      vv[k] = v[row + c];
+  for (int k = 0; k < K; ++k) {
+    const int o = min(64 * k + lane, g.n - 1), i = g.c0 + o, row = g.j * S;
+    int b = i;
+    if (tr <= g.c0 + 64 * k + 63 && i == tr && i > 1) {  // (the first: the same for all lanes)
+      b = i - 1;
+      uu[k] = a.u[row + b];
+      vv[k] = a.v[row + b];
     }
-    const Trace t = back_trace(sc.d, c, j, uu[k], vv[k]);
-    r0[k] = gather(d0, t, S);
-    r1[k] = gather(d1, t, S);
-    if (i == tr[k] && i == 1) {  // trigger in column 1: copies the ring cell d(0, j)
+    const Trace t = back_trace(d, b, g.j, uu[k], vv[k]);
+    r0[k] = gather(a.d0, t, S);
+    if constexpr (!DENSITY) {
+      r1[k] = gather(a.d1, t, S);
+      c[k] = code[o];
+    }
+    if (tr == 1 && i == 1) {  // trigger in column 1: copies the ring cell d(0, j)
       r0[k] = o0[row];
-      if (o1) r1[k] = o1[row];
+      if constexpr (!DENSITY) r1[k] = o1[row];
     }
   }
 #pragma unroll
-  for (int k = 0; k < CELL_K; ++k) {
-    if (!ok[k] || ci[k] > tr[k]) continue;  // right of the break: buffer keeps its content
-    const int q = cj[k] * S + ci[k];
-    o0[q] = r0[k];
-    if (o1) o1[q] = r1[k];
+  for (int k = 0; k < K; ++k) {
+    const int i = g.c0 + 64 * k + lane;
+    const uint32_t q = (uint32_t)(g.j * S + i);
+    const bool in = 64 * k + lane < g.n, keep = i > tr;
+    if constexpr (DENSITY) {
+      if (in && !keep) stg(o0, q, r0[k]);
+      else if (in && (i == 1 || i == d.N || g.j == 1 || g.j == d.N)) r0[k] = o0[q];
+    } else {
+      if (in && c[k] == R_INTERIOR) {
+        if (!keep) {
+          stg(o0, q, r0[k]);
+          stg(o1, q, r1[k]);
+        }
+      } else if (in) {
+        put_ruled(d, c[k], i, g.j, o0, o1, r0[k], r1[k], keep);
+      }
+    }
   }
+  if constexpr (DENSITY) put_ring_seg<K>(d, g, lane, o0, r0, true);
 }
-
-// set_boundaries as lists (built from the mask on the device): entry e of a
-// scene's mode0 list then of its mode1 list (role1 ROLE_NONE: none); bstart =
-// prefix of the scenes' entry counts for this (mode0, mode1).
-__global__ void k_bnd(const RbScene* __restrict__ scs, const int* __restrict__ bstart, int nsc, int mode0,
-                      int role0, int mode1, int role1) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= bstart[nsc]) return;
-  const int js = find_scene(bstart, nsc, e);
-  const RbScene& sc = scs[js];
+template <bool DENSITY, int K>
+__device__ __forceinline__ void adv_row(const SceneDesc& d, const Seg& g, int lane, const AdvArgs<DENSITY>& a) {
+  float uu[K], vv[K];
+  seg_load<K>(d, g, lane, a.u, a.v, uu, vv);
+  seg_gather<DENSITY, K>(d, g, lane, seg_break<K>(d, g, lane, uu, vv), a, uu, vv);
+}
+template <bool DENSITY, int NW>
+__global__ void __launch_bounds__(64 * NW) k_adv(const RbScene* __restrict__ scs, const int4* __restrict__ amap,
+                                                 int o0_role, int i0_role, int o1_role, int i1_role, int u_role,
+                                                 int v_role) {
+  __shared__ int brk;
+  const int4 at = amap[blockIdx.x];
+  const RbScene& sc = scs[at.x];
   const SceneDesc& d = sc.d;
-  const int off[3] = {0, d.nbnd[0], d.nbnd[0] + d.nbnd[1]};
-  const int k = e - bstart[js];
-  const bool first = k < d.nbnd[mode0];
-  const int mode = first ? mode0 : mode1;
-  float* x = role_ptr(sc, first ? role0 : role1);
-  const int2 p = d.bnd[off[mode] + (first ? k : k - d.nbnd[mode0])];
-  x[p.x] = (mode == M_PASSIVE ? 1.0f : -1.0f) * x[p.y];
-}
-
-// set_boundaries corners (fluid.rs:265-271): one thread per scene and field;
-// `diffused`: only scenes whose diffusion has sweeps.
-__global__ void k_corners(const RbScene* __restrict__ scs, int nsc, int role0, int role1, int diffused) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  const int js = t >> 1;
-  const int role = (t & 1) ? role1 : role0;
-  if (js >= nsc || role == ROLE_NONE) return;
-  const RbScene& sc = scs[js];
-  if (diffused && sc.d.diff_iters <= 0) return;
-  const int S = sc.d.S;
-  float* x = role_ptr(sc, role);
-  x[0] = 0.5f * (x[1] + x[S]);
-  x[(S - 1) * S] = 0.5f * (x[1 + (S - 1) * S] + x[(S - 2) * S]);
-  x[S - 1] = 0.5f * (x[S - 2] + x[S - 1 + S]);
-  x[S * S - 1] = 0.5f * (x[S - 2 + (S - 1) * S] + x[S - 1 + (S - 2) * S]);
+  const int N = d.N, lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  AdvArgs<DENSITY> a;
+  a.d0 = role_ptr(sc, i0_role);
+  a.d1 = DENSITY ? nullptr : role_ptr(sc, i1_role);
+  a.u = role_ptr(sc, u_role);
+  a.v = role_ptr(sc, v_role);
+  a.o0 = role_ptr(sc, o0_role);
+  a.o1 = DENSITY ? nullptr : role_ptr(sc, o1_role);
+  if (N <= SEG) {  // a row per wave
+    const Seg g{at.y + w, 1, at.y + w <= N ? N : 0};
+    if (g.n > 192) adv_row<DENSITY, 4>(d, g, lane, a);
+    else if (g.n > 128) adv_row<DENSITY, 3>(d, g, lane, a);
+    else if (g.n > 64) adv_row<DENSITY, 2>(d, g, lane, a);
+    else if (g.n > 0) adv_row<DENSITY, 1>(d, g, lane, a);
+    return;
+  }
+  if (threadIdx.x == 0) brk = N + 1;
+  __syncthreads();
+  constexpr int STEP = SEG * NW;
+  float uu[SEG_K], vv[SEG_K];
+  for (int c0 = 1 + w * SEG; c0 <= N; c0 += STEP) {
+    const Seg g{at.y, c0, min(SEG, N + 1 - c0)};
+    seg_load<SEG_K>(d, g, lane, a.u, a.v, uu, vv);
+    const int tr = seg_break<SEG_K>(d, g, lane, uu, vv);
+    if (tr <= N && lane == 0) atomicMin(&brk, tr);
+  }
+  __syncthreads();
+  const int tr = __builtin_amdgcn_readfirstlane(brk);
+  for (int c0 = 1 + w * SEG; c0 <= N; c0 += STEP) {
+    const Seg g{at.y, c0, min(SEG, N + 1 - c0)};
+    if (N > STEP) seg_load<SEG_K>(d, g, lane, a.u, a.v, uu, vv);
+    if (g.n > 192) {
+      seg_gather<DENSITY, SEG_K>(d, g, lane, tr, a, uu, vv);
+    } else {
+      float u1[3] = {uu[0], uu[1], uu[2]}, v1[3] = {vv[0], vv[1], vv[2]};
+      if (g.n > 128) {
+        seg_gather<DENSITY, 3>(d, g, lane, tr, a, u1, v1);
+      } else {
+        float u2[2] = {uu[0], uu[1]}, v2[2] = {vv[0], vv[1]}, u3[1] = {uu[0]}, v3[1] = {vv[0]};
+        if (g.n > 64) seg_gather<DENSITY, 2>(d, g, lane, tr, a, u2, v2);
+        else seg_gather<DENSITY, 1>(d, g, lane, tr, a, u3, v3);
+      }
+    }
+  }
 }
 
 // Frame sources (only the fields that were set; adding 0 would turn -0 into
@@ -725,9 +854,10 @@ struct RbGroup {
   size_t tab_bytes = 0;
   std::vector<char> h_tab;  // host image of the tables
   RbScene* d_scs = nullptr;
-  // work unit -> {scene, index in it}: band tiles, interior cell blocks, cell blocks
-  int2 *d_tmap = nullptr, *d_imap = nullptr, *d_cmap = nullptr;
-  int *d_bpp = nullptr, *d_brc = nullptr, *d_bp = nullptr;  // prefixes of list entries
+  // work unit -> {scene, index in it}: band tiles, cell blocks; -> {scene, row,
+  // segment, segments per row}: segments of rows, rows
+  int2 *d_tmap = nullptr, *d_cmap = nullptr;
+  int4 *d_imap = nullptr, *d_amap = nullptr;
   // exact mode: strips of the three diffusions and of a pressure solve, in
   // ticket order; counters; hand-off values; where a wait reports that it gave up
   bool exact = false;
@@ -736,11 +866,10 @@ struct RbGroup {
   void* d_lex = nullptr;
   size_t lex_bytes = 0;
   uint32_t* h_err = nullptr;
-  int n = 0, maxN = 0, tiles = 0, iblocks = 0, cblocks = 0, bpp = 0, brc = 0, bp = 0;
+  int n = 0, maxN = 0, tiles = 0, iblocks = 0, cblocks = 0, ablocks = 0;
   bool any_src = false;
   int diff_iters = 0, press_iters = 0;  // red-black: the same for every scene
   int diff_rounds = 0, press_rounds = 0;  // exact: the most of any scene
-  bool any_diff = false;
   int tile = 5, tsweeps = 5;  // band shape index (kBands) and sweeps per launch (untuned default)
   int tab_tile = -1, tab_T = -1;
   hipGraphExec_t graph = nullptr;
@@ -750,7 +879,6 @@ struct RbGroup {
 
 struct FrameWork {
   float* tmp = nullptr;  // ping-pong field
-  int* trig = nullptr;   // per-row break columns
   RbGroup one;           // the scene alone (eqf_step)
 };
 
@@ -760,6 +888,9 @@ struct BandCfg {
   int nw, r;
 };
 static const BandCfg kBands[] = {{8, 16}, {8, 32}, {16, 16}, {8, 18}, {8, 14}, {8, 10}};
+
+// Waves per workgroup of the advection: enough for a row of the largest scene.
+static int adv_waves(int maxN) { return maxN > 8 * rb::SEG ? 16 : maxN > 4 * rb::SEG ? 8 : 4; }
 
 static int band_tiles(int S, int tile, int T) {
   const BandCfg b = kBands[tile];
@@ -816,22 +947,21 @@ static void lex_order(std::vector<LexTask>& v, const std::vector<eqf_scene*>& sc
 static int group_tables(RbGroup& g, hipStream_t st, std::string& err) {
   const int n = (int)g.scenes.size();
   std::vector<RbScene> scs(n);
-  std::vector<int2> tmap, imap, cmap;
+  std::vector<int2> tmap, cmap;
+  std::vector<int4> imap, amap;
   std::vector<LexTask> ldiff, lpress;
   int64_t hd = 0, hp = 0;
   int fd = 0, fp = 0;
-  std::vector<int> bpp(n + 1, 0), brc(n + 1, 0), bp(n + 1, 0);
   g.any_src = false;
   g.maxN = 0;
+  for (const eqf_scene* s : g.scenes) g.maxN = std::max(g.maxN, s->N);
   g.diff_rounds = g.press_rounds = 0;
-  g.any_diff = false;
   for (int i = 0; i < n; ++i) {
     eqf_scene* s = g.scenes[i];
     auto* w = static_cast<FrameWork*>(s->work);
-    scs[i] = RbScene{s->desc, w->tmp, w->trig};
+    scs[i] = RbScene{s->desc, w->tmp};
     g.diff_rounds = std::max(g.diff_rounds, lex_rounds(s->desc.diff_iters));
     g.press_rounds = std::max(g.press_rounds, lex_rounds(s->desc.press_iters));
-    g.any_diff = g.any_diff || s->desc.diff_iters > 0;
     if (g.exact) {
       lex_tasks(i, s->S, s->desc.diff_iters, 3, ldiff, fd, hd);
       lex_tasks(i, s->S, s->desc.press_iters, 1, lpress, fp, hp);
@@ -839,17 +969,15 @@ static int group_tables(RbGroup& g, hipStream_t st, std::string& err) {
       const int nt = band_tiles(s->S, g.tile, g.tsweeps);
       for (int t = 0; t < nt; ++t) tmap.push_back(make_int2(i, t));
     }
-    const int64_t ni = ((int64_t)s->N * s->N + rb::CELL_BLOCK - 1) / rb::CELL_BLOCK;
-    for (int64_t k = 0; k < ni; ++k) imap.push_back(make_int2(i, (int)k));
+    const int nseg = (s->N + rb::SEG - 1) / rb::SEG;
+    for (int64_t k = 0; k < (int64_t)s->N * nseg; k += 4)
+      imap.push_back(make_int4(i, 1 + (int)(k / nseg), (int)(k % nseg), nseg));
     const int64_t nb = ((int64_t)s->S * s->S + rb::CELL_BLOCK - 1) / rb::CELL_BLOCK;
     for (int64_t k = 0; k < nb; ++k) cmap.push_back(make_int2(i, (int)k));
-    bpp[i + 1] = bpp[i] + 2 * s->nbnd[M_PASSIVE];
-    brc[i + 1] = brc[i] + s->nbnd[M_ROW] + s->nbnd[M_COL];
-    bp[i + 1] = bp[i] + s->nbnd[M_PASSIVE];
+    for (int j = 1; j <= s->N; j += nseg > 1 ? 1 : adv_waves(g.maxN)) amap.push_back(make_int4(i, j, 0, nseg));
     g.any_src = g.any_src || s->desc.has_src;
-    g.maxN = std::max(g.maxN, s->N);
   }
-  if (tmap.size() > INT32_MAX / 2 || cmap.size() > INT32_MAX / 2) {  // imap < cmap
+  if (tmap.size() > INT32_MAX / 2 || cmap.size() > INT32_MAX / 2 || imap.size() > INT32_MAX / 2) {  // amap <= imap * 4
     err = "launch group too large for one launch";
     return EQF_EINVAL;
   }
@@ -857,17 +985,16 @@ static int group_tables(RbGroup& g, hipStream_t st, std::string& err) {
   g.tiles = (int)tmap.size();
   g.iblocks = (int)imap.size();
   g.cblocks = (int)cmap.size();
-  g.bpp = bpp[n];
-  g.brc = brc[n];
-  g.bp = bp[n];
+  g.ablocks = (int)amap.size();
   auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
-  const size_t b_scs = up(sizeof(RbScene) * n), b_i = up(sizeof(int) * (n + 1));
+  const size_t b_scs = up(sizeof(RbScene) * n);
   const size_t b_t = up(sizeof(int2) * tmap.size());
-  const size_t b_m = up(sizeof(int2) * imap.size()), b_c = up(sizeof(int2) * cmap.size());
+  const size_t b_m = up(sizeof(int4) * imap.size()), b_c = up(sizeof(int2) * cmap.size());
+  const size_t b_a = up(sizeof(int4) * amap.size());
   lex_order(ldiff, g.scenes);
   lex_order(lpress, g.scenes);
   const size_t b_ld = up(sizeof(LexTask) * ldiff.size()), b_lp = up(sizeof(LexTask) * lpress.size());
-  const size_t bytes = b_scs + 3 * b_i + b_t + b_m + b_c + b_ld + b_lp;
+  const size_t bytes = b_scs + b_t + b_m + b_c + b_a + b_ld + b_lp;
   if (bytes > g.tab_bytes) {  // with headroom: a server's group changes size often
     (void)hipFree(g.d_tab);
     g.d_tab = nullptr;
@@ -890,22 +1017,18 @@ static int group_tables(RbGroup& g, hipStream_t st, std::string& err) {
     return at;
   };
   const size_t o_scs = put(scs.data(), sizeof(RbScene) * n, b_scs);
-  const size_t o_bpp = put(bpp.data(), sizeof(int) * (n + 1), b_i);
-  const size_t o_brc = put(brc.data(), sizeof(int) * (n + 1), b_i);
-  const size_t o_bp = put(bp.data(), sizeof(int) * (n + 1), b_i);
   const size_t o_t = put(tmap.data(), sizeof(int2) * tmap.size(), b_t);
-  const size_t o_m = put(imap.data(), sizeof(int2) * imap.size(), b_m);
+  const size_t o_m = put(imap.data(), sizeof(int4) * imap.size(), b_m);
   const size_t o_c = put(cmap.data(), sizeof(int2) * cmap.size(), b_c);
+  const size_t o_a = put(amap.data(), sizeof(int4) * amap.size(), b_a);
   const size_t o_ld = put(ldiff.data(), sizeof(LexTask) * ldiff.size(), b_ld);
   const size_t o_lp = put(lpress.data(), sizeof(LexTask) * lpress.size(), b_lp);
   char* d = (char*)g.d_tab;
   g.d_scs = (RbScene*)(d + o_scs);
-  g.d_bpp = (int*)(d + o_bpp);
-  g.d_brc = (int*)(d + o_brc);
-  g.d_bp = (int*)(d + o_bp);
   g.d_tmap = (int2*)(d + o_t);
-  g.d_imap = (int2*)(d + o_m);
+  g.d_imap = (int4*)(d + o_m);
   g.d_cmap = (int2*)(d + o_c);
+  g.d_amap = (int4*)(d + o_a);
   g.d_ldiff = (LexTask*)(d + o_ld);
   g.d_lpress = (LexTask*)(d + o_lp);
   g.n_ldiff = (int)ldiff.size();
@@ -999,11 +1122,6 @@ static void g_lin_solve(hipStream_t st, const RbGroup& g, int mode, int x, int x
   }
   if (a_ != x) g_copy(st, g, x, a_);
 }
-static void g_corners(hipStream_t st, const RbGroup& g, int c0, int c1, int diffused) {
-  hipLaunchKernelGGL(rb::k_corners, dim3((unsigned)((2 * g.n + 255) / 256)), dim3(256), 0, st, g.d_scs, g.n, c0, c1,
-                     diffused);
-}
-
 // Lexicographic lin_solves: the three diffusions of a frame in one launch per
 // round (they read and write different fields: u and v from the last frame's
 // velocity, density from the last frame's density), or a pressure solve.
@@ -1022,15 +1140,13 @@ static void g_pressure(hipStream_t st, const RbGroup& g, int p, int div) {
   else g_lin_solve(st, g, M_PASSIVE, p, div, 2, g.press_iters);
 }
 
-// set_boundaries lists of one or two fields, then the corners of the fields
-// c0 and c1 (ROLE_NONE: none).
-static void g_bnd(hipStream_t st, const RbGroup& g, int mode0, int x0, int mode1, int x1, int c0, int c1) {
-  const int* tab = x1 == rb::ROLE_NONE ? g.d_bp : mode0 == M_PASSIVE ? g.d_bpp : g.d_brc;
-  const int total = x1 == rb::ROLE_NONE ? g.bp : mode0 == M_PASSIVE ? g.bpp : g.brc;
-  if (total > 0)
-    hipLaunchKernelGGL(rb::k_bnd, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, g.d_scs, tab, g.n, mode0,
-                       x0, mode1, x1);
-  if (c0 != rb::ROLE_NONE || c1 != rb::ROLE_NONE) g_corners(st, g, c0, c1, 0);
+template <bool DENSITY>
+static void g_adv(hipStream_t st, const RbGroup& g, int o0, int i0, int o1, int i1, int u, int v) {
+  const dim3 rows((unsigned)g.ablocks);
+  const int nw = adv_waves(g.maxN);
+  if (nw == 4) hipLaunchKernelGGL((rb::k_adv<DENSITY, 4>), rows, dim3(256), 0, st, g.d_scs, g.d_amap, o0, i0, o1, i1, u, v);
+  else if (nw == 8) hipLaunchKernelGGL((rb::k_adv<DENSITY, 8>), rows, dim3(512), 0, st, g.d_scs, g.d_amap, o0, i0, o1, i1, u, v);
+  else hipLaunchKernelGGL((rb::k_adv<DENSITY, 16>), rows, dim3(1024), 0, st, g.d_scs, g.d_amap, o0, i0, o1, i1, u, v);
 }
 
 // One frame (fluid.rs:437-524) of every scene of the group.  All scenes share
@@ -1040,10 +1156,9 @@ static void g_bnd(hipStream_t st, const RbGroup& g, int mode0, int x0, int mode1
 // are part of the frame's final state; no sweep, divergence or gradient reads
 // them.  So a field's corners are computed only where a gather or the end of
 // the frame reads them before the field's next set_boundaries rewrites them:
-// U0 and V0 after the first gradient (advected from), V0 after the second
-// divergence, U0 after the second pressure solve (or after that divergence
-// when the solve has no sweeps), U and V after the second gradient, the
-// density scratch after its diffusion, the density after its advection.
+// U0 and V0 with the first gradient (advected from), V0 with the second
+// divergence, U0 and the density scratch with the second gradient (their solves
+// are done), U and V too, the density with its advection.
 static void g_frame(hipStream_t st, const RbGroup& g) {
   using rb::ROLE_NONE;
   const dim3 cells((unsigned)g.iblocks);  // interior cell blocks
@@ -1056,29 +1171,18 @@ static void g_frame(hipStream_t st, const RbGroup& g) {
     g_lin_solve(st, g, M_COL, F_V0, F_V, 0, g.diff_iters);  // fluid.rs:448
   }
   // project(U0, V0, p=U, div=V), fluid.rs:459
-  hipLaunchKernelGGL(rb::k_div, cells, dim3(256), 0, st, g.d_scs, g.d_imap, F_U0, F_V0, F_V, F_U);
-  g_bnd(st, g, M_PASSIVE, F_V, M_PASSIVE, F_U, ROLE_NONE, ROLE_NONE);
+  hipLaunchKernelGGL(rb::k_div, cells, dim3(256), 0, st, g.d_scs, g.d_imap, F_U0, F_V0, F_V, F_U, 0);
   g_pressure(st, g, F_U, F_V);
-  hipLaunchKernelGGL(rb::k_grad, cells, dim3(256), 0, st, g.d_scs, g.d_imap, F_U0, F_V0, F_U);
-  g_bnd(st, g, M_ROW, F_U0, M_COL, F_V0, F_U0, F_V0);
+  hipLaunchKernelGGL(rb::k_grad, cells, dim3(256), 0, st, g.d_scs, g.d_imap, F_U0, F_V0, F_U, 0, ROLE_NONE);
   // advect U from U0 and V from V0 with (U0, V0), fluid.rs:469-489
-  hipLaunchKernelGGL(rb::k_adv_trig, cells, dim3(256), 0, st, g.d_scs, g.d_imap, F_U0, F_V0);
-  hipLaunchKernelGGL(rb::k_adv, cells, dim3(256), 0, st, g.d_scs, g.d_imap, F_U, F_U0, F_V, F_V0, F_U0, F_V0);
-  g_bnd(st, g, M_ROW, F_U, M_COL, F_V, ROLE_NONE, ROLE_NONE);
+  g_adv<false>(st, g, F_U, F_U0, F_V, F_V0, F_U0, F_V0);
   // project(U, V, p=U0, div=V0), fluid.rs:491
-  hipLaunchKernelGGL(rb::k_div, cells, dim3(256), 0, st, g.d_scs, g.d_imap, F_U, F_V, F_V0, F_U0);
-  g_bnd(st, g, M_PASSIVE, F_V0, M_PASSIVE, F_U0, F_V0, ROLE_NONE);
+  hipLaunchKernelGGL(rb::k_div, cells, dim3(256), 0, st, g.d_scs, g.d_imap, F_U, F_V, F_V0, F_U0, 1);
   g_pressure(st, g, F_U0, F_V0);
-  g_corners(st, g, F_U0, ROLE_NONE, 0);
-  hipLaunchKernelGGL(rb::k_grad, cells, dim3(256), 0, st, g.d_scs, g.d_imap, F_U, F_V, F_U0);
-  g_bnd(st, g, M_ROW, F_U, M_COL, F_V, F_U, F_V);
-  // density, fluid.rs:501-523
-  if (!g.exact) g_lin_solve(st, g, M_PASSIVE, F_SC, F_D, 1, g.diff_iters);
-  if (g.any_diff) g_corners(st, g, F_SC, ROLE_NONE, 1);
-  hipLaunchKernelGGL(rb::k_adv_trig, cells, dim3(256), 0, st, g.d_scs, g.d_imap, F_U, F_V);
-  hipLaunchKernelGGL(rb::k_adv, cells, dim3(256), 0, st, g.d_scs, g.d_imap, F_D, F_SC, ROLE_NONE, ROLE_NONE,
-                     F_U, F_V);
-  g_bnd(st, g, M_PASSIVE, F_D, M_PASSIVE, ROLE_NONE, F_D, ROLE_NONE);
+  if (!g.exact) g_lin_solve(st, g, M_PASSIVE, F_SC, F_D, 1, g.diff_iters);  // density, fluid.rs:501
+  hipLaunchKernelGGL(rb::k_grad, cells, dim3(256), 0, st, g.d_scs, g.d_imap, F_U, F_V, F_U0, 1, F_SC);
+  // fluid.rs:511-523
+  g_adv<true>(st, g, F_D, F_SC, ROLE_NONE, ROLE_NONE, F_U, F_V);
   g_copy(st, g, F_SC, F_D);
 }
 
@@ -1121,7 +1225,7 @@ static int group_capture(RbGroup& g, hipStream_t st, std::string& err) {
 }
 
 // Advances every scene of the group by nframes on `st`.  The tables are
-// rebuilt when the scenes' parameters, lists or the tiling change.  The first
+// rebuilt when the scenes' parameters or the tiling change.  The first
 // frame after that is launched kernel by kernel; further ones replay a graph
 // captured once (a server's groups change membership often, and one frame's
 // launches cost less than a capture).
@@ -1176,11 +1280,9 @@ void* frame_create(eqf_scene* s, std::string& err) {
   const size_t n = (size_t)s->S * s->S;
   hipError_t e = hipSuccess;
   if (s->p.gs_mode == EQF_GS_REDBLACK) e = eqf_scene_malloc(s, (void**)&w->tmp, sizeof(float) * n);
-  if (e == hipSuccess) e = eqf_scene_malloc(s, (void**)&w->trig, sizeof(int) * (size_t)s->S);
   if (e != hipSuccess) {
     err = std::string("frame workspace: ") + hipGetErrorString(e);
     eqf_scene_mfree(s, w->tmp);
-    eqf_scene_mfree(s, w->trig);
     delete w;
     return nullptr;
   }
@@ -1195,7 +1297,6 @@ void frame_destroy(eqf_scene* s) {
   if (!w) return;
   group_release(w->one);
   eqf_scene_mfree(s, w->tmp);
-  eqf_scene_mfree(s, w->trig);
   delete w;
   s->work = nullptr;
 }

@@ -58,9 +58,7 @@ struct eqf_scene {
   int src_mask = 0;           // frame sources set: bit 0 density, 1 vx, 2 vy
   uint8_t* d_code = nullptr;
   uint8_t* d_rowf = nullptr;
-  int2* d_bnd = nullptr;
-  size_t bnd_cap = 0;
-  int nbnd[3] = {0, 0, 0};
+  int ring_copies = 0;        // Passive ring cells that copy their neighbour
   void* d_main = nullptr;     // one allocation: pad, fields, rule bytes, rowf
   float* d_stage = nullptr;   // staging for eqf_add_source (lazy)
   uint8_t* d_mask = nullptr;  // mask + scratch for the boundary build (lazy)
@@ -88,7 +86,7 @@ hipError_t eqf_scene_malloc(eqf_scene* s, void** p, size_t bytes);
 void eqf_scene_mfree(eqf_scene* s, void* p);
 
 // Runtime services shared with the server (eqf_runtime.hip).
-int eqf_internal_prepare(eqf_scene* s);  // boundary lists + descriptor
+int eqf_internal_prepare(eqf_scene* s);  // boundary rules + descriptor
 int eqf_internal_error(int code, const std::string& msg);
 // Device address of eqf_render_rgba_noalloc's fixed scratch on `device`
 // (eqf_render.hip), looked up once per device at context creation.
@@ -116,9 +114,8 @@ namespace eqf {
 // One scene of a launch group: a single scene, or every scene of a batch.
 // Each frame kernel covers all scenes of its group in one launch.
 struct RbScene {
-  SceneDesc d;  // the scene's descriptor (a copy): fields, sizes, coefficients, rule bytes, lists
+  SceneDesc d;  // the scene's descriptor (a copy): fields, sizes, coefficients, rule bytes
   float* tmp;   // its ping-pong field (red-black mode)
-  int* trig;    // its per-row break columns
 };
 
 // Lexicographic lin_solve (eqf_lex.hip).  A launch covers up to three

@@ -24,6 +24,7 @@ enum Mode { M_ROW = 0, M_COL = 1, M_PASSIVE = 2 };  // Orientation, fluid.rs:22-
 //   bit 0     interior cell (updated by the sweeps)
 //   bits 1-2  AdjustRow: 0 keep, 1 -(left), 2 -(right)  (right wins, fluid.rs:151-164)
 //   bits 3-4  AdjustColumn: 0 keep, 1 -(up), 2 -(down)  (up wins, fluid.rs:165-177)
+//             (either: 3 an interior wall cell, kept, that a fluid cell takes its value from)
 //   bits 5-7  Passive, ring cells whose row / column holds a NoWall cell
 //             (fluid.rs:179-187): 0 none, 1 copy the left, 2 the right, 3 the
 //             upper, 4 the lower neighbour
@@ -34,6 +35,7 @@ enum RuleBits : uint32_t {
   R_INTERIOR = 1u,
   R_ROW_SHIFT = 1, R_COL_SHIFT = 3, R_PAS_SHIFT = 5,
   R_NEG_FIRST = 1u, R_NEG_SECOND = 2u,  // left / up, right / down
+  R_SOURCE = 3u,
   R_COPY_LEFT = 1u, R_COPY_RIGHT = 2u, R_COPY_UP = 3u, R_COPY_DOWN = 4u,
 };
 
@@ -41,10 +43,9 @@ struct SceneDesc {
   float* fld;            // NFIELDS fields, `fstride` floats apart
   const float* src;      // per-frame sources (density, vx, vy) or nullptr
   const uint8_t* code;   // RuleBits at x + y*rm_code_stride(S), then the transposed array
-  const int2* bnd;       // (dst, src) field offsets: ROW list, COL list, PASSIVE list
   int64_t fstride;       // floats per field
   int S, N;              // size, interior size
-  int nbnd[3];           // list lengths per mode
+  int ring_copies;       // Passive ring cells that copy their neighbour (4 N: all but the corners)
   int diff_iters, press_iters;
   float a_visc, cr_visc; // diffuse coefficients for velocity (fluid.rs:286-294, 311)
   float a_diff, cr_diff; // diffuse coefficients for density

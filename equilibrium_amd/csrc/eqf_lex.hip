@@ -145,7 +145,7 @@ __device__ __forceinline__ void agent_store(T* p, T v) {
 }
 
 // Selector of a cell in LDS: 0 a plain cell; ROW / COL (logical): 1 -(left),
-// 2 -(right), 4 ring (keeps its value); PASSIVE ring: 8 keeps its value, 9
+// 2 -(right), 3 a plain one too, 4 ring (keeps its value); PASSIVE ring: 8 keeps its value, 9
 // copies the left, 10 the right, 11 the upper, 12 the lower neighbour.
 template <int MODE>
 __device__ __forceinline__ uint32_t selectors(uint32_t c) {  // four rule bytes -> four selectors
@@ -452,7 +452,7 @@ __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, const LexTa
     elo[z] = on ? pt.mlo : 1;
     ehi[z] = on ? pt.mhi : 0;
   }
-  const bool ring_copies = MODE == M_PASSIVE && d.nbnd[M_PASSIVE] == 4 * d.N;  // every ring cell copies its neighbour
+  const bool ring_copies = MODE == M_PASSIVE && d.ring_copies == 4 * d.N;  // every ring cell copies its neighbour
   const int hf = (lane & 1) * 4;  // the item's first row of the block's eight
   if (w == W) {  // x0
     const rsrc_t rx0 = make_rsrc(x0 - FLD_PAD, fbytes);
@@ -553,11 +553,11 @@ __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, const LexTa
           lu* cq = (lu*)L + (L_CODE + (row >> 2) * CP) + (hf >> 2) * CP + ((64 * z + lane) >> 1);
           cq[0] = sel;
           if (row == 0) cq[CR * CP] = sel;
-          any |= sel;
+          any |= MODE == M_PASSIVE ? sel : sel ^ (sel >> 1);  // (3 keeps its value)
           const int c = cc[z] + ub * B;
           cols = cols || (uint32_t)(c + 3) <= 3u || (uint32_t)(S - 1 - c) <= 3u;
         }
-      const bool rules = MODE == M_PASSIVE ? !ring_copies && any != 0 : (any & 0x03030303u) != 0;
+      const bool rules = MODE == M_PASSIVE ? !ring_copies && any != 0 : (any & 0x01010101u) != 0;
       h_rule = (h_rule << 1) | (__builtin_amdgcn_ballot_w64(rules) != 0 ? 1u : 0u);
       h_col = (h_col << 1) | (__builtin_amdgcn_ballot_w64(cols) != 0 ? 1u : 0u);
     };

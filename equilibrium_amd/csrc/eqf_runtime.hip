@@ -2,7 +2,7 @@
 //
 // Scene state lives on the device.  The host keeps only the parameters and the
 // obstacle mask (static during a run, fluid.rs:610-619), from which it derives
-// the per-cell boundary codes and the set_boundaries lists the kernels use.
+// the per-cell boundary codes the kernels use.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -110,8 +110,7 @@ static void host_init(int S, int times, std::vector<std::vector<float>>& F, std:
   }
 }
 
-// Boundary codes and set_boundaries lists derived from the mask (built on
-// the device from the host copy of the mask).
+// Boundary codes derived from the mask (built on the device from the host copy of the mask).
 static int rebuild_bnd(eqf_scene* s) { return eqf_dev_rebuild_bnd(s); }
 
 static void fill_desc(eqf_scene* s) {
@@ -120,11 +119,10 @@ static void fill_desc(eqf_scene* s) {
   d.fld = s->d_fld;
   d.src = s->d_src;
   d.code = s->d_code;
-  d.bnd = s->d_bnd;
   d.fstride = s->fstride;
   d.S = s->S;
   d.N = s->N;
-  for (int i = 0; i < 3; ++i) d.nbnd[i] = s->nbnd[i];
+  d.ring_copies = s->ring_copies;
   d.diff_iters = (int)resolved_gs(p);
   d.press_iters = (int)resolved_press(p);
   // diffuse (fluid.rs:286-294) and lin_solve's c_recip (fluid.rs:311), in f32
@@ -235,7 +233,6 @@ static void scene_free(eqf_scene* s) {
   if (s->ev_ops) (void)hipEventDestroy(s->ev_ops);
   eqf_scene_mfree(s, s->d_main);
   eqf_scene_mfree(s, s->d_src);
-  eqf_scene_mfree(s, s->d_bnd);
   eqf_scene_mfree(s, s->d_stage);
   eqf_scene_mfree(s, s->d_mask);
   if (s->stream && s->owns_stream) (void)hipStreamDestroy(s->stream);

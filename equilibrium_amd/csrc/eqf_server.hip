@@ -124,8 +124,8 @@ struct eqf_server {
 // Device bytes of a scene of this size and mode with frame sources.
 static uint64_t estimate_bytes(const eqf_params& p) {
   const int S = (int)p.size, N = S - 2;
-  // fields + sources, rule bytes, row flags, break columns, lists, and the
-  // ping-pong field (red-black) or the lin_solve hand-off (exact)
+  // fields + sources, rule bytes, row flags, tables, and the ping-pong field
+  // (red-black) or the lin_solve hand-off (exact)
   const uint64_t fs = (uint64_t)rm_field_floats(S), cells = (uint64_t)S * S;
   const uint64_t work = p.gs_mode == EQF_GS_REDBLACK ? cells * 4 : (uint64_t)lex_workspace_bytes(S);
   return (NFIELDS + 3) * fs * 4 + 2 * (uint64_t)rm_code_bytes(S) + work + (uint64_t)S * 5 + (uint64_t)N * 96 + 8192;

@@ -1,5 +1,5 @@
 // eqf_setup.hip -- device-side scene setup: initial state, uploads, downloads
-// and adds of whole fields, and the boundary rules / lists derived from the obstacle mask.  Keeping these on the device makes
+// and adds of whole fields, and the boundary rules derived from the obstacle mask.  Keeping these on the device makes
 // admitting a scene cost a few small launches instead of host loops over
 // every cell, which matters when the server admits hundreds of scenes/s.
 #include <hip/hip_runtime.h>
@@ -82,13 +82,11 @@ __global__ void k_rowcol_bytes(int S, const uint32_t* __restrict__ rowf32, const
   colf[k] = colf32[k] != 0;
 }
 
-// Per-cell rule bytes (eqf_layout.h RuleBits) and the set_boundaries
-// lists: AdjustRow (right wall wins over left, fluid.rs:151-164),
-// AdjustColumn (up wins over down, fluid.rs:165-177), Passive ring copies.
-// fill == 0 only counts entries.
+// Per-cell rule bytes (eqf_layout.h RuleBits): AdjustRow (right wall wins over
+// left, fluid.rs:151-164), AdjustColumn (up wins over down, fluid.rs:165-177),
+// Passive ring copies (counted).
 __global__ void k_codes(Geo g, const uint8_t* __restrict__ m, const uint8_t* __restrict__ rowf,
-                        const uint8_t* __restrict__ colf, uint8_t* __restrict__ code, int* __restrict__ cnt,
-                        int2* __restrict__ lrow, int2* __restrict__ lcol, int2* __restrict__ lpas, int fill) {
+                        const uint8_t* __restrict__ colf, uint8_t* __restrict__ code, int* __restrict__ copies) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int S = g.S, N = g.N;
   if (e >= (int64_t)S * S) return;
@@ -99,43 +97,19 @@ __global__ void k_codes(Geo g, const uint8_t* __restrict__ m, const uint8_t* __r
     code[rm_code_bytes(S) + (int64_t)i * rm_code_stride(S) + j] = (uint8_t)r;
   };
   if (x >= 1 && x <= N && y >= 1 && y <= N) {
-    const bool fl = !wall(x, y);
-    if (fill) {
-      uint32_t r = R_INTERIOR;
-      if (fl) {
-        r |= (wall(x + 1, y) ? R_NEG_SECOND : wall(x - 1, y) ? R_NEG_FIRST : 0u) << R_ROW_SHIFT;
-        r |= (wall(x, y - 1) ? R_NEG_FIRST : wall(x, y + 1) ? R_NEG_SECOND : 0u) << R_COL_SHIFT;
-      }
-      put(x, y, r);
+    uint32_t r = R_INTERIOR;
+    if (!wall(x, y)) {
+      r |= (wall(x + 1, y) ? R_NEG_SECOND : wall(x - 1, y) ? R_NEG_FIRST : 0u) << R_ROW_SHIFT;
+      r |= (wall(x, y - 1) ? R_NEG_FIRST : wall(x, y + 1) ? R_NEG_SECOND : 0u) << R_COL_SHIFT;
+    } else {
+      if (!wall(x - 1, y) || (!wall(x + 1, y) && !wall(x + 2, y))) r |= R_SOURCE << R_ROW_SHIFT;
+      if (!wall(x, y + 1) || (!wall(x, y - 1) && !wall(x, y - 2))) r |= R_SOURCE << R_COL_SHIFT;
     }
-    if (fl) {
-      int sx = -1;
-      if (wall(x + 1, y)) sx = x + 1;
-      else if (wall(x - 1, y)) sx = x - 1;
-      if (sx >= 0) {
-        const int k = atomicAdd(&cnt[0], 1);
-        if (fill) lrow[k] = make_int2((int)off_of(g, x, y), (int)off_of(g, sx, y));
-      }
-      int sy = -1;
-      if (wall(x, y - 1)) sy = y - 1;
-      else if (wall(x, y + 1)) sy = y + 1;
-      if (sy >= 0) {
-        const int k = atomicAdd(&cnt[1], 1);
-        if (fill) lcol[k] = make_int2((int)off_of(g, x, y), (int)off_of(g, x, sy));
-      }
-    }
+    put(x, y, r);
   } else if (!((x == 0 || x == S - 1) && (y == 0 || y == S - 1))) {  // non-corner ring cell
-    int sx = x, sy = y;
-    bool on = false;
-    if (y == 0) { sy = 1; on = colf[x]; }
-    else if (y == S - 1) { sy = S - 2; on = colf[x]; }
-    else if (x == 0) { sx = 1; on = rowf[y]; }
-    else { sx = S - 2; on = rowf[y]; }
-    if (on) {
-      const int k = atomicAdd(&cnt[2], 1);
-      if (fill) lpas[k] = make_int2((int)off_of(g, x, y), (int)off_of(g, sx, sy));
-      if (fill)
-        put(x, y, (y == 0 ? R_COPY_DOWN : y == S - 1 ? R_COPY_UP : x == 0 ? R_COPY_RIGHT : R_COPY_LEFT) << R_PAS_SHIFT);
+    if ((y == 0 || y == S - 1) ? colf[x] : rowf[y]) {
+      atomicAdd(copies, 1);
+      put(x, y, (y == 0 ? R_COPY_DOWN : y == S - 1 ? R_COPY_UP : x == 0 ? R_COPY_RIGHT : R_COPY_LEFT) << R_PAS_SHIFT);
     }
   }
 }
@@ -282,8 +256,8 @@ void eqf_dev_trim(eqf_scene* s) {
 }
 
 // Layout of the scene's d_mask buffer: the mask (S*S bytes), colf (S bytes),
-// then the 32-bit row/column flags (2*S) and the entry counters of the two
-// k_codes passes (3 + 3), zeroed by one memset.
+// then the 32-bit row/column flags (2*S) and k_codes' counter, zeroed by one
+// memset.
 struct MaskBuf {
   size_t colf, flags, cnt, bytes;
 };
@@ -294,7 +268,7 @@ static MaskBuf mask_buf(int S) {
   b.colf = up(n);
   b.flags = up(b.colf + (size_t)S);
   b.cnt = b.flags + 8 * (size_t)S;
-  b.bytes = b.cnt + 6 * sizeof(int);
+  b.bytes = b.cnt + sizeof(int);
   return b;
 }
 
@@ -311,40 +285,21 @@ int eqf_dev_rebuild_bnd(eqf_scene* s) {
   const Geo g = geo_of(s);
   e = hipMemcpyAsync(s->d_mask, s->mask.data(), (size_t)n, hipMemcpyHostToDevice, s->stream);
   if (e == hipSuccess) e = hipMemsetAsync(d_flags, 0, mb.bytes - mb.flags, s->stream);
+  if (e == hipSuccess) e = hipMemsetAsync(s->d_code, 0, 2 * (size_t)rm_code_bytes(S), s->stream);
   if (e == hipSuccess) {
     hipLaunchKernelGGL(k_rowcol_or, dim3((unsigned)((S + 255) / 256), (unsigned)((S + 63) / 64)), dim3(256), 0,
                        s->stream, g, s->d_mask, d_flags, d_flags + S);
     hipLaunchKernelGGL(k_rowcol_bytes, dim3(blocks_for(S)), dim3(256), 0, s->stream, S, d_flags, d_flags + S,
                        s->d_rowf, d_colf);
     hipLaunchKernelGGL(k_codes, dim3(blocks_for(n)), dim3(256), 0, s->stream, g, s->d_mask, s->d_rowf, d_colf,
-                       s->d_code, d_cnt, (int2*)nullptr, (int2*)nullptr, (int2*)nullptr, 0);
+                       s->d_code, d_cnt);
     e = hipGetLastError();
   }
-  int cnt[3] = {0, 0, 0};
-  if (e == hipSuccess) e = hipMemcpyAsync(cnt, d_cnt, sizeof(cnt), hipMemcpyDeviceToHost, s->stream);
+  int copies = 0;
+  if (e == hipSuccess) e = hipMemcpyAsync(&copies, d_cnt, sizeof(copies), hipMemcpyDeviceToHost, s->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
   if (e != hipSuccess) return eqf_internal_error(EQF_EDEVICE, std::string("boundary codes: ") + hipGetErrorString(e));
-  const size_t total = std::max<size_t>(1, (size_t)cnt[0] + cnt[1] + cnt[2]);
-  if (total > s->bnd_cap) {
-    eqf_scene_mfree(s, s->d_bnd);
-    s->d_bnd = nullptr;
-    e = eqf_scene_malloc(s, (void**)&s->d_bnd, sizeof(int2) * total);
-    if (e != hipSuccess) return eqf_internal_error(EQF_ENOMEM, std::string("boundary lists: ") + hipGetErrorString(e));
-    s->bnd_cap = total;
-  }
-  {
-    e = hipMemsetAsync(s->d_code, 0, 2 * (size_t)rm_code_bytes(S), s->stream);
-  }
-  if (e == hipSuccess) {  // the fill pass counts into the second, still zero, counters
-    hipLaunchKernelGGL(k_codes, dim3(blocks_for(n)), dim3(256), 0, s->stream, g, s->d_mask, s->d_rowf, d_colf,
-                       s->d_code, d_cnt + 3, s->d_bnd, s->d_bnd + cnt[0], s->d_bnd + cnt[0] + cnt[1], 1);
-    e = hipGetLastError();
-  }
-  if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
-  if (e != hipSuccess) return eqf_internal_error(EQF_EDEVICE, std::string("boundary lists: ") + hipGetErrorString(e));
-  s->nbnd[0] = cnt[0];
-  s->nbnd[1] = cnt[1];
-  s->nbnd[2] = cnt[2];
+  s->ring_copies = copies;
   s->bnd_dirty = false;
   return EQF_OK;
 }

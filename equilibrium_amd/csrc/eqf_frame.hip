@@ -8,14 +8,17 @@
 // first and the odd cells second, then applies set_boundaries, so all cells
 // of one colour are independent and the whole grid is updated in parallel by
 // many workgroups.  Sweeps are temporally blocked in registers (k_rb_band):
-// a workgroup loads a region (its output tile plus a halo of 3T cells on the
-// sides that face other tiles), runs T full sweeps (red, black,
+// a workgroup loads a region (its output tile plus a halo of 2T or 3T cells on
+// the sides that face other tiles, band_halo_x / _y), runs T full sweeps (red, black,
 // set_boundaries) on it, and writes the tile back, so x and x0 cross HBM once
 // per T sweeps instead of once per sweep.  Each full sweep shrinks the valid
-// region by 3 cells on every side with cells beyond it: red reads black
-// neighbours (1), black reads the new red neighbours (2), and set_boundaries
-// copies a wall neighbour (3).  A side on the grid's edge has nothing beyond
-// it, so the first and last tiles of a row or column of tiles reach the edge
+// region by 2 cells on every side with cells beyond it, red reading black
+// neighbours and black the new red ones, and by a third one in the direction in
+// which AdjustRow / AdjustColumn copy a wall neighbour.  (3 on all sides made a
+// frame of N=4096 with 40 sweeps 2.72 ms instead of 2.45, N=1501 0.460 instead
+// of 0.433: T=5 sweeps compute 1.6 to 1.9 times the output tile, not 2.1.)  A
+// side on the grid's edge has nothing beyond it, so the first and last tiles of
+// a row or column of tiles reach the edge
 // with no halo there.  A pass reads one buffer and writes another (ping-pong).
 //
 // The other phases (divergence, gradient, advection with its row `break`, each
@@ -133,6 +136,13 @@ __host__ __device__ __forceinline__ int band_span(int S, int W, int TX) {
   return S <= W ? 1 : (S - W + TX - 1) / TX + 1;
 }
 
+// Cells that T sweeps make invalid at a side of a region with cells beyond it:
+// red reads black neighbours, black the new red ones, and AdjustRow /
+// AdjustColumn a wall cell beside the cell in their direction.  (Passive only
+// writes the grid's own ring, from the cells inside it.)
+__host__ __device__ constexpr int band_halo_x(int mode, int T) { return (mode == M_ROW ? 3 : 2) * T; }
+__host__ __device__ constexpr int band_halo_y(int mode, int T) { return (mode == M_COL ? 3 : 2) * T; }
+
 // lin_solve coefficients (a, 1/c) of a scene: velocity diffusion, density
 // diffusion, pressure (fluid.rs:286-294, 311, 356).
 __device__ __forceinline__ void coefs(const SceneDesc& d, int coef, float& a, float& cr) {
@@ -148,10 +158,9 @@ __device__ __forceinline__ void coefs(const SceneDesc& d, int coef, float& a, fl
 // from the band's next register row; only the band's first and last rows
 // cross waves, through LDS (double-buffered, one barrier per exchange).
 // Red cells have (x + y) even; the region origin is chosen so that row i of
-// every band has its red cell in column (i & 1) of the lane.  Every full
-// sweep shrinks the valid region by 3 cells (red reads black, black reads the
-// new red, set_boundaries reads a neighbour) on each side that has cells
-// beyond it, so the launch stores the (128 - 6T) x (NW*R - 6T) interior of its
+// every band has its red cell in column (i & 1) of the lane.  Sweeps make cells
+// invalid from the sides that have cells beyond them (band_halo_x / _y), so the
+// launch stores the (128 - 2 HX) x (NW*R - 2 HY) interior of its
 // region, extended to the grid's edge on the sides where the region reaches
 // it (tile b of a dimension: region origin b*TX, so the first region starts
 // at the edge and the last one passes the far edge); the region reads one
@@ -161,8 +170,8 @@ template <int MODE, int T, int NW, int R>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu((NW == 8 && R <= 10) ? 8 : (NW == 8 && R <= 14) ? 6 : (NW == 8 && R <= 18) ? 4 : 1))) k_rb_band(const RbScene* __restrict__ scs, const int2* __restrict__ tmap,
                                                      int nt, int src_role, int dst_role, int x0_role, int coef,
                                                      int nsweeps) {
-  constexpr int H = 3 * T, W = 128, RH = NW * R;
-  constexpr int TX = W - 2 * H, TY = RH - 2 * H;
+  constexpr int HX = band_halo_x(MODE, T), HY = band_halo_y(MODE, T), W = 128, RH = NW * R;
+  constexpr int TX = W - 2 * HX, TY = RH - 2 * HY;
   static_assert(TX > 0 && TY > 0 && TX % 2 == 0 && TY % 2 == 0 && R % 2 == 0, "band geometry");
   // [buffer][first / last row][column of the lane's pair][wave][lane]: one
   // float per lane and store, so a wave's 64 accesses hit 64 distinct banks
@@ -388,12 +397,12 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu((N
   } while (++k < nsweeps);
 
   // (columns recomputed here rather than kept live through the sweeps)
-  // Output tile: [gx0 + H, gx0 + H + TX) x [gyb + H, gyb + H + TY), from the
+  // Output tile: [gx0 + HX, gx0 + HX + TX) x [gyb + HY, gyb + HY + TY), from the
   // grid's edge for the first tile of a dimension and to its far edge for
   // the last one.
   const int gxl = bx * TX + 2 * (int)(threadIdx.x & 63);
-  const int xlo = bx == 0 ? 0 : bx * TX + H, xhi = bx == tiles_x - 1 ? S : bx * TX + H + TX;
-  const int ylo = by == 0 ? 0 : gyb + H, yhi = by == tiles_y - 1 ? S : gyb + H + TY;
+  const int xlo = bx == 0 ? 0 : bx * TX + HX, xhi = bx == tiles_x - 1 ? S : bx * TX + HX + TX;
+  const int ylo = by == 0 ? 0 : gyb + HY, yhi = by == tiles_y - 1 ? S : gyb + HY + TY;
   bool cout[2];  // this lane's columns lie in the output tile
 #pragma unroll
   for (int b = 0; b < 2; ++b) {
@@ -856,7 +865,7 @@ struct RbGroup {
   RbScene* d_scs = nullptr;
   // work unit -> {scene, index in it}: band tiles, cell blocks; -> {scene, row,
   // segment, segments per row}: segments of rows, rows
-  int2 *d_tmap = nullptr, *d_cmap = nullptr;
+  int2 *d_tmap[3] = {nullptr, nullptr, nullptr}, *d_cmap = nullptr;
   int4 *d_imap = nullptr, *d_amap = nullptr;
   // exact mode: strips of the three diffusions and of a pressure solve, in
   // ticket order; counters; hand-off values; where a wait reports that it gave up
@@ -866,7 +875,7 @@ struct RbGroup {
   void* d_lex = nullptr;
   size_t lex_bytes = 0;
   uint32_t* h_err = nullptr;
-  int n = 0, maxN = 0, tiles = 0, iblocks = 0, cblocks = 0, ablocks = 0;
+  int n = 0, maxN = 0, tiles[3] = {0, 0, 0}, iblocks = 0, cblocks = 0, ablocks = 0;
   bool any_src = false;
   int diff_iters = 0, press_iters = 0;  // red-black: the same for every scene
   int diff_rounds = 0, press_rounds = 0;  // exact: the most of any scene
@@ -892,9 +901,9 @@ static const BandCfg kBands[] = {{8, 16}, {8, 32}, {16, 16}, {8, 18}, {8, 14}, {
 // Waves per workgroup of the advection: enough for a row of the largest scene.
 static int adv_waves(int maxN) { return maxN > 8 * rb::SEG ? 16 : maxN > 4 * rb::SEG ? 8 : 4; }
 
-static int band_tiles(int S, int tile, int T) {
+static int band_tiles(int S, int tile, int T, int mode) {
   const BandCfg b = kBands[tile];
-  const int TX = 128 - 6 * T, TY = b.nw * b.r - 6 * T;
+  const int TX = 128 - 2 * rb::band_halo_x(mode, T), TY = b.nw * b.r - 2 * rb::band_halo_y(mode, T);
   return rb::band_span(S, 128, TX) * rb::band_span(S, b.nw * b.r, TY);
 }
 
@@ -947,7 +956,7 @@ static void lex_order(std::vector<LexTask>& v, const std::vector<eqf_scene*>& sc
 static int group_tables(RbGroup& g, hipStream_t st, std::string& err) {
   const int n = (int)g.scenes.size();
   std::vector<RbScene> scs(n);
-  std::vector<int2> tmap, cmap;
+  std::vector<int2> tmap[3], cmap;
   std::vector<int4> imap, amap;
   std::vector<LexTask> ldiff, lpress;
   int64_t hd = 0, hp = 0;
@@ -966,8 +975,10 @@ static int group_tables(RbGroup& g, hipStream_t st, std::string& err) {
       lex_tasks(i, s->S, s->desc.diff_iters, 3, ldiff, fd, hd);
       lex_tasks(i, s->S, s->desc.press_iters, 1, lpress, fp, hp);
     } else {
-      const int nt = band_tiles(s->S, g.tile, g.tsweeps);
-      for (int t = 0; t < nt; ++t) tmap.push_back(make_int2(i, t));
+      for (int mode = 0; mode < 3; ++mode) {
+        const int nt = band_tiles(s->S, g.tile, g.tsweeps, mode);
+        for (int t = 0; t < nt; ++t) tmap[mode].push_back(make_int2(i, t));
+      }
     }
     const int nseg = (s->N + rb::SEG - 1) / rb::SEG;
     for (int64_t k = 0; k < (int64_t)s->N * nseg; k += 4)
@@ -977,24 +988,25 @@ static int group_tables(RbGroup& g, hipStream_t st, std::string& err) {
     for (int j = 1; j <= s->N; j += nseg > 1 ? 1 : adv_waves(g.maxN)) amap.push_back(make_int4(i, j, 0, nseg));
     g.any_src = g.any_src || s->desc.has_src;
   }
-  if (tmap.size() > INT32_MAX / 2 || cmap.size() > INT32_MAX / 2 || imap.size() > INT32_MAX / 2) {  // amap <= imap * 4
+  if (tmap[M_ROW].size() > INT32_MAX / 2 || tmap[M_COL].size() > INT32_MAX / 2 || cmap.size() > INT32_MAX / 2 || imap.size() > INT32_MAX / 2) {  // amap <= imap * 4
     err = "launch group too large for one launch";
     return EQF_EINVAL;
   }
   g.n = n;
-  g.tiles = (int)tmap.size();
+  for (int m = 0; m < 3; ++m) g.tiles[m] = (int)tmap[m].size();
   g.iblocks = (int)imap.size();
   g.cblocks = (int)cmap.size();
   g.ablocks = (int)amap.size();
   auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
   const size_t b_scs = up(sizeof(RbScene) * n);
-  const size_t b_t = up(sizeof(int2) * tmap.size());
+  size_t b_t[3];
+  for (int m = 0; m < 3; ++m) b_t[m] = up(sizeof(int2) * tmap[m].size());
   const size_t b_m = up(sizeof(int4) * imap.size()), b_c = up(sizeof(int2) * cmap.size());
   const size_t b_a = up(sizeof(int4) * amap.size());
   lex_order(ldiff, g.scenes);
   lex_order(lpress, g.scenes);
   const size_t b_ld = up(sizeof(LexTask) * ldiff.size()), b_lp = up(sizeof(LexTask) * lpress.size());
-  const size_t bytes = b_scs + b_t + b_m + b_c + b_a + b_ld + b_lp;
+  const size_t bytes = b_scs + b_t[0] + b_t[1] + b_t[2] + b_m + b_c + b_a + b_ld + b_lp;
   if (bytes > g.tab_bytes) {  // with headroom: a server's group changes size often
     (void)hipFree(g.d_tab);
     g.d_tab = nullptr;
@@ -1017,7 +1029,8 @@ static int group_tables(RbGroup& g, hipStream_t st, std::string& err) {
     return at;
   };
   const size_t o_scs = put(scs.data(), sizeof(RbScene) * n, b_scs);
-  const size_t o_t = put(tmap.data(), sizeof(int2) * tmap.size(), b_t);
+  size_t o_t[3];
+  for (int m = 0; m < 3; ++m) o_t[m] = put(tmap[m].data(), sizeof(int2) * tmap[m].size(), b_t[m]);
   const size_t o_m = put(imap.data(), sizeof(int4) * imap.size(), b_m);
   const size_t o_c = put(cmap.data(), sizeof(int2) * cmap.size(), b_c);
   const size_t o_a = put(amap.data(), sizeof(int4) * amap.size(), b_a);
@@ -1025,7 +1038,7 @@ static int group_tables(RbGroup& g, hipStream_t st, std::string& err) {
   const size_t o_lp = put(lpress.data(), sizeof(LexTask) * lpress.size(), b_lp);
   char* d = (char*)g.d_tab;
   g.d_scs = (RbScene*)(d + o_scs);
-  g.d_tmap = (int2*)(d + o_t);
+  for (int m = 0; m < 3; ++m) g.d_tmap[m] = (int2*)(d + o_t[m]);
   g.d_imap = (int4*)(d + o_m);
   g.d_cmap = (int2*)(d + o_c);
   g.d_amap = (int4*)(d + o_a);
@@ -1077,8 +1090,8 @@ static int group_tables(RbGroup& g, hipStream_t st, std::string& err) {
 
 template <int MODE, int T, int NW, int R>
 static void launch_band(hipStream_t st, const RbGroup& g, int src, int dst, int x0, int coef, int nsw) {
-  hipLaunchKernelGGL((rb::k_rb_band<MODE, T, NW, R>), dim3(g.tiles), dim3(64 * NW), 0, st, g.d_scs, g.d_tmap,
-                     g.tiles, src, dst, x0, coef, nsw);
+  hipLaunchKernelGGL((rb::k_rb_band<MODE, T, NW, R>), dim3(g.tiles[MODE]), dim3(64 * NW), 0, st, g.d_scs,
+                     g.d_tmap[MODE], g.tiles[MODE], src, dst, x0, coef, nsw);
 }
 
 template <int MODE, int NW, int R>

@@ -14,7 +14,7 @@ from helpers import FIELD_NAMES, assert_state_equal, download_all
 pytestmark = pytest.mark.gpu
 
 
-def _pair(N, mode, seed, walls=0.1, full=(), speed=1.0):
+def _pair(N, mode, seed, walls=0.1, full=(), speed=1.0, iters=2, press=3):
     S = N + 2
     rng = np.random.default_rng(seed)
     m = (rng.random((S, S)) >= walls).astype(np.uint8)
@@ -27,7 +27,7 @@ def _pair(N, mode, seed, walls=0.1, full=(), speed=1.0):
     m[:, 0] = m[:, -1] = 0
     p = _abi.default_params()
     p.size, p.delta_t, p.viscosity, p.diffusion = S, 0.1, 1.0 / N ** 2, 0.5 / N ** 2
-    p.gs_iters, p.pressure_iters, p.gs_mode = 2, 3, mode
+    p.gs_iters, p.pressure_iters, p.gs_mode = iters, press, mode
     s = _abi.Scene(p)
     s.set_mask(m.ravel())
     st = oracle.State(S)
@@ -37,7 +37,7 @@ def _pair(N, mode, seed, walls=0.1, full=(), speed=1.0):
         s.upload(i, f)
         st.f[k] = f.copy()
     order = oracle.RB if mode == _abi.GS_REDBLACK else oracle.LEX
-    return s, st, lambda n: st.run(p.delta_t, p.diffusion, p.viscosity, 2, n, press_iters=3, order=order)
+    return s, st, lambda n: st.run(p.delta_t, p.diffusion, p.viscosity, iters, n, press_iters=press, order=order)
 
 
 @pytest.mark.parametrize("N", [1, 2, 63, 64, 65, 128, 129, 192, 193, 255, 256, 257, 320, 449, 512, 513, 1024])
@@ -91,3 +91,18 @@ def test_batch_of_row_lengths_equals_oracle():
     b.close()
     for s, _, _ in trio:
         s.close()
+
+
+@pytest.mark.parametrize("N", [128, 300])  # several tiles in both directions
+@pytest.mark.parametrize("walls", [0.2, 0.5])
+@pytest.mark.parametrize("tile,tsw", [(5, 5), (0, 8), (1, 6), (2, 4)])
+def test_redblack_tile_halos_with_dense_walls(N, walls, tile, tsw):
+    """Every sweep of a launch carries values across tiles through walls too."""
+    print(f"[case] phases halo N={N} walls={walls} tile={tile} T={tsw}", flush=True)
+    s, st, run = _pair(N, _abi.GS_REDBLACK, 11, walls, iters=20, press=17)
+    s.set_tuning(tile, tsw)
+    s.step(2)
+    s.sync()
+    run(2)
+    assert_state_equal(download_all(s), st, f"N={N}")
+    s.close()

@@ -90,8 +90,8 @@ enum BandSel : uint32_t {
 // A workgroup finds its scene and its place in it with one load from a map
 // of the launch's work units (band tile or block of CELL_BLOCK cells, ring
 // included -> {scene, index in the scene}; segments of rows: seg_of).
-// Field roles in kernel arguments: F_* (eqf_layout.h), the ping-pong field, or none.
-constexpr int ROLE_TMP = NFIELDS;
+// Field roles in kernel arguments: F_* (eqf_layout.h), the ping-pong fields, or none.
+constexpr int ROLE_TMP = NFIELDS;  // .. + 2
 constexpr int ROLE_NONE = -1;
 // cells per workgroup of the whole-field kernels (256 threads x 4 cells)
 constexpr int CELL_K = 4;
@@ -127,7 +127,7 @@ __device__ __forceinline__ void stg(float* p, uint32_t i, float v) {
   *(GAS float*)((GAS char*)(GAS float*)p + (size_t)(i << 2)) = v;
 }
 __device__ __forceinline__ float* role_ptr(const RbScene& s, int role) {
-  return role == ROLE_TMP ? s.tmp : s.d.fld + (int64_t)role * s.d.fstride;
+  return role >= ROLE_TMP ? s.tmp[role - ROLE_TMP] : s.d.fld + (int64_t)role * s.d.fstride;
 }
 // Tiles along one dimension of S cells for regions of W cells and output
 // tiles of TX: region b starts at b*TX; the first needs no halo before it
@@ -150,6 +150,16 @@ __device__ __forceinline__ void coefs(const SceneDesc& d, int coef, float& a, fl
   cr = coef == 0 ? d.cr_visc : coef == 1 ? d.cr_diff : 0.25f;
 }
 
+// A lin_solve in a pass of k_rb_band: its tiles (workgroup -> {scene, tile}),
+// field roles and coefficients.
+struct BandSlot {
+  const int2* tmap;
+  int nt, mode, src, dst, x0, coef;
+};
+struct BandArgs {
+  BandSlot s[3];
+};
+
 // Red-black Gauss-Seidel with set_boundaries, T full sweeps per launch, all
 // in registers.  A workgroup of NW waves owns a region of 128 columns x
 // NW*R rows: lane l holds columns 2l and 2l+1 of its wave's band of R rows
@@ -167,23 +177,21 @@ __device__ __forceinline__ void coefs(const SceneDesc& d, int coef, float& a, fl
 // buffer and the tile is written to the other (ping-pong).  Corners are set
 // once after the lin_solve (nothing reads them during the sweeps).
 template <int MODE, int T, int NW, int R>
-__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu((NW == 8 && R <= 10) ? 8 : (NW == 8 && R <= 14) ? 6 : (NW == 8 && R <= 18) ? 4 : 1))) k_rb_band(const RbScene* __restrict__ scs, const int2* __restrict__ tmap,
-                                                     int nt, int src_role, int dst_role, int x0_role, int coef,
-                                                     int nsweeps) {
+__device__ __forceinline__ void band_tile(float (&edg)[2][2][2][NW][64], const RbScene* __restrict__ scs,
+                                          const BandSlot& sl, int L, int nsweeps) {
+  const int2* __restrict__ tmap = sl.tmap;
+  const int nt = sl.nt, src_role = sl.src, dst_role = sl.dst, x0_role = sl.x0, coef = sl.coef;
   constexpr int HX = band_halo_x(MODE, T), HY = band_halo_y(MODE, T), W = 128, RH = NW * R;
   constexpr int TX = W - 2 * HX, TY = RH - 2 * HY;
   static_assert(TX > 0 && TY > 0 && TX % 2 == 0 && TY % 2 == 0 && R % 2 == 0, "band geometry");
-  // [buffer][first / last row][column of the lane's pair][wave][lane]: one
-  // float per lane and store, so a wave's 64 accesses hit 64 distinct banks
-  __shared__ float edg[2][2][2][NW][64];
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // Tile order: workgroups are dealt to the 8 XCDs round-robin by linear id;
+  // Tile order: workgroup L of the slot's nt, one per tile; they are dealt to
+  // the 8 XCDs round-robin by linear id;
   // XCD k takes a contiguous run of the row-major tiles (scene after scene)
   // instead, so tiles that share halo columns run together on one L2.
   int t;
   {
-    const int L = blockIdx.x;  // nt workgroups, one per tile
     const int per = nt >> 3, rem = nt & 7, xcd = L & 7;
     t = __builtin_amdgcn_readfirstlane(xcd * per + min(xcd, rem) + (L >> 3));
   }
@@ -425,6 +433,23 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu((N
         if (cout[b]) *(GAS float*)(dp + 4u * (uint32_t)(gxl + b)) = x[i][b];
     }
   }
+}
+
+// One pass of up to three lin_solves that do not depend on each other: the
+// tiles of one after those of the other.
+template <int T, int NW, int R>
+__global__ void __launch_bounds__(64 * NW)
+    __attribute__((amdgpu_waves_per_eu((NW == 8 && R <= 10) ? 8 : (NW == 8 && R <= 14) ? 6 : (NW == 8 && R <= 18) ? 4 : 1)))
+    k_rb_band(const RbScene* __restrict__ scs, BandArgs args, int nsweeps) {
+  // [buffer][first / last row][column of the lane's pair][wave][lane]: one
+  // float per lane and store, so a wave's 64 accesses hit 64 distinct banks
+  __shared__ float edg[2][2][2][NW][64];
+  int L = blockIdx.x, k = 0;
+  while (L >= args.s[k].nt) L -= args.s[k++].nt;  // (the grid is the sum of the slots' tiles)
+  const BandSlot& sl = args.s[k];
+  if (sl.mode == M_ROW) band_tile<M_ROW, T, NW, R>(edg, scs, sl, L, nsweeps);
+  else if (sl.mode == M_COL) band_tile<M_COL, T, NW, R>(edg, scs, sl, L, nsweeps);
+  else band_tile<M_PASSIVE, T, NW, R>(edg, scs, sl, L, nsweeps);
 }
 
 // set_boundaries (fluid.rs:151-187) and its corners (fluid.rs:265-271) run
@@ -834,21 +859,27 @@ __global__ void __launch_bounds__(256) k_sources(const RbScene* __restrict__ scs
   if (m & 4) add_field(d.fld + F_V * n, d.src + 2 * n, e0, cells);
 }
 
-// dst = src over every cell of every scene (cmap as for k_sources).
+// dst = src over every cell of every scene (cmap as for k_sources), for up to
+// three pairs of fields (ROLE_NONE: fewer).
+struct CopyArgs {
+  int dst[3], src[3];
+};
 __global__ void __launch_bounds__(256) k_copy(const RbScene* __restrict__ scs, const int2* __restrict__ cmap,
-                                              int dst_role, int src_role) {
+                                              CopyArgs args) {
   const int2 cm = cmap[blockIdx.x];
   const RbScene& sc = scs[cm.x];
   const int64_t cells = (int64_t)sc.d.S * sc.d.S;
   const int64_t e0 = (int64_t)cm.y * CELL_BLOCK + threadIdx.x;
-  const float* __restrict__ src = role_ptr(sc, src_role);
-  float* __restrict__ dst = role_ptr(sc, dst_role);
-  float x[CELL_K];
+  for (int f = 0; f < 3 && args.dst[f] != ROLE_NONE; ++f) {
+    const float* __restrict__ src = role_ptr(sc, args.src[f]);
+    float* __restrict__ dst = role_ptr(sc, args.dst[f]);
+    float x[CELL_K];
 #pragma unroll
-  for (int k = 0; k < CELL_K; ++k) x[k] = src[min(e0 + k * 256, cells - 1)];
+    for (int k = 0; k < CELL_K; ++k) x[k] = src[min(e0 + k * 256, cells - 1)];
 #pragma unroll
-  for (int k = 0; k < CELL_K; ++k)
-    if (e0 + k * 256 < cells) dst[e0 + k * 256] = x[k];
+    for (int k = 0; k < CELL_K; ++k)
+      if (e0 + k * 256 < cells) dst[e0 + k * 256] = x[k];
+  }
 }
 
 }  // namespace rb
@@ -877,6 +908,7 @@ struct RbGroup {
   uint32_t* h_err = nullptr;
   int n = 0, maxN = 0, tiles[3] = {0, 0, 0}, iblocks = 0, cblocks = 0, ablocks = 0;
   bool any_src = false;
+  int ntmp = 1;  // red-black: ping-pong fields of every scene
   int diff_iters = 0, press_iters = 0;  // red-black: the same for every scene
   int diff_rounds = 0, press_rounds = 0;  // exact: the most of any scene
   int tile = 5, tsweeps = 5;  // band shape index (kBands) and sweeps per launch (untuned default)
@@ -887,7 +919,7 @@ struct RbGroup {
 };
 
 struct FrameWork {
-  float* tmp = nullptr;  // ping-pong field
+  float* tmp[3] = {nullptr, nullptr, nullptr};  // ping-pong fields: one, or one per diffusion
   RbGroup one;           // the scene alone (eqf_step)
 };
 
@@ -962,13 +994,15 @@ static int group_tables(RbGroup& g, hipStream_t st, std::string& err) {
   int64_t hd = 0, hp = 0;
   int fd = 0, fp = 0;
   g.any_src = false;
+  g.ntmp = 3;
   g.maxN = 0;
   for (const eqf_scene* s : g.scenes) g.maxN = std::max(g.maxN, s->N);
   g.diff_rounds = g.press_rounds = 0;
   for (int i = 0; i < n; ++i) {
     eqf_scene* s = g.scenes[i];
     auto* w = static_cast<FrameWork*>(s->work);
-    scs[i] = RbScene{s->desc, w->tmp};
+    scs[i] = RbScene{s->desc, {w->tmp[0], w->tmp[1], w->tmp[2]}};
+    if (!w->tmp[2]) g.ntmp = 1;
     g.diff_rounds = std::max(g.diff_rounds, lex_rounds(s->desc.diff_iters));
     g.press_rounds = std::max(g.press_rounds, lex_rounds(s->desc.press_iters));
     if (g.exact) {
@@ -1088,52 +1122,63 @@ static int group_tables(RbGroup& g, hipStream_t st, std::string& err) {
   return EQF_OK;
 }
 
-template <int MODE, int T, int NW, int R>
-static void launch_band(hipStream_t st, const RbGroup& g, int src, int dst, int x0, int coef, int nsw) {
-  hipLaunchKernelGGL((rb::k_rb_band<MODE, T, NW, R>), dim3(g.tiles[MODE]), dim3(64 * NW), 0, st, g.d_scs,
-                     g.d_tmap[MODE], g.tiles[MODE], src, dst, x0, coef, nsw);
+template <int T, int NW, int R>
+static void launch_band(hipStream_t st, const RbGroup& g, const rb::BandArgs& a, int nsw) {
+  hipLaunchKernelGGL((rb::k_rb_band<T, NW, R>), dim3((unsigned)(a.s[0].nt + a.s[1].nt + a.s[2].nt)), dim3(64 * NW), 0, st,
+                     g.d_scs, a, nsw);
 }
 
-template <int MODE, int NW, int R>
-static void launch_band_t(hipStream_t st, const RbGroup& g, int src, int dst, int x0, int coef, int nsw) {
+template <int NW, int R>
+static void launch_band_t(hipStream_t st, const RbGroup& g, const rb::BandArgs& a, int nsw) {
   const int T = g.tsweeps;
-  if (T == 1) launch_band<MODE, 1, NW, R>(st, g, src, dst, x0, coef, nsw);
-  else if (T == 2) launch_band<MODE, 2, NW, R>(st, g, src, dst, x0, coef, nsw);
-  else if (T == 4) launch_band<MODE, 4, NW, R>(st, g, src, dst, x0, coef, nsw);
-  else if (T == 5) launch_band<MODE, 5, NW, R>(st, g, src, dst, x0, coef, nsw);
-  else if (T == 6) launch_band<MODE, 6, NW, R>(st, g, src, dst, x0, coef, nsw);
-  else launch_band<MODE, 8, NW, R>(st, g, src, dst, x0, coef, nsw);
+  if (T == 1) launch_band<1, NW, R>(st, g, a, nsw);
+  else if (T == 2) launch_band<2, NW, R>(st, g, a, nsw);
+  else if (T == 4) launch_band<4, NW, R>(st, g, a, nsw);
+  else if (T == 5) launch_band<5, NW, R>(st, g, a, nsw);
+  else if (T == 6) launch_band<6, NW, R>(st, g, a, nsw);
+  else launch_band<8, NW, R>(st, g, a, nsw);
 }
 
-template <int MODE>
-static void launch_gs_mode(hipStream_t st, const RbGroup& g, int src, int dst, int x0, int coef, int nsw) {
-  if (g.tile == 1) launch_band_t<MODE, 8, 32>(st, g, src, dst, x0, coef, nsw);
-  else if (g.tile == 2) launch_band_t<MODE, 16, 16>(st, g, src, dst, x0, coef, nsw);
-  else if (g.tile == 3) launch_band_t<MODE, 8, 18>(st, g, src, dst, x0, coef, nsw);
-  else if (g.tile == 4) launch_band_t<MODE, 8, 14>(st, g, src, dst, x0, coef, nsw);
-  else if (g.tile == 5) launch_band_t<MODE, 8, 10>(st, g, src, dst, x0, coef, nsw);
-  else launch_band_t<MODE, 8, 16>(st, g, src, dst, x0, coef, nsw);
+static void launch_bands(hipStream_t st, const RbGroup& g, const rb::BandArgs& a, int nsw) {
+  if (g.tile == 1) launch_band_t<8, 32>(st, g, a, nsw);
+  else if (g.tile == 2) launch_band_t<16, 16>(st, g, a, nsw);
+  else if (g.tile == 3) launch_band_t<8, 18>(st, g, a, nsw);
+  else if (g.tile == 4) launch_band_t<8, 14>(st, g, a, nsw);
+  else if (g.tile == 5) launch_band_t<8, 10>(st, g, a, nsw);
+  else launch_band_t<8, 16>(st, g, a, nsw);
 }
 
-static void g_copy(hipStream_t st, const RbGroup& g, int dst, int src) {
-  hipLaunchKernelGGL(rb::k_copy, dim3((unsigned)g.cblocks), dim3(256), 0, st, g.d_scs, g.d_cmap, dst, src);
+static void g_copy(hipStream_t st, const RbGroup& g, const rb::CopyArgs& a) {
+  hipLaunchKernelGGL(rb::k_copy, dim3((unsigned)g.cblocks), dim3(256), 0, st, g.d_scs, g.d_cmap, a);
 }
 
-// lin_solve in red-black order on every scene of the group (one iteration
-// count): ceil(iters/T) tile passes ping-ponging between x and the scratch
-// field; an odd pass count ends with a copy back.
-static void g_lin_solve(hipStream_t st, const RbGroup& g, int mode, int x, int x0, int coef, int iters) {
+// A lin_solve: set_boundaries mode, fields and coefficients.
+struct Solve {
+  int mode, x, x0, coef;
+};
+// Up to three lin_solves in red-black order on every scene of the group (one
+// iteration count): ceil(iters/T) tile passes ping-ponging between x and a
+// scratch field; an odd pass count ends with a copy back.
+static void g_lin_solve(hipStream_t st, const RbGroup& g, const Solve* sv, int n, int iters) {
   if (iters <= 0) return;
-  int a_ = x, b_ = rb::ROLE_TMP;
-  for (int done = 0; done < iters;) {
+  rb::BandArgs a{};
+  for (int k = 0; k < n; ++k)
+    a.s[k] = rb::BandSlot{g.d_tmap[sv[k].mode], g.tiles[sv[k].mode], sv[k].mode, sv[k].x, rb::ROLE_TMP + k, sv[k].x0, sv[k].coef};
+  int passes = 0;
+  for (int done = 0; done < iters; ++passes) {
     const int nsw = std::min(g.tsweeps, iters - done);
-    if (mode == M_ROW) launch_gs_mode<M_ROW>(st, g, a_, b_, x0, coef, nsw);
-    else if (mode == M_COL) launch_gs_mode<M_COL>(st, g, a_, b_, x0, coef, nsw);
-    else launch_gs_mode<M_PASSIVE>(st, g, a_, b_, x0, coef, nsw);
-    std::swap(a_, b_);
+    launch_bands(st, g, a, nsw);
+    for (int k = 0; k < n; ++k) std::swap(a.s[k].src, a.s[k].dst);
     done += nsw;
   }
-  if (a_ != x) g_copy(st, g, x, a_);
+  if (passes & 1) {
+    rb::CopyArgs c;
+    for (int k = 0; k < 3; ++k) {
+      c.dst[k] = k < n ? sv[k].x : rb::ROLE_NONE;
+      c.src[k] = rb::ROLE_TMP + k;
+    }
+    g_copy(st, g, c);
+  }
 }
 // Lexicographic lin_solves: the three diffusions of a frame in one launch per
 // round (they read and write different fields: u and v from the last frame's
@@ -1150,7 +1195,10 @@ static void g_lex(hipStream_t st, const RbGroup& g, bool press, const LexSpec& s
 }
 static void g_pressure(hipStream_t st, const RbGroup& g, int p, int div) {
   if (g.exact) g_lex(st, g, true, LexSpec{M_PASSIVE, p, div, 2}, LexSpec{}, LexSpec{});
-  else g_lin_solve(st, g, M_PASSIVE, p, div, 2, g.press_iters);
+  else {
+    const Solve s{M_PASSIVE, p, div, 2};
+    g_lin_solve(st, g, &s, 1, g.press_iters);
+  }
 }
 
 template <bool DENSITY>
@@ -1177,11 +1225,13 @@ static void g_frame(hipStream_t st, const RbGroup& g) {
   const dim3 cells((unsigned)g.iblocks);  // interior cell blocks
   if (g.any_src)
     hipLaunchKernelGGL(rb::k_sources, dim3((unsigned)g.cblocks), dim3(256), 0, st, g.d_scs, g.d_cmap);
-  if (g.exact) {  // fluid.rs:438, 448, 501
+  // the three diffusions, fluid.rs:438, 448, 501 (the density's reads no velocity)
+  if (g.exact) {
     g_lex(st, g, false, LexSpec{M_ROW, F_U0, F_U, 0}, LexSpec{M_COL, F_V0, F_V, 0}, LexSpec{M_PASSIVE, F_SC, F_D, 1});
   } else {
-    g_lin_solve(st, g, M_ROW, F_U0, F_U, 0, g.diff_iters);  // fluid.rs:438
-    g_lin_solve(st, g, M_COL, F_V0, F_V, 0, g.diff_iters);  // fluid.rs:448
+    // each of them alone where the scenes have one ping-pong field
+    const Solve s[3] = {{M_ROW, F_U0, F_U, 0}, {M_COL, F_V0, F_V, 0}, {M_PASSIVE, F_SC, F_D, 1}};
+    for (int k = 0; k < 3; k += g.ntmp) g_lin_solve(st, g, s + k, g.ntmp, g.diff_iters);
   }
   // project(U0, V0, p=U, div=V), fluid.rs:459
   hipLaunchKernelGGL(rb::k_div, cells, dim3(256), 0, st, g.d_scs, g.d_imap, F_U0, F_V0, F_V, F_U, 0);
@@ -1192,11 +1242,10 @@ static void g_frame(hipStream_t st, const RbGroup& g) {
   // project(U, V, p=U0, div=V0), fluid.rs:491
   hipLaunchKernelGGL(rb::k_div, cells, dim3(256), 0, st, g.d_scs, g.d_imap, F_U, F_V, F_V0, F_U0, 1);
   g_pressure(st, g, F_U0, F_V0);
-  if (!g.exact) g_lin_solve(st, g, M_PASSIVE, F_SC, F_D, 1, g.diff_iters);  // density, fluid.rs:501
   hipLaunchKernelGGL(rb::k_grad, cells, dim3(256), 0, st, g.d_scs, g.d_imap, F_U, F_V, F_U0, 1, F_SC);
   // fluid.rs:511-523
   g_adv<true>(st, g, F_D, F_SC, ROLE_NONE, ROLE_NONE, F_U, F_V);
-  g_copy(st, g, F_SC, F_D);
+  g_copy(st, g, rb::CopyArgs{{F_SC, ROLE_NONE, ROLE_NONE}, {F_D, 0, 0}});
 }
 
 static void group_release(RbGroup& g) {
@@ -1292,10 +1341,15 @@ void* frame_create(eqf_scene* s, std::string& err) {
   auto* w = new FrameWork;
   const size_t n = (size_t)s->S * s->S;
   hipError_t e = hipSuccess;
-  if (s->p.gs_mode == EQF_GS_REDBLACK) e = eqf_scene_malloc(s, (void**)&w->tmp, sizeof(float) * n);
+  if (s->p.gs_mode == EQF_GS_REDBLACK) {
+    const int k = rb_scratch_fields(s->S);
+    const size_t fs = (size_t)rm_field_floats(s->S);
+    e = eqf_scene_malloc(s, (void**)&w->tmp[0], sizeof(float) * (k > 1 ? k * fs : n));
+    for (int i = 1; i < k && e == hipSuccess; ++i) w->tmp[i] = w->tmp[0] + i * fs;
+  }
   if (e != hipSuccess) {
     err = std::string("frame workspace: ") + hipGetErrorString(e);
-    eqf_scene_mfree(s, w->tmp);
+    eqf_scene_mfree(s, w->tmp[0]);
     delete w;
     return nullptr;
   }
@@ -1309,7 +1363,7 @@ void frame_destroy(eqf_scene* s) {
   auto* w = static_cast<FrameWork*>(s->work);
   if (!w) return;
   group_release(w->one);
-  eqf_scene_mfree(s, w->tmp);
+  eqf_scene_mfree(s, w->tmp[0]);
   delete w;
   s->work = nullptr;
 }

@@ -115,7 +115,7 @@ namespace eqf {
 // Each frame kernel covers all scenes of its group in one launch.
 struct RbScene {
   SceneDesc d;  // the scene's descriptor (a copy): fields, sizes, coefficients, rule bytes
-  float* tmp;   // its ping-pong field (red-black mode)
+  float* tmp[3];  // its ping-pong fields (red-black mode; rb_scratch_fields)
 };
 
 // Lexicographic lin_solve (eqf_lex.hip).  A launch covers up to three

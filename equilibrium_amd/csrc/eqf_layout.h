@@ -71,6 +71,14 @@ EQF_HD inline int rm_code_stride(int S) { return S + (S & 1); }
 EQF_HD inline int64_t rm_code_used(int S) { return (int64_t)S * rm_code_stride(S); }
 EQF_HD inline int64_t rm_code_bytes(int S) { return (rm_code_used(S) + 63) & ~(int64_t)63; }
 
+// ---- red-black lin_solve (eqf_frame.hip) ----
+// Ping-pong fields of a scene: one per diffusion, so that the three share their
+// launches, up to the size where one alone fills the device and the caches hold
+// more of one than of three.  ms per frame of 20 sweeps apart and together: N=250
+// 0.274 and 0.183, N=1501 0.436 and 0.346, N=2046 0.574 and 0.469, N=3000 0.948
+// and 0.909, N=4096 1.510 and 1.543.
+EQF_HD inline int rb_scratch_fields(int S) { return S <= 3072 ? 3 : 1; }
+
 // ---- lexicographic lin_solve (eqf_lex.hip) ----
 // Waves per workgroup, sweeps per round (five per wave), steps per block.
 constexpr int LEX_W = 4, LEX_KMAX = 20, LEX_B = 8;

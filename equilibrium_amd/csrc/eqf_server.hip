@@ -121,7 +121,8 @@ struct eqf_server {
   }
 };
 
-// Device bytes of a scene of this size and mode with frame sources.
+// Device bytes of a scene of this size and mode with frame sources (red-black:
+// with one ping-pong field).
 static uint64_t estimate_bytes(const eqf_params& p) {
   const int S = (int)p.size, N = S - 2;
   // fields + sources, rule bytes, row flags, tables, and the ping-pong field
@@ -465,7 +466,12 @@ extern "C" int eqf_server_submit(eqf_server* sv, const eqf_request* req, uint64_
     cp(req->init_vx, r->iu);
     cp(req->init_vy, r->iv);
   }
-  r->bytes = estimate_bytes(r->p);
+  const uint64_t least = estimate_bytes(r->p);
+  // A scene's further ping-pong fields count while it is resident, but do not
+  // keep a request out that fits without them.
+  const int more = r->p.gs_mode == EQF_GS_REDBLACK ? rb_scratch_fields((int)r->p.size) - 1 : 0;
+  r->bytes = std::min(least + more * (uint64_t)rm_field_floats((int)r->p.size) * 4,
+                      std::max(least, (uint64_t)sv->cfg.hbm_budget_bytes));
   std::lock_guard<std::mutex> lk(sv->mu);
   if (r->bytes > sv->cfg.hbm_budget_bytes)
     return eqf_internal_error(EQF_ENOMEM, "request does not fit the server's HBM budget");

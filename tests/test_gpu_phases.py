@@ -76,10 +76,11 @@ def test_walled_rows_and_breaks_equal_oracle(full, mode, speed):
     s.close()
 
 
-def test_batch_of_row_lengths_equals_oracle():
-    """Short rows (a wave each) beside rows of several waves in one launch."""
-    print("[case] phases batch", flush=True)
-    sizes = (1100, 30, 256, 257, 700)
+@pytest.mark.parametrize("sizes", [(1100, 30, 256, 257, 700), (3071, 40)])
+def test_batch_of_row_lengths_equals_oracle(sizes):
+    """Short rows (a wave each) beside rows of several waves in one launch; with
+    a scene of one ping-pong field in the batch the diffusions run apart."""
+    print(f"[case] phases batch {sizes}", flush=True)
     trio = [_pair(N, _abi.GS_REDBLACK, N) for N in sizes]
     b = _abi.Batch([s for s, _, _ in trio])
     for n in (1, 1):

@@ -80,8 +80,8 @@ EQF_HD inline int64_t rm_code_bytes(int S) { return (rm_code_used(S) + 63) & ~(i
 EQF_HD inline int rb_scratch_fields(int S) { return S <= 3072 ? 3 : 1; }
 
 // ---- lexicographic lin_solve (eqf_lex.hip) ----
-// Waves per workgroup, sweeps per round (five per wave), steps per block.
-constexpr int LEX_W = 4, LEX_KMAX = 20, LEX_B = 8;
+// Sweeps per round, steps per block.
+constexpr int LEX_KMAX = 20, LEX_B = 8;
 // Rounds of a lin_solve of `iters` sweeps, and the sweeps of each: as even as possible.
 EQF_HD inline int lex_rounds(int iters) { return iters > 0 ? (iters + LEX_KMAX - 1) / LEX_KMAX : 0; }
 EQF_HD inline int lex_round_sweeps(int iters, int round) {

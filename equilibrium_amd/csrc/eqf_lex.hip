@@ -3,8 +3,8 @@
 //
 // Work split.  The grid of S x S cells (ring included) is cut into strips of
 // 63 rows.  A workgroup takes one strip of one lin_solve through up to
-// LEX_KMAX = 20 sweeps (a round): lane r of a wave owns a row, each of four
-// waves runs up to five consecutive sweeps, two steps apart.  The strip moves
+// LEX_KMAX = 20 sweeps (a round): lane r of a wave owns a row, each of four or
+// eight waves runs up to five or three consecutive sweeps, two steps apart.  The strip moves
 // up by one row from sweep to sweep: in sweep k lane r holds row j = 63 s - 1 +
 // r - k.  A cell of sweep k at step t is column c = t - r - 2k.  Then everything
 // a cell reads comes from its own lane or the lane before it, at an earlier
@@ -23,14 +23,15 @@
 // sweeps of a strip 32 to 64 steps apart and moved 12 bytes per cell and sweep
 // through the caches: one workgroup per scene, 28.7 ms per frame at N=1024,
 // 0.86 at N=128, 0.44 at N=30 (16 sweeps), 11.0 for 512 scenes of N 64..512;
-// with moving strips on a CU each 1.91, 0.39, 0.16 and 5.8 ms.
+// with moving strips on a CU each 1.60, 0.29, 0.12 and 5.4 ms (the other phases
+// of a frame included).
 //
 // Lane 0 as a row of its own (63 rows per strip, one select per update) does
 // away with the first lane's neighbours as operands of their own: the lane
-// shifts become operands of the additions, 109 registers instead of 168 hold
-// a wave, and two workgroups share a CU.  With 64 rows, two values per cell in
-// the hand-off and the shifts as moves a frame took 2.20, 0.44, 0.18 and 8.1 ms
-// (7.6 where it was held to 128 registers, by spilling).
+// shifts become operands of the additions, 107 registers instead of 168 hold
+// a wave of five sweeps, and two workgroups share a CU.  With 64 rows, two values
+// per cell in the hand-off and the shifts as moves a frame took 2.20, 0.44, 0.18
+// and 8.1 ms, where this took 1.90, 0.39, 0.16 and 5.8.
 //
 // AdjustRow's walls are the left / right neighbours, known one step after the
 // cell: its final value is formed then (hence two steps from sweep to sweep).
@@ -40,14 +41,15 @@
 // value, or in Passive the copy of the interior neighbour.  Which of these a
 // block of eight steps can hold decides among four forms of the step (Class).
 //
-// Three more waves bring operands into LDS by anti-diagonals, where a step of a
+// Four more waves bring operands into LDS by anti-diagonals, where a step of a
 // wave reads 64 neighbours, write the results, and exchange lane 63's values
 // with the strips above and below, which run on other CUs: agent-scope stores
-// and loads in device memory, and a progress count per strip.  (Two waves for
-// it took 4400 cycles per block, more than the sweeps; with three the sweeps
-// bound it.)  A strip trails
-// the one above it by about 100 steps (64 of skew, the blocks of 8, two
-// memory latencies).  Workgroups take their strip from a ticket counter whose
+// and loads in device memory, and a progress count per strip.  (Two waves took
+// 4400 cycles per block for that and three 2900, when the sweeps took 3000 and
+// 2000.)  A strip trails the one above it by about 90 steps: 64 of skew, the
+// blocks of 8, a store and a load; taking lane 0's values a block earlier than
+// they are needed made it 8 more (N=1024 1.75 ms instead of 1.60).  Workgroups
+// take their strip from a ticket counter whose
 // order puts every strip after the one it reads from, so a waiting workgroup
 // always waits for one that already runs: the launch ends whatever share of
 // it is resident.
@@ -56,44 +58,19 @@
 // VALU instructions (6 of arithmetic, of which two shift a lane, one for lane
 // 0, one that gathers lane 63's value); a plain block of 5 sweeps x 8 steps
 // 2800 cycles with a wave alone on its SIMD, of which 500 are LDS reads of x0.
-// A lone scene is bound by its chain of S + 63 + 2K steps plus about 100 per
+// A lone scene is bound by its chain of S + 63 + 2K steps plus about 90 per
 // strip.
 //
 // Compiled with -ffp-contract=off: rustc does not contract a*b+c.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "eqf_internal.h"
 
 namespace eqf {
 namespace lex {
-
-constexpr int W = LEX_W, QMAX = 5, KMAX = LEX_KMAX, B = LEX_B;
-constexpr int NT = 64 * (W + 3);  // four waves of sweeps, three that move data
-static_assert(KMAX == W * QMAX && B == 8, "four waves of up to five sweeps, blocks of 8 steps");
-// x0 in LDS by anti-diagonals: row u = c + j - 63 s + 1 of a ring of XR rows,
-// position p = j - 63 s + KMAX (sweep k at step t reads row t - 3k, lane r
-// position r - k + KMAX - 1: 64 neighbours; lane 0 its value from the strip
-// above, at CP + k).  Rows are numbered u + UOFF >= 0.
-// A block of 8 steps may start anywhere in the ring, so the first 8 rows are
-// held twice.  Live at block b: rows 8b - 20 .. 8b + 79 (the last wave's last
-// sweep, words of four rules; the rows loaded during the block).
-constexpr int CP = 84, XP = CP + KMAX, XR = 104, UOFF = 64;
-static_assert(CP >= 64 + KMAX - 1 && XR % B == 0 && XR >= 3 * (KMAX - 1) + B * W + 11, "x0 ring too short");
-constexpr int CR = XR / 4;  // rule words: four rows of one position per word, first two rows held twice
-// hand-off from wave to wave: 16 step rows of 64 values; a pitch of 72 keeps the transposing accesses (8 steps x 8 lanes per
-// 64) in distinct banks
-constexpr int RP = 72, RR = 16;
-// LDS layout (4-byte words)
-constexpr int L_X0 = 0;
-constexpr int L_CODE = L_X0 + (XR + B) * XP;
-constexpr int L_RING = L_CODE + (CR + 2) * CP;
-constexpr int EN = W * QMAX * B;
-constexpr int L_P = L_RING + (W + 1) * RR * RP;  // lane 63's updated values: [block & 1][wave][sweep][8 steps]
-constexpr int L_CL = L_P + 2 * EN;  // class of the waves' blocks of steps, a byte each: [block & 3]
-constexpr int L_MISC = L_CL + 4;
-constexpr int L_WORDS = L_MISC + 4;
-static_assert(L_WORDS * 4 <= 80 * 1024, "two workgroups per CU");
 
 typedef __attribute__((address_space(3))) float lf;
 typedef __attribute__((address_space(3))) uint32_t lu;
@@ -144,11 +121,41 @@ __device__ __forceinline__ void agent_store(T* p, T v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// A workgroup with W waves of sweeps.
+template <int W>
+struct Lex {
+static constexpr int QMAX = (LEX_KMAX + W - 1) / W, KMAX = LEX_KMAX, B = LEX_B;
+static constexpr int NT = 64 * (W + 4);  // W waves of sweeps, four that move data
+static_assert(QMAX <= 5 && W <= 16 && B == 8, "waves of up to five sweeps, blocks of 8 steps");
+// x0 in LDS by anti-diagonals: row u = c + j - 63 s + 1 of a ring of XR rows,
+// position p = j - 63 s + KMAX (sweep k at step t reads row t - 3k, lane r
+// position r - k + KMAX - 1: 64 neighbours; lane 0 its value from the strip
+// above, at CP + k).  Rows are numbered u + UOFF >= 0.
+// A block of 8 steps may start anywhere in the ring, so the first 8 rows are
+// held twice.  Live at block b (W = 4): rows 8b - 20 .. 8b + 79 (the last wave's
+// last sweep, words of four rules; the rows loaded during the block).
+static constexpr int CP = 84, XP = CP + KMAX, XR = (3 * (KMAX - 1) + B * W + 11 + B - 1) / B * B, UOFF = 64;
+static_assert(CP >= 64 + KMAX - 1, "positions");
+static constexpr int CR = XR / 4;  // rule words: four rows of one position per word, first two rows held twice
+// hand-off from wave to wave: 16 step rows of 64 values; a pitch of 72 keeps the transposing accesses (8 steps x 8 lanes per
+// 64) in distinct banks
+static constexpr int RP = 72, RR = 16;
+// LDS layout (4-byte words)
+static constexpr int L_X0 = 0;
+static constexpr int L_CODE = L_X0 + (XR + B) * XP;
+static constexpr int L_RING = L_CODE + (CR + 2) * CP;
+static constexpr int EN = W * QMAX * B;
+static constexpr int L_P = L_RING + (W + 1) * RR * RP;  // lane 63's updated values: [block & 1][wave][sweep][8 steps]
+static constexpr int L_CL = L_P + 2 * EN;  // class of the waves' blocks of steps, a byte each: [block & 3]
+static constexpr int L_MISC = L_CL + 16;
+static constexpr int L_WORDS = L_MISC + 4;
+static_assert(L_WORDS * 4 <= (W == 4 ? 80 : 160) * 1024, "two workgroups per CU with four waves of sweeps");
+
 // Selector of a cell in LDS: 0 a plain cell; ROW / COL (logical): 1 -(left),
 // 2 -(right), 3 a plain one too, 4 ring (keeps its value); PASSIVE ring: 8 keeps its value, 9
 // copies the left, 10 the right, 11 the upper, 12 the lower neighbour.
 template <int MODE>
-__device__ __forceinline__ uint32_t selectors(uint32_t c) {  // four rule bytes -> four selectors
+static __device__ __forceinline__ uint32_t selectors(uint32_t c) {  // four rule bytes -> four selectors
   if constexpr (MODE == M_PASSIVE) return ((c >> R_PAS_SHIFT) & 0x07070707u) | ((~c & 0x01010101u) << 3);
   else return ((c >> (MODE == M_COL ? R_COL_SHIFT : R_ROW_SHIFT)) & 0x03030303u) | ((~c & 0x01010101u) << 2);
 }
@@ -181,7 +188,7 @@ struct Place {
 // .. 8m+7).  Where no cell has a rule, a cell's final value is the updated
 // one.
 template <int MODE, int Q, int CLS>
-__device__ __forceinline__ void steps(lf* L, Carry& s, int b, int w, int k0, const Place& pl) {
+static __device__ __forceinline__ void steps(lf* L, Carry& s, int b, int w, int k0, const Place& pl) {
   constexpr bool GEN = CLS == C_ALL;
   constexpr bool FIN = GEN && MODE != M_PASSIVE;  // final values other than the updated ones
   constexpr int G = 2;
@@ -348,19 +355,21 @@ __device__ __forceinline__ void steps(lf* L, Carry& s, int b, int w, int k0, con
 }
 
 template <int MODE, int Q>
-__device__ __forceinline__ void steps_c(int cls, lf* L, Carry& s, int b, int w, int k0, const Place& pl) {
+static __device__ __forceinline__ void steps_c(int cls, lf* L, Carry& s, int b, int w, int k0, const Place& pl) {
   if (cls == C_PLAIN) steps<MODE, Q, C_PLAIN>(L, s, b, w, k0, pl);
   else if (cls == C_ROWS) steps<MODE, Q, C_ROWS>(L, s, b, w, k0, pl);
   else if (MODE == M_PASSIVE && cls == C_RING) steps<M_PASSIVE, Q, C_RING>(L, s, b, w, k0, pl);
   else steps<MODE, Q, C_ALL>(L, s, b, w, k0, pl);
 }
 template <int MODE>
-__device__ __forceinline__ void steps_q(int Q, int cls, lf* L, Carry& s, int b, int w, int k0, const Place& pl) {
+static __device__ __forceinline__ void steps_q(int Q, int cls, lf* L, Carry& s, int b, int w, int k0, const Place& pl) {
   if (Q == 1) steps_c<MODE, 1>(cls, L, s, b, w, k0, pl);
   else if (Q == 2) steps_c<MODE, 2>(cls, L, s, b, w, k0, pl);
-  else if (Q == 3) steps_c<MODE, 3>(cls, L, s, b, w, k0, pl);
-  else if (Q == 4) steps_c<MODE, 4>(cls, L, s, b, w, k0, pl);
-  else steps_c<MODE, 5>(cls, L, s, b, w, k0, pl);
+  else if (QMAX == 3 || Q == 3) steps_c<MODE, 3>(cls, L, s, b, w, k0, pl);
+  else if constexpr (QMAX > 3) {
+    if (Q == 4) steps_c<MODE, 4>(cls, L, s, b, w, k0, pl);
+    else steps_c<MODE, 5>(cls, L, s, b, w, k0, pl);
+  }
 }
 
 // The sweeps of wave w of K: first sweep, count, and its first and last block of
@@ -368,7 +377,7 @@ __device__ __forceinline__ void steps_q(int Q, int cls, lf* L, Carry& s, int b, 
 struct Part {
   int k0, Q, mlo, mhi;
 };
-__device__ __forceinline__ Part part_of(int w, int steps, int K) {
+static __device__ __forceinline__ Part part_of(int w, int steps, int K) {
   const int Wn = min(W, K);
   Part r;
   r.Q = w < Wn ? K / Wn + (w < K % Wn ? 1 : 0) : 0;
@@ -378,13 +387,13 @@ __device__ __forceinline__ Part part_of(int w, int steps, int K) {
   return r;
 }
 
-// One strip of one round (K sweeps) of a lin_solve.  Waves 0..3 run the
-// sweeps; waves 4, 5 and 6 bring operands into LDS a block ahead, write the
+// One strip of one round (K sweeps) of a lin_solve.  Waves 0..W-1 run the
+// sweeps; waves W .. W+3 bring operands into LDS a block ahead, write the
 // results, and talk to the neighbouring strips, so that their loads'
 // latencies and the waits for the strip above stay out of the sweeps.
 // In block b of the workgroup wave w runs block m = b - w of its steps.
 template <int MODE>
-__device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, const LexTask& tk, const LexSpec& sp, int K,
+static __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, const LexTask& tk, const LexSpec& sp, int K,
                                            uint32_t* __restrict__ flags, float* __restrict__ Hb,
                                            uint32_t* __restrict__ err) {
   const SceneDesc& d = sc.d;
@@ -417,7 +426,7 @@ __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, const LexTa
     for (int b = -1; b < NI; ++b) {
       const int m = b - w;
       if (m >= pt.mlo && m <= pt.mhi) {
-        const int cls = (uni((int)((lu*)L)[L_CL + (b & 3)]) >> (8 * w)) & 255;
+        const int cls = uni((int)((const lb*)(L + L_CL))[(b & 3) * 16 + w]);
         steps_q<MODE>(pt.Q, cls, L, s, b, w, pt.k0, pl);
       }
       __syncthreads();
@@ -458,6 +467,20 @@ __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, const LexTa
   }
   const bool ring_copies = MODE == M_PASSIVE && d.ring_copies == 4 * d.N;  // every ring cell copies its neighbour
   const int hf = (lane & 1) * 4;  // the item's first row of the block's eight
+  constexpr int ZI = MODE == M_COL ? 3 : 2;                          // passes
+  constexpr int NIN = MODE == M_COL ? 2 * (64 + B - 1) : 2 * 64;     // items
+  // x before the round, as "sweep -1": row t of ring 0, lane r: x(t + 1 - r, base + r + 1)
+  int ir[ZI], ioff[ZI], oc[ZI], oj[ZI];
+#pragma unroll
+  for (int z = 0; z < ZI; ++z) {
+    const int it = (64 * z + lane) >> 1;
+    ir[z] = MODE == M_COL ? hf + it - (B - 1) : it;
+    const int ic = MODE == M_COL ? B - it : hf + 1 - it;  // + 8 m
+    ioff[z] = (MODE == M_COL ? ic * S + base + ir[z] + 1 : (base + ir[z] + 1) * S + ic) * 4 + FLD_PAD * 4;
+    // final values have the same shape
+    oc[z] = (MODE == M_COL ? B - 2 - it : hf - 1 - it) - 2 * (K - 1);  // + 8 m
+    oj[z] = base + ir[z] - (K - 1);
+  }
   if (w == W) {  // x0
     const rsrc_t rx0 = make_rsrc(x0 - FLD_PAD, fbytes);
     constexpr int NX = 2 * (CP - 1) + (MODE == M_COL ? 2 * (B - 1) : 0);
@@ -526,7 +549,86 @@ __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, const LexTa
     return;
   }
 
-  if (w == W + 2) {  // lane 63's values for the strip below; the rules
+  if (w == W + 2) {  // lane 63's values for the strip below, and the final values
+    float* hout = Hb + tk.hoff;
+    uint32_t* fown = flags + tk.flag;
+    for (int b = -1; b < NI; ++b) {
+      if (has_next && b > 0) {
+#pragma unroll
+        for (int z = 0; z < 3; ++z) {
+          const int m = b - 1 - ew[z], pb = (b - 1) & 1;
+          if (m >= elo[z] && m <= ehi[z]) agent_store(hout + (ek[z] * T + m * B + ei[z]), L[L_P + pb * EN + 64 * z + lane]);
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the stores are in memory: publish them
+        if (lane == 0) agent_store(fown, (uint32_t)b);
+      }
+      // Final values of the round's last sweep (ring Wn, the block before) to x:
+      // interior cells, and in Passive the ring cells that copy them.
+      if (b >= Wn) {
+        const int m = b - Wn;
+  #pragma unroll
+        for (int z = 0; z < ZI; ++z) {
+          if (64 * z + lane >= NIN) continue;
+          const lf* ring = L + (L_RING + (Wn * RR + (m & 1) * B) * RP) + hf * RP;
+          const int c = oc[z] + m * B, j = oj[z];
+          float v[4];
+          bool ok[4], all = true, some = false;
+  #pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int ci = MODE == M_COL ? c : c + i, ji = MODE == M_COL ? j + i : j;
+            const int ri = MODE == M_COL ? min(max(ir[z] + i, 0), 63) : ir[z];
+            v[i] = ring[i * RP + ri];
+            ok[i] = ci >= 1 && ci <= S - 2 && ji >= 1 && ji <= S - 2 && (uint32_t)(ir[z] + (MODE == M_COL ? i : 0) - 1) < 63u;
+            all = all && ok[i];
+            some = some || ok[i];
+          }
+          float* o = x + (MODE == M_COL ? c * S + j : j * S + c);
+          if (all) {
+            typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+            f4u vv;
+  #pragma unroll
+            for (int i = 0; i < 4; ++i) vv[i] = v[i];
+            *(f4u*)o = vv;
+          } else if (some) {
+  #pragma unroll
+            for (int i = 0; i < 4; ++i)
+              if (ok[i]) o[i] = v[i];
+          }
+          if constexpr (MODE == M_PASSIVE) {
+            if (some && (j == 1 || j == S - 2 || c <= 1 || c + 3 >= S - 2)) {
+              const int Sc = rm_code_stride(S);
+              if (j == 1 || j == S - 2) {  // the rows above / below the interior
+                for (int side = 0; side < 2; ++side) {
+                  if (j != (side ? S - 2 : 1)) continue;
+                  const int y = side ? S - 1 : 0;
+  #pragma unroll
+                  for (int i = 0; i < 4; ++i)
+                    if (ok[i] && (ring_copies || (d.code[y * Sc + c + i] >> R_PAS_SHIFT))) x[y * S + c + i] = v[i];
+                }
+              }
+              float e = v[0];  // the columns left / right of it
+  #pragma unroll
+              for (int i = 1; i < 4; ++i) e = c + i == 1 ? v[i] : e;
+              if (c <= 1 && c + 3 >= 1 && (ring_copies || (d.code[j * Sc] >> R_PAS_SHIFT))) x[j * S] = e;
+              e = v[0];
+  #pragma unroll
+              for (int i = 1; i < 4; ++i) e = c + i == S - 2 ? v[i] : e;
+              if (c <= S - 2 && c + 3 >= S - 2 && (ring_copies || (d.code[j * Sc + S - 1] >> R_PAS_SHIFT))) x[j * S + S - 1] = e;
+            }
+          }
+        }
+      }
+      __syncthreads();
+    }
+    if (has_next) {
+      if (lane == 0) agent_store(fown, 0x7fffffffu);
+      // in memory before this workgroup counts as ended (the flags are cleared then)
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    return;
+  }
+
+  if (w == W + 3) {  // the rules
     const int Sc = rm_code_stride(S);
     // the rule bytes, transposed for COL, from CODE_PAD bytes before to 8 after them
     const rsrc_t rc = make_rsrc(d.code + (MODE == M_COL ? rm_code_bytes(S) : 0) - CODE_PAD, rm_code_used(S) + CODE_PAD + 8);
@@ -580,23 +682,14 @@ __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, const LexTa
       uint32_t c = rows ? C_ROWS : C_PLAIN;
       c = (h_col & cmask) ? (MODE == M_PASSIVE ? C_RING : C_ALL) : c;
       c = (h_rule & cmask) ? C_ALL : c;
-      if (lane < W) ((lb*)(L + L_CL))[(nb & 3) * 4 + lane] = (uint8_t)c;
+      if (lane < W) ((lb*)(L + L_CL))[(nb & 3) * 16 + lane] = (uint8_t)c;
     };
     for (int ub = 5; ub < 8; ++ub) {  // rows of the cells left of column 0's diagonal
       load(ub);
       put(ub);
     }
-    float* hout = Hb + tk.hoff;
-    uint32_t* fown = flags + tk.flag;
     load(UOFF / B);
     for (int b = -1; b < NI; ++b) {
-      if (has_next) {
-#pragma unroll
-        for (int z = 0; z < 3; ++z) {
-          const int m = b - 1 - ew[z], pb = (b - 1) & 1;
-          if (m >= elo[z] && m <= ehi[z]) agent_store(hout + (ek[z] * T + m * B + ei[z]), L[L_P + pb * EN + 64 * z + lane]);
-        }
-      }
       if (b + 1 < NB) {
         put(b + 1 + UOFF / B);
       } else {
@@ -604,39 +697,17 @@ __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, const LexTa
         h_col <<= 1;
       }
       classes(b + 1);
-      if (has_next && b > 0) {  // the stores are in memory: publish them
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        if (lane == 0) agent_store(fown, (uint32_t)b);
-      }
       if (b + 2 < NB) load(b + 2 + UOFF / B);
       __syncthreads();
-    }
-    if (has_next) {
-      if (lane == 0) agent_store(fown, 0x7fffffffu);
-      // in memory before this workgroup counts as ended (the flags are cleared then)
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
     return;
   }
 
-  // Wave 5: x before the round, lane 0's values from the strip above, and the
-  // final values.
+  // x before the round, and lane 0's values from the strip above: these only in
+  // the block before they are needed, since every block that they come earlier
+  // puts every strip that much further behind the one above.
   const float* hin = Hb + (has_prev ? tk.hoff - (int64_t)KMAX * T : 0);
   const uint32_t* fprev = flags + (has_prev ? tk.flag - 1 : tk.flag);
-  constexpr int ZI = MODE == M_COL ? 3 : 2;                          // passes
-  constexpr int NIN = MODE == M_COL ? 2 * (64 + B - 1) : 2 * 64;     // items
-  // x before the round, as "sweep -1": row t of ring 0, lane r: x(t + 1 - r, base + r + 1)
-  int ir[ZI], ioff[ZI], oc[ZI], oj[ZI];
-#pragma unroll
-  for (int z = 0; z < ZI; ++z) {
-    const int it = (64 * z + lane) >> 1;
-    ir[z] = MODE == M_COL ? hf + it - (B - 1) : it;
-    const int ic = MODE == M_COL ? B - it : hf + 1 - it;  // + 8 m
-    ioff[z] = (MODE == M_COL ? ic * S + base + ir[z] + 1 : (base + ir[z] + 1) * S + ic) * 4 + FLD_PAD * 4;
-    // final values have the same shape
-    oc[z] = (MODE == M_COL ? B - 2 - it : hf - 1 - it) - 2 * (K - 1);  // + 8 m
-    oj[z] = base + ir[z] - (K - 1);
-  }
   u4 gin[ZI];
   float gu[3];
   int erow[3];  // x0 ring row of lane 0's values of the next block to be written
@@ -646,12 +717,13 @@ __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, const LexTa
   for (int z = 0; z < ZI; ++z) gin[z] = (u4)(0);
   uint32_t credit = 0, fnext = 0;  // the strip above has published this many blocks
   bool dead = false;
-  // operands of block nb of the workgroup
-  auto load = [&](int nb) {
-    if (nb < NB)
+  // operands of block nb of the workgroup (past the last: whatever is there, range-checked)
+  auto load_in = [&](int nb) {
 #pragma unroll
-      for (int z = 0; z < ZI; ++z)
-        gin[z] = __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(rx, ioff[z] + nb * B * stepc * 4, 0, 0));
+    for (int z = 0; z < ZI; ++z)
+      gin[z] = __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(rx, ioff[z] + nb * B * stepc * 4, 0, 0));
+  };
+  auto load_edge = [&](int nb) {
     // lane 0's values were made by the strip above in blocks up to nb + 8:
     // nb + 9 published blocks are needed
     if (has_prev) {
@@ -682,7 +754,7 @@ __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, const LexTa
       fnext = agent_load(fprev);
     }
   };
-  load(0);
+  load_in(0);
   for (int b = -1; b < NI; ++b) {
     if (b + 1 < NB) {
 #pragma unroll
@@ -698,6 +770,8 @@ __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, const LexTa
         }
       }
     }
+    load_edge(b + 1);
+    load_in(b + 2);
     if (has_prev) {
 #pragma unroll
       for (int z = 0; z < 3; ++z)
@@ -709,92 +783,38 @@ __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, const LexTa
           erow[z] -= erow[z] >= XR ? XR : 0;
         }
     }
-    load(b + 2);
-    // Final values of the round's last sweep (ring Wn, the block before) to x:
-    // interior cells, and in Passive the ring cells that copy them.
-    if (b >= Wn) {
-      const int m = b - Wn;
-#pragma unroll
-      for (int z = 0; z < ZI; ++z) {
-        if (64 * z + lane >= NIN) continue;
-        const lf* ring = L + (L_RING + (Wn * RR + (m & 1) * B) * RP) + hf * RP;
-        const int c = oc[z] + m * B, j = oj[z];
-        float v[4];
-        bool ok[4], all = true, some = false;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int ci = MODE == M_COL ? c : c + i, ji = MODE == M_COL ? j + i : j;
-          const int ri = MODE == M_COL ? min(max(ir[z] + i, 0), 63) : ir[z];
-          v[i] = ring[i * RP + ri];
-          ok[i] = ci >= 1 && ci <= S - 2 && ji >= 1 && ji <= S - 2 && (uint32_t)(ir[z] + (MODE == M_COL ? i : 0) - 1) < 63u;
-          all = all && ok[i];
-          some = some || ok[i];
-        }
-        float* o = x + (MODE == M_COL ? c * S + j : j * S + c);
-        if (all) {
-          typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
-          f4u vv;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) vv[i] = v[i];
-          *(f4u*)o = vv;
-        } else if (some) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (ok[i]) o[i] = v[i];
-        }
-        if constexpr (MODE == M_PASSIVE) {
-          if (some && (j == 1 || j == S - 2 || c <= 1 || c + 3 >= S - 2)) {
-            const int Sc = rm_code_stride(S);
-            if (j == 1 || j == S - 2) {  // the rows above / below the interior
-              for (int side = 0; side < 2; ++side) {
-                if (j != (side ? S - 2 : 1)) continue;
-                const int y = side ? S - 1 : 0;
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                  if (ok[i] && (ring_copies || (d.code[y * Sc + c + i] >> R_PAS_SHIFT))) x[y * S + c + i] = v[i];
-              }
-            }
-            float e = v[0];  // the columns left / right of it
-#pragma unroll
-            for (int i = 1; i < 4; ++i) e = c + i == 1 ? v[i] : e;
-            if (c <= 1 && c + 3 >= 1 && (ring_copies || (d.code[j * Sc] >> R_PAS_SHIFT))) x[j * S] = e;
-            e = v[0];
-#pragma unroll
-            for (int i = 1; i < 4; ++i) e = c + i == S - 2 ? v[i] : e;
-            if (c <= S - 2 && c + 3 >= S - 2 && (ring_copies || (d.code[j * Sc + S - 1] >> R_PAS_SHIFT))) x[j * S + S - 1] = e;
-          }
-        }
-      }
-    }
     __syncthreads();
   }
 }
+};
 
-__global__ void __launch_bounds__(NT, 4)
+template <int W>
+__global__ void __launch_bounds__(Lex<W>::NT, W == 4 ? 4 : 3)
     k_lex(const RbScene* __restrict__ scs, const LexTask* __restrict__ tasks, int ntasks, LexArgs args,
           uint32_t* __restrict__ ctl, uint32_t* __restrict__ flags, int nflags, float* __restrict__ H,
           uint32_t* __restrict__ err) {
+  typedef Lex<W> X;
   extern __shared__ float lex_lds[];
   lf* L = (lf*)lex_lds;
-  if (threadIdx.x == 0) ((lu*)L)[L_MISC] = atomicAdd(&ctl[0], 1u);
+  if (threadIdx.x == 0) ((lu*)L)[X::L_MISC] = atomicAdd(&ctl[0], 1u);
   __syncthreads();
-  const int t = uni((int)((lu*)L)[L_MISC]);
+  const int t = uni((int)((lu*)L)[X::L_MISC]);
   if (t >= ntasks) return;  // the counters were not zero at the start: nothing is sound then
   const LexTask tk = tasks[t];
   const RbScene& sc = scs[tk.scene];
   const LexSpec sp = args.sp[tk.slot];
   const int K = lex_round_sweeps(args.press ? sc.d.press_iters : sc.d.diff_iters, args.round);
   if (K > 0) {
-    if (sp.mode == M_ROW) strip_task<M_ROW>(L, sc, tk, sp, K, flags, H, err);
-    else if (sp.mode == M_COL) strip_task<M_COL>(L, sc, tk, sp, K, flags, H, err);
-    else strip_task<M_PASSIVE>(L, sc, tk, sp, K, flags, H, err);
+    if (sp.mode == M_ROW) X::template strip_task<M_ROW>(L, sc, tk, sp, K, flags, H, err);
+    else if (sp.mode == M_COL) X::template strip_task<M_COL>(L, sc, tk, sp, K, flags, H, err);
+    else X::template strip_task<M_PASSIVE>(L, sc, tk, sp, K, flags, H, err);
   }
   // The last workgroup to end leaves the counters as the next launch needs them.
   __syncthreads();
-  if (threadIdx.x == 0) ((lu*)L)[L_MISC] = atomicAdd(&ctl[1], 1u);
+  if (threadIdx.x == 0) ((lu*)L)[X::L_MISC] = atomicAdd(&ctl[1], 1u);
   __syncthreads();
-  if (uni((int)((lu*)L)[L_MISC]) == ntasks - 1) {
-    for (int i = threadIdx.x; i < nflags; i += NT) agent_store(flags + i, 0u);
+  if (uni((int)((lu*)L)[X::L_MISC]) == ntasks - 1) {
+    for (int i = threadIdx.x; i < nflags; i += X::NT) agent_store(flags + i, 0u);
     if (threadIdx.x < 2) agent_store(ctl + threadIdx.x, 0u);
   }
 }
@@ -804,8 +824,18 @@ __global__ void __launch_bounds__(NT, 4)
 void lex_launch(hipStream_t st, const RbScene* scs, const LexTask* tasks, int ntasks, const LexArgs& args,
                 uint32_t* ctl, int nflags, float* H, uint32_t* err) {
   if (ntasks <= 0) return;
-  hipLaunchKernelGGL(lex::k_lex, dim3((unsigned)ntasks), dim3(lex::NT), lex::L_WORDS * 4, st, scs, tasks, ntasks,
-                     args, ctl, ctl + 2, nflags, H, err);
+  auto launch = [&](auto w) {
+    typedef lex::Lex<decltype(w)::value> X;
+    hipLaunchKernelGGL(lex::k_lex<decltype(w)::value>, dim3((unsigned)ntasks), dim3(X::NT), X::L_WORDS * 4, st, scs, tasks,
+                       ntasks, args, ctl, ctl + 2, nflags, H, err);
+  };
+  // Up to one workgroup per CU (256 of them) the chain of blocks bounds the
+  // launch: eight waves of up to three sweeps take a block faster than four of up
+  // to five (a frame of N=1024 1.60 ms instead of 1.77, N=128 0.287 instead of
+  // 0.323; seven and ten waves lie within 3 % of eight).  Beyond that two
+  // workgroups of four fit a CU, one of eight does not leave room for another.
+  if (ntasks <= 256) launch(std::integral_constant<int, 8>());
+  else launch(std::integral_constant<int, 4>());
 }
 
 }  // namespace eqf

@@ -1,5 +1,5 @@
 // eqf_internal.h -- host-side objects of libeqfluid.so shared by the
-// runtime (eqf_runtime.hip) and the red-black driver (eqf_redblack.hip).
+// runtime (eqf_runtime.hip) and the kernels' drivers (eqf_frame.hip, eqf_lex.hip).
 #pragma once
 #include <hip/hip_runtime.h>
 

@@ -23,7 +23,7 @@
 // sweeps of a strip 32 to 64 steps apart and moved 12 bytes per cell and sweep
 // through the caches: one workgroup per scene, 28.7 ms per frame at N=1024,
 // 0.86 at N=128, 0.44 at N=30 (16 sweeps), 11.0 for 512 scenes of N 64..512;
-// with moving strips on a CU each 1.60, 0.29, 0.12 and 5.4 ms (the other phases
+// with moving strips on a CU each 1.45, 0.26, 0.12 and 5.4 ms (the other phases
 // of a frame included).
 //
 // Lane 0 as a row of its own (63 rows per strip, one select per update) does
@@ -41,14 +41,14 @@
 // value, or in Passive the copy of the interior neighbour.  Which of these a
 // block of eight steps can hold decides among four forms of the step (Class).
 //
-// Four more waves bring operands into LDS by anti-diagonals, where a step of a
+// Four or five more waves bring operands into LDS by anti-diagonals, where a step of a
 // wave reads 64 neighbours, write the results, and exchange lane 63's values
 // with the strips above and below, which run on other CUs: agent-scope stores
 // and loads in device memory, and a progress count per strip.  (Two waves took
 // 4400 cycles per block for that and three 2900, when the sweeps took 3000 and
 // 2000.)  A strip trails the one above it by about 90 steps: 64 of skew, the
 // blocks of 8, a store and a load; taking lane 0's values a block earlier than
-// they are needed made it 8 more (N=1024 1.75 ms instead of 1.60).  Workgroups
+// they are needed made it 8 more (N=1024 1.75 ms per frame, then 1.60).  Workgroups
 // take their strip from a ticket counter whose
 // order puts every strip after the one it reads from, so a waiting workgroup
 // always waits for one that already runs: the launch ends whatever share of
@@ -125,7 +125,11 @@ __device__ __forceinline__ void agent_store(T* p, T v) {
 template <int W>
 struct Lex {
 static constexpr int QMAX = (LEX_KMAX + W - 1) / W, KMAX = LEX_KMAX, B = LEX_B;
-static constexpr int NT = 64 * (W + 4);  // W waves of sweeps, four that move data
+// Waves that move data: with four waves of sweeps four (16 waves of two
+// workgroups fill a CU), else the final values have one of their own (with the
+// hand-off they took up to 3700 cycles per block, the sweeps 2600).
+static constexpr int NH = W == 4 ? 4 : 5;
+static constexpr int NT = 64 * (W + NH);
 static_assert(QMAX <= 5 && W <= 16 && B == 8, "waves of up to five sweeps, blocks of 8 steps");
 // x0 in LDS by anti-diagonals: row u = c + j - 63 s + 1 of a ring of XR rows,
 // position p = j - 63 s + KMAX (sweep k at step t reads row t - 3k, lane r
@@ -388,7 +392,7 @@ static __device__ __forceinline__ Part part_of(int w, int steps, int K) {
 }
 
 // One strip of one round (K sweeps) of a lin_solve.  Waves 0..W-1 run the
-// sweeps; waves W .. W+3 bring operands into LDS a block ahead, write the
+// sweeps; waves W and on bring operands into LDS a block ahead, write the
 // results, and talk to the neighbouring strips, so that their loads'
 // latencies and the waits for the strip above stay out of the sweeps.
 // In block b of the workgroup wave w runs block m = b - w of its steps.
@@ -481,6 +485,70 @@ static __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, cons
     oc[z] = (MODE == M_COL ? B - 2 - it : hf - 1 - it) - 2 * (K - 1);  // + 8 m
     oj[z] = base + ir[z] - (K - 1);
   }
+  // Final values of the round's last sweep (ring Wn, the block before) to x:
+  // interior cells, and in Passive the ring cells that copy them.
+  auto final_values = [&](int b) {
+    if (b < Wn) return;
+    const int m = b - Wn;
+#pragma unroll
+    for (int z = 0; z < ZI; ++z) {
+      if (64 * z + lane >= NIN) continue;
+      const lf* ring = L + (L_RING + (Wn * RR + (m & 1) * B) * RP) + hf * RP;
+      const int c = oc[z] + m * B, j = oj[z];
+      typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+      float v[4];
+      bool ok[4], all = true, some = false;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int ci = MODE == M_COL ? c : c + i, ji = MODE == M_COL ? j + i : j;
+        const int ri = MODE == M_COL ? min(max(ir[z] + i, 0), 63) : ir[z];
+        v[i] = ring[i * RP + ri];
+        ok[i] = ci >= 1 && ci <= S - 2 && ji >= 1 && ji <= S - 2 && (uint32_t)(ir[z] + (MODE == M_COL ? i : 0) - 1) < 63u;
+        all = all && ok[i];
+        some = some || ok[i];
+      }
+      f4u vv;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) vv[i] = v[i];
+      float* o = x + (MODE == M_COL ? c * S + j : j * S + c);
+      if (all) {
+        *(f4u*)o = vv;
+      } else if (some) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (ok[i]) o[i] = v[i];
+      }
+      if constexpr (MODE == M_PASSIVE) {
+        const int Sc = rm_code_stride(S);
+        if (some && (j == 1 || j == S - 2)) {  // the rows above / below the interior
+          for (int side = 0; side < 2; ++side) {
+            if (j != (side ? S - 2 : 1)) continue;
+            const int y = side ? S - 1 : 0;
+            if (all && ring_copies) {
+              *(f4u*)(x + y * S + c) = vv;
+            } else {
+#pragma unroll
+              for (int i = 0; i < 4; ++i)
+                if (ok[i] && (ring_copies || (d.code[y * Sc + c + i] >> R_PAS_SHIFT))) x[y * S + c + i] = v[i];
+            }
+          }
+        }
+        if (some && c <= 1) {  // the column left of it (c + 3 >= 1: some cell is in the interior)
+          float e = v[0];
+#pragma unroll
+          for (int i = 1; i < 4; ++i) e = c + i == 1 ? v[i] : e;
+          if (ring_copies || (d.code[j * Sc] >> R_PAS_SHIFT)) x[j * S] = e;
+        }
+        if (some && c + 3 >= S - 2) {  // the column right of it
+          float e = v[0];
+#pragma unroll
+          for (int i = 1; i < 4; ++i) e = c + i == S - 2 ? v[i] : e;
+          if (ring_copies || (d.code[j * Sc + S - 1] >> R_PAS_SHIFT)) x[j * S + S - 1] = e;
+        }
+      }
+    }
+  };
+
   if (w == W) {  // x0
     const rsrc_t rx0 = make_rsrc(x0 - FLD_PAD, fbytes);
     constexpr int NX = 2 * (CP - 1) + (MODE == M_COL ? 2 * (B - 1) : 0);
@@ -496,33 +564,34 @@ static __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, cons
       xoff[z] = (MODE == M_COL ? xc[z] * S + xj[z] : xj[z] * S + xc[z]) * 4 + FLD_PAD * 4;
       xring[z] = MODE == M_COL ? (uint32_t)(xj[z] + 3) <= 3u || (uint32_t)(S - 1 - xj[z]) <= 3u : xj[z] == 0 || xj[z] == S - 1;
     }
-    u4 gx0[3], gring[3];
-    bool ring_w[3] = {false, false, false};  // some item of the pass holds a ring cell (wave-uniform)
-#pragma unroll
-    for (int z = 0; z < 3; ++z) gx0[z] = gring[z] = (u4)(0);
-    auto load = [&](int ub) {  // rows 8 ub - UOFF .. of x0 (for ring cells, the value they hold)
+    struct Rows {
+      u4 x0[3], ring[3];
+      bool ring_w[3];  // some item of the pass holds a ring cell (wave-uniform)
+    };
+    auto load = [&](Rows& t, int ub) {  // rows 8 ub - UOFF .. of x0 (for ring cells, the value they hold)
 #pragma unroll
       for (int z = 0; z < 3; ++z) {
         const int c = xc[z] + ub * B, off = xoff[z] + ub * B * stepc * 4;
         // holds a ring cell (or one beyond the grid)
         const bool rg = xring[z] || (MODE == M_COL ? c == 0 || c == S - 1 : (uint32_t)(c + 3) <= 3u || (uint32_t)(S - 1 - c) <= 3u);
-        ring_w[z] = __builtin_amdgcn_ballot_w64(rg) != 0;
-        gx0[z] = __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(rx0, off, 0, 0));
-        if (ring_w[z]) gring[z] = __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(rx, off, 0, 0));
+        t.ring_w[z] = __builtin_amdgcn_ballot_w64(rg) != 0;
+        t.x0[z] = __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(rx0, off, 0, 0));
+        t.ring[z] = (u4)(0);
+        if (t.ring_w[z]) t.ring[z] = __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(rx, off, 0, 0));
       }
     };
-    auto put = [&](int ub) {
+    auto put = [&](const Rows& t, int ub) {
       const int row = (ub * B) % XR;
 #pragma unroll
       for (int z = 0; z < 3; ++z) {
         uint32_t v[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = gx0[z][i];
-        if (ring_w[z]) {
+        for (int i = 0; i < 4; ++i) v[i] = t.x0[z][i];
+        if (t.ring_w[z]) {
           const int c = xc[z] + ub * B;
 #pragma unroll
           for (int i = 0; i < 4; ++i)
-            v[i] = is_ring(MODE == M_COL ? c : c + i, MODE == M_COL ? xj[z] + i : xj[z]) ? gring[z][i] : v[i];
+            v[i] = is_ring(MODE == M_COL ? c : c + i, MODE == M_COL ? xj[z] + i : xj[z]) ? t.ring[z][i] : v[i];
         }
         lu* q = (lu*)L + (L_X0 + row * XP) + hf * XP;
         if (64 * z + lane < NX) {
@@ -536,20 +605,35 @@ static __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, cons
         }
       }
     };
-    for (int ub = 5; ub < 8; ++ub) {  // rows of the cells left of column 0's diagonal
-      load(ub);
-      put(ub);
-    }
-    load(UOFF / B);
+    // First the rows of the cells left of column 0's diagonal (5 .. 7), two groups
+    // in flight: a launch's start is a few memory latencies, of a solve of 32 us at
+    // N=30.
+    static_assert(UOFF / B == 8, "rows before the first block");
+    Rows g0, g1;
+    load(g0, 5);
+    load(g1, 6);
+    put(g0, 5);
+    load(g0, 7);
+    put(g1, 6);
+    load(g1, 8);
+    put(g0, 7);
     for (int b = -1; b < NI; ++b) {
-      if (b + 1 < NB) put(b + 1 + UOFF / B);
-      if (b + 2 < NB) load(b + 2 + UOFF / B);
+      if (b + 1 < NB) put(g1, b + 1 + UOFF / B);
+      if (b + 2 < NB) load(g1, b + 2 + UOFF / B);
       __syncthreads();
     }
     return;
   }
 
-  if (w == W + 2) {  // lane 63's values for the strip below, and the final values
+  if (NH > 4 && w == W + 4) {
+    for (int b = -1; b < NI; ++b) {
+      final_values(b);
+      __syncthreads();
+    }
+    return;
+  }
+
+  if (w == W + 2) {  // lane 63's values for the strip below (and the final values)
     float* hout = Hb + tk.hoff;
     uint32_t* fown = flags + tk.flag;
     for (int b = -1; b < NI; ++b) {
@@ -562,62 +646,7 @@ static __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, cons
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the stores are in memory: publish them
         if (lane == 0) agent_store(fown, (uint32_t)b);
       }
-      // Final values of the round's last sweep (ring Wn, the block before) to x:
-      // interior cells, and in Passive the ring cells that copy them.
-      if (b >= Wn) {
-        const int m = b - Wn;
-  #pragma unroll
-        for (int z = 0; z < ZI; ++z) {
-          if (64 * z + lane >= NIN) continue;
-          const lf* ring = L + (L_RING + (Wn * RR + (m & 1) * B) * RP) + hf * RP;
-          const int c = oc[z] + m * B, j = oj[z];
-          float v[4];
-          bool ok[4], all = true, some = false;
-  #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int ci = MODE == M_COL ? c : c + i, ji = MODE == M_COL ? j + i : j;
-            const int ri = MODE == M_COL ? min(max(ir[z] + i, 0), 63) : ir[z];
-            v[i] = ring[i * RP + ri];
-            ok[i] = ci >= 1 && ci <= S - 2 && ji >= 1 && ji <= S - 2 && (uint32_t)(ir[z] + (MODE == M_COL ? i : 0) - 1) < 63u;
-            all = all && ok[i];
-            some = some || ok[i];
-          }
-          float* o = x + (MODE == M_COL ? c * S + j : j * S + c);
-          if (all) {
-            typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
-            f4u vv;
-  #pragma unroll
-            for (int i = 0; i < 4; ++i) vv[i] = v[i];
-            *(f4u*)o = vv;
-          } else if (some) {
-  #pragma unroll
-            for (int i = 0; i < 4; ++i)
-              if (ok[i]) o[i] = v[i];
-          }
-          if constexpr (MODE == M_PASSIVE) {
-            if (some && (j == 1 || j == S - 2 || c <= 1 || c + 3 >= S - 2)) {
-              const int Sc = rm_code_stride(S);
-              if (j == 1 || j == S - 2) {  // the rows above / below the interior
-                for (int side = 0; side < 2; ++side) {
-                  if (j != (side ? S - 2 : 1)) continue;
-                  const int y = side ? S - 1 : 0;
-  #pragma unroll
-                  for (int i = 0; i < 4; ++i)
-                    if (ok[i] && (ring_copies || (d.code[y * Sc + c + i] >> R_PAS_SHIFT))) x[y * S + c + i] = v[i];
-                }
-              }
-              float e = v[0];  // the columns left / right of it
-  #pragma unroll
-              for (int i = 1; i < 4; ++i) e = c + i == 1 ? v[i] : e;
-              if (c <= 1 && c + 3 >= 1 && (ring_copies || (d.code[j * Sc] >> R_PAS_SHIFT))) x[j * S] = e;
-              e = v[0];
-  #pragma unroll
-              for (int i = 1; i < 4; ++i) e = c + i == S - 2 ? v[i] : e;
-              if (c <= S - 2 && c + 3 >= S - 2 && (ring_copies || (d.code[j * Sc + S - 1] >> R_PAS_SHIFT))) x[j * S + S - 1] = e;
-            }
-          }
-        }
-      }
+      if constexpr (NH == 4) final_values(b);
       __syncthreads();
     }
     if (has_next) {
@@ -635,27 +664,29 @@ static __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, cons
     constexpr int NC = 2 * (CP - 1);
     static_assert(NC <= 192, "three passes");
     int coff[3], cc[3];
-    u2 gc[3];
+    struct Words {
+      u2 c[3];
+    };
 #pragma unroll
     for (int z = 0; z < 3; ++z) {
       const int it = (64 * z + lane) >> 1;
       cc[z] = hf - it + KMAX - 1 - UOFF;  // + 8 ub: first logical column
       coff[z] = min(max(base + it - (KMAX - 1), 0), S - 1) * Sc + hf - it + KMAX - 1 - UOFF + CODE_PAD;
     }
-    auto load = [&](int ub) {
+    auto load = [&](Words& t, int ub) {
 #pragma unroll
       for (int z = 0; z < 3; ++z)
-        gc[z] = __builtin_bit_cast(u2, __builtin_amdgcn_raw_buffer_load_b64(rc, (coff[z] + ub * B) & ~3, 0, 0));
+        t.c[z] = __builtin_bit_cast(u2, __builtin_amdgcn_raw_buffer_load_b64(rc, (coff[z] + ub * B) & ~3, 0, 0));
     };
     uint32_t h_rule = 0, h_col = 0;
-    auto put = [&](int ub) {
+    auto put = [&](const Words& t, int ub) {
       const int row = (ub * B) % XR;
       uint32_t any = 0;
       bool cols = false;
 #pragma unroll
       for (int z = 0; z < 3; ++z)
         if (64 * z + lane < NC) {
-          const uint32_t sel = selectors<MODE>(__builtin_amdgcn_alignbyte(gc[z].y, gc[z].x, (uint32_t)((coff[z] + ub * B) & 3)));
+          const uint32_t sel = selectors<MODE>(__builtin_amdgcn_alignbyte(t.c[z].y, t.c[z].x, (uint32_t)((coff[z] + ub * B) & 3)));
           lu* cq = (lu*)L + (L_CODE + (row >> 2) * CP) + (hf >> 2) * CP + ((64 * z + lane) >> 1);
           cq[0] = sel;
           if (row == 0) cq[CR * CP] = sel;
@@ -684,20 +715,23 @@ static __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, cons
       c = (h_rule & cmask) ? C_ALL : c;
       if (lane < W) ((lb*)(L + L_CL))[(nb & 3) * 16 + lane] = (uint8_t)c;
     };
-    for (int ub = 5; ub < 8; ++ub) {  // rows of the cells left of column 0's diagonal
-      load(ub);
-      put(ub);
-    }
-    load(UOFF / B);
+    Words g5, g6, g7, g;
+    load(g5, 5);
+    load(g6, 6);
+    load(g7, 7);
+    load(g, 8);
+    put(g5, 5);
+    put(g6, 6);
+    put(g7, 7);
     for (int b = -1; b < NI; ++b) {
       if (b + 1 < NB) {
-        put(b + 1 + UOFF / B);
+        put(g, b + 1 + UOFF / B);
       } else {
         h_rule <<= 1;
         h_col <<= 1;
       }
       classes(b + 1);
-      if (b + 2 < NB) load(b + 2 + UOFF / B);
+      if (b + 2 < NB) load(g, b + 2 + UOFF / B);
       __syncthreads();
     }
     return;
@@ -831,8 +865,9 @@ void lex_launch(hipStream_t st, const RbScene* scs, const LexTask* tasks, int nt
   };
   // Up to one workgroup per CU (256 of them) the chain of blocks bounds the
   // launch: eight waves of up to three sweeps take a block faster than four of up
-  // to five (a frame of N=1024 1.60 ms instead of 1.77, N=128 0.287 instead of
-  // 0.323; seven and ten waves lie within 3 % of eight).  Beyond that two
+  // to five (a frame of N=1024 1.75 ms instead of 1.85, N=128 0.295 instead of
+  // 0.332, before what is said above of the other waves; seven and ten lie within
+  // 3 % of eight).  Beyond that two
   // workgroups of four fit a CU, one of eight does not leave room for another.
   if (ntasks <= 256) launch(std::integral_constant<int, 8>());
   else launch(std::integral_constant<int, 4>());

@@ -865,10 +865,10 @@ void lex_launch(hipStream_t st, const RbScene* scs, const LexTask* tasks, int nt
   };
   // Up to one workgroup per CU (256 of them) the chain of blocks bounds the
   // launch: eight waves of up to three sweeps take a block faster than four of up
-  // to five (a frame of N=1024 1.75 ms instead of 1.85, N=128 0.295 instead of
-  // 0.332, before what is said above of the other waves; seven and ten lie within
-  // 3 % of eight).  Beyond that two
-  // workgroups of four fit a CU, one of eight does not leave room for another.
+  // to five (a frame of N=1024 1.48 ms instead of 1.76, N=128 0.265 instead of
+  // 0.318, N=30 0.120 instead of 0.131; seven 1.58 at N=1024, ten as eight).
+  // Beyond that two workgroups of four fit a CU, one of eight does not leave room
+  // for another.
   if (ntasks <= 256) launch(std::integral_constant<int, 8>());
   else launch(std::integral_constant<int, 4>());
 }

@@ -1190,7 +1190,7 @@ static void g_lex(hipStream_t st, const RbGroup& g, bool press, const LexSpec& s
   for (int r = 0; r < (press ? g.press_rounds : g.diff_rounds); ++r) {
     const LexArgs a{{s0, s1, s2}, r, press ? 1 : 0};
     lex_launch(st, g.d_scs, press ? g.d_lpress : g.d_ldiff, press ? g.n_lpress : g.n_ldiff, a, ctl, g.n_lflags, H,
-               g.h_err);
+               g.h_err, g.maxN);
   }
 }
 static void g_pressure(hipStream_t st, const RbGroup& g, int p, int div) {

@@ -137,9 +137,9 @@ struct LexArgs {
 // Polls of about a microsecond a strip waits for the one above before it gives up (and reports).
 constexpr uint32_t LEX_SPIN_MAX = 1u << 22;
 // ctl: ticket, ended workgroups, then nflags progress counts, all zero before
-// the first launch; a launch leaves them zero.
+// the first launch; a launch leaves them zero.  maxN: the largest scene's.
 void lex_launch(hipStream_t st, const RbScene* scs, const LexTask* tasks, int ntasks, const LexArgs& args,
-                uint32_t* ctl, int nflags, float* H, uint32_t* err);
+                uint32_t* ctl, int nflags, float* H, uint32_t* err, int maxN);
 
 // Frames (eqf_frame.hip).  A launch group's scenes share one mode.
 void* frame_create(eqf_scene* s, std::string& err);

@@ -856,7 +856,7 @@ __global__ void __launch_bounds__(Lex<W>::NT, W == 4 ? 4 : 3)
 }  // namespace lex
 
 void lex_launch(hipStream_t st, const RbScene* scs, const LexTask* tasks, int ntasks, const LexArgs& args,
-                uint32_t* ctl, int nflags, float* H, uint32_t* err) {
+                uint32_t* ctl, int nflags, float* H, uint32_t* err, int maxN) {
   if (ntasks <= 0) return;
   auto launch = [&](auto w) {
     typedef lex::Lex<decltype(w)::value> X;
@@ -867,9 +867,14 @@ void lex_launch(hipStream_t st, const RbScene* scs, const LexTask* tasks, int nt
   // launch: eight waves of up to three sweeps take a block faster than four of up
   // to five (a frame of N=1024 1.48 ms instead of 1.76, N=128 0.265 instead of
   // 0.318, N=30 0.120 instead of 0.131; seven 1.58 at N=1024, ten as eight).
-  // Beyond that two workgroups of four fit a CU, one of eight does not leave room
-  // for another.
-  if (ntasks <= 256) launch(std::integral_constant<int, 8>());
+  // Two workgroups of four fit a CU, one of eight does not leave room for
+  // another, but up to three per CU the faster blocks still win (64 scenes of
+  // N=256 0.93 ms instead of 1.02, 24 of N=1024 3.42 instead of 3.81, a mix of 130
+  // 1.79 instead of 1.95) unless the strips are so short that filling eight
+  // waves weighs (100 scenes of N=128 0.595 instead of 0.565, 300 of N=64 0.574
+  // instead of 0.552).  Beyond that four waves win (the mix of 512 5.38 ms, 6.04
+  // with eight).
+  if (ntasks <= 256 || (ntasks <= 768 && maxN >= 192)) launch(std::integral_constant<int, 8>());
   else launch(std::integral_constant<int, 4>());
 }
 

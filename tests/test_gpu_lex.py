@@ -90,10 +90,11 @@ def test_batch_of_different_iteration_counts_equals_oracle():
         s.close()
 
 
-@pytest.mark.parametrize("n", [20, 90])  # fewer strips than CUs (eight waves of sweeps each), more (four)
-def test_batches_either_side_of_the_wave_count_equal_oracle(n):
-    print(f"[case] lex batch of {n}", flush=True)
-    specs = [(20 + 13 * (i % 9), 1 + i % 23, 1 + (7 * i) % 22) for i in range(n)]
+# fewer strips than CUs (eight waves of sweeps each); more (four); more, long ones (eight); many (four)
+@pytest.mark.parametrize("n,step", [(20, 13), (90, 13), (40, 40), (90, 40)])
+def test_batches_either_side_of_the_wave_count_equal_oracle(n, step):
+    print(f"[case] lex batch of {n}, {step}", flush=True)
+    specs = [(20 + step * (i % 9), 1 + i % 23, 1 + (7 * i) % 22) for i in range(n)]
     trio = [_pair(S, it, pr, 0.05, 900 + i) for i, (S, it, pr) in enumerate(specs)]
     b = _abi.Batch([s for s, _, _ in trio])
     b.step(2)

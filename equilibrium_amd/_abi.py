@@ -113,6 +113,7 @@ def lib():
             "eqf_last_error": (ctypes.c_char_p, []),
             "eqf_ctx_create": (I, [I, PP]),
             "eqf_ctx_destroy": (I, [P]),
+            "eqf_ctx_set_wait_limit": (I, [P, U32]),
             "eqf_ctx_device_key": (I, [P, ctypes.c_char_p, ctypes.c_size_t]),
             "eqf_scene_create": (I, [P, ctypes.POINTER(Params), PP]),
             "eqf_scene_clone": (I, [P, PP]),
@@ -197,6 +198,11 @@ class Context:
         h = ctypes.c_void_p()
         check(lib().eqf_ctx_create(device, ctypes.byref(h)))
         self.h = h
+
+    def set_wait_limit(self, polls):
+        """How often a strip of the exact mode looks for the one above it before
+        it gives up (eqf_ctx_set_wait_limit)."""
+        check(lib().eqf_ctx_set_wait_limit(self.h, polls))
 
     def device_key(self):
         """'<device name>/<gfx arch>/<CU count>' of the context's GPU."""

@@ -29,6 +29,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstring>
 #include <string>
 #include <vector>
@@ -906,6 +907,8 @@ struct RbGroup {
   void* d_lex = nullptr;
   size_t lex_bytes = 0;
   uint32_t* h_err = nullptr;
+  uint32_t polls = 0;              // eqf_ctx::wait_polls that the graph holds
+  std::atomic<bool> stale{false};  // a wait gave up: the counters have to be set up again
   int n = 0, maxN = 0, tiles[3] = {0, 0, 0}, iblocks = 0, cblocks = 0, ablocks = 0;
   bool any_src = false;
   int ntmp = 1;  // red-black: ping-pong fields of every scene
@@ -917,6 +920,8 @@ struct RbGroup {
   uint64_t key = 0;  // what the table and the graph were built for
   int64_t key_frames = 0;  // frames launched since
 };
+
+constexpr uint32_t kAllFields = (1u << NFIELDS) - 1;
 
 struct FrameWork {
   float* tmp[3] = {nullptr, nullptr, nullptr};  // ping-pong fields: one, or one per diffusion
@@ -954,6 +959,7 @@ static uint64_t group_key(const RbGroup& g) {
     for (uint64_t w : words) mix(w);
   }
   mix((uint64_t)g.tile * 16 + (uint64_t)g.tsweeps);
+  mix(g.polls);
   return key;
 }
 
@@ -1188,7 +1194,7 @@ static void g_lex(hipStream_t st, const RbGroup& g, bool press, const LexSpec& s
   uint32_t* ctl = (uint32_t*)g.d_lex;
   float* H = (float*)((char*)g.d_lex + lex_ctl_bytes(g.n_lflags));
   for (int r = 0; r < (press ? g.press_rounds : g.diff_rounds); ++r) {
-    const LexArgs a{{s0, s1, s2}, r, press ? 1 : 0};
+    const LexArgs a{{s0, s1, s2}, r, press ? 1 : 0, g.polls};
     lex_launch(st, g.d_scs, press ? g.d_lpress : g.d_ldiff, press ? g.n_lpress : g.n_ldiff, a, ctl, g.n_lflags, H,
                g.h_err, g.maxN);
   }
@@ -1302,8 +1308,11 @@ static int group_step(RbGroup& g, hipStream_t st, int64_t nframes, std::string& 
         err = "red-black scenes of one batch need the same iteration counts";
         return EQF_EINVAL;
       }
+  for (eqf_scene* s : g.scenes)
+    if (s->invalid.load()) s->invalid.store(kAllFields);  // a frame mixes the fields
+  g.polls = g.scenes[0]->ctx->wait_polls.load();
   const uint64_t key = group_key(g);
-  if (!g.d_tab || key != g.key || g.tab_tile != g.tile || g.tab_T != g.tsweeps) {
+  if (g.stale.exchange(false) || !g.d_tab || key != g.key || g.tab_tile != g.tile || g.tab_T != g.tsweeps) {
     int rc = group_tables(g, st, err);
     if (rc) {
       g.tab_tile = -1;  // not usable
@@ -1385,9 +1394,9 @@ int frame_step(eqf_scene* s, int64_t nframes, std::string& err) {
   return group_step(w->one, s->stream, nframes, err);
 }
 
-bool frame_failed(const eqf_scene* s) {
-  const auto* w = static_cast<const FrameWork*>(s->work);
-  return w && w->one.h_err && *(volatile const uint32_t*)w->one.h_err != 0;
+bool frame_collect(const eqf_scene* s) {
+  auto* w = static_cast<FrameWork*>(s->work);
+  return w && group_collect(&w->one);
 }
 
 // Batches (eqf_runtime.hip) and server lanes: one group over all scenes.
@@ -1424,9 +1433,15 @@ void group_set_scenes(void* p, const std::vector<eqf_scene*>& scenes) {
   auto* g = static_cast<RbGroup*>(p);
   g->scenes = scenes;  // a new membership changes the key: tables and graph are rebuilt
 }
-bool group_failed(const void* p) {
-  const auto* g = static_cast<const RbGroup*>(p);
-  return g && g->h_err && *(volatile const uint32_t*)g->h_err != 0;
+bool group_collect(void* p) {
+  auto* g = static_cast<RbGroup*>(p);
+  if (!g || !g->h_err || __atomic_exchange_n(g->h_err, 0u, __ATOMIC_ACQ_REL) == 0) return false;
+  for (eqf_scene* s : g->scenes) {
+    s->invalid.store(kAllFields);
+    s->failures.fetch_add(1);
+  }
+  g->stale.store(true);
+  return true;
 }
 
 }  // namespace eqf

@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <memory>
 #include <mutex>
 #include <string>
@@ -38,9 +39,14 @@ class HostStaging {
   int nfree_ = 0;
 };
 
+// Polls of about a microsecond that a strip of a lexicographic lin_solve waits
+// for the one above before it gives up and reports (eqf_ctx_set_wait_limit).
+constexpr uint32_t LEX_POLLS = 1u << 22;
+
 struct eqf_ctx {
   int device;
   std::shared_ptr<HostStaging> staging;
+  std::atomic<uint32_t> wait_polls{LEX_POLLS};
 };
 
 struct eqf_scene {
@@ -63,6 +69,10 @@ struct eqf_scene {
   float* d_stage = nullptr;   // staging for eqf_add_source (lazy)
   uint8_t* d_mask = nullptr;  // mask + scratch for the boundary build (lazy)
   eqf::SceneDesc desc{};
+  // Fields (a bit each) whose contents a failed frame left undefined, until they
+  // are uploaded whole; frames that failed so far (frame_collect).
+  std::atomic<uint32_t> invalid{0}, failures{0};
+  struct eqf_snapshot* rings = nullptr;  // its snapshot rings (eqf_render.hip)
   int in_batch = 0;
   // Batch membership: the batch advances the scene on its own stream.  Work
   // queued on the scene's stream meanwhile first waits for the batch's last
@@ -94,6 +104,11 @@ int eqf_internal_scratch_init(int device);
 // Orders work about to be queued on the scene's stream after the last step of
 // the scene's batch (no-op outside a batch).
 int eqf_internal_scene_enter(eqf_scene* s);
+// EQF_EDEVICE if a frame that has ended failed and left one of `fields` (a bit
+// each) undefined.
+int eqf_internal_check(const eqf_scene* s, uint32_t fields);
+// The scene goes; its snapshot rings keep their captures.
+void eqf_internal_rings_drop(eqf_scene* s);
 int eqf_internal_check_params(const eqf_params* p);
 // eqf_scene_create on a caller-owned stream (the server's admission stream),
 // allocating from `pool` in that stream's order when `pool` is set.
@@ -133,9 +148,8 @@ struct LexSpec {
 struct LexArgs {
   LexSpec sp[3];
   int round, press;  // round of sweeps; which iteration count (0 diffusion, 1 pressure)
+  uint32_t polls;    // how often a strip looks for the one above before it gives up (and reports)
 };
-// Polls of about a microsecond a strip waits for the one above before it gives up (and reports).
-constexpr uint32_t LEX_SPIN_MAX = 1u << 22;
 // ctl: ticket, ended workgroups, then nflags progress counts, all zero before
 // the first launch; a launch leaves them zero.  maxN: the largest scene's.
 void lex_launch(hipStream_t st, const RbScene* scs, const LexTask* tasks, int ntasks, const LexArgs& args,
@@ -152,9 +166,11 @@ void group_destroy(void* g);
 int group_set_tiling(void* g, int tile, int tsweeps);
 int group_step_frames(void* g, int64_t nframes, std::string& err);
 void group_set_scenes(void* g, const std::vector<eqf_scene*>& scenes);
-// Whether a wait inside a kernel of the group gave up (never in a sound run).
-bool group_failed(const void* g);
-bool frame_failed(const eqf_scene* s);
+// A wait inside a kernel of the group that gave up (never in a sound run): marks
+// its scenes (eqf_scene::invalid, failures), and lets the next step set the
+// group's counters up again.  For frames that have ended.
+bool group_collect(void* g);
+bool frame_collect(const eqf_scene* s);
 // Device bytes of the lexicographic hand-off of one scene.
 int64_t lex_workspace_bytes(int S);
 }  // namespace eqf

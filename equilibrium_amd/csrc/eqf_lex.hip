@@ -399,7 +399,7 @@ static __device__ __forceinline__ Part part_of(int w, int steps, int K) {
 template <int MODE>
 static __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, const LexTask& tk, const LexSpec& sp, int K,
                                            uint32_t* __restrict__ flags, float* __restrict__ Hb,
-                                           uint32_t* __restrict__ err) {
+                                           uint32_t* __restrict__ err, uint32_t polls) {
   const SceneDesc& d = sc.d;
   const int S = d.S;
   const int tid = threadIdx.x, lane = tid & 63, w = uni(tid >> 6);
@@ -768,7 +768,7 @@ static __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, cons
         credit = (uint32_t)uni((int)agent_load(fprev));
         if (credit < need) {
           __builtin_amdgcn_s_sleep(1);
-          if (++spins > LEX_SPIN_MAX) {  // cannot happen (see the file comment); never wait for ever
+          if (++spins > polls) {  // cannot happen (see the file comment); never wait for ever
             dead = true;
             if (lane == 0) __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
           }
@@ -833,15 +833,18 @@ __global__ void __launch_bounds__(Lex<W>::NT, W == 4 ? 4 : 3)
   if (threadIdx.x == 0) ((lu*)L)[X::L_MISC] = atomicAdd(&ctl[0], 1u);
   __syncthreads();
   const int t = uni((int)((lu*)L)[X::L_MISC]);
-  if (t >= ntasks) return;  // the counters were not zero at the start: nothing is sound then
+  if (t >= ntasks) {  // the counters were not zero at the start: nothing is sound then
+    if (threadIdx.x == 0) __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    return;
+  }
   const LexTask tk = tasks[t];
   const RbScene& sc = scs[tk.scene];
   const LexSpec sp = args.sp[tk.slot];
   const int K = lex_round_sweeps(args.press ? sc.d.press_iters : sc.d.diff_iters, args.round);
   if (K > 0) {
-    if (sp.mode == M_ROW) X::template strip_task<M_ROW>(L, sc, tk, sp, K, flags, H, err);
-    else if (sp.mode == M_COL) X::template strip_task<M_COL>(L, sc, tk, sp, K, flags, H, err);
-    else X::template strip_task<M_PASSIVE>(L, sc, tk, sp, K, flags, H, err);
+    if (sp.mode == M_ROW) X::template strip_task<M_ROW>(L, sc, tk, sp, K, flags, H, err, args.polls);
+    else if (sp.mode == M_COL) X::template strip_task<M_COL>(L, sc, tk, sp, K, flags, H, err, args.polls);
+    else X::template strip_task<M_PASSIVE>(L, sc, tk, sp, K, flags, H, err, args.polls);
   }
   // The last workgroup to end leaves the counters as the next launch needs them.
   __syncthreads();

@@ -122,12 +122,14 @@ extern "C" int eqf_render_rgba(eqf_scene* s, const eqf_colors* c, uint8_t* rgba_
     if (e != hipSuccess) rc = eqf_internal_error(EQF_EDEVICE, std::string("render copy: ") + hipGetErrorString(e));
   }
   (void)hipFree(d_dens);
-  return rc;
+  return rc ? rc : eqf_internal_check(s, 1u << F_D);
 }
 
 // ---------------------------------------------------------------- snapshots
 struct eqf_snapshot {
-  eqf_scene* scene = nullptr;
+  eqf_scene* scene = nullptr;     // null once it is destroyed
+  eqf_snapshot* next = nullptr;   // the scene's next ring
+  uint32_t failures = 0;          // of a scene that is destroyed
   int device = 0;
   int depth = 0, with_rgba = 0;
   eqf_colors colors{};
@@ -139,12 +141,29 @@ struct eqf_snapshot {
     uint8_t* h_rgba = nullptr;
     hipEvent_t ready = nullptr, done = nullptr;
     int64_t frame = 0;
+    bool invalid = false;   // the density was known to be undefined when it was captured
+    uint32_t failures = 0;  // of the scene, known then
   };
   std::vector<Slot> slots;
   int head = 0, count = 0;  // oldest capture, captures held
 };
 
+void eqf_internal_rings_drop(eqf_scene* s) {
+  if (s->rings) (void)eqf_internal_check(s, 0);
+  for (eqf_snapshot* sn = s->rings; sn; sn = sn->next) {
+    sn->failures = s->failures.load();
+    sn->scene = nullptr;
+  }
+  s->rings = nullptr;
+}
+
 static void snapshot_free(eqf_snapshot* sn) {
+  if (sn->scene)
+    for (eqf_snapshot** p = &sn->scene->rings; *p; p = &(*p)->next)
+      if (*p == sn) {
+        *p = sn->next;
+        break;
+      }
   for (auto& sl : sn->slots) {
     (void)hipFree(sl.d_dens);
     (void)hipHostFree(sl.h_dens);
@@ -160,6 +179,8 @@ extern "C" int eqf_snapshot_create(eqf_scene* s, int depth, int with_rgba, const
   hipError_t e = hipSetDevice(s->ctx->device);
   auto* sn = new eqf_snapshot;
   sn->scene = s;
+  sn->next = s->rings;
+  s->rings = sn;
   sn->device = s->ctx->device;
   sn->depth = depth;
   sn->with_rgba = with_rgba ? 1 : 0;
@@ -191,6 +212,7 @@ extern "C" int eqf_snapshot_capture(eqf_snapshot* sn, int64_t frame) {
   if (!sn) return eqf_internal_error(EQF_EINVAL, "snapshot is NULL");
   if (sn->count == sn->depth) return eqf_internal_error(EQF_EBUSY, "every snapshot slot holds an unreleased capture");
   eqf_scene* s = sn->scene;
+  if (!s) return eqf_internal_error(EQF_EINVAL, "the snapshot's scene is destroyed");
   if (int rc = eqf_internal_scene_enter(s)) return rc;
   hipError_t e = hipSetDevice(s->ctx->device);
   if (e != hipSuccess) return eqf_internal_error(EQF_EDEVICE, hipGetErrorString(e));
@@ -210,6 +232,8 @@ extern "C" int eqf_snapshot_capture(eqf_snapshot* sn, int64_t frame) {
   if (e == hipSuccess) e = hipEventRecord(sl.done, sn->copy);
   if (e != hipSuccess) return eqf_internal_error(EQF_EDEVICE, std::string("snapshot: ") + hipGetErrorString(e));
   sl.frame = frame;
+  sl.invalid = s->invalid.load() & (1u << F_D);
+  sl.failures = s->failures.load();
   ++sn->count;
   return EQF_OK;
 }
@@ -220,6 +244,12 @@ extern "C" int eqf_snapshot_acquire(eqf_snapshot* sn, int64_t* frame, const floa
   auto& sl = sn->slots[sn->head];
   hipError_t e = hipEventSynchronize(sl.done);
   if (e != hipSuccess) return eqf_internal_error(EQF_EDEVICE, std::string("snapshot wait: ") + hipGetErrorString(e));
+  if (sn->scene) {
+    (void)eqf_internal_check(sn->scene, 0);
+    sn->failures = sn->scene->failures.load();
+  }
+  if (sl.invalid || sn->failures != sl.failures)
+    return eqf_internal_error(EQF_EDEVICE, "a lin_solve strip gave up waiting; the capture is not valid");
   if (frame) *frame = sl.frame;
   if (density) *density = sl.h_dens;
   if (rgba) *rgba = sn->with_rgba ? sl.h_rgba : nullptr;
@@ -323,5 +353,5 @@ extern "C" int eqf_render_rgba_noalloc(eqf_scene* s, const eqf_colors* c, uint8_
   e = hipMemcpyAsync(rgba_host, d_rgba, 4 * n, hipMemcpyDeviceToHost, s->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(s->stream);  // the next call may reuse the scratch
   if (e != hipSuccess) return eqf_internal_error(EQF_EDEVICE, std::string("render copy: ") + hipGetErrorString(e));
-  return EQF_OK;
+  return eqf_internal_check(s, 1u << F_D);
 }

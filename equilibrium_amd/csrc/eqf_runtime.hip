@@ -60,16 +60,6 @@ static int upload_rm(eqf_scene* s, float* dfield, const float* host) {
   return eqf_dev_upload(s, dfield, nullptr, host, 0);
 }
 
-// Reported by the calls that wait for frames if a strip gave up waiting for
-// the one above it (see eqf_lex.hip: its order of work rules that out).
-static const char* const kGaveUp = "a lin_solve strip gave up waiting; the scene's fields are not valid";
-static int check_frames(const eqf_scene* s);
-
-static int download_rm(const eqf_scene* cs, const float* dfield, float* host) {
-  const int rc = eqf_dev_download(const_cast<eqf_scene*>(cs), dfield, host);
-  return rc ? rc : check_frames(cs);
-}
-
 // Reference initial state (fluid.rs:93-110, 527-570, 602-606), on the host.
 static void host_init(int S, int times, std::vector<std::vector<float>>& F, std::vector<uint8_t>& m) {
   const size_t n = (size_t)S * S;
@@ -198,6 +188,12 @@ extern "C" int eqf_ctx_destroy(eqf_ctx* ctx) {
   return EQF_OK;
 }
 
+extern "C" int eqf_ctx_set_wait_limit(eqf_ctx* ctx, uint32_t polls) {
+  if (!ctx) return fail(EQF_EINVAL, "ctx is NULL");
+  ctx->wait_polls.store(polls);
+  return EQF_OK;
+}
+
 extern "C" int eqf_ctx_device_key(const eqf_ctx* ctx, char* buf, size_t len) {
   if (!ctx || !buf || len == 0) return fail(EQF_EINVAL, "ctx or buf is NULL, or len is 0");
   hipDeviceProp_t prop;
@@ -229,6 +225,7 @@ void eqf_scene_mfree(eqf_scene* s, void* p) {
 
 static void scene_free(eqf_scene* s) {
   if (!s) return;
+  eqf_internal_rings_drop(s);
   if (s->work) frame_destroy(s);
   if (s->ev_ops) (void)hipEventDestroy(s->ev_ops);
   eqf_scene_mfree(s, s->d_main);
@@ -353,6 +350,8 @@ extern "C" int eqf_scene_clone(const eqf_scene* src, eqf_scene** out) {
     scene_free(s);
     return fail(EQF_EDEVICE, std::string("clone: ") + hipGetErrorString(e));
   }
+  (void)eqf_internal_check(src, 0);  // (its stream has ended)
+  s->invalid.store(src->invalid.load());
   std::string err;
   s->work = frame_create(s, err);
   if (!s->work) {
@@ -536,7 +535,11 @@ extern "C" int eqf_upload(eqf_scene* s, int field, const float* host) {
   int rc = check_field(field);
   if (!rc) rc = eqf_internal_scene_enter(s);
   if (rc) return rc;
-  return upload_rm(s, field_ptr(s, field), host);
+  rc = upload_rm(s, field_ptr(s, field), host);
+  if (rc) return rc;
+  (void)eqf_internal_check(s, 0);  // what frames before the upload left
+  s->invalid.fetch_and(~(1u << field));
+  return EQF_OK;
 }
 
 extern "C" int eqf_download(eqf_scene* s, int field, float* host) {
@@ -544,7 +547,8 @@ extern "C" int eqf_download(eqf_scene* s, int field, float* host) {
   int rc = check_field(field);
   if (!rc) rc = eqf_internal_scene_enter(s);
   if (rc) return rc;
-  return download_rm(s, field_ptr(s, field), host);
+  rc = eqf_dev_download(s, field_ptr(s, field), host);
+  return rc ? rc : eqf_internal_check(s, 1u << field);
 }
 
 extern "C" int eqf_step(eqf_scene* s, int64_t nframes) {
@@ -572,7 +576,7 @@ extern "C" int eqf_sync(eqf_scene* s) {
   if (!s) return fail(EQF_EINVAL, "scene is NULL");
   if (int rc = eqf_internal_scene_enter(s)) return rc;
   HIPCHK(hipStreamSynchronize(s->stream));
-  return check_frames(s);
+  return eqf_internal_check(s, ~0u);
 }
 
 // ------------------------------------------------------------------ batch --
@@ -586,8 +590,13 @@ struct eqf_batch {
   double last_ms = 0.0;
 };
 
-static int check_frames(const eqf_scene* s) {
-  return frame_failed(s) || (s->batch && group_failed(s->batch->group)) ? fail(EQF_EDEVICE, kGaveUp) : EQF_OK;
+// A strip that gave up waiting for the one above it (eqf_lex.hip: its order of
+// work rules that out) makes the fields of its launch's scenes undefined.
+static const char* const kGaveUp = "a lin_solve strip gave up waiting; the scene's fields are not valid";
+int eqf_internal_check(const eqf_scene* s, uint32_t fields) {
+  (void)frame_collect(s);
+  if (s->batch) (void)group_collect(s->batch->group);
+  return s->invalid.load() & fields ? fail(EQF_EDEVICE, kGaveUp) : EQF_OK;
 }
 
 extern "C" int eqf_batch_create(eqf_ctx* ctx, eqf_scene* const* scenes, int n, eqf_batch** out) {
@@ -715,7 +724,10 @@ extern "C" int eqf_batch_sync(eqf_batch* b) {
   HIPCHK(hipStreamSynchronize(b->stream));
   float ms = 0.f;
   if (hipEventElapsedTime(&ms, b->ev0, b->ev1) == hipSuccess) b->last_ms = ms;
-  return group_failed(b->group) ? fail(EQF_EDEVICE, kGaveUp) : EQF_OK;
+  (void)group_collect(b->group);
+  for (const eqf_scene* s : b->scenes)
+    if (s->invalid.load()) return fail(EQF_EDEVICE, kGaveUp);
+  return EQF_OK;
 }
 
 extern "C" int eqf_batch_last_ms(const eqf_batch* b, double* ms) {
@@ -729,6 +741,7 @@ extern "C" int eqf_batch_destroy(eqf_batch* b) {
   (void)hipStreamSynchronize(b->stream);
   for (auto* s : b->scenes)  // work that waits on the batch's events ends before they go
     if (s->ops_pending) (void)hipStreamSynchronize(s->stream);
+  (void)group_collect(b->group);  // its scenes keep what its frames left
   group_destroy(b->group);
   for (auto* s : b->scenes) {
     s->in_batch = 0;

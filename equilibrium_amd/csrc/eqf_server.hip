@@ -221,7 +221,7 @@ static std::string lane_launch(eqf_server* sv, int li) {
     if (!g) break;
     group_set_scenes(g, members);
     if (group_step_frames(g, 1, err) != EQF_OK) break;
-    if (group_failed(g)) {
+    if (group_collect(g)) {
       err = "a lin_solve strip gave up waiting";
       break;
     }

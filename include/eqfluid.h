@@ -88,6 +88,16 @@ int eqf_ctx_destroy(eqf_ctx *ctx);
  * fit in len bytes. */
 int eqf_ctx_device_key(const eqf_ctx *ctx, char *buf, size_t len);
 
+/* No counterpart in the reference.  In the exact mode a strip of rows waits for
+ * the one above it, which always runs or has ended; the wait is bounded all the
+ * same.  Sets how often a strip looks before it gives up (about a microsecond
+ * each; 2^22 until set), for the steps that the context's scenes, batches and
+ * servers queue from then on.  A frame in which a strip gave up leaves all six
+ * fields of its scenes undefined: eqf_sync, eqf_batch_sync, eqf_download, the
+ * renders and eqf_snapshot_acquire (of every capture queued before it was seen)
+ * return EQF_EDEVICE.  A field is valid again once it is uploaded whole. */
+int eqf_ctx_set_wait_limit(eqf_ctx *ctx, uint32_t polls);
+
 /* Fluid::new / Fluid::default (fluid.rs:83-110): allocates the six fields and
  * the mask on the device and writes the reference's initial state. */
 int eqf_scene_create(eqf_ctx *ctx, const eqf_params *p, eqf_scene **out);

@@ -46,6 +46,9 @@ struct Req {
   bool keep_vel = false;
   int state = EQF_REQ_QUEUED;
   bool cancel = false;
+  // a frame or the read-back failed: EQF_REQ_FAILED once retired (until then the
+  // state stays EQF_REQ_ACTIVE: the server's threads use the request)
+  bool failed = false;
   bool forget = false;  // released while queued or resident: dropped from the ticket map once retired
   int64_t frames_done = 0;
   int tick_frames = 1;  // frames of the tick in flight
@@ -172,23 +175,35 @@ static void finish(eqf_server* sv, Req* r) {
   const size_t n = (size_t)r->p.size * r->p.size;
   if (!r->cancel) {
     r->out_d.resize(n);
-    if (eqf_download(r->scene, EQF_DENSITY, r->out_d.data()) != EQF_OK) r->state = EQF_REQ_FAILED;
+    bool ok = eqf_download(r->scene, EQF_DENSITY, r->out_d.data()) == EQF_OK;
     if (r->keep_vel) {
       r->out_u.resize(n);
       r->out_v.resize(n);
-      (void)eqf_download(r->scene, EQF_VX, r->out_u.data());
-      (void)eqf_download(r->scene, EQF_VY, r->out_v.data());
+      ok = ok && eqf_download(r->scene, EQF_VX, r->out_u.data()) == EQF_OK;
+      ok = ok && eqf_download(r->scene, EQF_VY, r->out_v.data()) == EQF_OK;
     }
+    if (!ok) r->failed = true;
   }
   eqf_scene_destroy(r->scene);
   r->scene = nullptr;
 }
 
-// A lane's tick has ended (called with sv->mu held).
-static void lane_tick_done(eqf_server* sv, Lane& L, double now) {
+// State of a retired request.
+static int end_state(const Req* r) {
+  return r->failed ? EQF_REQ_FAILED : r->cancel ? EQF_REQ_CANCELLED : EQF_REQ_DONE;
+}
+
+// A lane's tick has ended (called with sv->mu held); its scenes know whether
+// they failed in it.
+static void lane_tick_done(eqf_server* sv, Lane& L, double now, hipError_t status) {
   const float ms = (float)(now - L.t_launch);
   sv->ticks++;
   for (Req* r : L.ticking) {
+    if (status != hipSuccess || r->scene->invalid.load()) {
+      r->failed = r->cancel = true;
+      sv->thread_error = status != hipSuccess ? hipGetErrorString(status) : "a lin_solve strip gave up waiting";
+      continue;
+    }
     const int f = r->tick_frames;
     r->frames_done += f;
     sv->scene_frames += f;
@@ -221,16 +236,13 @@ static std::string lane_launch(eqf_server* sv, int li) {
     if (!g) break;
     group_set_scenes(g, members);
     if (group_step_frames(g, 1, err) != EQF_OK) break;
-    if (group_collect(g)) {
-      err = "a lin_solve strip gave up waiting";
-      break;
-    }
   }
   if (err.empty()) {
     e = hipEventRecord(L.ev, L.st);
     if (e != hipSuccess) err = hipGetErrorString(e);
   }
   if (!err.empty()) {
+    (void)hipStreamSynchronize(L.st);  // what was queued uses scenes that are retired next
     L.ticking.clear();
     return err;
   }
@@ -275,7 +287,7 @@ static bool admit_one(eqf_server* sv) {
     finish(sv, r);
     std::lock_guard<std::mutex> lk(sv->mu);
     sv->used_bytes -= r->bytes;
-    r->state = r->cancel ? EQF_REQ_CANCELLED : EQF_REQ_DONE;
+    r->state = end_state(r);
     r->t_done = sv->now_ms();
     if (r->forget) sv->reqs.erase(r->ticket);
     return true;
@@ -298,13 +310,14 @@ static void tick_loop(eqf_server* sv) {
   (void)hipSetDevice(sv->ctx->device);
   for (;;) {
     bool progress = false;
-    for (Lane& L : sv->lanes) {
+    for (int li = 0; li < NLANES; ++li) {
+      Lane& L = sv->lanes[li];
       if (!L.busy) continue;
       const hipError_t q = hipEventQuery(L.ev);
       if (q == hipErrorNotReady) continue;
+      for (auto& kv : sv->groups[li]) (void)group_collect(kv.second);
       std::lock_guard<std::mutex> lk(sv->mu);
-      if (q != hipSuccess) sv->thread_error = hipGetErrorString(q);
-      lane_tick_done(sv, L, sv->now_ms());
+      lane_tick_done(sv, L, sv->now_ms(), q);
       progress = true;
     }
     for (int li = 0; li < NLANES; ++li) {
@@ -333,8 +346,7 @@ static void tick_loop(eqf_server* sv) {
         std::lock_guard<std::mutex> lk(sv->mu);
         sv->thread_error = err;
         for (Req* r : L.members) {
-          r->state = EQF_REQ_FAILED;
-          r->cancel = true;  // retired at the next pass
+          r->failed = r->cancel = true;  // retired at the next pass
         }
       }
       progress = true;
@@ -387,7 +399,7 @@ static void work_loop(eqf_server* sv) {
         // never returns while a request still reads as resident
         sv->active.erase(std::find(sv->active.begin(), sv->active.end(), r));
         sv->used_bytes -= r->bytes;
-        if (r->state != EQF_REQ_FAILED) r->state = r->cancel ? EQF_REQ_CANCELLED : EQF_REQ_DONE;
+        r->state = end_state(r);
         r->t_done = sv->now_ms();
         if (r->forget) sv->reqs.erase(r->ticket);
       }

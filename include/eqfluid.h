@@ -95,7 +95,8 @@ int eqf_ctx_device_key(const eqf_ctx *ctx, char *buf, size_t len);
  * servers queue from then on.  A frame in which a strip gave up leaves all six
  * fields of its scenes undefined: eqf_sync, eqf_batch_sync, eqf_download, the
  * renders and eqf_snapshot_acquire (of every capture queued before it was seen)
- * return EQF_EDEVICE.  A field is valid again once it is uploaded whole. */
+ * return EQF_EDEVICE, a served request ends as EQF_REQ_FAILED.  A field is valid
+ * again once it is uploaded whole. */
 int eqf_ctx_set_wait_limit(eqf_ctx *ctx, uint32_t polls);
 
 /* Fluid::new / Fluid::default (fluid.rs:83-110): allocates the six fields and

@@ -2,11 +2,13 @@
 allowed (eqf_ctx_set_wait_limit(0)) makes the second strip give up in its first
 block, every kernel ends as always, and everything that hands the scene's fields
 out says so until they are uploaded again."""
+import time
+
 import numpy as np
 import pytest
 
-from equilibrium_amd import _abi
-from helpers import FIELD_NAMES, assert_bit_equal, download_all
+from equilibrium_amd import _abi, scenes
+from helpers import FIELD_NAMES, assert_bit_equal, download_all, gpu_scene
 
 pytestmark = pytest.mark.gpu
 
@@ -124,4 +126,44 @@ def test_batch_leaves_the_failure_to_its_scenes():
         ctx.set_wait_limit(0)
     for s, _ in pairs:
         s.close()
+    ctx.close()
+
+
+def _until(srv, t, states):
+    for _ in range(20000):
+        st = srv.poll(t)
+        if st.state in states:
+            return st
+        time.sleep(0.001)
+    raise AssertionError(f"ticket {t} still in state {st.state}")
+
+
+def test_served_request_fails_in_the_frame_that_gave_up():
+    """The failure in a request's only (so last) frame is its own; the lane goes on
+    with the next requests, and a cancelled one beside it is not held up."""
+    print("[case] gave up: server", flush=True)
+    ctx = _abi.Context(0)
+    srv = _abi.Server(4 << 30, ctx=ctx)
+    sc = [scenes.stam_scene(500, scenes.derive_seed(60, i), iters=20, frames=1 + i, n_rects=2) for i in range(3)]
+    small = scenes.stam_scene(60, scenes.derive_seed(61), iters=20, frames=3)  # one lane further
+    ended = (_abi.REQ_DONE, _abi.REQ_FAILED, _abi.REQ_CANCELLED)
+    ctx.set_wait_limit(0)
+    ts = [srv.submit(s, keep_velocity=True) for s in sc]
+    for t in ts:
+        st = _until(srv, t, ended)
+        assert st.state == _abi.REQ_FAILED and st.frames_done == 0
+        with pytest.raises(_abi.EqfError):
+            srv.result(t)
+        srv.release(t)
+    ctx.set_wait_limit(1 << 22)
+    ts = [srv.submit(s, keep_velocity=True) for s in sc + [small]]
+    for t, s in zip(ts, sc + [small]):
+        assert _until(srv, t, ended).state == _abi.REQ_DONE
+        g = gpu_scene(s)
+        g.step(s["frames"])
+        g.sync()
+        for f in (_abi.DENSITY, _abi.VX, _abi.VY):
+            assert_bit_equal(srv.result(t, f), g.download(f), f"N={s['size'] - 2} field {f}")
+        g.close()
+    srv.close()
     ctx.close()

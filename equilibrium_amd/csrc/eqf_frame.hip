@@ -899,19 +899,19 @@ struct RbGroup {
   // segment, segments per row}: segments of rows, rows
   int2 *d_tmap[3] = {nullptr, nullptr, nullptr}, *d_cmap = nullptr;
   int4 *d_imap = nullptr, *d_amap = nullptr;
-  // exact mode: strips of the three diffusions and of a pressure solve, in
-  // ticket order; counters; hand-off values; where a wait reports that it gave up
+  // exact mode: strips of the three diffusions (of one of them where a scene has
+  // one slot) and of a pressure solve, in ticket order; counters; where a wait
+  // reports that it gave up
   bool exact = false;
   LexTask *d_ldiff = nullptr, *d_lpress = nullptr;
   int n_ldiff = 0, n_lpress = 0, n_lflags = 0;
-  void* d_lex = nullptr;
-  size_t lex_bytes = 0;
+  uint32_t* d_ctl = nullptr;
   uint32_t* h_err = nullptr;
   uint32_t polls = 0;              // eqf_ctx::wait_polls that the graph holds
   std::atomic<bool> stale{false};  // a wait gave up: the counters have to be set up again
   int n = 0, maxN = 0, tiles[3] = {0, 0, 0}, iblocks = 0, cblocks = 0, ablocks = 0;
   bool any_src = false;
-  int ntmp = 1;  // red-black: ping-pong fields of every scene
+  int slots = 1;  // lin_solves that every scene has workspaces for
   int diff_iters = 0, press_iters = 0;  // red-black: the same for every scene
   int diff_rounds = 0, press_rounds = 0;  // exact: the most of any scene
   int tile = 5, tsweeps = 5;  // band shape index (kBands) and sweeps per launch (untuned default)
@@ -964,19 +964,22 @@ static uint64_t group_key(const RbGroup& g) {
 }
 
 // The strips of `nslots` lin_solves of scene i, `iters` sweeps each.
-static void lex_tasks(int i, int S, int iters, int nslots, std::vector<LexTask>& v, int& nflags, int64_t& hfloats) {
+static void lex_tasks(int i, int S, int iters, int nslots, std::vector<LexTask>& v, int& nflags) {
   const int K = lex_round_sweeps(iters, 0);  // the longest round
   if (K == 0) return;
   const int n = lex_strips(S, K);
   for (int slot = 0; slot < nslots; ++slot)
-    for (int strip = 0; strip < n; ++strip) {
-      v.push_back(LexTask{i, slot, strip, n, nflags++, 0, hfloats});
-      if (strip + 1 < n) hfloats += lex_handoff_floats(S);
-    }
+    for (int strip = 0; strip < n; ++strip)
+      v.push_back(LexTask{i, slot, strip, n, nflags++, 0, slot * lex_solve_floats(S) + strip * lex_handoff_floats(S)});
 }
 static size_t lex_ctl_bytes(int nflags) { return (sizeof(uint32_t) * (size_t)(nflags + 2) + 255) & ~(size_t)255; }
-int64_t lex_workspace_bytes(int S) {
-  return 3 * ((int64_t)(lex_strips(S, LEX_KMAX) - 1) * lex_handoff_floats(S) * 4 + lex_strips(S, LEX_KMAX) * 36);
+int64_t frame_table_bytes(int S, bool exact) {
+  const int64_t N = S - 2, nseg = (N + rb::SEG - 1) / rb::SEG;
+  int64_t b = sizeof(RbScene) + sizeof(int4) * ((N * nseg + 3) / 4 + (nseg > 1 ? N : (N + 3) / 4)) +
+              sizeof(int2) * (((int64_t)S * S + rb::CELL_BLOCK - 1) / rb::CELL_BLOCK);
+  if (exact) b += 4 * lex_strips(S, LEX_KMAX) * (int64_t)(sizeof(LexTask) + sizeof(uint32_t));
+  else for (int mode = 0; mode < 3; ++mode) b += sizeof(int2) * (int64_t)band_tiles(S, 5, 5, mode);
+  return 2 * b;  // with the headroom of group_tables
 }
 
 // Ticket order: the longest remaining chain of a scene first (a strip waits
@@ -997,23 +1000,24 @@ static int group_tables(RbGroup& g, hipStream_t st, std::string& err) {
   std::vector<int2> tmap[3], cmap;
   std::vector<int4> imap, amap;
   std::vector<LexTask> ldiff, lpress;
-  int64_t hd = 0, hp = 0;
   int fd = 0, fp = 0;
   g.any_src = false;
-  g.ntmp = 3;
+  g.slots = 3;
   g.maxN = 0;
-  for (const eqf_scene* s : g.scenes) g.maxN = std::max(g.maxN, s->N);
+  for (const eqf_scene* s : g.scenes) {
+    g.maxN = std::max(g.maxN, s->N);
+    if (s->slots < 3) g.slots = 1;
+  }
   g.diff_rounds = g.press_rounds = 0;
   for (int i = 0; i < n; ++i) {
     eqf_scene* s = g.scenes[i];
     auto* w = static_cast<FrameWork*>(s->work);
-    scs[i] = RbScene{s->desc, {w->tmp[0], w->tmp[1], w->tmp[2]}};
-    if (!w->tmp[2]) g.ntmp = 1;
+    scs[i] = RbScene{s->desc, {w->tmp[0], w->tmp[1], w->tmp[2]}, s->d_hand};
     g.diff_rounds = std::max(g.diff_rounds, lex_rounds(s->desc.diff_iters));
     g.press_rounds = std::max(g.press_rounds, lex_rounds(s->desc.press_iters));
     if (g.exact) {
-      lex_tasks(i, s->S, s->desc.diff_iters, 3, ldiff, fd, hd);
-      lex_tasks(i, s->S, s->desc.press_iters, 1, lpress, fp, hp);
+      lex_tasks(i, s->S, s->desc.diff_iters, g.slots, ldiff, fd);
+      lex_tasks(i, s->S, s->desc.press_iters, 1, lpress, fp);
     } else {
       for (int mode = 0; mode < 3; ++mode) {
         const int nt = band_tiles(s->S, g.tile, g.tsweeps, mode);
@@ -1046,7 +1050,9 @@ static int group_tables(RbGroup& g, hipStream_t st, std::string& err) {
   lex_order(ldiff, g.scenes);
   lex_order(lpress, g.scenes);
   const size_t b_ld = up(sizeof(LexTask) * ldiff.size()), b_lp = up(sizeof(LexTask) * lpress.size());
-  const size_t bytes = b_scs + b_t[0] + b_t[1] + b_t[2] + b_m + b_c + b_a + b_ld + b_lp;
+  g.n_lflags = std::max(fd, fp);
+  const size_t b_ctl = lex_ctl_bytes(g.n_lflags);  // zero at first; every launch leaves it so
+  const size_t bytes = b_ctl + b_scs + b_t[0] + b_t[1] + b_t[2] + b_m + b_c + b_a + b_ld + b_lp;
   if (bytes > g.tab_bytes) {  // with headroom: a server's group changes size often
     (void)hipFree(g.d_tab);
     g.d_tab = nullptr;
@@ -1061,7 +1067,7 @@ static int group_tables(RbGroup& g, hipStream_t st, std::string& err) {
   }
   g.h_tab.assign(bytes, 0);
   char* base = g.h_tab.data();
-  size_t off = 0;
+  size_t off = b_ctl;
   auto put = [&](const void* src, size_t len, size_t slot) {
     if (len) std::memcpy(base + off, src, len);
     const size_t at = off;
@@ -1077,6 +1083,7 @@ static int group_tables(RbGroup& g, hipStream_t st, std::string& err) {
   const size_t o_ld = put(ldiff.data(), sizeof(LexTask) * ldiff.size(), b_ld);
   const size_t o_lp = put(lpress.data(), sizeof(LexTask) * lpress.size(), b_lp);
   char* d = (char*)g.d_tab;
+  g.d_ctl = (uint32_t*)d;
   g.d_scs = (RbScene*)(d + o_scs);
   for (int m = 0; m < 3; ++m) g.d_tmap[m] = (int2*)(d + o_t[m]);
   g.d_imap = (int4*)(d + o_m);
@@ -1086,35 +1093,13 @@ static int group_tables(RbGroup& g, hipStream_t st, std::string& err) {
   g.d_lpress = (LexTask*)(d + o_lp);
   g.n_ldiff = (int)ldiff.size();
   g.n_lpress = (int)lpress.size();
-  if (g.exact) {
-    g.n_lflags = std::max(fd, fp);
-    const size_t need = lex_ctl_bytes(g.n_lflags) + 4 * (size_t)std::max(hd, hp);
-    if (need > g.lex_bytes) {
-      (void)hipFree(g.d_lex);
-      g.d_lex = nullptr;
-      g.lex_bytes = 0;
-      const size_t cap = g.stream ? need + need / 2 : need;  // with headroom where scenes come and go
-      hipError_t e = hipMalloc(&g.d_lex, cap);
-      if (e != hipSuccess) {
-        err = std::string("lin_solve workspace: ") + hipGetErrorString(e);
-        return EQF_ENOMEM;
-      }
-      g.lex_bytes = cap;
-    }
-    if (!g.h_err) {
-      hipError_t e = hipHostMalloc((void**)&g.h_err, sizeof(uint32_t), hipHostMallocDefault);
-      if (e != hipSuccess) {
-        err = std::string("lin_solve status: ") + hipGetErrorString(e);
-        return EQF_ENOMEM;
-      }
-      *g.h_err = 0;
-    }
-    // counters start at zero; every launch leaves them so
-    hipError_t e = hipMemsetAsync(g.d_lex, 0, lex_ctl_bytes(g.n_lflags), st);
+  if (g.exact && !g.h_err) {
+    hipError_t e = hipHostMalloc((void**)&g.h_err, sizeof(uint32_t), hipHostMallocDefault);
     if (e != hipSuccess) {
-      err = std::string("lin_solve counters: ") + hipGetErrorString(e);
-      return EQF_EDEVICE;
+      err = std::string("lin_solve status: ") + hipGetErrorString(e);
+      return EQF_ENOMEM;
     }
+    *g.h_err = 0;
   }
   // behind the frames already queued on `st` (they read the old tables)
   hipError_t e = hipMemcpyAsync(g.d_tab, base, bytes, hipMemcpyHostToDevice, st);
@@ -1191,11 +1176,9 @@ static void g_lin_solve(hipStream_t st, const RbGroup& g, const Solve* sv, int n
 // velocity, density from the last frame's density), or a pressure solve.
 static void g_lex(hipStream_t st, const RbGroup& g, bool press, const LexSpec& s0, const LexSpec& s1,
                   const LexSpec& s2) {
-  uint32_t* ctl = (uint32_t*)g.d_lex;
-  float* H = (float*)((char*)g.d_lex + lex_ctl_bytes(g.n_lflags));
   for (int r = 0; r < (press ? g.press_rounds : g.diff_rounds); ++r) {
     const LexArgs a{{s0, s1, s2}, r, press ? 1 : 0, g.polls};
-    lex_launch(st, g.d_scs, press ? g.d_lpress : g.d_ldiff, press ? g.n_lpress : g.n_ldiff, a, ctl, g.n_lflags, H,
+    lex_launch(st, g.d_scs, press ? g.d_lpress : g.d_ldiff, press ? g.n_lpress : g.n_ldiff, a, g.d_ctl, g.n_lflags,
                g.h_err, g.maxN);
   }
 }
@@ -1232,12 +1215,14 @@ static void g_frame(hipStream_t st, const RbGroup& g) {
   if (g.any_src)
     hipLaunchKernelGGL(rb::k_sources, dim3((unsigned)g.cblocks), dim3(256), 0, st, g.d_scs, g.d_cmap);
   // the three diffusions, fluid.rs:438, 448, 501 (the density's reads no velocity)
+  // together, or each of them alone where a scene has one slot
   if (g.exact) {
-    g_lex(st, g, false, LexSpec{M_ROW, F_U0, F_U, 0}, LexSpec{M_COL, F_V0, F_V, 0}, LexSpec{M_PASSIVE, F_SC, F_D, 1});
+    const LexSpec s[3] = {{M_ROW, F_U0, F_U, 0}, {M_COL, F_V0, F_V, 0}, {M_PASSIVE, F_SC, F_D, 1}};
+    if (g.slots == 3) g_lex(st, g, false, s[0], s[1], s[2]);
+    else for (int k = 0; k < 3; ++k) g_lex(st, g, false, s[k], LexSpec{}, LexSpec{});
   } else {
-    // each of them alone where the scenes have one ping-pong field
     const Solve s[3] = {{M_ROW, F_U0, F_U, 0}, {M_COL, F_V0, F_V, 0}, {M_PASSIVE, F_SC, F_D, 1}};
-    for (int k = 0; k < 3; k += g.ntmp) g_lin_solve(st, g, s + k, g.ntmp, g.diff_iters);
+    for (int k = 0; k < 3; k += g.slots) g_lin_solve(st, g, s + k, g.slots, g.diff_iters);
   }
   // project(U0, V0, p=U, div=V), fluid.rs:459
   hipLaunchKernelGGL(rb::k_div, cells, dim3(256), 0, st, g.d_scs, g.d_imap, F_U0, F_V0, F_V, F_U, 0);
@@ -1257,13 +1242,10 @@ static void g_frame(hipStream_t st, const RbGroup& g) {
 static void group_release(RbGroup& g) {
   if (g.graph) (void)hipGraphExecDestroy(g.graph);
   g.graph = nullptr;
-  (void)hipFree(g.d_tab);
+  if (g.d_tab) (void)hipFree(g.d_tab);
   g.d_tab = nullptr;
   g.tab_bytes = 0;
-  (void)hipFree(g.d_lex);
-  g.d_lex = nullptr;
-  g.lex_bytes = 0;
-  (void)hipHostFree(g.h_err);
+  if (g.h_err) (void)hipHostFree(g.h_err);
   g.h_err = nullptr;
 }
 
@@ -1351,7 +1333,7 @@ void* frame_create(eqf_scene* s, std::string& err) {
   const size_t n = (size_t)s->S * s->S;
   hipError_t e = hipSuccess;
   if (s->p.gs_mode == EQF_GS_REDBLACK) {
-    const int k = rb_scratch_fields(s->S);
+    const int k = s->slots;
     const size_t fs = (size_t)rm_field_floats(s->S);
     e = eqf_scene_malloc(s, (void**)&w->tmp[0], sizeof(float) * (k > 1 ? k * fs : n));
     for (int i = 1; i < k && e == hipSuccess; ++i) w->tmp[i] = w->tmp[0] + i * fs;

@@ -64,8 +64,10 @@ struct eqf_scene {
   int src_mask = 0;           // frame sources set: bit 0 density, 1 vx, 2 vy
   uint8_t* d_code = nullptr;
   uint8_t* d_rowf = nullptr;
+  float* d_hand = nullptr;    // exact mode: hand-off values of its lin_solves
+  int slots = 1;              // lin_solves of a frame that may run at once (scene_slots)
   int ring_copies = 0;        // Passive ring cells that copy their neighbour
-  void* d_main = nullptr;     // one allocation: pad, fields, rule bytes, rowf
+  void* d_main = nullptr;     // one allocation: pad, fields, rule bytes, rowf, hand-off
   float* d_stage = nullptr;   // staging for eqf_add_source (lazy)
   uint8_t* d_mask = nullptr;  // mask + scratch for the boundary build (lazy)
   eqf::SceneDesc desc{};
@@ -111,9 +113,13 @@ int eqf_internal_check(const eqf_scene* s, uint32_t fields);
 void eqf_internal_rings_drop(eqf_scene* s);
 int eqf_internal_check_params(const eqf_params* p);
 // eqf_scene_create on a caller-owned stream (the server's admission stream),
-// allocating from `pool` in that stream's order when `pool` is set.
-int eqf_internal_scene_create(eqf_ctx* ctx, const eqf_params* p, hipStream_t stream, hipMemPool_t pool,
+// allocating from `pool` in that stream's order when `pool` is set; `slots` as
+// scene_slots or 1.
+int eqf_internal_scene_create(eqf_ctx* ctx, const eqf_params* p, hipStream_t stream, hipMemPool_t pool, int slots,
                               eqf_scene** out);
+// Device memory of a scene that was prepared (with frame sources or without) and
+// of its share of a launch group's tables.
+uint64_t eqf_internal_scene_bytes(const eqf_params* p, int slots, bool sources);
 
 // Device-side setup (eqf_setup.hip).
 int eqf_dev_init_fields(eqf_scene* s, int times);
@@ -122,6 +128,7 @@ int eqf_dev_download(eqf_scene* s, const float* src, float* host);
 // src field -> another device array, queued on the scene's stream.
 int eqf_dev_copy_async(eqf_scene* s, const float* src, float* dst);
 int eqf_dev_rebuild_bnd(eqf_scene* s);
+size_t eqf_dev_mask_bytes(int S);
 void eqf_dev_trim(eqf_scene* s);
 
 namespace eqf {
@@ -130,7 +137,8 @@ namespace eqf {
 // Each frame kernel covers all scenes of its group in one launch.
 struct RbScene {
   SceneDesc d;  // the scene's descriptor (a copy): fields, sizes, coefficients, rule bytes
-  float* tmp[3];  // its ping-pong fields (red-black mode; rb_scratch_fields)
+  float* tmp[3];  // its ping-pong fields (red-black mode)
+  float* hand;    // its hand-off values (exact mode)
 };
 
 // Lexicographic lin_solve (eqf_lex.hip).  A launch covers up to three
@@ -140,7 +148,7 @@ struct LexTask {
   int strip, nstrips;
   int flag;      // its progress count; the strip above has the one before
   int pad;
-  int64_t hoff;  // its hand-off values (the strip above: lex_handoff_floats before)
+  int64_t hoff;  // its hand-off values in the scene's (the strip above: lex_handoff_floats before)
 };
 struct LexSpec {
   int mode, x_role, x0_role, coef;
@@ -153,7 +161,7 @@ struct LexArgs {
 // ctl: ticket, ended workgroups, then nflags progress counts, all zero before
 // the first launch; a launch leaves them zero.  maxN: the largest scene's.
 void lex_launch(hipStream_t st, const RbScene* scs, const LexTask* tasks, int ntasks, const LexArgs& args,
-                uint32_t* ctl, int nflags, float* H, uint32_t* err, int maxN);
+                uint32_t* ctl, int nflags, uint32_t* err, int maxN);
 
 // Frames (eqf_frame.hip).  A launch group's scenes share one mode.
 void* frame_create(eqf_scene* s, std::string& err);
@@ -171,6 +179,6 @@ void group_set_scenes(void* g, const std::vector<eqf_scene*>& scenes);
 // group's counters up again.  For frames that have ended.
 bool group_collect(void* g);
 bool frame_collect(const eqf_scene* s);
-// Device bytes of the lexicographic hand-off of one scene.
-int64_t lex_workspace_bytes(int S);
+// Device bytes of a scene's share of its group's tables.
+int64_t frame_table_bytes(int S, bool exact);
 }  // namespace eqf

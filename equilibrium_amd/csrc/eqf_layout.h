@@ -70,14 +70,16 @@ constexpr int CODE_PAD = 16;
 EQF_HD inline int rm_code_stride(int S) { return S + (S & 1); }
 EQF_HD inline int64_t rm_code_used(int S) { return (int64_t)S * rm_code_stride(S); }
 EQF_HD inline int64_t rm_code_bytes(int S) { return (rm_code_used(S) + 63) & ~(int64_t)63; }
+EQF_HD inline int rm_code_arrays(bool exact) { return exact ? 2 : 1; }
 
-// ---- red-black lin_solve (eqf_frame.hip) ----
-// Ping-pong fields of a scene: one per diffusion, so that the three share their
-// launches, up to the size where one alone fills the device and the caches hold
+// Lin_solves that a scene has workspaces for at once (red-black: ping-pong fields;
+// exact: hand-off values): the three diffusions, which then share their launches, or
+// one (a server's scene whose budget does not hold more).  Red-black scenes have one
+// from the size where one diffusion fills the device and the caches hold
 // more of one than of three.  ms per frame of 20 sweeps apart and together: N=250
 // 0.274 and 0.183, N=1501 0.436 and 0.346, N=2046 0.574 and 0.469, N=3000 0.948
 // and 0.909, N=4096 1.510 and 1.543.
-EQF_HD inline int rb_scratch_fields(int S) { return S <= 3072 ? 3 : 1; }
+EQF_HD inline int scene_slots(bool exact, int S) { return exact || S <= 3072 ? 3 : 1; }
 
 // ---- lexicographic lin_solve (eqf_lex.hip) ----
 // Sweeps per round, steps per block.
@@ -96,5 +98,7 @@ EQF_HD inline int lex_strips(int S, int K) { return (S + K - 1 + LEX_ROWS - 1) /
 EQF_HD inline int lex_blocks(int S, int K) { return ((S + 63 + 2 * (K - 1)) >> 3) + 1; }
 // Hand-off values a strip leaves for the next one: one per sweep and step.
 EQF_HD inline int64_t lex_handoff_floats(int S) { return (int64_t)LEX_KMAX * lex_blocks(S, LEX_KMAX) * LEX_B; }
+// ... of a lin_solve of any number of sweeps.
+EQF_HD inline int64_t lex_solve_floats(int S) { return (lex_strips(S, LEX_KMAX) - 1) * lex_handoff_floats(S); }
 
 }  // namespace eqf

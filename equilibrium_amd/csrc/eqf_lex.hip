@@ -398,7 +398,7 @@ static __device__ __forceinline__ Part part_of(int w, int steps, int K) {
 // In block b of the workgroup wave w runs block m = b - w of its steps.
 template <int MODE>
 static __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, const LexTask& tk, const LexSpec& sp, int K,
-                                           uint32_t* __restrict__ flags, float* __restrict__ Hb,
+                                           uint32_t* __restrict__ flags,
                                            uint32_t* __restrict__ err, uint32_t polls) {
   const SceneDesc& d = sc.d;
   const int S = d.S;
@@ -634,7 +634,7 @@ static __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, cons
   }
 
   if (w == W + 2) {  // lane 63's values for the strip below (and the final values)
-    float* hout = Hb + tk.hoff;
+    float* hout = sc.hand + tk.hoff;
     uint32_t* fown = flags + tk.flag;
     for (int b = -1; b < NI; ++b) {
       if (has_next && b > 0) {
@@ -740,7 +740,7 @@ static __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, cons
   // x before the round, and lane 0's values from the strip above: these only in
   // the block before they are needed, since every block that they come earlier
   // puts every strip that much further behind the one above.
-  const float* hin = Hb + (has_prev ? tk.hoff - (int64_t)KMAX * T : 0);
+  const float* hin = sc.hand + (has_prev ? tk.hoff - (int64_t)KMAX * T : 0);
   const uint32_t* fprev = flags + (has_prev ? tk.flag - 1 : tk.flag);
   u4 gin[ZI];
   float gu[3];
@@ -825,8 +825,7 @@ static __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, cons
 template <int W>
 __global__ void __launch_bounds__(Lex<W>::NT, W == 4 ? 4 : 3)
     k_lex(const RbScene* __restrict__ scs, const LexTask* __restrict__ tasks, int ntasks, LexArgs args,
-          uint32_t* __restrict__ ctl, uint32_t* __restrict__ flags, int nflags, float* __restrict__ H,
-          uint32_t* __restrict__ err) {
+          uint32_t* __restrict__ ctl, uint32_t* __restrict__ flags, int nflags, uint32_t* __restrict__ err) {
   typedef Lex<W> X;
   extern __shared__ float lex_lds[];
   lf* L = (lf*)lex_lds;
@@ -842,9 +841,9 @@ __global__ void __launch_bounds__(Lex<W>::NT, W == 4 ? 4 : 3)
   const LexSpec sp = args.sp[tk.slot];
   const int K = lex_round_sweeps(args.press ? sc.d.press_iters : sc.d.diff_iters, args.round);
   if (K > 0) {
-    if (sp.mode == M_ROW) X::template strip_task<M_ROW>(L, sc, tk, sp, K, flags, H, err, args.polls);
-    else if (sp.mode == M_COL) X::template strip_task<M_COL>(L, sc, tk, sp, K, flags, H, err, args.polls);
-    else X::template strip_task<M_PASSIVE>(L, sc, tk, sp, K, flags, H, err, args.polls);
+    if (sp.mode == M_ROW) X::template strip_task<M_ROW>(L, sc, tk, sp, K, flags, err, args.polls);
+    else if (sp.mode == M_COL) X::template strip_task<M_COL>(L, sc, tk, sp, K, flags, err, args.polls);
+    else X::template strip_task<M_PASSIVE>(L, sc, tk, sp, K, flags, err, args.polls);
   }
   // The last workgroup to end leaves the counters as the next launch needs them.
   __syncthreads();
@@ -859,12 +858,12 @@ __global__ void __launch_bounds__(Lex<W>::NT, W == 4 ? 4 : 3)
 }  // namespace lex
 
 void lex_launch(hipStream_t st, const RbScene* scs, const LexTask* tasks, int ntasks, const LexArgs& args,
-                uint32_t* ctl, int nflags, float* H, uint32_t* err, int maxN) {
+                uint32_t* ctl, int nflags, uint32_t* err, int maxN) {
   if (ntasks <= 0) return;
   auto launch = [&](auto w) {
     typedef lex::Lex<decltype(w)::value> X;
     hipLaunchKernelGGL(lex::k_lex<decltype(w)::value>, dim3((unsigned)ntasks), dim3(X::NT), X::L_WORDS * 4, st, scs, tasks,
-                       ntasks, args, ctl, ctl + 2, nflags, H, err);
+                       ntasks, args, ctl, ctl + 2, nflags, err);
   };
   // Up to one workgroup per CU (256 of them) the chain of blocks bounds the
   // launch: eight waves of up to three sweeps take a block faster than four of up

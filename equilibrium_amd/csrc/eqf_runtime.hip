@@ -236,8 +236,32 @@ static void scene_free(eqf_scene* s) {
   delete s;
 }
 
+// A scene's main allocation.
+struct MainBytes {
+  size_t fld, code, rowf, hand, total;
+};
+static MainBytes main_bytes(int S, bool exact, int slots) {
+  auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
+  MainBytes b;
+  b.fld = up(sizeof(float) * NFIELDS * (size_t)rm_field_floats(S));
+  b.code = up(rm_code_arrays(exact) * (size_t)rm_code_bytes(S));
+  b.rowf = up((size_t)S);
+  b.hand = exact ? up(sizeof(float) * slots * (size_t)lex_solve_floats(S)) : 0;
+  b.total = sizeof(float) * FLD_PAD + b.fld + b.code + b.rowf + b.hand;
+  return b;
+}
+
+uint64_t eqf_internal_scene_bytes(const eqf_params* p, int slots, bool sources) {
+  const int S = (int)p->size;
+  const bool exact = p->gs_mode == EQF_GS_WAVEFRONT;
+  uint64_t b = main_bytes(S, exact, slots).total + eqf_dev_mask_bytes(S) + (uint64_t)frame_table_bytes(S, exact);
+  if (!exact) b += sizeof(float) * slots * (uint64_t)rm_field_floats(S);
+  if (sources) b += sizeof(float) * 3 * (uint64_t)rm_field_floats(S);
+  return b;
+}
+
 static int scene_alloc(eqf_ctx* ctx, const eqf_params* p, eqf_scene** out, hipStream_t stream = nullptr,
-                       hipMemPool_t pool = nullptr) {
+                       hipMemPool_t pool = nullptr, int slots = 0) {
   int rc = check_params(p);
   if (rc) return rc;
   HIPCHK(hipSetDevice(ctx->device));
@@ -251,6 +275,8 @@ static int scene_alloc(eqf_ctx* ctx, const eqf_params* p, eqf_scene** out, hipSt
   s->S = (int)p->size;
   s->N = s->S - 2;
   s->fstride = rm_field_floats(s->S);
+  const bool exact = p->gs_mode == EQF_GS_WAVEFRONT;
+  s->slots = slots ? slots : scene_slots(exact, s->S);
   hipError_t e = hipSuccess;
   if (stream) {
     s->stream = stream;
@@ -266,15 +292,14 @@ static int scene_alloc(eqf_ctx* ctx, const eqf_params* p, eqf_scene** out, hipSt
     scene_free(s);
     return fail(EQF_EDEVICE, std::string("hipStreamCreate: ") + hipGetErrorString(e));
   }
-  auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
-  const size_t b_pad = sizeof(float) * FLD_PAD, b_fld = up(sizeof(float) * NFIELDS * (size_t)s->fstride);
-  const size_t b_code = up(2 * (size_t)rm_code_bytes(s->S)), b_rowf = up((size_t)s->S);
-  e = eqf_scene_malloc(s, &s->d_main, b_pad + b_fld + b_code + b_rowf);
+  const MainBytes mb = main_bytes(s->S, exact, s->slots);
+  e = eqf_scene_malloc(s, &s->d_main, mb.total);
   if (e == hipSuccess) {
-    char* base = (char*)s->d_main + b_pad;
+    char* base = (char*)s->d_main + sizeof(float) * FLD_PAD;
     s->d_fld = (float*)base;
-    s->d_code = (uint8_t*)(base + b_fld);
-    s->d_rowf = (uint8_t*)(base + b_fld + b_code);
+    s->d_code = (uint8_t*)(base + mb.fld);
+    s->d_rowf = (uint8_t*)(base + mb.fld + mb.code);
+    if (exact) s->d_hand = (float*)(base + mb.fld + mb.code + mb.rowf);
     e = hipMemsetAsync(s->d_fld, 0, sizeof(float) * NFIELDS * s->fstride, s->stream);
   }
   if (e != hipSuccess) {
@@ -287,14 +312,14 @@ static int scene_alloc(eqf_ctx* ctx, const eqf_params* p, eqf_scene** out, hipSt
 }
 
 extern "C" int eqf_scene_create(eqf_ctx* ctx, const eqf_params* p, eqf_scene** out) {
-  return eqf_internal_scene_create(ctx, p, nullptr, nullptr, out);
+  return eqf_internal_scene_create(ctx, p, nullptr, nullptr, 0, out);
 }
 
-int eqf_internal_scene_create(eqf_ctx* ctx, const eqf_params* p, hipStream_t stream, hipMemPool_t pool,
+int eqf_internal_scene_create(eqf_ctx* ctx, const eqf_params* p, hipStream_t stream, hipMemPool_t pool, int slots,
                               eqf_scene** out) {
   if (!ctx || !out) return fail(EQF_EINVAL, "ctx/out is NULL");
   eqf_scene* s = nullptr;
-  int rc = scene_alloc(ctx, p, &s, stream, pool);
+  int rc = scene_alloc(ctx, p, &s, stream, pool, slots);
   if (rc) return rc;
   if (s->S >= 22) {
     // No index clamping in init_density at this size: write the state on the

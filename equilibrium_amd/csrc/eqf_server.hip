@@ -56,6 +56,7 @@ struct Req {
   eqf_scene* scene = nullptr;
   int lane = 0;
   uint64_t bytes = 0;
+  int slots = 0;  // of its scene: three where the budget holds them, else one
   int64_t cells = 0;
   std::vector<float> out_d, out_u, out_v;
 };
@@ -124,20 +125,22 @@ struct eqf_server {
   }
 };
 
-// Device bytes of a scene of this size and mode with frame sources (red-black:
-// with one ping-pong field).
-static uint64_t estimate_bytes(const eqf_params& p) {
-  const int S = (int)p.size, N = S - 2;
-  // fields + sources, rule bytes, row flags, tables, and the ping-pong field
-  // (red-black) or the lin_solve hand-off (exact)
-  const uint64_t fs = (uint64_t)rm_field_floats(S), cells = (uint64_t)S * S;
-  const uint64_t work = p.gs_mode == EQF_GS_REDBLACK ? cells * 4 : (uint64_t)lex_workspace_bytes(S);
-  return (NFIELDS + 3) * fs * 4 + 2 * (uint64_t)rm_code_bytes(S) + work + (uint64_t)S * 5 + (uint64_t)N * 96 + 8192;
+// What a request may not exceed the budget by when it is submitted.  This rule is
+// older than the present layout (exact scenes: rows in strips of 64, columns rounded
+// up to 16) and stays, so that a budget goes on taking the requests that it took;
+// what a resident scene is charged are its own bytes (eqf_internal_scene_bytes).
+static uint64_t accept_bytes(const eqf_params& p) {
+  const uint64_t S = p.size, N = S - 2;
+  if (p.gs_mode == EQF_GS_REDBLACK)
+    return (NFIELDS + 3) * (uint64_t)rm_field_floats((int)S) * 4 + (uint64_t)rm_code_bytes((int)S) + S * S * 4 + S * 5 +
+           N * 96 + 128 + 8192;
+  const uint64_t cells = (N + 63) / 64 * 64 * ((N + 15) / 16 * 16);
+  return (NFIELDS + 3) * ((cells + 4 * S + 63) & ~(uint64_t)63) * 4 + cells * 3 / 4 + S + N * 96 + 128 + 4096;
 }
 
 static int admit(eqf_server* sv, Req* r, std::string& err) {
   eqf_scene* s = nullptr;
-  int rc = eqf_internal_scene_create(sv->ctx, &r->p, sv->astream, sv->pool, &s);
+  int rc = eqf_internal_scene_create(sv->ctx, &r->p, sv->astream, sv->pool, r->slots, &s);
   for (size_t k = 0; !rc && k + 4 <= r->rects.size(); k += 4)
     rc = eqf_fill_rect(s, r->rects[k], r->rects[k + 1], r->rects[k + 2], r->rects[k + 3]);
   auto in = [](const std::vector<float>& v, const float* b) { return v.empty() ? b : v.data(); };
@@ -253,6 +256,12 @@ static std::string lane_launch(eqf_server* sv, int li) {
   return "";
 }
 
+// Whether the budget has room for a request (one that was accepted runs alone
+// where its own bytes are more than the rule of acceptance counts).
+static bool fits(const eqf_server* sv, const Req* r) {
+  return sv->used_bytes == 0 || sv->used_bytes + r->bytes <= sv->cfg.hbm_budget_bytes;
+}
+
 // Admits the queue's head if its memory fits; true if one was admitted (or
 // dropped).
 static bool admit_one(eqf_server* sv) {
@@ -268,7 +277,7 @@ static bool admit_one(eqf_server* sv) {
     if (sv->queue.empty()) return false;
     Req* h = sv->queue.front();
     if (sv->cfg.max_active > 0 && sv->active.size() >= (size_t)sv->cfg.max_active) return false;
-    if (sv->used_bytes + h->bytes > sv->cfg.hbm_budget_bytes) return false;
+    if (!fits(sv, h)) return false;
     sv->queue.pop_front();
     sv->used_bytes += h->bytes;
     sv->peak_bytes = std::max(sv->peak_bytes, sv->used_bytes);
@@ -384,7 +393,7 @@ static void work_loop(eqf_server* sv) {
         const Req* h = sv->queue.front();
         if (h->cancel) return true;
         if (sv->cfg.max_active > 0 && sv->active.size() >= (size_t)sv->cfg.max_active) return false;
-        return sv->used_bytes + h->bytes <= sv->cfg.hbm_budget_bytes;
+        return fits(sv, h);
       };
       if (sv->queue.empty() && sv->active.empty()) sv->cv_idle.notify_all();
       sv->cv_work.wait(lk, ready);
@@ -478,14 +487,13 @@ extern "C" int eqf_server_submit(eqf_server* sv, const eqf_request* req, uint64_
     cp(req->init_vx, r->iu);
     cp(req->init_vy, r->iv);
   }
-  const uint64_t least = estimate_bytes(r->p);
-  // A scene's further ping-pong fields count while it is resident, but do not
-  // keep a request out that fits without them.
-  const int more = r->p.gs_mode == EQF_GS_REDBLACK ? rb_scratch_fields((int)r->p.size) - 1 : 0;
-  r->bytes = std::min(least + more * (uint64_t)rm_field_floats((int)r->p.size) * 4,
-                      std::max(least, (uint64_t)sv->cfg.hbm_budget_bytes));
+  const uint64_t budget = sv->cfg.hbm_budget_bytes;
+  const bool sources = req->src_density || req->src_vx || req->src_vy;
+  r->slots = scene_slots(r->p.gs_mode == EQF_GS_WAVEFRONT, (int)r->p.size);
+  if (eqf_internal_scene_bytes(&r->p, r->slots, sources) > budget) r->slots = 1;
+  r->bytes = eqf_internal_scene_bytes(&r->p, r->slots, sources);
   std::lock_guard<std::mutex> lk(sv->mu);
-  if (r->bytes > sv->cfg.hbm_budget_bytes)
+  if (accept_bytes(r->p) > budget)
     return eqf_internal_error(EQF_ENOMEM, "request does not fit the server's HBM budget");
   r->ticket = sv->next_ticket++;
   r->t_submit = sv->now_ms();

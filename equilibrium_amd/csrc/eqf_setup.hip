@@ -86,7 +86,7 @@ __global__ void k_rowcol_bytes(int S, const uint32_t* __restrict__ rowf32, const
 // left, fluid.rs:151-164), AdjustColumn (up wins over down, fluid.rs:165-177),
 // Passive ring copies (counted).
 __global__ void k_codes(Geo g, const uint8_t* __restrict__ m, const uint8_t* __restrict__ rowf,
-                        const uint8_t* __restrict__ colf, uint8_t* __restrict__ code, int* __restrict__ copies) {
+                        const uint8_t* __restrict__ colf, uint8_t* __restrict__ code, int arrays, int* __restrict__ copies) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int S = g.S, N = g.N;
   if (e >= (int64_t)S * S) return;
@@ -94,7 +94,7 @@ __global__ void k_codes(Geo g, const uint8_t* __restrict__ m, const uint8_t* __r
   auto wall = [&](int i, int j) { return m[(int64_t)j * S + i] == EQF_DEFAULT_WALL; };
   auto put = [&](int i, int j, uint32_t r) {
     code[(int64_t)j * rm_code_stride(S) + i] = (uint8_t)r;
-    code[rm_code_bytes(S) + (int64_t)i * rm_code_stride(S) + j] = (uint8_t)r;
+    if (arrays > 1) code[rm_code_bytes(S) + (int64_t)i * rm_code_stride(S) + j] = (uint8_t)r;
   };
   if (x >= 1 && x <= N && y >= 1 && y <= N) {
     uint32_t r = R_INTERIOR;
@@ -272,8 +272,10 @@ static MaskBuf mask_buf(int S) {
   return b;
 }
 
+size_t eqf_dev_mask_bytes(int S) { return mask_buf(S).bytes; }
+
 int eqf_dev_rebuild_bnd(eqf_scene* s) {
-  const int S = s->S;
+  const int S = s->S, arrays = rm_code_arrays(s->p.gs_mode == EQF_GS_WAVEFRONT);
   const int64_t n = (int64_t)S * S;
   const MaskBuf mb = mask_buf(S);
   hipError_t e = hipSuccess;
@@ -285,14 +287,14 @@ int eqf_dev_rebuild_bnd(eqf_scene* s) {
   const Geo g = geo_of(s);
   e = hipMemcpyAsync(s->d_mask, s->mask.data(), (size_t)n, hipMemcpyHostToDevice, s->stream);
   if (e == hipSuccess) e = hipMemsetAsync(d_flags, 0, mb.bytes - mb.flags, s->stream);
-  if (e == hipSuccess) e = hipMemsetAsync(s->d_code, 0, 2 * (size_t)rm_code_bytes(S), s->stream);
+  if (e == hipSuccess) e = hipMemsetAsync(s->d_code, 0, arrays * (size_t)rm_code_bytes(S), s->stream);
   if (e == hipSuccess) {
     hipLaunchKernelGGL(k_rowcol_or, dim3((unsigned)((S + 255) / 256), (unsigned)((S + 63) / 64)), dim3(256), 0,
                        s->stream, g, s->d_mask, d_flags, d_flags + S);
     hipLaunchKernelGGL(k_rowcol_bytes, dim3(blocks_for(S)), dim3(256), 0, s->stream, S, d_flags, d_flags + S,
                        s->d_rowf, d_colf);
     hipLaunchKernelGGL(k_codes, dim3(blocks_for(n)), dim3(256), 0, s->stream, g, s->d_mask, s->d_rowf, d_colf,
-                       s->d_code, d_cnt);
+                       s->d_code, arrays, d_cnt);
     e = hipGetLastError();
   }
   int copies = 0;

@@ -206,7 +206,12 @@ int eqf_batch_set_band(eqf_batch *b, int tile, int sweeps_per_block);
  * its own stream); scenes join and leave at tick boundaries.  Admission
  * uploads overlap the running tick. */
 typedef struct eqf_server_config {
-    uint64_t hbm_budget_bytes; /* device memory the resident scenes may use */
+    /* Device memory the resident scenes may use.  A request is refused
+     * (EQF_ENOMEM) when ten fields of its size and what goes with them exceed it.
+     * A scene is charged what it allocates; one that would not fit with workspaces
+     * for three lin_solves at once gets them for one (slower), and one that does not
+     * fit even so (by at most a ninth) runs alone. */
+    uint64_t hbm_budget_bytes;
     int32_t max_active;        /* resident scenes at most (0: no limit) */
     int32_t reserved;
 } eqf_server_config;

@@ -212,6 +212,16 @@ void HostStaging::give(Buf* b) {
   drop(b);
 }
 
+// Memory that the device writes by itself: pinned, managed or its own.
+static bool device_writes(const void* p) {
+  hipPointerAttribute_t a;
+  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return a.type != hipMemoryTypeUnregistered;
+}
+
 // Field -> the caller's memory, through pinned chunks: one is copied out while
 // the next arrives.  The runtime's own copy to memory that is not pinned pins
 // it for the time, or goes through small chunks: 512 fields of S 66..514 (178
@@ -219,10 +229,12 @@ void HostStaging::give(Buf* b) {
 // 238 us; this takes 14 ms and 180 us, about 40 us per MB of which is the host
 // reading what just arrived, on top of 10 us for the first copy.  Chunks of 1
 // MB took 15 ms and 185 us, of 512 KB 16 ms and 225 us: each costs the wait for
-// its event.
+// its event.  Where the device writes the caller's memory by itself the copy goes
+// straight there: 67 MB into pinned memory 1.19 ms, through the chunks 2.51.
 int eqf_dev_download(eqf_scene* s, const float* src, float* host) {
   const size_t bytes = sizeof(float) * (size_t)s->S * s->S;
-  HostStaging::Buf* b = s->staging ? s->staging->take() : nullptr;
+  const bool direct = device_writes(host) && device_writes((const char*)host + bytes - 1);
+  HostStaging::Buf* b = s->staging && !direct ? s->staging->take() : nullptr;
   hipError_t e = hipSuccess;
   if (!b) {
     e = hipMemcpyAsync(host, src, bytes, hipMemcpyDeviceToHost, s->stream);

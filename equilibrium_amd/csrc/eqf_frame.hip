@@ -883,6 +883,9 @@ __global__ void __launch_bounds__(256) k_copy(const RbScene* __restrict__ scs, c
   }
 }
 
+// A scene's entry of the tables.
+__global__ void k_put_scene(RbScene* __restrict__ at, RbScene v) { *at = v; }
+
 }  // namespace rb
 
 // ------------------------------------------------------------------ host --
@@ -917,7 +920,8 @@ struct RbGroup {
   int tile = 5, tsweeps = 5;  // band shape index (kBands) and sweeps per launch (untuned default)
   int tab_tile = -1, tab_T = -1;
   hipGraphExec_t graph = nullptr;
-  uint64_t key = 0;  // what the table and the graph were built for
+  uint64_t key = 0;   // what the work maps and the graph were built for
+  uint64_t dkey = 0;  // the descriptors that the tables hold
   int64_t key_frames = 0;  // frames launched since
 };
 
@@ -944,23 +948,37 @@ static int band_tiles(int S, int tile, int T, int mode) {
   return rb::band_span(S, 128, TX) * rb::band_span(S, b.nw * b.r, TY);
 }
 
-static uint64_t group_key(const RbGroup& g) {
+struct Hash {
   uint64_t key = 1469598103934665603ull;
-  auto mix = [&key](uint64_t v) { key = (key ^ v) * 1099511628211ull; };
+  void mix(uint64_t v) { key = (key ^ v) * 1099511628211ull; }
+};
+// What the work maps and the graph are made for.
+static uint64_t group_key(const RbGroup& g) {
+  Hash h;
   for (const eqf_scene* s : g.scenes) {
-    // The tables embed a copy of every descriptor, so every byte of it is
-    // part of the key (dt0 included: with zero viscosity and diffusion a new
-    // delta_t changes only dt0).  The descriptor is value-initialised, so
-    // its padding bytes are zero.
-    const SceneDesc& d = s->desc;
-    uint64_t words[(sizeof(SceneDesc) + 7) / 8] = {};
-    std::memcpy(words, &d, sizeof(SceneDesc));
-    mix(s->uid);
-    for (uint64_t w : words) mix(w);
+    h.mix(s->uid);
+    h.mix((uint64_t)s->desc.diff_iters << 32 | (uint32_t)s->desc.press_iters);
+    h.mix(s->desc.has_src != 0);
   }
-  mix((uint64_t)g.tile * 16 + (uint64_t)g.tsweeps);
-  mix(g.polls);
-  return key;
+  h.mix((uint64_t)g.tile * 16 + (uint64_t)g.tsweeps);
+  h.mix(g.polls);
+  return h.key;
+}
+// What the tables' copies of the descriptors hold: every byte counts (dt0
+// included: with zero viscosity and diffusion a new delta_t changes only dt0).
+// A descriptor is value-initialised, so its padding bytes are zero.
+static uint64_t desc_key(const RbGroup& g) {
+  Hash h;
+  for (const eqf_scene* s : g.scenes) {
+    uint64_t words[(sizeof(SceneDesc) + 7) / 8] = {};
+    std::memcpy(words, &s->desc, sizeof(SceneDesc));
+    for (uint64_t w : words) h.mix(w);
+  }
+  return h.key;
+}
+static RbScene scene_entry(const eqf_scene* s) {
+  const auto* w = static_cast<const FrameWork*>(s->work);
+  return RbScene{s->desc, {w->tmp[0], w->tmp[1], w->tmp[2]}, s->d_hand};
 }
 
 // The strips of `nslots` lin_solves of scene i, `iters` sweeps each.
@@ -1011,8 +1029,7 @@ static int group_tables(RbGroup& g, hipStream_t st, std::string& err) {
   g.diff_rounds = g.press_rounds = 0;
   for (int i = 0; i < n; ++i) {
     eqf_scene* s = g.scenes[i];
-    auto* w = static_cast<FrameWork*>(s->work);
-    scs[i] = RbScene{s->desc, {w->tmp[0], w->tmp[1], w->tmp[2]}, s->d_hand};
+    scs[i] = scene_entry(s);
     g.diff_rounds = std::max(g.diff_rounds, lex_rounds(s->desc.diff_iters));
     g.press_rounds = std::max(g.press_rounds, lex_rounds(s->desc.press_iters));
     if (g.exact) {
@@ -1274,12 +1291,22 @@ static int group_capture(RbGroup& g, hipStream_t st, std::string& err) {
   return EQF_OK;
 }
 
+// Kernels of a frame, and up to how many of them it is worth a graph: the sweep
+// counts have no bound that would keep a graph's size reasonable (2^24 sweeps are
+// 2.5 million launches), and a frame this long hides its launches.
+static constexpr int64_t GRAPH_MAX = 4096;
+static int64_t frame_launches(const RbGroup& g) {
+  auto solve = [&g](int iters) { return (int64_t)(iters + g.tsweeps - 1) / g.tsweeps + 1; };
+  const int64_t d = g.exact ? g.diff_rounds : solve(g.diff_iters), p = g.exact ? g.press_rounds : solve(g.press_iters);
+  return 8 + d * (3 / g.slots) + 2 * p;
+}
+
 // Advances every scene of the group by nframes on `st`.  The tables are
-// rebuilt when the scenes' parameters or the tiling change.  The first
+// rebuilt when the scenes, their iteration counts or the tiling change.  The first
 // frame after that is launched kernel by kernel; further ones replay a graph
 // captured once (a server's groups change membership often, and one frame's
 // launches cost less than a capture).
-static int group_step(RbGroup& g, hipStream_t st, int64_t nframes, std::string& err) {
+static int group_step_all(RbGroup& g, hipStream_t st, int64_t nframes, std::string& err) {
   if (nframes <= 0 || g.scenes.empty()) return EQF_OK;
   g.diff_iters = g.scenes[0]->desc.diff_iters;
   g.press_iters = g.scenes[0]->desc.press_iters;
@@ -1293,8 +1320,10 @@ static int group_step(RbGroup& g, hipStream_t st, int64_t nframes, std::string& 
   for (eqf_scene* s : g.scenes)
     if (s->invalid.load()) s->invalid.store(kAllFields);  // a frame mixes the fields
   g.polls = g.scenes[0]->ctx->wait_polls.load();
-  const uint64_t key = group_key(g);
-  if (g.stale.exchange(false) || !g.d_tab || key != g.key || g.tab_tile != g.tile || g.tab_T != g.tsweeps) {
+  const uint64_t key = group_key(g), dkey = desc_key(g);
+  const bool descs = dkey != g.dkey;
+  if (g.stale.exchange(false) || !g.d_tab || key != g.key || g.tab_tile != g.tile || g.tab_T != g.tsweeps ||
+      (descs && g.n > 1)) {
     int rc = group_tables(g, st, err);
     if (rc) {
       g.tab_tile = -1;  // not usable
@@ -1303,10 +1332,18 @@ static int group_step(RbGroup& g, hipStream_t st, int64_t nframes, std::string& 
     if (g.graph) (void)hipGraphExecDestroy(g.graph);
     g.graph = nullptr;
     g.key = key;
+    g.dkey = dkey;
     g.key_frames = 0;
+  } else if (descs) {
+    // A lone scene's parameters (the scenes of a group keep theirs): behind the
+    // queued frames, without a wait, and the graph stays.  Tables made anew wait for
+    // the frames before them.
+    hipLaunchKernelGGL(rb::k_put_scene, dim3(1), dim3(1), 0, st, g.d_scs, scene_entry(g.scenes[0]));
+    g.dkey = dkey;
   }
+  const bool graph = frame_launches(g) <= GRAPH_MAX;
   for (int64_t f = 0; f < nframes; ++f) {
-    if (g.key_frames++ == 0) {
+    if (g.key_frames++ == 0 || !graph) {
       g_frame(st, g);
       hipError_t e = hipGetLastError();
       if (e != hipSuccess) {
@@ -1326,6 +1363,16 @@ static int group_step(RbGroup& g, hipStream_t st, int64_t nframes, std::string& 
     }
   }
   return EQF_OK;
+}
+
+static int group_step(RbGroup& g, hipStream_t st, int64_t nframes, std::string& err) {
+  try {
+    return group_step_all(g, st, nframes, err);
+  } catch (...) {  // std::bad_alloc of the tables' host image
+    g.tab_tile = -1;
+    err = "out of memory";
+    return EQF_ENOMEM;
+  }
 }
 
 void* frame_create(eqf_scene* s, std::string& err) {

@@ -147,7 +147,11 @@ int eqf_upload(eqf_scene *s, int field, const float *host);
 int eqf_download(eqf_scene *s, int field, float *host);
 
 /* Fluid::step (fluid.rs:437-524), `nframes` times, each preceded by the
- * frame sources.  Asynchronous on the scene's stream. */
+ * frame sources.  Asynchronous on the scene's stream, also after a change of
+ * delta_t, diffusion, viscosity or of a source's amounts.  The first step, and the
+ * next one after a change of the iteration counts, the tiling, the mask or whether
+ * there are sources, sets up launch tables: it may allocate (EQF_ENOMEM) and waits
+ * for the frames queued before. */
 int eqf_step(eqf_scene *s, int64_t nframes);
 /* Waits for the scene's queued work. */
 int eqf_sync(eqf_scene *s);

@@ -1380,10 +1380,16 @@ void* frame_create(eqf_scene* s, std::string& err) {
   const size_t n = (size_t)s->S * s->S;
   hipError_t e = hipSuccess;
   if (s->p.gs_mode == EQF_GS_REDBLACK) {
-    const int k = s->slots;
     const size_t fs = (size_t)rm_field_floats(s->S);
-    e = eqf_scene_malloc(s, (void**)&w->tmp[0], sizeof(float) * (k > 1 ? k * fs : n));
-    for (int i = 1; i < k && e == hipSuccess; ++i) w->tmp[i] = w->tmp[0] + i * fs;
+    auto alloc = [&] { return eqf_scene_malloc(s, (void**)&w->tmp[0], sizeof(float) * (s->slots > 1 ? s->slots * fs : n)); };
+    e = alloc();
+    if (e == hipErrorOutOfMemory && s->slots > 1) {  // the diffusions one after the other then
+      (void)hipGetLastError();
+      w->tmp[0] = nullptr;
+      s->slots = 1;
+      e = alloc();
+    }
+    for (int i = 1; i < s->slots && e == hipSuccess; ++i) w->tmp[i] = w->tmp[0] + i * fs;
   }
   if (e != hipSuccess) {
     err = std::string("frame workspace: ") + hipGetErrorString(e);

@@ -66,7 +66,7 @@ struct Req {
 namespace {
 // Lanes of resident scenes (see the file comment).  With the admission stream
 // that is four streams, the number of hardware queues HIP gives a process by
-// default: streams sharing a queue would run their ticks one after the other.
+// default: streams sharing a queue run one after the other (own_queue_stream).
 enum { LANE_SMALL = 0, LANE_LARGE = 1, LANE_RB = 2, NLANES = 3 };
 constexpr int kSmallMaxSize = 258;
 
@@ -78,6 +78,50 @@ struct Lane {
   bool busy = false;
   double t_launch = 0;
 };
+
+// Holds a stream for `ticks` of the 100 MHz clock (bounded in rounds of about a
+// quarter of a microsecond too).
+__global__ void k_hold(uint64_t ticks) {
+  const uint64_t t0 = wall_clock64();
+  for (int i = 0; i < (1 << 14) && wall_clock64() - t0 < ticks; ++i) __builtin_amdgcn_s_sleep(8);
+}
+__global__ void k_pass() {}
+
+// Whether work on b runs while a is held.
+bool side_by_side(hipStream_t a, hipStream_t b, hipEvent_t ev) {
+  for (int k = 0; k < 3; ++k) {  // (a host that is late to look sees a free again)
+    hipLaunchKernelGGL(k_hold, dim3(1), dim3(64), 0, a, (uint64_t)10000);  // 100 us
+    hipLaunchKernelGGL(k_pass, dim3(1), dim3(64), 0, b);
+    bool beside = hipEventRecord(ev, a) == hipSuccess && hipStreamSynchronize(b) == hipSuccess;
+    beside = beside && hipEventQuery(ev) == hipErrorNotReady;
+    (void)hipStreamSynchronize(a);
+    (void)hipGetLastError();
+    if (beside) return true;
+  }
+  return false;
+}
+
+// A stream that runs beside those of `taken`.  The runtime gives a new stream one of
+// its hardware queues by what exists already (other streams, graphs), and an
+// admission that shares a busy lane's queue waits for its tick at each of its waits:
+// 16 ms instead of 0.2 beside ticks of 8 to 15 ms.  So candidates are tried; the
+// last is taken where none runs beside all.
+hipError_t own_queue_stream(const std::vector<hipStream_t>& taken, hipEvent_t ev, hipStream_t* out) {
+  constexpr int TRIES = 12;
+  std::vector<hipStream_t> others;
+  hipError_t e = hipSuccess;
+  for (int k = 0; k < TRIES; ++k) {
+    e = hipStreamCreate(out);
+    if (e != hipSuccess || k == TRIES - 1) break;
+    hipLaunchKernelGGL(k_hold, dim3(1), dim3(64), 0, *out, (uint64_t)0);  // the first launch takes longer
+    hipLaunchKernelGGL(k_pass, dim3(1), dim3(64), 0, *out);
+    (void)hipStreamSynchronize(*out);
+    if (std::all_of(taken.begin(), taken.end(), [&](hipStream_t t) { return side_by_side(t, *out, ev); })) break;
+    others.push_back(*out);  // kept while the next is made: it gets another queue
+  }
+  for (hipStream_t s : others) (void)hipStreamDestroy(s);
+  return e;
+}
 
 int lane_of(const eqf_scene* s) {
   if (s->p.gs_mode == EQF_GS_REDBLACK) return LANE_RB;
@@ -426,7 +470,14 @@ extern "C" int eqf_server_create(eqf_ctx* ctx, const eqf_server_config* cfg, eqf
   sv->ctx = ctx;
   sv->cfg = *cfg;
   sv->t0 = Clock::now();
-  bool ok = hipStreamCreate(&sv->astream) == hipSuccess;
+  bool ok = true;
+  std::vector<hipStream_t> taken;
+  for (Lane& L : sv->lanes) {
+    ok = ok && hipEventCreateWithFlags(&L.ev, hipEventDisableTiming) == hipSuccess;
+    ok = ok && own_queue_stream(taken, L.ev, &L.st) == hipSuccess;
+    taken.push_back(L.st);
+  }
+  ok = ok && own_queue_stream(taken, sv->lanes[0].ev, &sv->astream) == hipSuccess;
   if (ok) {
     hipMemPoolProps props;
     std::memset(&props, 0, sizeof(props));
@@ -438,10 +489,6 @@ extern "C" int eqf_server_create(eqf_ctx* ctx, const eqf_server_config* cfg, eqf
     // keep freed memory in the pool for the next admissions (the budget bounds it)
     uint64_t keep = UINT64_MAX;
     ok = ok && hipMemPoolSetAttribute(sv->pool, hipMemPoolAttrReleaseThreshold, &keep) == hipSuccess;
-  }
-  for (Lane& L : sv->lanes) {
-    ok = ok && hipStreamCreate(&L.st) == hipSuccess;
-    ok = ok && hipEventCreateWithFlags(&L.ev, hipEventDisableTiming) == hipSuccess;
   }
   if (!ok) {
     if (sv->pool) (void)hipMemPoolDestroy(sv->pool);

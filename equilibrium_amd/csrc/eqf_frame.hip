@@ -908,6 +908,11 @@ struct RbGroup {
   bool exact = false;
   LexTask *d_ldiff = nullptr, *d_lpress = nullptr;
   int n_ldiff = 0, n_lpress = 0, n_lflags = 0;
+  // ... and by class the solves of small scenes where there are many (eqf_lex_small.hip)
+  struct {
+    int2 *diff, *press;
+    int ndiff, npress;
+  } small[LEX_SMALL_CLASSES] = {};
   uint32_t* d_ctl = nullptr;
   uint32_t* h_err = nullptr;
   uint32_t polls = 0;              // eqf_ctx::wait_polls that the graph holds
@@ -990,6 +995,23 @@ static void lex_tasks(int i, int S, int iters, int nslots, std::vector<LexTask>&
     for (int strip = 0; strip < n; ++strip)
       v.push_back(LexTask{i, slot, strip, n, nflags++, 0, slot * lex_solve_floats(S) + strip * lex_handoff_floats(S)});
 }
+// Solves of small scenes: by class, kinds apart, whole waves.
+static void small_tasks(const std::vector<int>& scenes, int cls, int nslots, std::vector<int2>& v) {
+  const size_t w = (size_t)lex_small_group(cls);
+  for (int slot = 0; slot < nslots; ++slot) {
+    for (int i : scenes) v.push_back(make_int2(i, slot));
+    while (v.size() % w) v.push_back(make_int2(-1, slot));
+  }
+}
+// From how many small scenes on they are solved by waves of their own: a lone solve
+// takes a wave longer than a strip's eight (N=62 266 us per frame of 20 sweeps instead
+// of 180, N=8 97 instead of 105), the strips fill the CUs much sooner.  us by strips and
+// by waves, 20 sweeps (4 sweeps): 128 scenes of N=30 175 and 157 (101 and 93), N=48 256
+// and 280 (123 and 148), N=64 344 and 411 (231 and 205); 192 scenes 212 and 162, 356 and
+// 293 (155 and 162), 413 and 433; 256 scenes 224 and 169 (137 and 105), 412 and 305
+// (175 and 173), 483 and 445 (322 and 239); 512 scenes 370 and 195, 643 and 363, 751
+// and 539.
+static constexpr int SMALL_MIN = 256;
 static size_t lex_ctl_bytes(int nflags) { return (sizeof(uint32_t) * (size_t)(nflags + 2) + 255) & ~(size_t)255; }
 int64_t frame_table_bytes(int S, bool exact) {
   const int64_t N = S - 2, nseg = (N + rb::SEG - 1) / rb::SEG;
@@ -1026,16 +1048,27 @@ static int group_tables(RbGroup& g, hipStream_t st, std::string& err) {
     g.maxN = std::max(g.maxN, s->N);
     if (s->slots < 3) g.slots = 1;
   }
+  std::vector<int2> sdiff[LEX_SMALL_CLASSES], spress[LEX_SMALL_CLASSES];
+  std::vector<int> sd[LEX_SMALL_CLASSES], spr[LEX_SMALL_CLASSES];
+  int nsmall = 0;
+  for (const eqf_scene* s : g.scenes) nsmall += lex_small_class(s->S) >= 0;
+  const bool small = g.exact && nsmall >= SMALL_MIN;
   g.diff_rounds = g.press_rounds = 0;
   for (int i = 0; i < n; ++i) {
     eqf_scene* s = g.scenes[i];
     scs[i] = scene_entry(s);
-    g.diff_rounds = std::max(g.diff_rounds, lex_rounds(s->desc.diff_iters));
-    g.press_rounds = std::max(g.press_rounds, lex_rounds(s->desc.press_iters));
-    if (g.exact) {
+    const int cls = small ? lex_small_class(s->S) : -1;
+    if (cls >= 0) {
+      if (s->desc.diff_iters > 0) sd[cls].push_back(i);
+      if (s->desc.press_iters > 0) spr[cls].push_back(i);
+    } else {
+      g.diff_rounds = std::max(g.diff_rounds, lex_rounds(s->desc.diff_iters));
+      g.press_rounds = std::max(g.press_rounds, lex_rounds(s->desc.press_iters));
+    }
+    if (g.exact && cls < 0) {
       lex_tasks(i, s->S, s->desc.diff_iters, g.slots, ldiff, fd);
       lex_tasks(i, s->S, s->desc.press_iters, 1, lpress, fp);
-    } else {
+    } else if (!g.exact) {
       for (int mode = 0; mode < 3; ++mode) {
         const int nt = band_tiles(s->S, g.tile, g.tsweeps, mode);
         for (int t = 0; t < nt; ++t) tmap[mode].push_back(make_int2(i, t));
@@ -1067,9 +1100,15 @@ static int group_tables(RbGroup& g, hipStream_t st, std::string& err) {
   lex_order(ldiff, g.scenes);
   lex_order(lpress, g.scenes);
   const size_t b_ld = up(sizeof(LexTask) * ldiff.size()), b_lp = up(sizeof(LexTask) * lpress.size());
+  size_t b_small = 0;
+  for (int c = 0; c < LEX_SMALL_CLASSES; ++c) {
+    small_tasks(sd[c], c, g.slots, sdiff[c]);
+    small_tasks(spr[c], c, 1, spress[c]);
+    b_small += up(sizeof(int2) * sdiff[c].size()) + up(sizeof(int2) * spress[c].size());
+  }
   g.n_lflags = std::max(fd, fp);
   const size_t b_ctl = lex_ctl_bytes(g.n_lflags);  // zero at first; every launch leaves it so
-  const size_t bytes = b_ctl + b_scs + b_t[0] + b_t[1] + b_t[2] + b_m + b_c + b_a + b_ld + b_lp;
+  const size_t bytes = b_ctl + b_scs + b_t[0] + b_t[1] + b_t[2] + b_m + b_c + b_a + b_ld + b_lp + b_small;
   if (bytes > g.tab_bytes) {  // with headroom: a server's group changes size often
     (void)hipFree(g.d_tab);
     g.d_tab = nullptr;
@@ -1108,6 +1147,13 @@ static int group_tables(RbGroup& g, hipStream_t st, std::string& err) {
   g.d_amap = (int4*)(d + o_a);
   g.d_ldiff = (LexTask*)(d + o_ld);
   g.d_lpress = (LexTask*)(d + o_lp);
+  for (int c = 0; c < LEX_SMALL_CLASSES; ++c) {
+    auto& sm = g.small[c];
+    sm.diff = (int2*)(d + put(sdiff[c].data(), sizeof(int2) * sdiff[c].size(), up(sizeof(int2) * sdiff[c].size())));
+    sm.press = (int2*)(d + put(spress[c].data(), sizeof(int2) * spress[c].size(), up(sizeof(int2) * spress[c].size())));
+    sm.ndiff = (int)sdiff[c].size();
+    sm.npress = (int)spress[c].size();
+  }
   g.n_ldiff = (int)ldiff.size();
   g.n_lpress = (int)lpress.size();
   if (g.exact && !g.h_err) {
@@ -1198,6 +1244,9 @@ static void g_lex(hipStream_t st, const RbGroup& g, bool press, const LexSpec& s
     lex_launch(st, g.d_scs, press ? g.d_lpress : g.d_ldiff, press ? g.n_lpress : g.n_ldiff, a, g.d_ctl, g.n_lflags,
                g.h_err, g.maxN);
   }
+  const LexArgs a{{s0, s1, s2}, 0, press ? 1 : 0, 0};
+  for (int c = 0; c < LEX_SMALL_CLASSES; ++c)
+    lex_small_launch(st, g.d_scs, press ? g.small[c].press : g.small[c].diff, c, press ? g.small[c].npress : g.small[c].ndiff, a);
 }
 static void g_pressure(hipStream_t st, const RbGroup& g, int p, int div) {
   if (g.exact) g_lex(st, g, true, LexSpec{M_PASSIVE, p, div, 2}, LexSpec{}, LexSpec{});

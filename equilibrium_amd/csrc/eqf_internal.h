@@ -163,6 +163,14 @@ struct LexArgs {
 void lex_launch(hipStream_t st, const RbScene* scs, const LexTask* tasks, int ntasks, const LexArgs& args,
                 uint32_t* ctl, int nflags, uint32_t* err, int maxN);
 
+// ... of many small scenes, whole solves (eqf_lex_small.hip).  Class of a size (-1:
+// none), solves of one kind that a wave takes (ntasks is a multiple of them;
+// tasks: {scene, slot}, scene -1: none, not the first of a wave).
+int lex_small_class(int S);
+int lex_small_group(int cls);
+constexpr int LEX_SMALL_CLASSES = 5;
+void lex_small_launch(hipStream_t st, const RbScene* scs, const int2* tasks, int cls, int ntasks, const LexArgs& args);
+
 // Frames (eqf_frame.hip).  A launch group's scenes share one mode.
 void* frame_create(eqf_scene* s, std::string& err);
 void frame_destroy(eqf_scene* s);

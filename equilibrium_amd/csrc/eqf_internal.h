@@ -138,7 +138,6 @@ namespace eqf {
 struct RbScene {
   SceneDesc d;  // the scene's descriptor (a copy): fields, sizes, coefficients, rule bytes
   float* tmp[3];  // its ping-pong fields (red-black mode)
-  float* hand;    // its hand-off values (exact mode)
 };
 
 // Lexicographic lin_solve (eqf_lex.hip).  A launch covers up to three
@@ -148,7 +147,7 @@ struct LexTask {
   int strip, nstrips;
   int flag;      // its progress count; the strip above has the one before
   int pad;
-  int64_t hoff;  // its hand-off values in the scene's (the strip above: lex_handoff_floats before)
+  float* hand;  // its hand-off values (of the strip above: lex_handoff_floats before)
 };
 struct LexSpec {
   int mode, x_role, x0_role, coef;

@@ -634,7 +634,7 @@ static __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, cons
   }
 
   if (w == W + 2) {  // lane 63's values for the strip below (and the final values)
-    float* hout = sc.hand + tk.hoff;
+    float* hout = tk.hand;
     uint32_t* fown = flags + tk.flag;
     for (int b = -1; b < NI; ++b) {
       if (has_next && b > 0) {
@@ -740,7 +740,7 @@ static __device__ __forceinline__ void strip_task(lf* L, const RbScene& sc, cons
   // x before the round, and lane 0's values from the strip above: these only in
   // the block before they are needed, since every block that they come earlier
   // puts every strip that much further behind the one above.
-  const float* hin = sc.hand + (has_prev ? tk.hoff - (int64_t)KMAX * T : 0);
+  const float* hin = tk.hand - (has_prev ? KMAX * T : 0);
   const uint32_t* fprev = flags + (has_prev ? tk.flag - 1 : tk.flag);
   u4 gin[ZI];
   float gu[3];

@@ -983,17 +983,18 @@ static uint64_t desc_key(const RbGroup& g) {
 }
 static RbScene scene_entry(const eqf_scene* s) {
   const auto* w = static_cast<const FrameWork*>(s->work);
-  return RbScene{s->desc, {w->tmp[0], w->tmp[1], w->tmp[2]}, s->d_hand};
+  return RbScene{s->desc, {w->tmp[0], w->tmp[1], w->tmp[2]}};
 }
 
 // The strips of `nslots` lin_solves of scene i, `iters` sweeps each.
-static void lex_tasks(int i, int S, int iters, int nslots, std::vector<LexTask>& v, int& nflags) {
+static void lex_tasks(int i, const eqf_scene* s, int iters, int nslots, std::vector<LexTask>& v, int& nflags) {
+  const int S = s->S;
   const int K = lex_round_sweeps(iters, 0);  // the longest round
   if (K == 0) return;
   const int n = lex_strips(S, K);
   for (int slot = 0; slot < nslots; ++slot)
     for (int strip = 0; strip < n; ++strip)
-      v.push_back(LexTask{i, slot, strip, n, nflags++, 0, slot * lex_solve_floats(S) + strip * lex_handoff_floats(S)});
+      v.push_back(LexTask{i, slot, strip, n, nflags++, 0, s->d_hand + slot * lex_solve_floats(S) + strip * lex_handoff_floats(S)});
 }
 // Solves of small scenes: by class, kinds apart, whole waves.
 static void small_tasks(const std::vector<int>& scenes, int cls, int nslots, std::vector<int2>& v) {
@@ -1066,8 +1067,8 @@ static int group_tables(RbGroup& g, hipStream_t st, std::string& err) {
       g.press_rounds = std::max(g.press_rounds, lex_rounds(s->desc.press_iters));
     }
     if (g.exact && cls < 0) {
-      lex_tasks(i, s->S, s->desc.diff_iters, g.slots, ldiff, fd);
-      lex_tasks(i, s->S, s->desc.press_iters, 1, lpress, fp);
+      lex_tasks(i, s, s->desc.diff_iters, g.slots, ldiff, fd);
+      lex_tasks(i, s, s->desc.press_iters, 1, lpress, fp);
     } else if (!g.exact) {
       for (int mode = 0; mode < 3; ++mode) {
         const int nt = band_tiles(s->S, g.tile, g.tsweeps, mode);
@@ -1265,8 +1266,9 @@ static void g_adv(hipStream_t st, const RbGroup& g, int o0, int i0, int o1, int 
   else hipLaunchKernelGGL((rb::k_adv<DENSITY, 16>), rows, dim3(1024), 0, st, g.d_scs, g.d_amap, o0, i0, o1, i1, u, v);
 }
 
-// One frame (fluid.rs:437-524) of every scene of the group.  All scenes share
-// the iteration counts, so the sequence of launches is the same for all.
+// One frame (fluid.rs:437-524) of every scene of the group.  Red-black scenes share
+// the iteration counts; exact ones need not: the launches are those of the scene
+// with the most rounds of sweeps, the others have no work in the last of them.
 //
 // Corners (fluid.rs:265-271) are read only by advect's bilinear gathers and
 // are part of the frame's final state; no sweep, divergence or gradient reads

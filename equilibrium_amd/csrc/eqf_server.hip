@@ -51,7 +51,6 @@ struct Req {
   bool failed = false;
   bool forget = false;  // released while queued or resident: dropped from the ticket map once retired
   int64_t frames_done = 0;
-  int tick_frames = 1;  // frames of the tick in flight
   double t_submit = 0, t_admit = 0, t_done = 0;
   eqf_scene* scene = nullptr;
   int lane = 0;
@@ -112,6 +111,7 @@ hipError_t own_queue_stream(const std::vector<hipStream_t>& taken, hipEvent_t ev
   hipError_t e = hipSuccess;
   for (int k = 0; k < TRIES; ++k) {
     e = hipStreamCreate(out);
+    if (e != hipSuccess) *out = nullptr;  // (it still named the last of the others)
     if (e != hipSuccess || k == TRIES - 1) break;
     hipLaunchKernelGGL(k_hold, dim3(1), dim3(64), 0, *out, (uint64_t)0);  // the first launch takes longer
     hipLaunchKernelGGL(k_pass, dim3(1), dim3(64), 0, *out);
@@ -251,11 +251,10 @@ static void lane_tick_done(eqf_server* sv, Lane& L, double now, hipError_t statu
       sv->thread_error = status != hipSuccess ? hipGetErrorString(status) : "a lin_solve strip gave up waiting";
       continue;
     }
-    const int f = r->tick_frames;
-    r->frames_done += f;
-    sv->scene_frames += f;
-    sv->cell_updates += (double)r->cells * f;
-    for (int k = 0; k < f; ++k) sv->frame_lat.emplace_back(r->p.size, ms / f);
+    r->frames_done++;
+    sv->scene_frames++;
+    sv->cell_updates += (double)r->cells;
+    sv->frame_lat.emplace_back(r->p.size, ms);
   }
   L.ticking.clear();
   L.busy = false;
@@ -273,7 +272,6 @@ static std::string lane_launch(eqf_server* sv, int li) {
   std::stable_sort(L.ticking.begin(), L.ticking.end(),
                    [](const Req* a, const Req* b) { return a->cells > b->cells; });
   for (Req* r : L.ticking) {
-    r->tick_frames = 1;
     const SceneDesc& d = r->scene->desc;
     by_iters[li == LANE_RB ? std::make_pair(d.diff_iters, d.press_iters) : std::make_pair(0, 0)].push_back(r->scene);
   }

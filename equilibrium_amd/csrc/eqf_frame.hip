@@ -1243,7 +1243,7 @@ static void g_lex(hipStream_t st, const RbGroup& g, bool press, const LexSpec& s
   for (int r = 0; r < (press ? g.press_rounds : g.diff_rounds); ++r) {
     const LexArgs a{{s0, s1, s2}, r, press ? 1 : 0, g.polls};
     lex_launch(st, g.d_scs, press ? g.d_lpress : g.d_ldiff, press ? g.n_lpress : g.n_ldiff, a, g.d_ctl, g.n_lflags,
-               g.h_err, g.maxN);
+               g.h_err, g.maxN, g.scenes[0]->ctx->cus);
   }
   const LexArgs a{{s0, s1, s2}, 0, press ? 1 : 0, 0};
   for (int c = 0; c < LEX_SMALL_CLASSES; ++c)
@@ -1521,12 +1521,15 @@ void group_set_scenes(void* p, const std::vector<eqf_scene*>& scenes) {
 }
 bool group_collect(void* p) {
   auto* g = static_cast<RbGroup*>(p);
-  if (!g || !g->h_err || __atomic_exchange_n(g->h_err, 0u, __ATOMIC_ACQ_REL) == 0) return false;
+  if (!g || !g->h_err || __atomic_load_n(g->h_err, __ATOMIC_ACQUIRE) == 0) return false;
+  // cleared last: a thread that has another of the scenes and finds the status clear
+  // finds its scene marked (two threads that see it set both mark, which does no harm)
   for (eqf_scene* s : g->scenes) {
     s->invalid.store(kAllFields);
     s->failures.fetch_add(1);
   }
   g->stale.store(true);
+  __atomic_store_n(g->h_err, 0u, __ATOMIC_RELEASE);
   return true;
 }
 

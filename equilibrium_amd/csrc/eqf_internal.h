@@ -45,6 +45,7 @@ constexpr uint32_t LEX_POLLS = 1u << 22;
 
 struct eqf_ctx {
   int device;
+  int cus = 256;  // its compute units
   std::shared_ptr<HostStaging> staging;
   std::atomic<uint32_t> wait_polls{LEX_POLLS};
 };
@@ -158,9 +159,10 @@ struct LexArgs {
   uint32_t polls;    // how often a strip looks for the one above before it gives up (and reports)
 };
 // ctl: ticket, ended workgroups, then nflags progress counts, all zero before
-// the first launch; a launch leaves them zero.  maxN: the largest scene's.
+// the first launch; a launch leaves them zero.  maxN: the largest scene's; cus: the
+// device's compute units.
 void lex_launch(hipStream_t st, const RbScene* scs, const LexTask* tasks, int ntasks, const LexArgs& args,
-                uint32_t* ctl, int nflags, uint32_t* err, int maxN);
+                uint32_t* ctl, int nflags, uint32_t* err, int maxN, int cus);
 
 // ... of many small scenes, whole solves (eqf_lex_small.hip).  Class of a size (-1:
 // none), solves of one kind that a wave takes (ntasks is a multiple of them;

@@ -54,12 +54,25 @@
 // always waits for one that already runs: the launch ends whatever share of
 // it is resident.
 //
-// Bound: instruction issue of the sweeps.  An update of a plain cell takes 8
-// VALU instructions (6 of arithmetic, of which two shift a lane, one for lane
-// 0, one that gathers lane 63's value); a plain block of 5 sweeps x 8 steps
-// 2800 cycles with a wave alone on its SIMD, of which 500 are LDS reads of x0.
-// A lone scene is bound by its chain of S + 63 + 2K steps plus about 90 per
-// strip.
+// Bound: a launch that fills the device by instruction issue.  For 512 scenes of N
+// 64..512 and 20 sweeps the SIMDs issue a VALU instruction in 73% of their cycles
+// (LDS is accessed in 25%, 7% are bank conflicts).  An update of a plain cell takes 8
+// of them (6 of arithmetic, of which two shift a lane, one for lane 0, one that
+// gathers lane 63's value), 186 M of a launch's 520 M; the others are steps of
+// the skew and of rows beyond the grid, cells beside walls and the ring, and the waves
+// that move data.  A plain block of 5 sweeps x 8 steps takes 2800 cycles with a wave
+// alone on its SIMD, of which 500 are LDS reads of x0.  A lone scene is bound by its
+// chain of S + 63 + 2K steps plus about 90 per strip.
+//
+// With few sweeps a launch that fills the device is bound by its loads and stores, 32
+// bytes of a row per block (512 scenes of N=128: VALU 77% of the cycles with 20
+// sweeps, 49 with 4, 26 with one; 33 bytes per cell and solve at 2.2 TB/s where 13
+// would do).  There walking the grid once per sweep, a workgroup per scene, was faster;
+// us per frame then and now: 512 scenes of N=128 564 and 875 (one sweep), 763 and 961
+// (4), 960 and 1060 (8), 1528 and 1556 (20); of N=256 2203 and 2997, 3115 and 3115,
+// 4115 and 3229, 6886 and 3986; of N=512 7.2 and 11.3 ms, 9.6 and 11.5, 13.2 and 11.8.
+// More workgroups do not help: four of two waves of sweeps per CU, for up to 8 sweeps,
+// took 0.92 to 1.32 of the time of these.
 //
 // Compiled with -ffp-contract=off: rustc does not contract a*b+c.
 #include <hip/hip_runtime.h>
@@ -858,25 +871,27 @@ __global__ void __launch_bounds__(Lex<W>::NT, W == 4 ? 4 : 3)
 }  // namespace lex
 
 void lex_launch(hipStream_t st, const RbScene* scs, const LexTask* tasks, int ntasks, const LexArgs& args,
-                uint32_t* ctl, int nflags, uint32_t* err, int maxN) {
+                uint32_t* ctl, int nflags, uint32_t* err, int maxN, int cus) {
   if (ntasks <= 0) return;
   auto launch = [&](auto w) {
     typedef lex::Lex<decltype(w)::value> X;
     hipLaunchKernelGGL(lex::k_lex<decltype(w)::value>, dim3((unsigned)ntasks), dim3(X::NT), X::L_WORDS * 4, st, scs, tasks,
                        ntasks, args, ctl, ctl + 2, nflags, err);
   };
-  // Up to one workgroup per CU (256 of them) the chain of blocks bounds the
+  // Up to one workgroup per CU the chain of blocks bounds the
   // launch: eight waves of up to three sweeps take a block faster than four of up
   // to five (a frame of N=1024 1.48 ms instead of 1.76, N=128 0.265 instead of
   // 0.318, N=30 0.120 instead of 0.131; seven 1.58 at N=1024, ten as eight).
   // Two workgroups of four fit a CU, one of eight does not leave room for
   // another, but up to three per CU the faster blocks still win (64 scenes of
   // N=256 0.93 ms instead of 1.02, 24 of N=1024 3.42 instead of 3.81, a mix of 130
-  // 1.79 instead of 1.95) unless the strips are so short that filling eight
+  // 1.79 instead of 1.95; also where the large ones are few: one of N=200 beside 200 of
+  // N=30 0.387 instead of 0.456, of N=62 0.530 instead of 0.542, four of N=400 beside
+  // 200 of N=128 1.14 instead of 1.18) unless the strips are so short that filling eight
   // waves weighs (100 scenes of N=128 0.595 instead of 0.565, 300 of N=64 0.574
   // instead of 0.552).  Beyond that four waves win (the mix of 512 5.38 ms, 6.04
   // with eight).
-  if (ntasks <= 256 || (ntasks <= 768 && maxN >= 192)) launch(std::integral_constant<int, 8>());
+  if (ntasks <= cus || (ntasks <= 3 * cus && maxN >= 192)) launch(std::integral_constant<int, 8>());
   else launch(std::integral_constant<int, 4>());
 }
 

@@ -138,8 +138,10 @@ static int sync_desc(eqf_scene* s) {
   return EQF_OK;
 }
 
-// The exact mode takes grids of up to 16 strips of 64 rows; a batch's
-// max_waves is at least the strips of its largest scene.
+// What the exact mode takes and refuses is older than its present kernels, which
+// have no such limits: grids of up to 16 strips of 64 rows, sweep counts by the
+// steps that one workgroup took for a whole scene, and a batch's max_waves from
+// the strips of its largest scene.  Callers rely on both, so the rules stay.
 static int exact_strips(int N) { return (N + 63) / 64; }
 
 static int check_params(const eqf_params* p) {
@@ -172,6 +174,10 @@ extern "C" int eqf_ctx_create(int device, eqf_ctx** out) {
   auto* c = new (std::nothrow) eqf_ctx;
   if (!c) return fail(EQF_ENOMEM, "host allocation failed");
   c->device = device;
+  if (hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) {
+    (void)hipGetLastError();
+    c->cus = 256;
+  }
   try {
     c->staging = std::make_shared<HostStaging>(device);
   } catch (...) {

@@ -10,7 +10,7 @@ counted).
 
 Also reported beside it: the single-grid drop-in on the same mix (one scene
 at a time), the N=1024 single grid, the red-black legs, snapshots, serving,
-the HBM roofline of the frame kernel and the CPU leg.  The CPU leg ("cpu") is
+the HBM traffic of the frame's kernels and the CPU leg.  The CPU leg ("cpu") is
 the only part of this script that runs the oracle: it checks the red-black
 legs' GPU outputs against the f64 oracle (their vs_fp64 and Poisson residual
 fields) and times the oracle on this host as cpu_baseline.
@@ -48,9 +48,8 @@ def b_alg(iters):
 
 def profiled_traffic(kernel, shape=None):
     """HBM bytes per launch measured by the committed rocprofv3 PMC runs, for
-    the launch shape (batch: "max_waves:order:schedule", red-black:
-    "band:sweeps") the run used; None when no profile
-    was taken at that shape.  Returns (bytes, profile entry)."""
+    the launch shape (red-black: "band:sweeps") the run used; None when no
+    profile was taken at that shape.  Returns (bytes, profile entry)."""
     try:
         with open(os.path.join(REPO, "profiles", "traffic.json")) as f:
             ent = json.load(f)[kernel]
@@ -58,8 +57,6 @@ def profiled_traffic(kernel, shape=None):
         return None, None
     if "by_shape" in ent:
         ent = ent["by_shape"].get(shape)
-    elif ent.get("shape") != shape:
-        ent = None
     if ent is None:
         return None, None
     return ent.get("traffic_bytes_per_launch", ent.get("traffic_bytes_per_frame")), ent
@@ -99,9 +96,6 @@ def device_sync():
         pass
 
 
-SCHED_NAMES = {0: "auto", 1: "wide", 2: "ring", 3: "fine"}  # eqf_batch_set_schedule
-
-
 def make_scenes(scs):
     hs = []
     for sc in scs:
@@ -113,19 +107,9 @@ def make_scenes(scs):
     return hs
 
 
-def bench_batch(scs, steps, warmup, tuning=None):
-    from equilibrium_amd import tune
-
+def bench_batch(scs, steps, warmup):
     hs = make_scenes(scs)
-    if tuning:
-        (w, o, sch), timings = (tuning + (_abi.SCHED_AUTO,))[:3], {}
-        log(f"batch: max waves {w}, order {o}, schedule {SCHED_NAMES[sch]} (given)")
-    else:
-        w, o, sch, timings = tune.tune_batch(hs)
-        log(f"batch: autotuned max waves {w}, order {o}, schedule {SCHED_NAMES[sch]}: {timings}")
     b = _abi.Batch(hs)
-    b.set_tuning(w, o)
-    b.set_schedule(sch)
     if warmup:
         b.step(warmup)
         b.sync()
@@ -145,8 +129,7 @@ def bench_batch(scs, steps, warmup, tuning=None):
         ("density", "scratch", "vx", "vy", "vx0", "vy0"))}) for i in sorted(picks.values())], warmup + steps)
     for h in hs:
         h.close()
-    return wall, ev_ms, {"max_waves": w, "order": "largest first" if o == 0 else "given",
-                         "schedule": SCHED_NAMES[sch], "shape": f"{w}:{o}:{sch}", "trial_ms": timings}
+    return wall, ev_ms
 
 
 def check_batch_exact(samples, frames, threads):
@@ -607,8 +590,7 @@ def main():
     ap.add_argument("--rb-frames", type=int, default=10)
     ap.add_argument("--rb-check-frames", type=int, default=20)
     ap.add_argument("--batch-tuning", type=str, default="",
-                    help="max_waves:order[:schedule] for the batch instead of autotuning (e.g. 16:0:2; "
-                         "schedule 0 auto, 1 wide, 2 ring, 3 fine)")
+                    help="accepted and not used: the exact batch has nothing to choose")
     ap.add_argument("--rb-tiling", type=str, default="",
                     help="band:sweeps for the N=4096 red-black grid instead of autotuning (e.g. 0:5)")
     ap.add_argument("--rb-batch-band", type=str, default="",
@@ -647,13 +629,13 @@ def main():
         iters = mix[0]["iters"]
         cells = sum((sc["size"] - 2) ** 2 for sc in mix)
         log(f"batched mix: {len(mix)} scenes, {cells} interior cells, {iters} sweeps")
-        given = tuple(int(x) for x in args.batch_tuning.split(":")) if args.batch_tuning else None
-        wall, ev_ms, tuning = bench_batch(mix, args.steps, args.warmup, given)
+        wall, ev_ms = bench_batch(mix, args.steps, args.warmup)
         value = cells * args.steps / wall
         ms_per_step = wall * 1e3 / args.steps
         launch_ms = ev_ms / args.steps  # HIP events on the batch stream around the K launches
         alg_bytes = cells * b_alg(iters)
-        achieved = alg_bytes / (launch_ms * 1e-3) / 1e9
+        traffic, ent = profiled_traffic("exact_frame_mix") if args.scenes == 512 else (None, None)
+        achieved = traffic / (launch_ms * 1e-3) / 1e9 if traffic else None
         log(f"batch: {value:.4g} cell-updates/s, {ms_per_step:.3f} ms/frame, kernel {launch_ms:.3f} ms")
 
         out.update({
@@ -678,32 +660,30 @@ def main():
                 "gs_sweeps": iters,
                 "mode": "wavefront, bit-exact: the CPU leg checks one timed scene per size against the "
                         "oracle after all frames (config.bit_exact_check)",
-                "batch_tuning": tuning,
             },
+            # The lin_solves keep up to 20 sweeps on chip: `frac` is what the frame's
+            # kernels really move, `streaming_model_frac` what they would if every
+            # sweep crossed memory (it can exceed 1 and is no HBM fraction).
             "roofline": {
-                "bound": "hbm",
-                "kernel": "the frame's kernels (k_lex for the lin_solves, one workgroup per strip of 63 rows)",
-                "frac_basis": "algorithmic bytes (B_alg per cell-update) / launch time; traffic_frac: "
-                              "measured HBM bytes (rocprofv3) / launch time.  The strips keep the sweeps on chip, so "
-                              "the algorithmic figure can exceed 1 and is no HBM fraction",
+                "bound": "k_lex (the lin_solves): instruction issue (VALU in 73% of the cycles, profiles/exact_frames.md); "
+                         "the other phases: memory",
+                "kernel": "the frame's kernels (k_lex: one workgroup per strip of 63 rows)",
+                "frac_basis": "measured HBM bytes per frame (rocprofv3) / launch time",
                 "achieved": achieved,
                 "peak": HBM_PEAK_GBS,
                 "unit": "GB/s",
-                "frac": achieved / HBM_PEAK_GBS,
-                "alg_bytes_per_launch": alg_bytes,
+                "frac": achieved / HBM_PEAK_GBS if traffic else None,
+                "traffic": traffic,
+                "traffic_source": (f"{ent['source']} (rocprofv3 --pmc FETCH_SIZE, WRITE_SIZE)" if ent
+                                   else "no rocprofv3 profile of this batch"),
                 "launch_ms": launch_ms,
+                "streaming_model_bytes": alg_bytes,
+                "streaming_model_frac": alg_bytes / (launch_ms * 1e-3) / 1e9 / HBM_PEAK_GBS,
             },
         })
-        shape = tuning["shape"]
-        traffic, ent = profiled_traffic("exact_frame_mix", shape)
-        out["roofline"]["traffic"] = traffic
-        out["roofline"]["traffic_frac"] = (traffic / (launch_ms * 1e-3) / 1e9 / HBM_PEAK_GBS) if traffic else None
-        out["roofline"]["traffic_source"] = (
-            f"{ent['source']} at launch shape {shape} (rocprofv3 --pmc FETCH_SIZE, WRITE_SIZE, scaled by a copy "
-            "of known size)" if ent else f"no rocprofv3 profile at launch shape {shape}")
         if bw:
             out["roofline"]["practical_peak"] = bw["copy"]
-            out["roofline"]["frac_of_practical"] = achieved / bw["copy"]
+            out["roofline"]["frac_of_practical"] = achieved / bw["copy"] if traffic else None
 
     if "rbmix" in legs:
         # the batched mix in red-black mode (<= 1e-5 vs FP64 instead of bit-exact)

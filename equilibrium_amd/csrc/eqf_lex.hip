@@ -58,7 +58,7 @@
 // 64..512 and 20 sweeps the SIMDs issue a VALU instruction in 73% of their cycles
 // (LDS is accessed in 25%, 7% are bank conflicts).  An update of a plain cell takes 8
 // of them (6 of arithmetic, of which two shift a lane, one for lane 0, one that
-// gathers lane 63's value), 186 M of a launch's 520 M; the others are steps of
+// gathers lane 63's value), 180 M of a launch's 520 M; the others are steps of
 // the skew and of rows beyond the grid, cells beside walls and the ring, and the waves
 // that move data.  A plain block of 5 sweeps x 8 steps takes 2800 cycles with a wave
 // alone on its SIMD, of which 500 are LDS reads of x0.  A lone scene is bound by its

@@ -187,9 +187,8 @@ int eqf_batch_last_ms(const eqf_batch *b, double *ms);
 /* Launch shape of a wavefront-mode batch (no counterpart in the reference):
  * waves per workgroup at most (1..16, at least the largest scene's strip count
  * of ceil(N/64)) and the scene-to-workgroup order.  The arguments are checked;
- * neither results nor launches depend on them: a lin_solve always gives a
- * workgroup to each strip of 64 rows, in the order of the scenes' longest
- * remaining chains. */
+ * neither results nor launches depend on them: what a lin_solve's workgroups and
+ * waves take follows from the scenes' sizes and number. */
 enum { EQF_BATCH_LARGEST_FIRST = 0, EQF_BATCH_GIVEN_ORDER = 1 };
 int eqf_batch_set_tuning(eqf_batch *b, int max_waves, int order);
 /* Wavefront schedule of a wavefront-mode batch (no counterpart in the

@@ -915,7 +915,7 @@ struct RbGroup {
   } small[LEX_SMALL_CLASSES] = {};
   uint32_t* d_ctl = nullptr;
   uint32_t* h_err = nullptr;
-  uint32_t polls = 0;              // eqf_ctx::wait_polls that the graph holds
+  uint32_t polls = 0;              // LaunchLimits::wait_polls that the graph holds
   std::atomic<bool> stale{false};  // a wait gave up: the counters have to be set up again
   int n = 0, maxN = 0, tiles[3] = {0, 0, 0}, iblocks = 0, cblocks = 0, ablocks = 0;
   bool any_src = false;
@@ -1243,7 +1243,7 @@ static void g_lex(hipStream_t st, const RbGroup& g, bool press, const LexSpec& s
   for (int r = 0; r < (press ? g.press_rounds : g.diff_rounds); ++r) {
     const LexArgs a{{s0, s1, s2}, r, press ? 1 : 0, g.polls};
     lex_launch(st, g.d_scs, press ? g.d_lpress : g.d_ldiff, press ? g.n_lpress : g.n_ldiff, a, g.d_ctl, g.n_lflags,
-               g.h_err, g.maxN, g.scenes[0]->ctx->cus);
+               g.h_err, g.maxN, g.scenes[0]->limits->cus);
   }
   const LexArgs a{{s0, s1, s2}, 0, press ? 1 : 0, 0};
   for (int c = 0; c < LEX_SMALL_CLASSES; ++c)
@@ -1370,7 +1370,7 @@ static int group_step_all(RbGroup& g, hipStream_t st, int64_t nframes, std::stri
       }
   for (eqf_scene* s : g.scenes)
     if (s->invalid.load()) s->invalid.store(kAllFields);  // a frame mixes the fields
-  g.polls = g.scenes[0]->ctx->wait_polls.load();
+  g.polls = g.scenes[0]->limits->wait_polls.load();
   const uint64_t key = group_key(g), dkey = desc_key(g);
   const bool descs = dkey != g.dkey;
   if (g.stale.exchange(false) || !g.d_tab || key != g.key || g.tab_tile != g.tile || g.tab_T != g.tsweeps ||

@@ -43,16 +43,23 @@ class HostStaging {
 // for the one above before it gives up and reports (eqf_ctx_set_wait_limit).
 constexpr uint32_t LEX_POLLS = 1u << 22;
 
+// What launches read of a context; held by its scenes too, which a batch of another
+// context may step after it is gone.
+struct LaunchLimits {
+  int cus = 256;  // compute units of the device
+  std::atomic<uint32_t> wait_polls{LEX_POLLS};
+};
+
 struct eqf_ctx {
   int device;
-  int cus = 256;  // its compute units
   std::shared_ptr<HostStaging> staging;
-  std::atomic<uint32_t> wait_polls{LEX_POLLS};
+  std::shared_ptr<LaunchLimits> limits;
 };
 
 struct eqf_scene {
   eqf_ctx* ctx = nullptr;
   std::shared_ptr<HostStaging> staging;  // the context's
+  std::shared_ptr<LaunchLimits> limits;  // the context's
   uint64_t uid = 0;  // unique per scene object of the process (never reused)
   eqf_params p{};
   int S = 0, N = 0;

@@ -174,15 +174,16 @@ extern "C" int eqf_ctx_create(int device, eqf_ctx** out) {
   auto* c = new (std::nothrow) eqf_ctx;
   if (!c) return fail(EQF_ENOMEM, "host allocation failed");
   c->device = device;
-  if (hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) {
-    (void)hipGetLastError();
-    c->cus = 256;
-  }
   try {
     c->staging = std::make_shared<HostStaging>(device);
+    c->limits = std::make_shared<LaunchLimits>();
   } catch (...) {
     delete c;
     return fail(EQF_ENOMEM, "host allocation failed");
+  }
+  if (hipDeviceGetAttribute(&c->limits->cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) {
+    (void)hipGetLastError();
+    c->limits->cus = 256;
   }
   c->staging->give(c->staging->take());  // one is there from the start
   *out = c;
@@ -196,7 +197,7 @@ extern "C" int eqf_ctx_destroy(eqf_ctx* ctx) {
 
 extern "C" int eqf_ctx_set_wait_limit(eqf_ctx* ctx, uint32_t polls) {
   if (!ctx) return fail(EQF_EINVAL, "ctx is NULL");
-  ctx->wait_polls.store(polls);
+  ctx->limits->wait_polls.store(polls);
   return EQF_OK;
 }
 
@@ -277,6 +278,7 @@ static int scene_alloc(eqf_ctx* ctx, const eqf_params* p, eqf_scene** out, hipSt
   s->uid = next_uid++;
   s->ctx = ctx;
   s->staging = ctx->staging;
+  s->limits = ctx->limits;
   s->p = *p;
   s->S = (int)p->size;
   s->N = s->S - 2;

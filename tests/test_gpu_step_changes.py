@@ -6,8 +6,8 @@ import numpy as np
 import pytest
 
 import oracle
-from equilibrium_amd import _abi
-from helpers import FIELD_NAMES, assert_state_equal, download_all
+from equilibrium_amd import _abi, scenes
+from helpers import FIELD_NAMES, assert_state_equal, download_all, oracle_state
 
 pytestmark = pytest.mark.gpu
 
@@ -123,3 +123,24 @@ def test_more_launches_than_a_graph_holds_equal_oracle(mode, iters):
            order=oracle.RB if mode == _abi.GS_REDBLACK else oracle.LEX)
     assert_state_equal(download_all(s), st, "long solves")
     s.close()
+
+
+def test_a_batch_steps_scenes_whose_context_is_gone():
+    """A batch belongs to its own context; what its scenes need of theirs they hold."""
+    print("[case] scenes of a context that is destroyed", flush=True)
+    sc = scenes.stam_scene(70, scenes.derive_seed(65), iters=5, frames=2, n_rects=1)
+    a, b = _abi.Context(0), _abi.Context(0)
+    s = _abi.Scene(scenes.scene_params(sc), a)
+    scenes.apply_to_scene(s, sc)
+    batch = _abi.Batch([s], b)
+    a.close()
+    batch.step(1)
+    batch.step(1)
+    batch.sync()
+    st = oracle_state(sc)
+    st.run(sc["dt"], sc["diffusion"], sc["viscosity"], sc["iters"], 2, src_d=sc["src_d"], src_u=sc["src_u"],
+           src_v=sc["src_v"])
+    assert_state_equal(download_all(s), st, "context gone")
+    batch.close()
+    s.close()
+    b.close()

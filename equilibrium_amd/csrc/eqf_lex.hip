@@ -64,10 +64,12 @@
 // alone on its SIMD, of which 500 are LDS reads of x0.  A lone scene is bound by its
 // chain of S + 63 + 2K steps plus about 90 per strip.
 //
-// With few sweeps a launch that fills the device is bound by its loads and stores, 32
-// bytes of a row per block (512 scenes of N=128: VALU 77% of the cycles with 20
-// sweeps, 49 with 4, 26 with one; 33 bytes per cell and solve at 2.2 TB/s where 13
-// would do).  There walking the grid once per sweep, a workgroup per scene, was faster;
+// With few sweeps a launch that fills the device is bound by the length of a block
+// (1.1 us at N=128 with one sweep, 2.0 with 20; 512 scenes: VALU 77% of the cycles with
+// 20 sweeps, 49 with 4, 26 with one): the data waves' chains from barrier to barrier
+// and their loads and stores of 32 bytes of a row (33 bytes per cell and solve at 2.2
+// TB/s where 13 would do; without any of the fields' loads and stores a frame takes 10%
+// less at N=128, 27% at N=256).  There walking the grid once per sweep, a workgroup per scene, was faster;
 // us per frame then and now: 512 scenes of N=128 564 and 875 (one sweep), 763 and 961
 // (4), 960 and 1060 (8), 1528 and 1556 (20); of N=256 2203 and 2997, 3115 and 3115,
 // 4115 and 3229, 6886 and 3986; of N=512 7.2 and 11.3 ms, 9.6 and 11.5, 13.2 and 11.8.
